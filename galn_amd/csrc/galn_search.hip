@@ -45,6 +45,7 @@
 #include <cstring>
 #include <mutex>
 #include <numeric>
+#include <type_traits>
 #include <vector>
 
 #include "galn_hip.h"
@@ -80,20 +81,9 @@ constexpr uint64_t TR_PRIME = 1099511628211ull;
 
 struct DMeta {
     uint64_t primary;
-    uint64_t L2[5];
     uint64_t seq_len;
-};
-
-// The cumulative symbol counts held in registers: a lane's count for its own symbol is picked
-// by selects. Indexing the kernel-argument copy by a per-lane symbol is a vector memory load,
-// whose wait also waits for every store the wave still has in flight.
-struct L2Sel {
-    uint64_t v0, v1, v2, v3, v4;
-    __device__ explicit L2Sel(const DMeta &m) : v0(m.L2[0]), v1(m.L2[1]), v2(m.L2[2]), v3(m.L2[3]), v4(m.L2[4]) {}
-    __device__ __forceinline__ uint64_t operator[](int c) const
-    {
-        return c == 0 ? v0 : c == 1 ? v1 : c == 2 ? v2 : c == 3 ? v3 : v4;
-    }
+    const uint64_t *ext;  // counts at the start of each epoch of blocks, or null (one epoch, 32-bit counts)
+    uint32_t eshift;      // log2 of an epoch's blocks
 };
 
 // packed stack entry (layout below)
@@ -167,56 +157,139 @@ __device__ __forceinline__ T cold_ld(const __attribute__((address_space(4))) T *
 #define CA(f) cold_ld(&A->f)
 
 // ---------------------------------------------------------------------------
-// Occurrence counts. Device index layout: 128-symbol blocks of 16 u32 words, 4 x u64
-// exclusive counts, then the block's symbols as two bit planes: 4 words of high bits, then 4
-// words of low bits, symbol s at bit 31 - (s & 31) of word s >> 5 of each plane. The .bwt body
-// (BWA's layout: 8 words of 16 two-bit symbols, first symbol in bits 31-30) is uploaded as is and
-// converted in place by k_planes. Position p of the $-inclusive BWT is at p - (p >= primary).
+// Occurrence counts. Device index layout: blocks of 128 symbols in 64 bytes,
+//   4 x u32  C[c]: row of the first suffix that starts with base c, plus the c's before the block
+//   4 x {high bits, low bits, prefix}, one per 32 symbols: the symbols' two bit planes (symbol s of the
+//            word at bit 31 - s) and, 7 bits each, the set high bits, set low bits and base 3's of the
+//            block before this word.
+// A count needs C and one 12-byte word, two loads of one 64-byte line and one masked popcount per
+// plane; with the counts as u64 and the planes whole (four 16-byte loads, a masked popcount of every
+// plane word) it was 55 vector instructions a position against 25, and 16 registers of loaded data
+// against 7. An index of 2^32 symbols or more counts C from the start of its epoch (2^24 blocks), and
+// `ext` holds the epochs' own counts; 32-bit counts are all a smaller index needs.
+//
+// Counts are of the first P symbols of the $-less BWT. Row r of the BWT with $ is symbol r - (r > primary)
+// (for r != primary), so the symbols at or before row k - 1 are P = k - (k > primary), k = 0 included, and
+// those at or before row l are P = l + (l < primary).
 
-__device__ __forceinline__ void load_block(const uint32_t *__restrict__ bwt, uint64_t blk, uint4 (&b)[4])
-{
-    const uint4 *p = reinterpret_cast<const uint4 *>(bwt + (blk << 4));
-    b[0] = p[0];
-    b[1] = p[1];
-    b[2] = p[2];
-    b[3] = p[3];
-}
+// what a position's count is computed from
+struct OccWord {
+    uint4 C;
+    uint32_t h, l, pre;
+};
 
-// counts of all 4 bases among symbols 0..r of a loaded block, plus its prefix counts: per plane
-// word, the high bits count bases 2 and 3, the low bits 1 and 3, both together base 3
-__device__ __forceinline__ void block_occ4(const uint4 (&b)[4], int r, uint64_t c[4])
+struct Sub {
+    uint32_t h, l, pre;
+};
+
+template <class K>
+__device__ __forceinline__ void occ_load(const uint32_t *__restrict__ bwt, K P, OccWord &o)
 {
-    const uint32_t hp[4] = {b[2].x, b[2].y, b[2].z, b[2].w};
-    const uint32_t lp[4] = {b[3].x, b[3].y, b[3].z, b[3].w};
-    uint32_t nh = 0, nl = 0, n3 = 0;
-#pragma unroll
-    for (int j = 0; j < 4; ++j) {
-        // the top t bits of word j: t = symbols of the word at or before r, 0..32
-        const uint32_t t = (uint32_t)min(max(r + 1 - 32 * j, 0), 32);
-        const uint32_t valid = (uint32_t)(0xffffffff00000000ull >> t);
-        const uint32_t h = hp[j] & valid, l = lp[j] & valid;
-        nh += __builtin_popcount(h);
-        nl += __builtin_popcount(l);
-        n3 += __builtin_popcount(h & l);
+    const uint32_t in = 16u + 12u * ((uint32_t)(P >> 5) & 3u);
+    const char *const base = reinterpret_cast<const char *>(bwt);
+    Sub sub;
+    if constexpr (sizeof(K) == 4) {
+        const uint32_t off = ((uint32_t)P >> 7) << 6;  // below 2^31
+        o.C = *reinterpret_cast<const uint4 *>(base + off);
+        sub = *reinterpret_cast<const Sub *>(base + (off + in));
+    } else {
+        const uint64_t off = ((uint64_t)P >> 7) << 6;
+        o.C = *reinterpret_cast<const uint4 *>(base + off);
+        sub = *reinterpret_cast<const Sub *>(base + off + in);
     }
-    const uint32_t n2 = nh - n3, n1 = nl - n3;
-    const uint32_t n0 = (uint32_t)(r + 1) - n1 - n2 - n3;
-    c[0] = ((uint64_t)b[0].y << 32 | b[0].x) + n0;
-    c[1] = ((uint64_t)b[0].w << 32 | b[0].z) + n1;
-    c[2] = ((uint64_t)b[1].y << 32 | b[1].x) + n2;
-    c[3] = ((uint64_t)b[1].w << 32 | b[1].z) + n3;
+    o.h = sub.h;
+    o.l = sub.l;
+    o.pre = sub.pre;
 }
 
-// In-place conversion of the uploaded .bwt body's symbol words to bit planes, one block per
-// thread (a last, shorter block included: its missing words were zero-filled).
-__global__ void __launch_bounds__(256) k_planes(uint32_t *bwt, uint64_t n_blocks)
+// counts of all four bases among the first P symbols, each plus its base's first row; `wide`: the index
+// has epochs (a constant in the wave engine)
+template <class K>
+__device__ __forceinline__ void occ_count(const DMeta &m, bool wide, const OccWord &o, K P, K (&c)[4])
+{
+    const uint32_t out = 0xffffffffu >> ((uint32_t)P & 31u);  // the symbols of the word from P on
+    const uint32_t h = o.h & ~out, l = o.l & ~out;
+    const uint32_t nh = __builtin_popcount(h) + (o.pre & 127u), nl = __builtin_popcount(l) + ((o.pre >> 7) & 127u);
+    const uint32_t n3 = __builtin_popcount(h & l) + ((o.pre >> 14) & 127u);
+    const uint32_t n0 = ((uint32_t)P & 127u) - nh - nl + n3;
+    c[0] = (K)(o.C.x + n0);
+    c[1] = (K)(o.C.y + (nl - n3));
+    c[2] = (K)(o.C.z + (nh - n3));
+    c[3] = (K)(o.C.w + n3);
+    if constexpr (sizeof(K) == 8) {
+        if (wide) {
+            const ulonglong2 *const e = reinterpret_cast<const ulonglong2 *>(m.ext + 4 * ((P >> 7) >> m.eshift));
+            const ulonglong2 e01 = e[0], e23 = e[1];
+            c[0] += e01.x;
+            c[1] += e01.y;
+            c[2] += e23.x;
+            c[3] += e23.y;
+        }
+    }
+}
+
+template <class K>
+__device__ __forceinline__ K pick4(const K (&v)[4], int c)
+{
+    // (all four are read first: a choice between elements would become an indexed load of the array,
+    // which then lives in scratch memory)
+    const K v0 = v[0], v1 = v[1], v2 = v[2], v3 = v[3];
+    const K a = (c & 1) ? v1 : v0, b = (c & 1) ? v3 : v2;
+    return (c & 2) ? b : a;
+}
+
+template <class K>
+__device__ __forceinline__ K pos_k(const DMeta &m, K k) { return k - (K)(k > (K)m.primary); }
+template <class K>
+__device__ __forceinline__ K pos_l(const DMeta &m, K l) { return l + (K)(l < (K)m.primary); }
+
+// 64-byte units of an occurrence query at (k - 1, l) as the reference counts them: one block when
+// k = 0 or both positions lie in one 128-symbol block of the .bwt, else two (src/bwtgap_hd.h:158-192)
+template <class K>
+__device__ __forceinline__ uint32_t occ_units(K Pk, K Pl)
+{
+    return Pk != 0 && (((Pk - 1) ^ (Pl - 1)) >> 7) != 0 ? 2u : 1u;
+}
+
+// bwt_2occ4 (src/bwtgap_hd.h:158-192) of the interval [k, l] on an index of any size: ca, cb are the
+// counts at rows k - 1 and l, each plus the base's first row, so that a child's interval is
+// [ca[c] + 1, cb[c]]. Returns the query's algorithmic bytes.
+__device__ __forceinline__ uint32_t lf_pair(const uint32_t *__restrict__ bwt, const DMeta &m, uint64_t k, uint64_t l,
+                                            uint64_t (&ca)[4], uint64_t (&cb)[4])
+{
+    const uint64_t Pk = pos_k<uint64_t>(m, k), Pl = pos_l<uint64_t>(m, l);
+    OccWord A, B;
+    occ_load<uint64_t>(bwt, Pk, A);
+    occ_load<uint64_t>(bwt, Pl, B);
+    occ_count<uint64_t>(m, m.ext != nullptr, A, Pk, ca);
+    occ_count<uint64_t>(m, m.ext != nullptr, B, Pl, cb);
+    return occ_units<uint64_t>(Pk, Pl) << 6;
+}
+
+// `ext` of an uploaded .bwt body (before k_planes rewrites it): per epoch and base, the base's first row
+// plus its count before the epoch's first block
+__global__ void k_epochs(const uint32_t *bwt, uint64_t n_blocks, uint32_t eshift, uint4 l2lo, uint4 l2hi, uint64_t *ext, uint32_t n)
+{
+    const uint32_t t = blockIdx.x * blockDim.x + threadIdx.x;
+    if (t >= 4 * n) return;
+    const uint64_t blk = (uint64_t)(t >> 2) << eshift;
+    const int c = (int)(t & 3);
+    const uint32_t lo[4] = {l2lo.x, l2lo.y, l2lo.z, l2lo.w}, hi[4] = {l2hi.x, l2hi.y, l2hi.z, l2hi.w};
+    const uint64_t before = blk < n_blocks ? reinterpret_cast<const uint64_t *>(bwt + (blk << 4))[c] : 0;
+    ext[t] = ((uint64_t)hi[c] << 32 | lo[c]) + before;
+}
+
+// In-place conversion of the uploaded .bwt body (BWA's blocks: 4 x u64 exclusive counts, 8 words of 16
+// two-bit symbols, first symbol in bits 31-30) to the device layout, one block per thread (a last, shorter
+// block included: what lies past its symbols is never counted).
+__global__ void __launch_bounds__(256) k_planes(uint32_t *bwt, uint64_t n_blocks, const uint64_t *ext, uint32_t eshift, int wide)
 {
     const uint64_t i = (uint64_t)blockIdx.x * blockDim.x + threadIdx.x;
     if (i >= n_blocks) return;
     uint4 *const p = reinterpret_cast<uint4 *>(bwt + (i << 4));
-    const uint4 s0 = p[2], s1 = p[3];
+    const uint4 c0 = p[0], c1 = p[1], s0 = p[2], s1 = p[3];
     const uint32_t w[8] = {s0.x, s0.y, s0.z, s0.w, s1.x, s1.y, s1.z, s1.w};
-    uint32_t hp[4] = {0, 0, 0, 0}, lp[4] = {0, 0, 0, 0};
+    uint32_t hp[4] = {0, 0, 0, 0}, lp[4] = {0, 0, 0, 0}, pre[4];
 #pragma unroll
     for (int k = 0; k < 8; ++k) {
 #pragma unroll
@@ -227,84 +300,23 @@ __global__ void __launch_bounds__(256) k_planes(uint32_t *bwt, uint64_t n_blocks
             lp[sym >> 5] |= (c & 1u) << (31 - (sym & 31));
         }
     }
-    p[2] = make_uint4(hp[0], hp[1], hp[2], hp[3]);
-    p[3] = make_uint4(lp[0], lp[1], lp[2], lp[3]);
-}
-
-// Occ of all four bases at positions a (may be -1) and b >= 0: bwt_2occ4, src/bwtgap_hd.h:158-192.
-// One 64-byte block when both fall in it, else two independent loads issued together.
-__device__ __forceinline__ uint32_t lf_pair(const uint32_t *__restrict__ bwt, const DMeta &m, uint64_t a, uint64_t b,
-                                            uint64_t ca[4], uint64_t cb[4])
-{
-    const uint64_t bp = b - (b >= m.primary);
-    const uint64_t bb = bp >> 7;
-    const bool aneg = a == ~0ull;
-    const uint64_t ap = a - (a >= m.primary);
-    const uint64_t ab = ap >> 7;
-    const bool same = !aneg && ab == bb;
-    uint4 B[4], A[4];
-    load_block(bwt, bb, B);
-    if (!aneg && !same) load_block(bwt, ab, A);
-    block_occ4(B, (int)(bp & 127), cb);
-    // a's block, picked per lane, so that one count serves lanes of both kinds
-#pragma unroll
-    for (int t = 0; t < 4; ++t) {
-        A[t].x = same ? B[t].x : A[t].x;
-        A[t].y = same ? B[t].y : A[t].y;
-        A[t].z = same ? B[t].z : A[t].z;
-        A[t].w = same ? B[t].w : A[t].w;
-    }
-    block_occ4(A, (int)(ap & 127), ca);
-    if (aneg) ca[0] = ca[1] = ca[2] = ca[3] = 0;
-    return (aneg || same) ? 64u : 128u;
-}
-
-// Occ of base c alone at positions a (may be -1) and b, for the steps that follow one symbol (an
-// exact tail, a width): one popcount per plane word, the planes flipped so that base c reads as
-// ones. Same block loads and byte count as lf_pair.
-__device__ __forceinline__ uint64_t block_occ1(const uint4 (&b)[4], int r, int c)
-{
-    const uint32_t hp[4] = {b[2].x, b[2].y, b[2].z, b[2].w};
-    const uint32_t lp[4] = {b[3].x, b[3].y, b[3].z, b[3].w};
-    const uint32_t hx = (c & 2) ? 0u : ~0u, lx = (c & 1) ? 0u : ~0u;
-    uint32_t n = 0;
+    uint32_t nh = 0, nl = 0, n3 = 0;
 #pragma unroll
     for (int j = 0; j < 4; ++j) {
-        const uint32_t t = (uint32_t)min(max(r + 1 - 32 * j, 0), 32);
-        const uint32_t valid = (uint32_t)(0xffffffff00000000ull >> t);
-        n += __builtin_popcount((hp[j] ^ hx) & (lp[j] ^ lx) & valid);
+        pre[j] = nh | nl << 7 | n3 << 14;
+        nh += __builtin_popcount(hp[j]);
+        nl += __builtin_popcount(lp[j]);
+        n3 += __builtin_popcount(hp[j] & lp[j]);
     }
-    // base c's count at the block start, by masks (a select between the block's words would be
-    // turned into an indexed load of the block, which then lives in scratch memory)
-    const uint32_t m0 = 0u - (uint32_t)(c == 0), m1 = 0u - (uint32_t)(c == 1), m2 = 0u - (uint32_t)(c == 2),
-                   m3 = 0u - (uint32_t)(c == 3);
-    const uint32_t lo = (b[0].x & m0) | (b[0].z & m1) | (b[1].x & m2) | (b[1].z & m3);
-    const uint32_t hi = (b[0].y & m0) | (b[0].w & m1) | (b[1].y & m2) | (b[1].w & m3);
-    return ((uint64_t)hi << 32 | lo) + n;
-}
-
-__device__ __forceinline__ uint32_t lf_one(const uint32_t *__restrict__ bwt, const DMeta &m, uint64_t a, uint64_t b,
-                                           int c, uint64_t &oa, uint64_t &ob)
-{
-    const uint64_t bp = b - (b >= m.primary);
-    const uint64_t bb = bp >> 7;
-    const bool aneg = a == ~0ull;
-    const uint64_t ap = a - (a >= m.primary);
-    const uint64_t ab = ap >> 7;
-    const bool same = !aneg && ab == bb;
-    uint4 B[4], A[4];
-    load_block(bwt, bb, B);
-    if (!aneg && !same) load_block(bwt, ab, A);
-    ob = block_occ1(B, (int)(bp & 127), c);
+    // 32 bits: the count from the epoch's start, or (one epoch) the base's first row and the count
+    const uint64_t *const e = ext + (wide ? 4 * (i >> eshift) : 0);
+    uint64_t C[4] = {(uint64_t)c0.y << 32 | c0.x, (uint64_t)c0.w << 32 | c0.z, (uint64_t)c1.y << 32 | c1.x, (uint64_t)c1.w << 32 | c1.z};
 #pragma unroll
-    for (int t = 0; t < 4; ++t) {
-        A[t].x = same ? B[t].x : A[t].x;
-        A[t].y = same ? B[t].y : A[t].y;
-        A[t].z = same ? B[t].z : A[t].z;
-        A[t].w = same ? B[t].w : A[t].w;
-    }
-    oa = aneg ? 0 : block_occ1(A, (int)(ap & 127), c);
-    return (aneg || same) ? 64u : 128u;
+    for (int c = 0; c < 4; ++c) C[c] = wide ? C[c] + ext[c] - e[c] : C[c] + ext[c];
+    p[0] = make_uint4((uint32_t)C[0], (uint32_t)C[1], (uint32_t)C[2], (uint32_t)C[3]);
+    p[1] = make_uint4(hp[0], lp[0], pre[0], hp[1]);
+    p[2] = make_uint4(lp[1], pre[1], hp[2], lp[2]);
+    p[3] = make_uint4(pre[2], hp[3], lp[3], pre[3]);
 }
 
 // ---------------------------------------------------------------------------
@@ -778,9 +790,9 @@ __global__ void __launch_bounds__(128) k_search(KArgs a)
                 hl = e_l(e);
                 return HITP;
             }
-            // the LF lookup at (k-1, l), whether the entry expands or starts an exact tail,
+            // the occurrence query of (k, l), whether the entry expands or starts an exact tail,
             // with the widths and the query bytes it needs
-            qa = e_k(e) - 1;
+            qa = e_k(e);
             qb = e_l(e);
             rq_lf = true;
             rq_w = true;
@@ -856,7 +868,7 @@ __global__ void __launch_bounds__(128) k_search(KArgs a)
             if (!in_seed) nN += c0 > 3;
             if (c0 <= 3) {
                 cbase = 3 - c0;
-                qa = ck - 1;
+                qa = ck;
                 qb = cl;
                 rq_lf = true;
                 c1p = cj + 1 < plen ? pstr + (cj + 1) : nullptr;
@@ -967,7 +979,7 @@ __global__ void __launch_bounds__(128) k_search(KArgs a)
                 if (had_lf) {
                     obytes += lf_bytes;
                     const int c = cbase;
-                    uint64_t k = M.L2[c] + ca[c] + 1, l = M.L2[c] + cb[c];
+                    uint64_t k = pick4(ca, c) + 1, l = pick4(cb, c);
                     if (k > l) {
                         k = 0;
                         l = seq_len;
@@ -990,7 +1002,7 @@ __global__ void __launch_bounds__(128) k_search(KArgs a)
                 // one step of an exact tail (bwt_match_exact_alt, src/bwtgap_hd.h:201-208)
                 obytes += lf_bytes;
                 const int c = cbase;
-                const uint64_t k = M.L2[c] + ca[c] + 1, l = M.L2[c] + cb[c];
+                const uint64_t k = pick4(ca, c) + 1, l = pick4(cb, c);
                 want_pop = true;
                 if (k <= l) {
                     if (cj == 0) {
@@ -1000,7 +1012,7 @@ __global__ void __launch_bounds__(128) k_search(KArgs a)
                     } else if (ch1 <= 3) {
                         --cj;
                         cbase = ch1;
-                        qa = k - 1;
+                        qa = k;
                         qb = l;
                         rq_lf = true;
                         c1p = cj >= 1 ? q + (cj - 1) : nullptr;
@@ -1019,7 +1031,7 @@ __global__ void __launch_bounds__(128) k_search(KArgs a)
                     // exact tail: its first step is this lookup
                     if (qbase <= 3) {
                         obytes += lf_bytes;
-                        const uint64_t k = M.L2[qbase] + ca[qbase] + 1, l = M.L2[qbase] + cb[qbase];
+                        const uint64_t k = pick4(ca, qbase) + 1, l = pick4(cb, qbase);
                         if (k <= l) {
                             if (i0 < 2) {
                                 want_hit = (int)(uint32_t)(l - k + 1) != 0;
@@ -1028,7 +1040,7 @@ __global__ void __launch_bounds__(128) k_search(KArgs a)
                             } else if (ch2 <= 3) {
                                 cj = i0 - 2;
                                 cbase = ch2;
-                                qa = k - 1;
+                                qa = k;
                                 qb = l;
                                 rq_lf = true;
                                 c1p = cj >= 1 ? q + (cj - 1) : nullptr;
@@ -1065,17 +1077,7 @@ __global__ void __launch_bounds__(128) k_search(KArgs a)
                     // bit 0 insertion, bits 1-4 deletions (bases 0..3), bits 5-8 the bases
                     // qbase+1 .. qbase+4 (the last one is the exact child), bit 9 the exact child
                     // alone (when differences are not allowed here)
-                    // the children's intervals per base (constant indices: the counts come from
-                    // scalar loads, not per-lane loads of the kernel arguments)
-                    uint64_t KK[4], LL[4];
-#pragma unroll
-                    for (int j = 0; j < 4; ++j) {
-                        KK[j] = M.L2[j] + ca[j] + 1;
-                        LL[j] = M.L2[j] + cb[j];
-                    }
-                    auto pick = [](const uint64_t(&v)[4], int j) __attribute__((always_inline)) {
-                        return j == 0 ? v[0] : j == 1 ? v[1] : j == 2 ? v[2] : v[3];
-                    };
+                    // the children's intervals are [ca + 1, cb] per base
                     uint32_t mask = 0;
                     if (gap_ok) {
                         const bool open = st == ST_M && go < max_gapo;
@@ -1083,16 +1085,16 @@ __global__ void __launch_bounds__(128) k_search(KArgs a)
                         if (open || (st == ST_D && ge < max_gape && (ge + go < max_diff || occ < (uint64_t)(int64_t)mdo))) {
     #pragma unroll
                             for (int j = 0; j < 4; ++j)
-                                if (KK[j] <= LL[j]) mask |= 2u << j;
+                                if (ca[j] < cb[j]) mask |= 2u << j;
                         }
                     }
                     if (allow_diff && allow_M) {
     #pragma unroll
                         for (int j = 1; j <= 4; ++j) {
                             const int c = (qbase + j) & 3;
-                            if (ca[c] + 1 <= cb[c]) mask |= 16u << j;
+                            if (pick4(ca, c) < pick4(cb, c)) mask |= 16u << j;
                         }
-                    } else if (qbase < 4 && ca[qbase] + 1 <= cb[qbase]) {
+                    } else if (qbase < 4 && pick4(ca, qbase) < pick4(cb, qbase)) {
                         mask |= 512u;
                     }
                     // Pushes, in bwt_match_gap's order: the gap children (bits 0-4) all score sg
@@ -1124,12 +1126,12 @@ __global__ void __launch_bounds__(128) k_search(KArgs a)
                                 ch = mk_ent(k, l, i, i, mm, go2, ge2, ins + 1, ST_I);
                             } else if (bit <= 4) {
                                 const int j = bit - 1;
-                                const uint64_t kk = pick(KK, j), ll = pick(LL, j);
+                                const uint64_t kk = pick4(ca, j) + 1, ll = pick4(cb, j);
                                 const int go2 = st == ST_M ? go + 1 : go, ge2 = st == ST_M ? ge : ge + 1;
                                 ch = mk_ent(kk, ll, i + 1, i + 1, mm, go2, ge2, ins, ST_D);
                             } else {
                                 const int c = (qbase + bit - 4) & 3;
-                                const uint64_t kk = pick(KK, c), ll = pick(LL, c);
+                                const uint64_t kk = pick4(ca, c) + 1, ll = pick4(cb, c);
                                 ch = mk_ent(kk, ll, i, i, mm + 1, go, ge, ins, ST_M);
                             }
                             if (bit <= 4)
@@ -1142,7 +1144,7 @@ __global__ void __launch_bounds__(128) k_search(KArgs a)
                             CHK[slot_] = ch;
                         }
                         if (mx) {
-                            const uint64_t kk = pick(KK, qbase & 3), ll = pick(LL, qbase & 3);  // (qbase <= 3 here)
+                            const uint64_t kk = pick4(ca, qbase) + 1, ll = pick4(cb, qbase);  // (qbase <= 3 here)
                             const Ent ch = mk_ent(kk, ll, i, 0, mm, go, ge, ins, ST_M);
                             if (a.fuse) {
                                 // pushed last with the parent's score: the next pop; kept in registers
@@ -1199,7 +1201,6 @@ __global__ void __launch_bounds__(256) k_sa_walk(const uint32_t *__restrict__ bw
                                                   const uint64_t *__restrict__ rows, uint64_t n, uint64_t *__restrict__ pos,
                                                   const int32_t *__restrict__ ref_len, int32_t *__restrict__ strand)
 {
-    const L2Sel L2(m);
     for (uint64_t i = (uint64_t)blockIdx.x * blockDim.x + threadIdx.x; i < n; i += (uint64_t)gridDim.x * blockDim.x) {
         uint64_t k = rows[i], sa = 0;
         while (k & (intv - 1)) {
@@ -1208,15 +1209,15 @@ __global__ void __launch_bounds__(256) k_sa_walk(const uint32_t *__restrict__ bw
                 k = 0;
                 break;
             }
-            const uint64_t x = k - (k > m.primary);
-            uint4 B[4];
-            load_block(bwt, x >> 7, B);
-            const int r = (int)(x & 127);
-            const uint32_t hw = r < 32 ? B[2].x : r < 64 ? B[2].y : r < 96 ? B[2].z : B[2].w;
-            const uint32_t lw = r < 32 ? B[3].x : r < 64 ? B[3].y : r < 96 ? B[3].z : B[3].w;
-            const int sh = 31 - (r & 31);
-            const int c = (int)(((hw >> sh) & 1u) << 1 | ((lw >> sh) & 1u));
-            k = L2[c] + block_occ1(B, r, c);
+            // the row's symbol, the one after the first k - (k > primary) symbols, and its rank
+            const uint64_t P = pos_k<uint64_t>(m, k);
+            OccWord o;
+            occ_load<uint64_t>(bwt, P, o);
+            uint64_t cnt[4];
+            occ_count<uint64_t>(m, m.ext != nullptr, o, P, cnt);
+            const uint32_t sh = 31u - ((uint32_t)P & 31u);
+            const int c = (int)(((o.h >> sh) & 1u) << 1 | ((o.l >> sh) & 1u));
+            k = pick4(cnt, c) + 1;
         }
         uint64_t p = sa + (k == 0 ? ~0ull : samples[k / intv - 1]);
         if (ref_len) {
@@ -1240,32 +1241,41 @@ __global__ void __launch_bounds__(256) k_sa_walk(const uint32_t *__restrict__ bw
 }
 
 // ---------------------------------------------------------------------------
-// Wave-per-read engine for heavy reads.
+// Wave-per-read engine.
 //
-// Between two hits the search's state (max_diff, widths, best score) is fixed,
-// and with positive penalties every non-exact child lands in a higher bucket
-// than its parent. So the entries of the lowest bucket b each start an
-// independent "chain" -- the entry, then its exact child, then that child's
-// exact child, ... (the sequential search pops exactly this chain next, LIFO) --
-// whose pushes all go to buckets above b. A wave takes the top K <= 64 entries
-// of bucket b, runs the K chains in parallel (one lane each, pushes logged),
-// then commits them in the sequential order: pops, pushes (placed by a
-// per-bucket scan so every bucket keeps its LIFO order), removal of the K
-// entries, and the first hit, which changes the state and ends the commit.
-// Chains after that hit are discarded and re-run in the next round. The
-// result, the pop count and the trace are those of the sequential search.
+// Between two hits the search's state (max_diff, widths, best score) is fixed, and with positive
+// penalties every non-exact child lands in a higher bucket than its parent. So the entries of the lowest
+// bucket b each start an independent "chain" -- the entry, then its exact child, then that child's exact
+// child, ... (the sequential search pops exactly this chain next, LIFO) -- whose pushes all go to buckets
+// above b. A workgroup of NW waves takes up to CPL chains per thread from the top of bucket b, runs them
+// (a thread takes the next chain when its own has ended), then commits them in the sequential order: pops,
+// pushes (placed by scans so that every bucket keeps its LIFO order), removal of the heads, and the first
+// hit, which changes the state and ends the commit. Chains after that hit are discarded and run again in
+// the next round. The result, the pop count and the trace are those of the sequential search.
 //
-// Buckets are LIFO lists of segments (a 16-byte header naming the segment
-// below, then the entries) in granules the wave takes from the stack pool.
+// Buckets are LIFO lists of segments (a 16-byte header naming the segment below, then the entries) in
+// granules the workgroup takes from the stack pool.
+//
+// What bounds it: vector issue, then the lookups' latency on a round's longest chain. A wave pays a full
+// iteration while one lane has a lookup left, and the chains of a heavy read are 2.3 steps long on average,
+// 5.5 the longest of 64: with one chain per lane and round 37% of the lane slots did work. Taking the next
+// chain when one ends, pruning dead heads before the loop, tails as iterations of the same loop (a nested
+// one held the wave for the longest tail of every step), 32-bit intervals and packed fields kept in
+// registers below 2^32 symbols, and one log per bucket code (a placed push needs no ranks, ballots or score)
+// took 2M ancient DNA reads on 100 Mbp from 308 ms of this kernel to 238, and 262,144 from 130 to 80.
 
-constexpr int HW = 64;         // lanes, one wave per workgroup
-constexpr int H_STEPS = 32;    // chain steps per lane per round
-constexpr int H_PUSH = 128;    // logged pushes per lane per round
-constexpr int H_CAP = 4096;    // pushes committed per round
-static_assert(H_CAP < 65536, "a round's bucket totals are summed in 16-bit fields");
-constexpr int H_KEEP = 64;     // granules a wave keeps between reads
-constexpr int H_PIECES = 48;    // segment pieces one round may add (three buckets)
+constexpr int HW = 64;         // lanes of a wave
+constexpr int H_STEPS = 32;    // chain steps per round
+constexpr int H_LOG = 64;      // logged pushes per thread and bucket code
+constexpr int H_SPUSH = 9;     // pushes of one step at most
+constexpr int H_SLOG = 64;     // trace build: steps logged per thread
+constexpr int H_CAP = 4096;    // pushes committed per round and wave
+constexpr int H_KEEP = 64;     // granules a workgroup keeps between reads
+constexpr int H_PIECES = 48;   // segment pieces one round may add (three buckets)
+constexpr int H_MINCAP = 128;  // the lowest push cap a test may set
 constexpr uint32_t GENT = (uint32_t)GRAN * CH;  // entries per granule
+static_assert(H_LOG <= 120 && H_LOG > 2 * H_SPUSH, "push counts and offsets are 7-bit fields");
+static_assert(H_SLOG >= 2 * H_STEPS, "a chain's steps fit the rest of a thread's step log");
 
 enum : int { K_END = 0, K_HIT = 1, K_TRUNC = 2, K_ESCORE = 3 };
 
@@ -1279,10 +1289,11 @@ struct HArgs {
     const int32_t *batch;
     const galn_search_opt_t *bopts;
     const int32_t *nstacks;
-    const int32_t *list;
+    const int32_t *list;        // read ids by position, or null (the position)
+    const int32_t *poslist;     // positions to search, or null (0 .. n_list - 1)
     int32_t n_list;
-    const int32_t *n_list_dev;  // when set, the number of reads is read here (written by k_search)
-    const uint64_t *hand;       // widths handed over by k_search (slot = list position), or null
+    const int32_t *n_list_dev;  // when set, the number of reads is read here
+    const uint64_t *hand;       // widths by position (k_search or k_widths), or null
     uint32_t hand_stride;
     int32_t hand_cap;
     int32_t *qnext;
@@ -1306,24 +1317,28 @@ struct HArgs {
     int32_t buckets;  // LDS buckets: the largest n_stacks of the launch
     int32_t wlen;     // LDS widths: longest read + 1
     int32_t swlen;    // LDS seed widths
-    int32_t push_cap; // pushes committed per round, H_PUSH..H_CAP (H_CAP unless a test lowers it)
-    unsigned long long *stats;  // [8] engine counters (rounds, chains, steps, cycles)
+    int32_t push_cap; // pushes committed per round (H_CAP per wave unless a test lowers it)
+    uint32_t deep_pops;  // > 0: a read that has popped this many goes to deep_list (its position)
+    int32_t *deep_list, *deep_n;
+    unsigned long long *stats;  // [16] engine counters (rounds, chains, steps, cycles)
 };
 
 struct HShared {
-    int rid, len, n_stacks, md_read, seeding, seed_len;
+    int len, n_stacks, md_read, seeding, seed_len;
     int s_mm, s_gapo, s_gape, mode, ies, mdo, max_entries, max_gapo, max_gape, msd, max_top2;
     int best_score, best_diff, max_diff, best_cnt, n_aln, n_entries;
     unsigned long long pops, trace, obytes;
     unsigned long long bm[4];
-    int has_pend, claim, status, result, K, b, J, jcap, jcut, tcut, n_piece, n_own, n_used, aleft;
+    int has_pend, claim, status, result, K, b, n_piece, n_own, n_used, aleft, nN, bad;
     uint32_t abase;
-    int nN;
-    int l_full;             // the last committed chain's stop kind
+    int next, stop, lim, l_kind, cut;  // the round's claims, first stopping chain, commit limit
+    uint32_t tot01, tot2s, totb;       // committed pushes (16 bits per bucket code), pops, index bytes / 64
+    int fp[3];                         // first piece of each bucket code
+    uint32_t wsum[3][16];              // per wave: scan totals
+    int wlive[16];
     unsigned long long st[16];
-    uint64_t hk, hl;
-    Ent pend, he;
-    int he_score;
+    uint64_t hk, hl;                   // the last committed chain's hit, or its pending child
+    uint32_t hx, hy;
 };
 
 __device__ __forceinline__ int hbm_low(const unsigned long long *bm)
@@ -1332,60 +1347,125 @@ __device__ __forceinline__ int hbm_low(const unsigned long long *bm)
                  : bm[3] ? 192 + __builtin_ctzll(bm[3]) : -1;
 }
 
-// wave-wide (64-lane) scans and reductions; every lane of the wave must call them
-__device__ __forceinline__ int wave_excl_scan(int v)
+// lanes below this one that are set in m
+__device__ __forceinline__ int lanes_below(uint64_t m)
 {
-    const int lane = threadIdx.x & (HW - 1);
-    int x = v;
-    for (int d = 1; d < HW; d <<= 1) {
-        const int t = __shfl_up(x, d, HW);
-        if (lane >= d) x += t;
+    return (int)__builtin_amdgcn_mbcnt_hi((uint32_t)(m >> 32), __builtin_amdgcn_mbcnt_lo((uint32_t)m, 0u));
+}
+
+// inclusive sum over a wave's lanes in six row moves (no LDS); every lane of the wave must call it
+__device__ __forceinline__ uint32_t wave_incl_scan(uint32_t x)
+{
+    x += (uint32_t)__builtin_amdgcn_update_dpp(0, (int)x, 0x111, 0xf, 0xf, false);  // row_shr:1
+    x += (uint32_t)__builtin_amdgcn_update_dpp(0, (int)x, 0x112, 0xf, 0xf, false);  // row_shr:2
+    x += (uint32_t)__builtin_amdgcn_update_dpp(0, (int)x, 0x114, 0xf, 0xf, false);  // row_shr:4
+    x += (uint32_t)__builtin_amdgcn_update_dpp(0, (int)x, 0x118, 0xf, 0xf, false);  // row_shr:8
+    x += (uint32_t)__builtin_amdgcn_update_dpp(0, (int)x, 0x142, 0xa, 0xf, false);  // row_bcast:15
+    x += (uint32_t)__builtin_amdgcn_update_dpp(0, (int)x, 0x143, 0xc, 0xf, false);  // row_bcast:31
+    return x;
+}
+
+// A stack entry in registers: the interval, x = i | n_mm << 10 | n_gapo << 17 | state << 24 and
+// y = last_diff_pos | n_gape << 10 | n_ins << 18. In memory an index of 2^32 symbols or more packs k and x
+// into one 64-bit word, l and y into the other (the layout above); a smaller one stores the four words.
+template <bool WIDE>
+struct Item {
+    using K = typename std::conditional<WIDE, uint64_t, uint32_t>::type;
+    K k, l;
+    uint32_t x, y;
+};
+constexpr uint32_t X_I = 1023u, X_MM = 1u << 10, X_GO = 1u << 17, X_ST = 3u << 24, X_INS = 1u << 24, X_DEL = 2u << 24;
+constexpr uint32_t Y_LDP = 1023u, Y_GE = 1u << 10, Y_IN = 1u << 18;
+__device__ __forceinline__ int x_mm(uint32_t x) { return (int)((x >> 10) & 127u); }
+__device__ __forceinline__ int x_go(uint32_t x) { return (int)((x >> 17) & 127u); }
+__device__ __forceinline__ int x_st(uint32_t x) { return (int)((x >> 24) & 3u); }
+__device__ __forceinline__ int y_ge(uint32_t y) { return (int)((y >> 10) & 255u); }
+__device__ __forceinline__ int y_ins(uint32_t y) { return (int)((y >> 18) & 255u); }
+
+template <bool WIDE>
+__device__ __forceinline__ void put_item(Ent *p, typename Item<WIDE>::K k, typename Item<WIDE>::K l, uint32_t x, uint32_t y)
+{
+    if constexpr (WIDE) {
+        Ent e;
+        e.w0 = (uint64_t)k | (uint64_t)x << 38;
+        e.w1 = (uint64_t)l | (uint64_t)y << 38;
+        *p = e;
+    } else {
+        *reinterpret_cast<uint4 *>(p) = make_uint4((uint32_t)k, (uint32_t)l, x, y);
     }
-    return x - v;
 }
 
-
-__device__ __forceinline__ unsigned long long wave_sum_u64(unsigned long long v)
+template <bool WIDE>
+__device__ __forceinline__ Item<WIDE> get_item(const Ent *p)
 {
-    for (int d = HW / 2; d > 0; d >>= 1) v += __shfl_xor(v, d, HW);
-    return v;
+    Item<WIDE> r;
+    if constexpr (WIDE) {
+        const Ent e = *p;
+        r.k = e.w0 & KMASK;
+        r.l = e.w1 & KMASK;
+        r.x = (uint32_t)(e.w0 >> 38);
+        r.y = (uint32_t)(e.w1 >> 38);
+    } else {
+        const uint4 v = *reinterpret_cast<const uint4 *>(p);
+        r.k = v.x;
+        r.l = v.y;
+        r.x = v.z;
+        r.y = v.w;
+    }
+    return r;
 }
 
-__device__ __forceinline__ int wave_max_i32(int v)
+// a popped entry's share of the trace hash
+__device__ __forceinline__ uint64_t trace_item(uint64_t t, int score, uint64_t k, uint64_t l, uint32_t x, uint32_t y, int n_entries)
 {
-    for (int d = HW / 2; d > 0; d >>= 1) v = max(v, __shfl_xor(v, d, HW));
-    return v;
+    const int mm = x_mm(x), go = x_go(x), ge = y_ge(y), st = x_st(x), ins = y_ins(y);
+    t = tr_mix(t, (uint64_t)((uint32_t)score << 21 | (x & X_I)));
+    t = tr_mix(t, k);
+    t = tr_mix(t, l);
+    t = tr_mix(t, (uint64_t)((uint32_t)mm | (uint32_t)go << 8 | (uint32_t)ge << 16 | (uint32_t)st << 24));
+    t = tr_mix(t, (uint64_t)ins | (uint64_t)(go + ge - ins) << 16);
+    t = tr_mix(t, (uint64_t)(y & Y_LDP));
+    return tr_mix(t, (uint64_t)(uint32_t)n_entries);
 }
 
-// bwt_cal_width by one lane (src/bwtgap_hd.h:216-242); returns the algorithmic bytes
-__device__ uint64_t cal_width_one(const uint32_t *bwt, const DMeta &M, int len, const uint8_t *str, uint64_t *w)
+// widths in LDS: the value in the low part, the bound above it (32 bits each below 2^32 symbols, so that
+// neither needs a shift; the 48 | 16 of the hand-off slots otherwise)
+template <bool WIDE>
+__device__ __forceinline__ uint32_t lw_bid(uint64_t v) { return WIDE ? (uint32_t)(v >> 48) : (uint32_t)(v >> 32); }
+template <bool WIDE>
+__device__ __forceinline__ uint64_t lw_val(uint64_t v) { return WIDE ? v & W48 : v & 0xffffffffull; }
+template <bool WIDE>
+__device__ __forceinline__ uint64_t lw_make(uint64_t w, uint32_t bid) { return WIDE ? w | (uint64_t)bid << 48 : w | (uint64_t)bid << 32; }
+
+// bwt_cal_width by one thread (src/bwtgap_hd.h:216-242); returns the algorithmic bytes. put(i, w, bid)
+// stores position i's width.
+template <class Put>
+__device__ __forceinline__ uint64_t cal_width_one(const uint32_t *bwt, const DMeta &M, int len, const uint8_t *str, Put put)
 {
-    const L2Sel L2s(M);
     uint64_t k = 0, l = M.seq_len, bytes = 0;
     int bid = 0;
     for (int i = 0; i < len; ++i) {
         const int c0 = str[i];
-        const int c = c0 > 3 ? 4 : 3 - c0;
-        if (c < 4) {
-            uint64_t oa, ob;
-            bytes += lf_one(bwt, M, k - 1, l, c, oa, ob);
-            k = L2s[c] + oa + 1;
-            l = L2s[c] + ob;
+        if (c0 <= 3) {
+            uint64_t ca[4], cb[4];
+            bytes += lf_pair(bwt, M, k, l, ca, cb);
+            k = pick4(ca, 3 - c0) + 1;
+            l = pick4(cb, 3 - c0);
         }
-        if (k > l || c > 3) {
+        if (k > l || c0 > 3) {
             k = 0;
             l = M.seq_len;
             ++bid;
         }
-        w[i] = wpack(l - k + 1, bid);
+        put(i, l - k + 1, bid);
     }
-    w[len] = wpack(0, ++bid);
+    put(len, 0, ++bid);
     return bytes;
 }
 
-// Widths of the reads given to the wave engine whose hand-off slot is empty (a record found by
-// k_search had already changed them): one thread per read, all reads at once, so that the wave
-// engine does not hold 64 lanes while one of them walks a read's sequential width pass.
+// Widths of the reads given to the wave engine, into their hand-off slots (those that k_search has not
+// filled): one thread per read, all reads at once, so that the wave engine does not hold 64 lanes while one
+// of them walks a read's sequential width pass.
 struct WArgs {
     const uint32_t *bwt;
     DMeta meta;
@@ -1401,6 +1481,7 @@ struct WArgs {
     uint32_t hand_stride;
     int32_t hand_cap;
     int32_t wlen, swlen;
+    int32_t check;  // slots may hold widths already
 };
 
 __global__ void __launch_bounds__(256) k_widths(WArgs a)
@@ -1408,82 +1489,86 @@ __global__ void __launch_bounds__(256) k_widths(WArgs a)
     const int n = min(a.n_list_dev ? *a.n_list_dev : a.n_list, a.hand_cap);
     for (int pos = blockIdx.x * blockDim.x + threadIdx.x; pos < n; pos += gridDim.x * blockDim.x) {
         uint64_t *const dst = a.hand + (uint64_t)pos * a.hand_stride;
-        if (dst[0] >> 63) continue;  // handed over by k_search
-        const int rid = a.list[pos];
+        if (a.check && (dst[0] >> 63)) continue;  // handed over by k_search
+        const int rid = a.list ? a.list[pos] : pos;
         const int len = a.qlen[rid];
-        if (len < 1 || len + 1 > a.wlen) continue;  // the wave engine rejects it
         const int sl = a.bopts[a.batch[rid]].seed_len;
-        if (sl < len && sl + 1 > a.swlen) continue;
+        // (a read the wave engine rejects, or a seed it has no room for: no widths)
+        if (len < 1 || len + 1 > a.wlen || (sl < len && sl + 1 > a.swlen)) {
+            dst[0] = 0;
+            continue;
+        }
         const uint8_t *const q = a.query + a.qoff[rid];
-        uint64_t wb = cal_width_one(a.bwt, a.meta, len, q, dst + 1);
-        if (sl < len) wb += cal_width_one(a.bwt, a.meta, sl, q + (len - sl), dst + 2 + len);
+        uint64_t *w = dst + 1;
+        uint64_t wb = cal_width_one(a.bwt, a.meta, len, q, [w](int i, uint64_t v, int bid) { w[i] = wpack(v, bid); });
+        w = dst + 2 + len;
+        if (sl < len) wb += cal_width_one(a.bwt, a.meta, sl, q + (len - sl), [w](int i, uint64_t v, int bid) { w[i] = wpack(v, bid); });
         dst[0] = wb | (1ull << 63);
     }
 }
 
-// WPE waves per SIMD: 4 (16 per CU) at 128 VGPRs, the compiler spilling a few values to scratch; the
-// extra resident waves hide more of the index latency than the spills cost (measured 3.4% against 3
-// per SIMD on the 100 Mbp workload, where 5 was 10% slower: that index sits in the MALL and the
-// engine is bound by instruction issue). 5 (96 VGPRs, more spills) for indexes in HBM, where a wave
-// waits on its loads: 20% faster on the 3.1 Gbp human-like workload, 25% slower on the 20 Gbp one.
-template <bool TRACE, int WPE>
-__global__ void __launch_bounds__(64) __attribute__((amdgpu_waves_per_eu(WPE))) k_heavy(HArgs a)
+// LDS of a workgroup of nw waves, cpl chains per thread (k_heavy carves it up in this order)
+constexpr size_t heavy_chain_bytes = 16 + 4 + 4 + 4 + 2 + 2;  // head | counts | log place | steps | id | trace place
+
+// NW waves per read; WPE waves per SIMD: 4 at 128 VGPRs, or 5 (96 VGPRs) for indexes in HBM, where a wave
+// waits on its loads.
+template <bool TRACE, bool WIDE, int NW, int CPL, int WPE>
+__global__ void __launch_bounds__(64 * NW) __attribute__((amdgpu_waves_per_eu(WPE))) k_heavy(HArgs a)
 {
+    using K = typename Item<WIDE>::K;
+    constexpr int T = 64 * NW, KMAX = T * CPL;
+    static_assert(T <= 256, "a thread's index takes 8 bits of its chains' records");
     extern __shared__ __align__(16) uint8_t hlds[];
     HShared &F = *reinterpret_cast<HShared *>(hlds);
     uint8_t *lp = hlds + ((sizeof(HShared) + 15) & ~(size_t)15);
-    const int NB = a.buckets;
-    uint32_t *seg_base = reinterpret_cast<uint32_t *>(lp);
-    uint32_t *seg_cnt = seg_base + NB;
-    int32_t *first_piece = reinterpret_cast<int32_t *>(seg_cnt + NB);
-    lp = reinterpret_cast<uint8_t *>(first_piece + NB);
-    lp = hlds + (((size_t)(lp - hlds) + 15) & ~(size_t)15);
-    uint4 *pieces = reinterpret_cast<uint4 *>(lp);  // {bucket, rank0, len, base}
-    uint64_t *W = reinterpret_cast<uint64_t *>(pieces + H_PIECES);
-    uint64_t *SW = W + a.wlen;
-    int32_t *lcommit = reinterpret_cast<int32_t *>(SW + a.swlen);  // per chain, for the trace hash
-    int32_t *lnstart = lcommit + HW;
-    // per chain step: pushes (4 bits) | index bytes / 64 << 4 (a step's bytes are whole 64-byte
-    // blocks, at most 2 per position of a read of at most 1023: under 4096 units)
-    uint16_t *const SINFO_ALL = reinterpret_cast<uint16_t *>(lnstart + HW);
-    uint8_t *const QL = reinterpret_cast<uint8_t *>(SINFO_ALL + HW * H_STEPS);  // the read's query
+    uint4 *const pieces = reinterpret_cast<uint4 *>(lp);  // {bucket code, rank0, len, base}
+    Ent *const hent = reinterpret_cast<Ent *>(pieces + H_PIECES);  // live chains' heads, in order
+    uint16_t *const epre = reinterpret_cast<uint16_t *>(hent);     // after them: pushes before each chain, by code
+    uint32_t *const cA = reinterpret_cast<uint32_t *>(hent + KMAX);  // pushes by code (8 bits each) | stop kind << 24
+    uint32_t *const cB = cA + KMAX;                                  // place in the thread's logs (8 bits each) | thread << 24
+    uint32_t *const cC = cB + KMAX;                                  // steps | index bytes / 64 << 6
+    uint16_t *const hcid = reinterpret_cast<uint16_t *>(cC + KMAX);  // live chains' ids
+    uint16_t *const cS = hcid + KMAX;                                // trace build: place in the thread's step log
+    uint64_t *const Wp = reinterpret_cast<uint64_t *>(cS + KMAX);    // Wp[i] = width of position i - 1
+    uint64_t *const SW = Wp + a.wlen + 1;
+    uint32_t *const seg_base = reinterpret_cast<uint32_t *>(SW + a.swlen);
+    uint32_t *const seg_cnt = seg_base + a.buckets;
+    uint16_t *const s0info = reinterpret_cast<uint16_t *>(seg_cnt + a.buckets);  // chain 0's steps: pushes | index bytes / 64 << 4
+    uint8_t *const QL = reinterpret_cast<uint8_t *>(s0info + H_STEPS);           // the read's query
+    static_assert(MAXLEN * 2 + 2 < 4096, "a step's index bytes fit the step info");
 
-    const int lane = threadIdx.x;
+    const int tid = threadIdx.x, lane = tid & (HW - 1), wave = tid >> 6;
     if ((int)blockIdx.x >= a.n_slots) return;
     uint8_t *const base = a.scratch + (uint64_t)blockIdx.x * a.slot_bytes;
     galn_aln_rec_t *const REC = reinterpret_cast<galn_aln_rec_t *>(base + a.rec_off);
     uint32_t *const OWN = reinterpret_cast<uint32_t *>(base + a.own_off);
-    Ent *const PLOG = reinterpret_cast<Ent *>(base + a.plog_off) + lane * H_PUSH;
-    Ent *const SLOG_ALL = reinterpret_cast<Ent *>(base + a.slog_off);
-    Ent *const SLOG = SLOG_ALL + lane * H_STEPS;
-    uint16_t *const SINFO = SINFO_ALL + lane * H_STEPS;
-    static_assert(MAXLEN * 128 / 64 < 4096, "a step's index bytes fit the step info");
+    Ent *const LOG = reinterpret_cast<Ent *>(base + a.plog_off);     // code c, thread t: [(c * T + t) * H_LOG]
+    Ent *const SLOG = reinterpret_cast<Ent *>(base + a.slog_off);    // trace build: thread t's steps at t * H_SLOG
+    uint8_t *const SINFO = reinterpret_cast<uint8_t *>(SLOG + T * H_SLOG);  // and their push counts
     Ent *const POOL = a.pool;
     const DMeta &M = a.meta;
-    const L2Sel L2s(M);
-    const uint64_t seq_len = M.seq_len;
+    const K seq_len = (K)M.seq_len;
 
-    if (lane == 0) {
+    if (tid == 0) {
         for (int j = 0; j < 16; ++j) F.st[j] = 0;
-        F.n_own = 0;  // granules this wave holds; a read reuses them before taking more
+        F.n_own = 0;  // granules this workgroup holds; a read reuses them before taking more
     }
     const int n_list = a.n_list_dev ? *a.n_list_dev : a.n_list;
     for (;;) {
         const long long t_read = a.stats ? wall_clock64() : 0;
-        if (lane == 0) F.claim = atomicAdd(a.qnext, 1);
+        if (tid == 0) F.claim = atomicAdd(a.qnext, 1);
         __syncthreads();
-        const int pos = F.claim;
-        if (pos >= n_list) break;
-        // ---- read set-up (lane 0), widths (lanes 0 and 1) ----
-        const int rid = a.list[pos];
+        const int claim = F.claim;
+        if (claim >= n_list) break;
+        // ---- read set-up ----
+        const int pos = a.poslist ? a.poslist[claim] : claim;
+        const int rid = a.list ? a.list[pos] : pos;
         const int len = a.qlen[rid];
         const uint8_t *const qg = a.query + a.qoff[rid];
-        const uint8_t *const q = QL;
-        for (int j = lane; j < len && j < a.wlen; j += HW) QL[j] = qg[j];
-        if (lane == 0) {
+        for (int j = tid; j < len && j < a.wlen; j += T) QL[j] = qg[j];
+        if (tid == 0) {
             const int b0 = a.batch[rid];
             const galn_search_opt_t o = a.bopts[b0];
-            F.rid = rid;
             F.len = len;
             F.s_mm = o.s_mm;
             F.s_gapo = o.s_gapo;
@@ -1506,33 +1591,36 @@ __global__ void __launch_bounds__(64) __attribute__((amdgpu_waves_per_eu(WPE))) 
             F.aleft = 0;
             F.abase = 0;
             F.status = 0;
+            F.bad = 0;
         }
         __syncthreads();
-        const bool unsup = len < 1 || len > MAXLEN || len + 1 > a.wlen || F.n_stacks > NB || F.md_read > MAXDIFF ||
+        const bool unsup = len < 1 || len > MAXLEN || len + 1 > a.wlen || F.n_stacks > a.buckets || F.md_read > MAXDIFF ||
                            F.max_gapo > MAXDIFF || F.max_gapo + F.max_gape > 255;
         const uint64_t h0 = (!unsup && a.hand && pos < a.hand_cap) ? a.hand[(uint64_t)pos * a.hand_stride] : 0;
-        if (!unsup && (h0 >> 63)) {
-            // the widths k_search computed for this read
-            const uint64_t *src = a.hand + (uint64_t)pos * a.hand_stride;
-            for (int j = lane; j <= len; j += HW) W[j] = src[1 + j];
-            if (F.seeding)
-                for (int j = lane; j <= F.seed_len; j += HW) SW[j] = src[2 + len + j];
-            if (lane == 0) F.obytes = h0 & ~(1ull << 63);
+        if (!unsup) {
+            if (h0 >> 63) {
+                // the widths computed for this read
+                const uint64_t *src = a.hand + (uint64_t)pos * a.hand_stride;
+                for (int j = tid; j <= len; j += T) Wp[1 + j] = lw_make<WIDE>(wval(src[1 + j]), (uint32_t)wbid(src[1 + j]));
+                if (F.seeding)
+                    for (int j = tid; j <= F.seed_len; j += T)
+                        SW[j] = lw_make<WIDE>(wval(src[2 + len + j]), (uint32_t)wbid(src[2 + len + j]));
+                if (tid == 0) F.obytes = h0 & ~(1ull << 63);
+            } else {
+                uint64_t wb = 0;
+                auto putw = [Wp](int i, uint64_t v, int bid) { Wp[1 + i] = lw_make<WIDE>(v, (uint32_t)bid); };
+                auto puts = [SW](int i, uint64_t v, int bid) { SW[i] = lw_make<WIDE>(v, (uint32_t)bid); };
+                if (tid == 0) wb = cal_width_one(a.bwt, M, len, QL, putw);
+                if (tid == 1 && F.seeding) wb = cal_width_one(a.bwt, M, F.seed_len, QL + (len - F.seed_len), puts);
+                if (wb) atomicAdd(&F.obytes, (unsigned long long)wb);
+            }
             int nN = 0;
-            for (int j = lane; j < len; j += HW) nN += q[j] > 3;
+            for (int j = tid; j < len; j += T) nN += QL[j] > 3;
             if (nN) atomicAdd(&F.nN, nN);
-        } else if (!unsup) {
-            uint64_t wb = 0;
-            if (lane == 0) wb = cal_width_one(a.bwt, M, len, q, W);
-            if (lane == 1 && F.seeding) wb = cal_width_one(a.bwt, M, F.seed_len, q + (len - F.seed_len), SW);
-            int nN = 0;
-            for (int j = lane; j < len; j += HW) nN += q[j] > 3;
-            if (nN) atomicAdd(&F.nN, nN);
-            if (wb) atomicAdd(&F.obytes, (unsigned long long)wb);
         }
         __syncthreads();
         // ---- search set-up ----
-        if (lane == 0) {
+        if (tid == 0) {
             F.best_score = (F.md_read + 1) * F.s_mm + (F.max_gapo + 1) * F.s_gapo + (F.max_gape + 1) * F.s_gape;
             F.best_diff = F.md_read + 1;
             F.max_diff = F.md_read;
@@ -1543,6 +1631,7 @@ __global__ void __launch_bounds__(64) __attribute__((amdgpu_waves_per_eu(WPE))) 
             F.bm[0] = F.bm[1] = F.bm[2] = F.bm[3] = 0;
             F.has_pend = 0;
             F.n_entries = 0;
+            Wp[0] = 0;
             if (unsup) {
                 F.status = 1;
                 F.result = ERR_UNSUP;
@@ -1554,28 +1643,28 @@ __global__ void __launch_bounds__(64) __attribute__((amdgpu_waves_per_eu(WPE))) 
                 F.result = ERR_SCORE;
             } else {
                 F.has_pend = 1;
-                F.pend = mk_ent(0, seq_len, len, 0, 0, 0, 0, 0, ST_M);
+                F.hk = 0;
+                F.hl = M.seq_len;
+                F.hx = (uint32_t)len;
+                F.hy = 0;
                 F.b = 0;
                 F.n_entries = 1;
             }
         }
         __syncthreads();
-        if (a.stats && lane == 0) {
+        if (a.stats && tid == 0) {
             F.st[12] += (unsigned long long)(wall_clock64() - t_read);
             F.st[15] += 1;
         }
         // ---- rounds ----
         long long t_round_end = 0;  // with stats: end of the last round's commit
-        while (F.status == 0) {
+        for (;;) {
             const long long t_round = a.stats ? wall_clock64() : 0;
-            if (a.stats && lane == 0 && t_round_end) F.st[14] += (unsigned long long)(t_round - t_round_end);
-            if (lane == 0) {
+            if (a.stats && tid == 0 && t_round_end) F.st[14] += (unsigned long long)(t_round - t_round_end);
+            if (tid == 0 && F.status == 0) {  // (the others read the status after the barrier)
                 // a pending exact child is the top of the lowest bucket (the bucket it came from)
                 const int b = F.has_pend ? F.b : hbm_low(F.bm);
-                if (F.has_pend == 0 && b < 0) {
-                    F.status = 1;
-                    F.result = F.n_aln;
-                } else if (F.n_entries > F.max_entries) {
+                if (b < 0 || F.n_entries > F.max_entries) {
                     F.status = 1;
                     F.result = F.n_aln;
                 } else {
@@ -1584,349 +1673,499 @@ __global__ void __launch_bounds__(64) __attribute__((amdgpu_waves_per_eu(WPE))) 
                     const uint32_t avail = (uint32_t)F.has_pend + (bit ? seg_cnt[b] : 0u);
                     if (!(F.mode & MODE_NONSTOP) && (uint32_t)b > (uint32_t)(F.best_score + F.s_mm)) {
                         // this pop ends the search (src/bwtgap_hd.h:366)
-                        const Ent e = F.has_pend ? F.pend : POOL[seg_base[b] + seg_cnt[b] - 1];
                         F.pops += 1;
                         F.n_entries -= 1;
                         if (TRACE) {
-                            const int i0 = e_i(e), mm = e_mm(e), go = e_go(e), ge = e_ge(e), st = e_st(e), ins = e_ins(e);
-                            uint64_t t = F.trace;
-                            t = tr_mix(t, (uint64_t)((uint32_t)b << 21 | (uint32_t)i0));
-                            t = tr_mix(t, e_k(e));
-                            t = tr_mix(t, e_l(e));
-                            t = tr_mix(t, (uint64_t)((uint32_t)mm | (uint32_t)go << 8 | (uint32_t)ge << 16 | (uint32_t)st << 24));
-                            t = tr_mix(t, (uint64_t)ins | (uint64_t)(go + ge - ins) << 16);
-                            t = tr_mix(t, (uint64_t)(uint32_t)e_ldp(e));
-                            t = tr_mix(t, (uint64_t)(uint32_t)F.n_entries);
-                            F.trace = t;
+                            Item<WIDE> e;
+                            if (F.has_pend) {
+                                e.k = (K)F.hk;
+                                e.l = (K)F.hl;
+                                e.x = F.hx;
+                                e.y = F.hy;
+                            } else {
+                                e = get_item<WIDE>(POOL + seg_base[b] + seg_cnt[b] - 1);
+                            }
+                            F.trace = trace_item(F.trace, b, e.k, e.l, e.x, e.y, F.n_entries);
                         }
                         F.status = 1;
                         F.result = F.n_aln;
                     } else {
-                        F.K = (int)min(avail, (uint32_t)HW);
+                        F.K = (int)min(avail, (uint32_t)KMAX);
+                        F.next = T;
+                        F.stop = 0x7fffffff;
+                        F.lim = 0x7fffffff;
+                        F.l_kind = K_END;
+                        F.cut = -1;
                     }
                 }
             }
             __syncthreads();
             if (F.status) break;
-            // ---- speculation: lane j runs the chain of the j-th entry from the top of bucket b ----
-            const int b = F.b, K = F.K, hp = F.has_pend;
+            const int b = F.b, nK = F.K, hp = F.has_pend;
             const long long t_spec = a.stats ? wall_clock64() : 0;
-            if (a.stats && lane == 0) F.st[13] += (unsigned long long)(t_spec - t_round);
+            if (a.stats && tid == 0) F.st[13] += (unsigned long long)(t_spec - t_round);
             const int s_mm = F.s_mm, s_gapo = F.s_gapo, s_gape = F.s_gape, mode = F.mode, max_diff = F.max_diff;
             const int n_stacks = F.n_stacks, max_gapo = F.max_gapo, max_gape = F.max_gape, ies = F.ies, mdo = F.mdo;
-            const int msd = F.msd, seed_len = F.seed_len;
+            const int msd = F.msd, sofs = len - F.seed_len;
             const bool seeding = F.seeding != 0;
-            int steps = 0, np = 0, kind = K_END;
-            uint32_t sby = 0;    // index bytes of the chain's steps
-            uint32_t ccnt = 0;   // logged pushes per bucket code, 8 bits each
-            uint64_t hk = 0, hl = 0;
-            Ent nxt{0, 0};
-            if (lane < K) {
-                Ent e = (lane == 0 && hp) ? F.pend : POOL[seg_base[b] + seg_cnt[b] - 1 - (uint32_t)(lane - hp)];
-                for (;;) {
-                    if (steps == H_STEPS || np > H_PUSH - 9) {
-                        kind = K_TRUNC;
-                        nxt = e;
-                        break;
-                    }
-                    if (TRACE) SLOG[steps] = e;  // the trace hash runs over every committed pop
-                    uint32_t sp = 0, sbytes = 0;
-                    bool cont = false;
-                    Ent child{0, 0};
-                    const int i0 = e_i(e), mm = e_mm(e), go = e_go(e), ge = e_ge(e), st = e_st(e), ins = e_ins(e);
-                    int m = max_diff - (mm + go);
-                    if (mode & MODE_GAPE) m -= ge;
-                    if (m >= 0) {
-                        int m_seed = 0;
-                        if (seeding) {
-                            m_seed = msd - (mm + go);
-                            if (mode & MODE_GAPE) m_seed -= ge;
-                        }
-                        if (i0 == 0) {
-                            kind = K_HIT;
-                            hk = e_k(e);
-                            hl = e_l(e);
+            // the buckets that pushes go to and their log codes: 0 a mismatch, 1 a gap open, 2 a gap
+            // extension, or the lower code of the same bucket (one log, so that its order is kept)
+            const int tg0 = b + s_mm, tg1 = b + s_gapo, tg2 = b + s_gape;
+            const int sh1 = s_gapo == s_mm ? 0 : 8, sh2 = s_gape == s_mm ? 0 : s_gape == s_gapo ? 8 : 16;
+            // differences still allowed to a chain (constant along it)
+            auto left = [&](int lim, uint32_t x, uint32_t y) __attribute__((always_inline)) {
+                return lim - x_mm(x) - x_go(x) - ((mode & MODE_GAPE) ? y_ge(y) : 0);
+            };
+            // ---- chain heads, from the top of bucket b; those that cannot go on end here. Wave w loads
+            // heads w * 64 * CPL on; the live ones are listed in order ----
+            {
+                const uint32_t top = hp ? 0u : 1u;  // head c is entry seg_cnt - top - c + ... of the top segment
+                uint64_t lm[CPL];
+                int cnt = 0;
+                Item<WIDE> h[CPL];
+#pragma unroll
+                for (int r = 0; r < CPL; ++r) {
+                    const int c = (wave * CPL + r) * HW + lane;
+                    if (c < nK) {
+                        if (c == 0 && hp) {
+                            h[r].k = (K)F.hk;
+                            h[r].l = (K)F.hl;
+                            h[r].x = F.hx;
+                            h[r].y = F.hy;
                         } else {
-                            const uint64_t wB = W[i0 - 1], wA = i0 >= 2 ? W[i0 - 2] : 0;
-                            const int qbase = q[i0 - 1];
-                            uint64_t ca[4], cb[4];
-                            const uint32_t lfb = lf_pair(a.bwt, M, e_k(e) - 1, e_l(e), ca, cb);
-                            if (m < wbid(wB)) {
-                                // pruned
-                            } else if (m == 0 && (st == ST_M || (mode & MODE_GAPE) || ge == max_gape)) {
-                                // exact tail: bwt_match_exact_alt, src/bwtgap_hd.h:195-211
-                                if (qbase <= 3) {
-                                    sbytes += lfb;
-                                    uint64_t k = L2s[qbase] + ca[qbase] + 1, l = L2s[qbase] + cb[qbase];
-                                    bool ok = k <= l;
-                                    for (int jn = i0 - 2; ok && jn >= 0; --jn) {
-                                        const int c = q[jn];
-                                        if (c > 3) {
-                                            ok = false;
-                                            break;
-                                        }
-                                        uint64_t oa, ob;
-                                        sbytes += lf_one(a.bwt, M, k - 1, l, c, oa, ob);
-                                        k = L2s[c] + oa + 1;
-                                        l = L2s[c] + ob;
-                                        ok = k <= l;
-                                    }
-                                    if (ok && (int)(uint32_t)(l - k + 1) != 0) {
-                                        kind = K_HIT;
-                                        hk = k;
-                                        hl = l;
-                                    }
-                                }
-                            } else {
-                                // expansion: src/bwtgap_hd.h:412-470
-                                sbytes += lfb;
-                                const int i = i0 - 1;
-                                const uint64_t k = e_k(e), l = e_l(e), occ = l - k + 1;
-                                bool allow_diff = true, allow_M = true;
-                                if (i > 0) {
-                                    if (wbid(wA) > m - 1)
-                                        allow_diff = false;
-                                    else if (wbid(wA) == m - 1 && wbid(wB) == m - 1 && wval(wA) == wval(wB))
-                                        allow_M = false;
-                                    if (seeding) {
-                                        const int ii = i - (len - seed_len);
-                                        if (ii > 0) {
-                                            const uint64_t sA = SW[ii - 1], sB = SW[ii];
-                                            if (wbid(sA) > m_seed - 1)
-                                                allow_diff = false;
-                                            else if (wbid(sA) == m_seed - 1 && wbid(sB) == m_seed - 1 && wval(sA) == wval(sB))
-                                                allow_M = false;
-                                        }
-                                    }
-                                }
-                                const int tmp = (mode & MODE_LOGGAP) ? int_log2((uint32_t)(ge + go)) / 2 + 1 : go + ge;
-                                // the children's intervals per base
-                                uint64_t KK[4], LL[4];
+                            h[r] = get_item<WIDE>(POOL + seg_base[b] + seg_cnt[b] - top - (uint32_t)c);
+                        }
+                    }
+                }
 #pragma unroll
-                                for (int j = 0; j < 4; ++j) {
-                                    KK[j] = L2s[j] + ca[j] + 1;
-                                    LL[j] = L2s[j] + cb[j];
-                                }
-                                auto logp = [&](int s, const Ent &en) __attribute__((always_inline)) {
-                                    if (kind != K_END) return;
-                                    if (s < 0 || s >= n_stacks) {
-                                        kind = K_ESCORE;
-                                        return;
-                                    }
-                                    PLOG[np] = en;
-                                    // its bucket as the commit numbers them: 0 b+s_mm, 1 b+s_gapo,
-                                    // 2 b+s_gape, 3 none of them (not possible with positive penalties)
-                                    const int d = s - b;
-                                    const int code = d == s_mm ? 0 : d == s_gapo ? 1 : d == s_gape ? 2 : 3;
-                                    ccnt += 1u << (8 * code);  // at most H_PUSH of each
-                                    ++np;
-                                    ++sp;
-                                };
-                                if (allow_diff && i >= ies + tmp && len - i >= ies + tmp) {
-                                    if (st == ST_M) {
-                                        if (go < max_gapo) {
-                                            const int sc = mm * s_mm + (go + 1) * s_gapo + ge * s_gape;
-                                            logp(sc, mk_ent(k, l, i, i, mm, go + 1, ge, ins + 1, ST_I));
-                                            for (int j = 0; j < 4; ++j)
-                                                if (KK[j] <= LL[j]) logp(sc, mk_ent(KK[j], LL[j], i + 1, i + 1, mm, go + 1, ge, ins, ST_D));
-                                        }
-                                    } else if (st == ST_I) {
-                                        if (ge < max_gape)
-                                            logp(mm * s_mm + go * s_gapo + (ge + 1) * s_gape,
-                                                 mk_ent(k, l, i, i, mm, go, ge + 1, ins + 1, ST_I));
-                                    } else {
-                                        if (ge < max_gape && (ge + go < max_diff || occ < (uint64_t)(int64_t)mdo)) {
-                                            const int sc = mm * s_mm + go * s_gapo + (ge + 1) * s_gape;
-                                            for (int j = 0; j < 4; ++j)
-                                                if (KK[j] <= LL[j]) logp(sc, mk_ent(KK[j], LL[j], i + 1, i + 1, mm, go, ge + 1, ins, ST_D));
-                                        }
-                                    }
-                                }
-                                // the intervals rotated so that slot t holds base (qbase + t) & 3, the
-                                // order of the mismatch loop (the deletions above are done with them)
-                                uint64_t RK[4], RL[4];
-                                {
-                                    const bool r1 = (qbase & 1) != 0, r2 = (qbase & 2) != 0;
-                                    uint64_t TK[4], TL[4];
+                for (int r = 0; r < CPL; ++r) {
+                    const int c = (wave * CPL + r) * HW + lane;
+                    bool live = c < nK;
+                    if (!TRACE && live) {
+                        const int m = left(max_diff, h[r].x, h[r].y);
+                        const uint32_t i0 = h[r].x & X_I;
+                        if (m < 0 || (i0 > 0 && m < (int)lw_bid<WIDE>(Wp[i0]))) {
+                            live = false;
+                            cA[c] = 0;
+                            cB[c] = 0;
+                            cC[c] = 1;  // one pop, no lookup
+                            if (c == 0) s0info[0] = 0;
+                        }
+                    }
+                    lm[r] = __ballot(live);
+                    cnt += __builtin_popcountll(lm[r]);
+                }
+                int at = 0;
+                if (NW > 1) {
+                    if (lane == 0) F.wlive[wave] = cnt;
+                    __syncthreads();
+                    for (int w = 0; w < wave; ++w) at += F.wlive[w];
+                }
 #pragma unroll
-                                    for (int t = 0; t < 4; ++t) {
-                                        TK[t] = r1 ? KK[(t + 1) & 3] : KK[t];
-                                        TL[t] = r1 ? LL[(t + 1) & 3] : LL[t];
-                                    }
+                for (int r = 0; r < CPL; ++r) {
+                    const int c = (wave * CPL + r) * HW + lane;
+                    if ((lm[r] >> lane) & 1ull) {
+                        const int p = at + lanes_below(lm[r]);
+                        put_item<WIDE>(hent + p, h[r].k, h[r].l, h[r].x, h[r].y);
+                        hcid[p] = (uint16_t)c;
+                    }
+                    at += __builtin_popcountll(lm[r]);
+                }
+                if (NW == 1 && lane == 0) F.wlive[0] = cnt;
+            }
+            __syncthreads();
+            int nlive = 0;
 #pragma unroll
-                                    for (int t = 0; t < 4; ++t) {
-                                        RK[t] = r2 ? TK[(t + 2) & 3] : TK[t];
-                                        RL[t] = r2 ? TL[(t + 2) & 3] : TL[t];
-                                    }
-                                }
-                                if (allow_diff && allow_M) {
-                                    for (int j = 1; j <= 4; ++j) {
-                                        // base (qbase + j) & 3: slot j & 3 of the rotated intervals
-                                        const int is_mm = (j != 4 || qbase > 3);
-                                        const uint64_t kk = RK[j & 3], ll = RL[j & 3];
-                                        if (kk > ll) continue;
-                                        if (is_mm) {
-                                            logp((mm + 1) * s_mm + go * s_gapo + ge * s_gape,
-                                                 mk_ent(kk, ll, i, i, mm + 1, go, ge, ins, ST_M));
-                                        } else if (kind == K_END) {
-                                            child = mk_ent(kk, ll, i, 0, mm, go, ge, ins, ST_M);
-                                            cont = true;
-                                        }
-                                    }
-                                } else if (qbase < 4) {
-                                    const uint64_t kk = RK[0], ll = RL[0];  // base qbase
-                                    if (kk <= ll && kind == K_END) {
-                                        child = mk_ent(kk, ll, i, 0, mm, go, ge, ins, ST_M);
-                                        cont = true;
-                                    }
-                                }
+            for (int w = 0; w < NW; ++w) nlive += F.wlive[w];
+            // ---- speculation: every thread runs chains, one lookup an iteration, and takes the next live
+            // one when its own has ended ----
+            int next = T, stop = 0x7fffffff, its = 0;  // (NW > 1: the claims and the stop are F.next, F.stop)
+            uint32_t np3 = 0, o3 = 0;                  // logged pushes by code, 8 bits each; at the chain's start
+            int cid = -1, kind = K_END, steps = 0, m = 0, m_seed = 0, so = 0, sl = 0;
+            uint32_t sby = 0, sp = 0, spb = 0;  // index bytes / 64 of the chain; pushes, bytes of its last pop
+            bool busy = false, fin = false, tail = false;
+            K k = 0, l = 0;
+            uint32_t x = 0, y = 0;
+            constexpr uint32_t ROOM = 0x010101u * (uint32_t)(127 - (H_LOG - H_SPUSH));  // sets bit 7 of a full log's count
+            bool first = true;
+            for (;;) {
+                const bool want = !busy && !fin && ((np3 + ROOM) & 0x808080u) == 0 && (!TRACE || sl <= H_SLOG - H_STEPS);
+                if (!busy && !want) fin = true;
+                const uint64_t wm = __ballot(want);
+                if (wm) {
+                    int p;
+                    if (first) {
+                        p = tid;
+                    } else if (NW == 1) {
+                        p = next + lanes_below(wm);
+                        next += __builtin_popcountll(wm);
+                    } else {
+                        int g = 0;
+                        const int leader = __builtin_ctzll(wm);
+                        if (lane == leader) g = atomicAdd(&F.next, __builtin_popcountll(wm));
+                        p = __shfl(g, leader) + lanes_below(wm);
+                    }
+                    if (want) {
+                        fin = true;
+                        if (p < nlive) {
+                            const int c = hcid[p];
+                            if (c < (NW == 1 ? stop : __hip_atomic_load(&F.stop, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_WORKGROUP))) {
+                                const Item<WIDE> e = get_item<WIDE>(hent + p);
+                                fin = false;
+                                busy = true;
+                                tail = false;
+                                cid = c;
+                                k = e.k;
+                                l = e.l;
+                                x = e.x;
+                                y = e.y;
+                                m = left(max_diff, x, y);
+                                m_seed = left(msd, x, y);
+                                steps = 0;
+                                sby = 0;
+                                o3 = np3;
+                                so = sl;
                             }
                         }
                     }
-                    if (!TRACE && (kind == K_HIT || kind == K_ESCORE)) SLOG[steps] = e;  // read by the commit
-                    SINFO[steps] = (uint16_t)(sp | (sbytes >> 6) << 4);
-                    sby += sbytes;
-                    ++steps;
-                    if (kind != K_END || !cont) break;
-                    e = child;
                 }
-            }
-            // ---- commit plan, by wave-wide scans over the chains ----
-            if (lane >= K) {
-                steps = 0;
-                np = 0;
-                sby = 0;
-                kind = K_END;
+                first = false;
+                if (!__ballot(busy)) break;
+                ++its;
+                bool ended = false;
+                if (busy) {
+                    const uint32_t i0 = x & X_I;
+                    uint64_t wB = 0;
+                    if (!tail) {
+                        // a pop
+                        if (TRACE) {
+                            put_item<WIDE>(SLOG + tid * H_SLOG + sl, k, l, x, y);
+                            ++sl;
+                        }
+                        ++steps;
+                        sp = 0;
+                        spb = 0;
+                        wB = Wp[i0];
+                        if (i0 == 0 && m >= 0) {
+                            ended = true;
+                            kind = K_HIT;
+                        } else if (m < 0 || m < (int)lw_bid<WIDE>(wB)) {
+                            ended = true;  // pruned
+                        } else if (m == 0 && ((x & X_ST) == 0 || (mode & MODE_GAPE) || y_ge(y) == max_gape)) {
+                            tail = true;
+                        }
+                    }
+                    if (!ended) {
+                        const uint32_t qb = QL[i0 - 1];
+                        const K Pk = pos_k<K>(M, k), Pl = pos_l<K>(M, l);
+                        OccWord A, B;
+                        occ_load<K>(a.bwt, Pk, A);
+                        occ_load<K>(a.bwt, Pl, B);
+                        const uint64_t wA = Wp[i0 - 1];
+                        const uint32_t units = occ_units<K>(Pk, Pl);
+                        K ca[4], cb[4];
+                        occ_count<K>(M, WIDE, A, Pk, ca);
+                        occ_count<K>(M, WIDE, B, Pl, cb);
+                        if (tail) {
+                            // exact tail: bwt_match_exact_alt, src/bwtgap_hd.h:195-211
+                            ended = true;
+                            if (qb <= 3) {
+                                spb += units;
+                                const K kk = pick4(ca, (int)qb) + 1, ll = pick4(cb, (int)qb);
+                                if (kk <= ll) {
+                                    k = kk;
+                                    l = ll;
+                                    x -= 1;
+                                    if (i0 > 1)
+                                        ended = false;
+                                    else if ((uint32_t)(ll - kk + 1) != 0)
+                                        kind = K_HIT;
+                                }
+                            }
+                        } else {
+                            // expansion: src/bwtgap_hd.h:412-470
+                            spb = units;
+                            const int i = (int)i0 - 1;
+                            bool allow_diff = true, allow_M = true;
+                            if (i > 0) {
+                                const int bA = (int)lw_bid<WIDE>(wA);
+                                if (bA > m - 1)
+                                    allow_diff = false;
+                                else if (bA == m - 1 && wA == wB)
+                                    allow_M = false;
+                                if (seeding) {
+                                    const int ii = i - sofs;
+                                    if (ii > 0) {
+                                        const uint64_t sA = SW[ii - 1], sB = SW[ii];
+                                        const int b_s = (int)lw_bid<WIDE>(sA);
+                                        if (b_s > m_seed - 1)
+                                            allow_diff = false;
+                                        else if (b_s == m_seed - 1 && sA == sB)
+                                            allow_M = false;
+                                    }
+                                }
+                            }
+                            const int ge = y_ge(y), go = x_go(x);
+                            const uint32_t st = x & X_ST, xb = x & ~X_ST, yb = y & ~Y_LDP;
+                            if (allow_diff) {
+                                const int tmp = (mode & MODE_LOGGAP) ? int_log2((uint32_t)(ge + go)) / 2 + 1 : go + ge;
+                                if (i >= ies + tmp && len - i >= ies + tmp) {
+                                    // gap children: opened by an entry that ends in a match, or extended
+                                    const bool open = st == 0;
+                                    const bool may = open ? go < max_gapo : ge < max_gape;
+                                    const bool ins = may && st != X_DEL;
+                                    const bool del = may && st != X_INS &&
+                                                     (open || ge + go < max_diff || (uint64_t)(K)(l - k + 1) < (uint64_t)(int64_t)mdo);
+                                    const uint32_t dm = !del ? 0u
+                                                             : (ca[0] < cb[0] ? 1u : 0u) | (ca[1] < cb[1] ? 2u : 0u) |
+                                                                   (ca[2] < cb[2] ? 4u : 0u) | (ca[3] < cb[3] ? 8u : 0u);
+                                    if (ins || dm) {
+                                        const int tg = open ? tg1 : tg2, sh = open ? sh1 : sh2;
+                                        if (tg < 0 || tg >= n_stacks) {
+                                            kind = K_ESCORE;
+                                        } else {
+                                            Ent *d = LOG + ((sh >> 3) * T + tid) * H_LOG + ((np3 >> sh) & 127u);
+                                            const uint32_t xg = xb + (open ? X_GO : 0u), yg = yb + (open ? 0u : Y_GE);
+                                            if (ins) put_item<WIDE>(d++, k, l, (xg - 1) | X_INS, (yg + Y_IN) | (uint32_t)i);
+#pragma unroll
+                                            for (int j = 0; j < 4; ++j)
+                                                if (dm >> j & 1u) put_item<WIDE>(d++, ca[j] + 1, cb[j], xg | X_DEL, yg | i0);
+                                            const uint32_t n = (ins ? 1u : 0u) + __builtin_popcount(dm);
+                                            np3 += n << sh;
+                                            sp += n;
+                                        }
+                                    }
+                                }
+                            }
+                            ended = true;
+                            if (kind == K_END) {
+                                // the intervals rotated so that slot t holds base (qb + t) & 3, the order of the
+                                // mismatch loop
+                                const bool r1 = (qb & 1u) != 0, r2 = (qb & 2u) != 0;
+                                K RK[4], RL[4], TK[4], TL[4];
+#pragma unroll
+                                for (int t = 0; t < 4; ++t) {
+                                    TK[t] = r1 ? ca[(t + 1) & 3] : ca[t];
+                                    TL[t] = r1 ? cb[(t + 1) & 3] : cb[t];
+                                }
+#pragma unroll
+                                for (int t = 0; t < 4; ++t) {
+                                    RK[t] = r2 ? TK[(t + 2) & 3] : TK[t];
+                                    RL[t] = r2 ? TL[(t + 2) & 3] : TL[t];
+                                }
+                                const bool x0 = RK[0] < RL[0];
+                                if (allow_diff && allow_M) {
+                                    // mismatches: the other bases in order, and all four of them at an N
+                                    const uint32_t mmk = (RK[1] < RL[1] ? 1u : 0u) | (RK[2] < RL[2] ? 2u : 0u) |
+                                                         (RK[3] < RL[3] ? 4u : 0u) | (qb > 3 && x0 ? 8u : 0u);
+                                    if (mmk) {
+                                        if (tg0 < 0 || tg0 >= n_stacks) {
+                                            kind = K_ESCORE;
+                                        } else {
+                                            Ent *d = LOG + tid * H_LOG + (np3 & 127u);
+                                            const uint32_t xm = xb - 1 + X_MM, ym = yb | (uint32_t)i;
+#pragma unroll
+                                            for (int t = 1; t <= 4; ++t)
+                                                if (mmk >> (t - 1) & 1u) put_item<WIDE>(d++, RK[t & 3] + 1, RL[t & 3], xm, ym);
+                                            const uint32_t n = __builtin_popcount(mmk);
+                                            np3 += n;
+                                            sp += n;
+                                        }
+                                    }
+                                }
+                                if (kind == K_END && qb <= 3 && x0) {
+                                    // the exact child, popped next
+                                    k = RK[0] + 1;
+                                    l = RL[0];
+                                    x = xb - 1;
+                                    y = yb;
+                                    ended = false;
+                                    if (steps == H_STEPS || ((np3 + ROOM) & 0x808080u) != 0) {
+                                        ended = true;
+                                        kind = K_TRUNC;  // it goes on in the next round
+                                    }
+                                }
+                            }
+                            sby += spb;
+                        }
+                    }
+                    if (tail && ended) sby += spb;
+                    if (cid == 0) s0info[steps - 1] = (uint16_t)(sp | spb << 4);
+                    if (TRACE) SINFO[tid * H_SLOG + sl - 1] = (uint8_t)sp;
+                    if (ended) {
+                        cA[cid] = (np3 - o3) | (uint32_t)kind << 24;
+                        cB[cid] = o3 | (uint32_t)tid << 24;
+                        cC[cid] = (uint32_t)steps | sby << 6;
+                        if (TRACE) cS[cid] = (uint16_t)so;
+                        busy = false;
+                        if (kind != K_END) fin = true;  // what it stopped with stays in its registers
+                    }
+                }
+                // the first chain that stops (a hit, a truncation, a score error): those after it run again
+                // in the next round
+                const uint64_t sm = __ballot(ended && kind != K_END);
+                if (sm) {
+                    if (NW == 1) {
+                        for (uint64_t t = sm; t; t &= t - 1) stop = min(stop, __builtin_amdgcn_readlane(cid, __builtin_ctzll(t)));
+                    } else if (ended && kind != K_END) {
+                        atomicMin(&F.stop, cid);
+                    }
+                }
+                if (busy && cid > (NW == 1 ? stop : __hip_atomic_load(&F.stop, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_WORKGROUP))) {
+                    busy = false;
+                    fin = true;
+                }
             }
             const long long t_commit = a.stats ? wall_clock64() : 0;
-            // J: the first chain that stops (a hit, a truncation, a score error); the chains after
-            // it are re-run in the next round
-            const uint64_t stopm = __ballot(kind != K_END);
-            const int J = stopm ? __builtin_ctzll(stopm) : K - 1;
-            const bool inJ = lane <= J;
-            const int pex = wave_excl_scan(inJ ? np : 0);  // pushes of the chains before this one
-            // entries before this chain's first pop: each chain pops its head, pushes its logged
-            // children and, when truncated, leaves its next exact child pending
-            const int nstart = F.n_entries + wave_excl_scan(inJ ? np - 1 + (kind == K_TRUNC ? 1 : 0) : 0);
-            // the push cap falls in chain jcap, which waits for the next round with the chains
-            // after it (chain 0 always fits: a chain logs at most H_PUSH pushes)
-            const uint64_t capm = __ballot(inJ && pex + np > a.push_cap);
-            const int jcap = capm ? max(1, __builtin_ctzll(capm)) : J + 1;
-            const bool cand = inJ && lane < jcap;
-            int c = 0, cut = -1;
-            if (cand) {
-                c = steps;
-                // the max_entries check before each pop (src/bwtgap_hd.h:360): the entries before a
-                // pop are nstart plus the chain's earlier pushes, so only a chain whose pushes could
-                // cross the limit is walked
-                if ((long)nstart + np > F.max_entries) {
-                    long nb = nstart;
-                    for (int t = 0; t < c; ++t) {
+            __syncthreads();
+            // ---- commit plan, by scans over the chains (thread t: chains t * CPL on) ----
+            if (NW > 1) {
+                next = F.next;
+                stop = F.stop;
+            }
+            const int run = next < nlive ? (int)hcid[next] : nK;  // chains before the first one not taken
+            const int J = min(stop, run - 1);
+            uint32_t v01[CPL], v2s[CPL], vb[CPL];
+            uint32_t s01 = 0, s2s = 0, sb = 0;
+#pragma unroll
+            for (int r = 0; r < CPL; ++r) {
+                const int c = tid * CPL + r;
+                const bool in = c <= J;
+                const uint32_t A = in ? cA[c] : 0u, C = in ? cC[c] : 0u;
+                v01[r] = (A & 255u) | ((A >> 8) & 255u) << 16;
+                v2s[r] = ((A >> 16) & 255u) | (C & 63u) << 16;
+                vb[r] = C >> 6;
+                s01 += v01[r];
+                s2s += v2s[r];
+                sb += vb[r];
+            }
+            uint32_t e01 = wave_incl_scan(s01), e2s = wave_incl_scan(s2s), eb = wave_incl_scan(sb);
+            if (NW > 1) {
+                if (lane == HW - 1) {
+                    F.wsum[0][wave] = e01;
+                    F.wsum[1][wave] = e2s;
+                    F.wsum[2][wave] = eb;
+                }
+                __syncthreads();
+                for (int w = 0; w < wave; ++w) {
+                    e01 += F.wsum[0][w];
+                    e2s += F.wsum[1][w];
+                    eb += F.wsum[2][w];
+                }
+            }
+            e01 -= s01;
+            e2s -= s2s;
+            eb -= sb;
+            // pushes before each chain by code (over the heads, which are not needed any more), and the first
+            // chain that must wait for the next round: the push cap falls in it (chain 0 always fits), or
+            // the max_entries check before a pop could (src/bwtgap_hd.h:360); chain 0 is walked step by step
+            {
+                uint32_t p01 = e01, p2s = e2s;
+                int wait = 0x7fffffff;
+                bool walk0 = false;
+#pragma unroll
+                for (int r = 0; r < CPL; ++r) {
+                    const int c = tid * CPL + r;
+                    if (c <= J) {
+                        epre[c] = (uint16_t)p01;
+                        epre[KMAX + c] = (uint16_t)(p01 >> 16);
+                        epre[2 * KMAX + c] = (uint16_t)p2s;
+                        const int pex = (int)((p01 & 0xffffu) + (p01 >> 16) + (p2s & 0xffffu));
+                        const int np = (int)((v01[r] & 0xffffu) + (v01[r] >> 16) + (v2s[r] & 0xffffu));
+                        // each chain before this one popped its head and left its pushes
+                        const bool over = (long)F.n_entries + pex - c + np > (long)F.max_entries;
+                        if (c == 0)
+                            walk0 = over;
+                        else if ((over || pex + np > a.push_cap) && wait == 0x7fffffff)
+                            wait = c;
+                        p01 += v01[r];
+                        p2s += v2s[r];
+                    }
+                }
+                if (wait != 0x7fffffff) atomicMin(&F.lim, wait);
+                if (walk0) {
+                    const int s0 = (int)(cC[0] & 63u);
+                    long nb = F.n_entries;
+                    unsigned long long by = 0;
+                    for (int t = 0; t < s0; ++t) {
                         if (nb > F.max_entries) {
-                            cut = t;
+                            F.cut = t;
                             break;
                         }
-                        nb += SINFO[t] & 0xf;
+                        nb += s0info[t] & 15;
+                        by += s0info[t] >> 4;
+                    }
+                    if (F.cut >= 0) {
+                        // the search stops inside chain 0
+                        F.pops += (unsigned long long)F.cut;
+                        F.obytes += by << 6;
+                        F.status = 1;
+                        F.result = F.n_aln;
+                    } else {
+                        atomicMin(&F.lim, 1);
                     }
                 }
-                if (c > 0 && c == steps && (kind == K_HIT || kind == K_ESCORE)) {
-                    F.hk = hk;
-                    F.hl = hl;
-                    F.he = SLOG[steps - 1];
+            }
+            __syncthreads();
+            const int last = min(J, F.lim - 1);  // chains 0..last commit
+            if (TRACE && tid == 0) {
+                // the trace hash runs over the committed pops in order
+                uint64_t tr = F.trace;
+                int nb = F.n_entries;
+                const int cut = F.cut;
+                for (int j = 0; j <= (cut >= 0 ? 0 : last); ++j) {
+                    const int t0 = (int)(cB[j] >> 24) * H_SLOG + (int)cS[j], n = cut >= 0 ? cut : (int)(cC[j] & 63u);
+                    for (int t = 0; t < n; ++t) {
+                        const Item<WIDE> e = get_item<WIDE>(SLOG + t0 + t);
+                        nb -= 1;
+                        tr = trace_item(tr, b, e.k, e.l, e.x, e.y, nb);
+                        nb += (int)SINFO[t0 + t] + (t + 1 < n ? 1 : 0);  // its pushes, and its exact child
+                    }
                 }
-                if (c > 0 && c == steps && kind == K_TRUNC) F.pend = nxt;
+                F.trace = tr;
             }
-            // the search stops inside chain jcut (max_entries); otherwise chains 0..last commit
-            const uint64_t cutm = __ballot(cand && cut >= 0);
-            const int jcut = cutm ? __builtin_ctzll(cutm) : -1;
-            const uint64_t posm = __ballot(cand && c > 0);
-            const int last = jcut >= 0 ? jcut : (posm ? 63 - __builtin_clzll(posm) : -1);
-            const int cj = lane <= last ? (lane == jcut ? cut : c) : 0;  // committed steps of this chain
-            int ncp = 0;  // committed pushes of this chain
-            uint64_t by = 0;
-            if (cj == steps) {  // the whole chain
-                ncp = np;
-                by = sby;
-            } else {
-                for (int t = 0; t < cj; ++t) {
-                    by += (uint64_t)(SINFO[t] >> 4) << 6;
-                    ncp += SINFO[t] & 0xf;
-                }
+            if (F.status) break;
+            if (last / CPL == tid) {
+                uint32_t p01 = e01, p2s = e2s, pb = eb;
+#pragma unroll
+                for (int r = 0; r < CPL; ++r)
+                    if (tid * CPL + r <= last) {
+                        p01 += v01[r];
+                        p2s += v2s[r];
+                        pb += vb[r];
+                    }
+                F.tot01 = p01;
+                F.tot2s = p2s;
+                F.totb = pb;
             }
-            // pops and entry changes in one sum: pops in bits 0-31, entry change + 1 (>= 0) above
-            const unsigned long long pe_sum =
-                wave_sum_u64((unsigned long long)cj | (unsigned long long)(cj > 0 ? ncp : 1) << 32);
-            const unsigned long long sum_pops = pe_sum & 0xffffffffull, sum_by = wave_sum_u64(by);
-            const int sum_ne = (int)(pe_sum >> 32) - HW;
-            if (TRACE) {
-                lcommit[lane] = cj;
-                lnstart[lane] = nstart;
+            if (kind != K_END && cid == last) {
+                F.l_kind = kind;
+                F.hk = k;
+                F.hl = l;
+                F.hx = x;
+                F.hy = y;
             }
-            // a committed chain commits whole (a cut at max_entries ends the search instead)
-            if (lane == last) F.l_full = kind;
             __syncthreads();
             const long long t_c1 = a.stats ? wall_clock64() : 0;
-            if (lane == 0) {
-                if (TRACE) {
-                    // the trace hash runs over the committed pops in order
-                    uint64_t tr = F.trace;
-                    for (int j = 0; j <= last; ++j) {
-                        long nb = lnstart[j];
-                        for (int t = 0; t < lcommit[j]; ++t) {
-                            const uint32_t info = SINFO_ALL[j * H_STEPS + t];
-                            nb -= 1;
-                            const Ent e = SLOG_ALL[j * H_STEPS + t];
-                            const int i0 = e_i(e), mm = e_mm(e), go = e_go(e), ge = e_ge(e), st = e_st(e), ins = e_ins(e);
-                            tr = tr_mix(tr, (uint64_t)((uint32_t)b << 21 | (uint32_t)i0));
-                            tr = tr_mix(tr, e_k(e));
-                            tr = tr_mix(tr, e_l(e));
-                            tr = tr_mix(tr, (uint64_t)((uint32_t)mm | (uint32_t)go << 8 | (uint32_t)ge << 16 | (uint32_t)st << 24));
-                            tr = tr_mix(tr, (uint64_t)ins | (uint64_t)(go + ge - ins) << 16);
-                            tr = tr_mix(tr, (uint64_t)(uint32_t)e_ldp(e));
-                            tr = tr_mix(tr, (uint64_t)(uint32_t)nb);
-                            nb += (info & 0xf) + 1;  // its pushes, and its exact child (popped next, if any)
-                        }
-                    }
-                    F.trace = tr;
-                }
-                F.pops += sum_pops;
-                F.obytes += sum_by;
-                if (jcut >= 0) {
-                    F.status = 1;
-                    F.result = F.n_aln;
-                }
-            }
-            __syncthreads();
-            if (F.status) break;
-            // ---- pushes: a committed push goes to bucket b + s_mm, b + s_gapo or b + s_gape
-            // (a mismatch, a gap open, a gap extension); its rank in the bucket is its place in
-            // the sequential push order, chain by chain ----
-            const int tg0 = b + s_mm, tg1 = b + s_gapo, tg2 = b + s_gape;
-            // pushes per bucket, counted while the log was written: a round commits a chain whole,
-            // or ends the search (max_entries) before its pushes are placed
-            const uint32_t cc = ncp > 0 ? ccnt : 0u;
-            const int n0 = (int)(cc & 0xff), n1 = (int)((cc >> 8) & 0xff), n2 = (int)((cc >> 16) & 0xff);
-            const bool bad = (cc >> 24) != 0 || (ncp != 0 && ncp != np);
-            // the three totals in one sum (16-bit fields: a round commits at most H_CAP pushes)
-            const unsigned long long tsum =
-                wave_sum_u64((unsigned long long)n0 | (unsigned long long)n1 << 16 | (unsigned long long)n2 << 32);
-            const int T0 = (int)(tsum & 0xffff), T1 = (int)((tsum >> 16) & 0xffff), T2 = (int)((tsum >> 32) & 0xffff);
-            const bool badw = __ballot(bad) != 0;
-            if (lane == 0) {
-                // pieces of the wave's current granule for each bucket that receives pushes; a
+            const uint32_t tot01 = F.tot01, tot2s = F.tot2s;
+            const int T0 = (int)(tot01 & 0xffffu), T1 = (int)(tot01 >> 16), T2 = (int)(tot2s & 0xffffu);
+            if (tid == 0) {
+                // pieces of the workgroup's current granule for each bucket that receives pushes; a
                 // bucket's new piece links to its previous top segment
                 int np_ = 0;
                 bool oom = false;
-                for (int x = 0; x < 3 && !oom && !badw; ++x) {
-                    // (selects: arrays indexed by x would live in scratch memory)
-                    const int sb = x == 0 ? tg0 : x == 1 ? tg1 : tg2;
-                    uint32_t rem = (uint32_t)(x == 0 ? T0 : x == 1 ? T1 : T2);
+                uint32_t abase = F.abase;
+                int aleft = F.aleft;
+                for (int c = 0; c < 3 && !oom; ++c) {
+                    // (selects: arrays indexed by c would live in scratch memory)
+                    const int sbk = c == 0 ? tg0 : c == 1 ? tg1 : tg2;
+                    uint32_t rem = (uint32_t)(c == 0 ? T0 : c == 1 ? T1 : T2);
                     if (!rem) continue;
-                    const bool bit = (F.bm[sb >> 6] >> (sb & 63)) & 1ull;
-                    uint32_t prev_base = bit ? seg_base[sb] : NIL, prev_size = bit ? seg_cnt[sb] : 0u, rk = 0;
-                    first_piece[sb] = np_;
+                    const bool bit = (F.bm[sbk >> 6] >> (sbk & 63)) & 1ull;
+                    uint32_t prev_base = bit ? seg_base[sbk] : NIL, prev_size = bit ? seg_cnt[sbk] : 0u, rk = 0;
+                    F.fp[c] = np_;
                     while (rem > 0) {
-                        if (F.aleft < 2) {
+                        if (aleft < 2) {
                             uint32_t g;
                             if (F.n_used < F.n_own) {
                                 g = OWN[F.n_used];
@@ -1944,109 +2183,81 @@ __global__ void __launch_bounds__(64) __attribute__((amdgpu_waves_per_eu(WPE))) 
                                 OWN[F.n_own++] = g;
                             }
                             ++F.n_used;
-                            F.abase = g * GENT;
-                            F.aleft = (int)GENT;
+                            abase = g * GENT;
+                            aleft = (int)GENT;
                         }
-                        const uint32_t plen = min(rem, (uint32_t)F.aleft - 1);
+                        if (np_ == H_PIECES) {  // (not possible: the push cap spans fewer pieces)
+                            oom = true;
+                            break;
+                        }
+                        const uint32_t plen = min(rem, (uint32_t)aleft - 1);
                         Ent hdr;
                         hdr.w0 = (uint64_t)prev_base | (uint64_t)prev_size << 32;
                         hdr.w1 = 0;
-                        POOL[F.abase] = hdr;
-                        pieces[np_++] = make_uint4((uint32_t)sb, rk, plen, F.abase + 1);
-                        prev_base = F.abase + 1;
+                        POOL[abase] = hdr;
+                        pieces[np_++] = make_uint4((uint32_t)c, rk, plen, abase + 1);
+                        prev_base = abase + 1;
                         prev_size = plen;
-                        F.abase += plen + 1;
-                        F.aleft -= (int)plen + 1;
+                        abase += plen + 1;
+                        aleft -= (int)plen + 1;
                         rem -= plen;
                         rk += plen;
                     }
-                    seg_base[sb] = prev_base;
-                    seg_cnt[sb] = prev_size;
-                    F.bm[sb >> 6] |= 1ull << (sb & 63);
+                    seg_base[sbk] = prev_base;
+                    seg_cnt[sbk] = prev_size;
+                    F.bm[sbk >> 6] |= 1ull << (sbk & 63);
                 }
+                F.abase = abase;
+                F.aleft = aleft;
                 F.n_piece = np_;
-                if (badw) {  // a push outside the three buckets: not possible with positive penalties
-                    F.status = 1;
-                    F.result = ERR_INTERNAL;
-                } else if (oom) {
+                if (oom) {
                     F.status = 1;
                     F.result = ERR_STACK;
                 }
+                F.pops += tot2s >> 16;
+                F.obytes += (unsigned long long)F.totb << 6;
             }
             __syncthreads();
             if (F.status) break;
             const long long t_c2 = a.stats ? wall_clock64() : 0;
+            // ---- placement: a bucket's push g of the round comes from the last chain with at most g pushes
+            // to the bucket before it, at its place in that chain's log ----
             {
                 const int npieces = F.n_piece;
-                const Ent *const PLOG_W = reinterpret_cast<const Ent *>(base + a.plog_off);  // lane j's log at j * H_PUSH
-                bool bad_piece = false;
-                // rank R of bucket tg's pushes this round to its pool slot, within this round's pieces
-                auto place = [&](int tg, uint32_t R, const Ent &pe) __attribute__((always_inline)) {
-                    int p = first_piece[tg];
-                    while (p < npieces && R >= pieces[p].y + pieces[p].z) ++p;
-                    if (p < npieces && (int)pieces[p].x == tg)
-                        POOL[pieces[p].w + (R - pieces[p].y)] = pe;
-                    else
-                        bad_piece = true;
-                };
-                // every committed push, spread over the wave: push g of the round in the sequential
-                // order (chain by chain, each in log order) is placed by lane g % 64. Its rank in
-                // its bucket is the number of earlier pushes to that bucket in this order: a ballot
-                // per bucket within a spread, plus the counts of the spreads before it.
-                const int E = wave_excl_scan(ncp);
-                const int M = __shfl(E + ncp, HW - 1);
-                const uint64_t lt = (1ull << lane) - 1ull;  // the lanes before this one
-                uint32_t c0 = 0, c1 = 0, c2 = 0;
-                for (int g0 = 0; g0 < M; g0 += HW) {
-                    const int g = g0 + lane;
-                    int L = 0;  // the owner: the last lane whose first push is at or before g
 #pragma unroll
-                    for (int step = 32; step > 0; step >>= 1) {
-                        const int el = __shfl(E, L + step);
-                        if (el <= g) L += step;
-                    }
-                    const int u = g - __shfl(E, L);
-                    const bool valid = g < M;
-                    if (valid && (u < 0 || u >= H_PUSH)) bad_piece = true;  // (not possible: E is a scan)
-                    Ent pe{0, 0};
-                    int x = 3;
-                    if (valid && u >= 0 && u < H_PUSH) {
-                        pe = PLOG_W[L * H_PUSH + u];
-                        const int sc = e_mm(pe) * s_mm + e_go(pe) * s_gapo + e_ge(pe) * s_gape;  // its bucket
-                        x = sc == tg0 ? 0 : sc == tg1 ? 1 : sc == tg2 ? 2 : 3;
-                    }
-                    const uint64_t b0 = __ballot(x == 0), b1 = __ballot(x == 1), b2 = __ballot(x == 2);
-                    if (valid && u >= 0 && u < H_PUSH) {
-                        if (x == 3) {
-                            bad_piece = true;  // (ruled out when the round was sized)
+                for (int c = 0; c < 3; ++c) {
+                    const int Tc = c == 0 ? T0 : c == 1 ? T1 : T2;
+                    const uint16_t *const ep = epre + c * KMAX;
+                    for (int g = tid; g < Tc; g += T) {
+                        int lo = 0;
+#pragma unroll
+                        for (int step = KMAX / 2; step > 0; step >>= 1)
+                            if (lo + step <= last && (int)ep[lo + step] <= g) lo += step;
+                        const uint32_t B = cB[lo];
+                        const int u = (int)((B >> (8 * c)) & 127u) + (g - (int)ep[lo]);
+                        int p = F.fp[c];
+                        while (p + 1 < npieces && (uint32_t)g >= pieces[p].y + pieces[p].z) ++p;
+                        const uint4 pc = pieces[p];
+                        if (u < H_LOG && pc.x == (uint32_t)c && (uint32_t)g - pc.y < pc.z) {
+                            POOL[pc.w + ((uint32_t)g - pc.y)] = LOG[(c * T + (int)(B >> 24)) * H_LOG + u];
                         } else {
-                            const uint32_t R = x == 0   ? c0 + (uint32_t)__builtin_popcountll(b0 & lt)
-                                               : x == 1 ? c1 + (uint32_t)__builtin_popcountll(b1 & lt)
-                                                        : c2 + (uint32_t)__builtin_popcountll(b2 & lt);
-                            place(x == 0 ? tg0 : x == 1 ? tg1 : tg2, R, pe);
+                            F.bad = 1;  // a rank outside this round's pieces: not possible
                         }
                     }
-                    c0 += (uint32_t)__builtin_popcountll(b0);
-                    c1 += (uint32_t)__builtin_popcountll(b1);
-                    c2 += (uint32_t)__builtin_popcountll(b2);
-                }
-                if (bad_piece) {  // a rank outside this round's pieces: not possible
-                    F.status = 1;
-                    F.result = ERR_INTERNAL;
                 }
             }
-            const int mxs = a.stats ? wave_max_i32(steps) : 0;
             __syncthreads();
-            if (F.status) break;
             const long long t_c3 = a.stats ? wall_clock64() : 0;
             // ---- bucket b: the committed start entries leave its top; the state moves on ----
-            if (lane == 0) {
-                const int taken = __builtin_popcountll(posm);
-                const int from_seg = taken - (F.has_pend && taken > 0 ? 1 : 0);
-                if (taken > 0) F.has_pend = 0;
+            const int l_kind = F.l_kind;
+            if (tid == 0) {
+                const int taken = last + 1;
+                const int from_seg = taken - hp;
+                F.has_pend = 0;
                 if (from_seg > 0) {
-                    seg_cnt[b] -= (uint32_t)from_seg;
-                    if (seg_cnt[b] == 0) {
+                    const uint32_t left_n = seg_cnt[b] - (uint32_t)from_seg;
+                    seg_cnt[b] = left_n;
+                    if (left_n == 0) {
                         const Ent hdr = POOL[seg_base[b] - 1];
                         const uint32_t pb = (uint32_t)hdr.w0, ps = (uint32_t)(hdr.w0 >> 32);
                         if (pb == NIL) {
@@ -2057,20 +2268,23 @@ __global__ void __launch_bounds__(64) __attribute__((amdgpu_waves_per_eu(WPE))) 
                         }
                     }
                 }
-                // entries: every committed pop -1, every committed push +1, a pending child +1
-                long ne = F.n_entries + sum_ne;
-                const int lfull = last >= 0 ? F.l_full : -1;
-                if (last >= 0 && lfull == K_TRUNC) {
+                // entries: every chain's head left, its pushes came; a pending child is one more
+                int ne = F.n_entries + T0 + T1 + T2 - taken;
+                if (l_kind == K_TRUNC) {
                     F.has_pend = 1;
                     ne += 1;
                 }
-                F.n_entries = (int)ne;
+                F.n_entries = ne;
+                if (l_kind == K_ESCORE || F.bad) {
+                    F.status = 1;
+                    F.result = F.bad ? ERR_INTERNAL : ERR_SCORE;
+                }
                 if (a.stats) {
                     F.st[0] += 1;
-                    F.st[1] += (unsigned long long)K;
-                    F.st[2] += (unsigned long long)(last + 1);
-                    F.st[3] += sum_pops;
-                    F.st[4] += (unsigned long long)mxs;
+                    F.st[1] += (unsigned long long)nK;
+                    F.st[2] += (unsigned long long)taken;
+                    F.st[3] += tot2s >> 16;
+                    F.st[4] += (unsigned long long)its;
                     F.st[5] += (unsigned long long)(t_commit - t_spec);
                     const long long t_end = wall_clock64();
                     t_round_end = t_end;
@@ -2080,96 +2294,97 @@ __global__ void __launch_bounds__(64) __attribute__((amdgpu_waves_per_eu(WPE))) 
                     F.st[9] += (unsigned long long)(t_c3 - t_c2);
                     F.st[10] += (unsigned long long)(t_end - t_c3);
                 }
-                // a hit or a score error ends the last committed chain
-                if (lfull == K_ESCORE) {
-                    F.status = 1;
-                    F.result = ERR_SCORE;
-                } else if (lfull == K_HIT) {
-                    const Ent e = F.he;
-                    const uint64_t k = F.hk, l = F.hl;
-                    const int mm = e_mm(e), go = e_go(e), ge = e_ge(e);
-                    const int score = b;
-                    bool do_add = true, stop = false;
-                    if (F.n_aln == 0) {
-                        F.best_score = score;
-                        F.best_diff = mm + go + ((F.mode & MODE_GAPE) ? ge : 0);
-                        if (!(F.mode & MODE_NONSTOP))
-                            F.max_diff = (F.best_diff + 1 > F.md_read) ? F.md_read : F.best_diff + 1;
-                    }
-                    if (score == F.best_score) {
-                        F.best_cnt = (int)(uint32_t)((uint64_t)(int64_t)F.best_cnt + (l - k + 1));
-                    } else if (F.best_cnt > F.max_top2) {
-                        stop = true;
-                    }
-                    if (!stop) {
-                        if (go) {
-                            for (int j = 0; j < F.n_aln; ++j)
-                                if (REC[j].k == k && REC[j].l == l) {
-                                    do_add = false;
-                                    break;
-                                }
-                        }
-                        if (do_add) {
-                            const int x = (int)(uint32_t)(l - k + 1);
-                            const uint64_t ux = (uint64_t)(int64_t)x;
-                            int jj = 0;
-                            for (int i = 0; i < e_ldp(e); ++i) {
-                                uint64_t w = wval(W[i]);
-                                int bid = wbid(W[i]);
-                                if (w > ux) w -= ux;
-                                else if (w == ux) {
-                                    bid = 1;
-                                    w = seq_len - (uint64_t)(++jj);
-                                } else continue;
-                                W[i] = wpack(w, bid);
-                            }
-                            if (F.n_aln == a.rec_cap) {
-                                F.status = 1;
-                                F.result = ERR_ALN;
-                            } else {
-                                const int ins = e_ins(e), del = go + ge - ins;
-                                galn_aln_rec_t r;
-                                r.packed = ((uint64_t)(mm & 0xff)) | ((uint64_t)(go & 0xff) << 8) |
-                                           ((uint64_t)(ge & 0xff) << 16) | ((uint64_t)(score & 0xfffff) << 24) |
-                                           ((uint64_t)(ins & 0x3ff) << 44) | ((uint64_t)(del & 0x3ff) << 54);
-                                r.k = k;
-                                r.l = l;
-                                REC[F.n_aln] = r;
-                                F.n_aln += 1;
-                            }
-                        }
-                    } else {
-                        F.status = 1;
-                        F.result = F.n_aln;
+            }
+            if (l_kind == K_HIT && wave == 0 && F.status == 0) {
+                // a hit ends the last committed chain (src/bwtgap_hd.h:385-409); one wave applies it
+                const uint64_t hk = F.hk, hl = F.hl;
+                const uint32_t hx = F.hx, hy = F.hy;
+                const int n_aln = F.n_aln, mm = x_mm(hx), go = x_go(hx), ge = y_ge(hy);
+                const bool same = n_aln == 0 || b == F.best_score;
+                const bool stop_hits = !same && F.best_cnt > F.max_top2;
+                bool dup = false;
+                if (!stop_hits && go) {
+                    for (int j0 = 0; j0 < n_aln && !dup; j0 += HW) {
+                        const int j = j0 + lane;
+                        dup = __ballot(j < n_aln && REC[j].k == hk && REC[j].l == hl) != 0;
                     }
                 }
+                if (!stop_hits && !dup) {
+                    // gap_shadow (src/bwtgap_hd.h:309-320); the widths equal to the hit's are numbered in order
+                    const uint64_t ux = (uint64_t)(int64_t)(int)(uint32_t)(hl - hk + 1);
+                    const int ldp = (int)(hy & Y_LDP);
+                    uint64_t eq = 0;
+                    for (int j0 = 0; j0 < ldp; j0 += HW) {
+                        const int j = j0 + lane;
+                        const uint64_t v = j < ldp ? Wp[1 + j] : 0, w = lw_val<WIDE>(v);
+                        const uint64_t em = __ballot(j < ldp && w == ux);
+                        if (j < ldp && w > ux) Wp[1 + j] = lw_make<WIDE>(w - ux, lw_bid<WIDE>(v));
+                        if (j < ldp && w == ux) Wp[1 + j] = lw_make<WIDE>(M.seq_len - (eq + (uint64_t)lanes_below(em) + 1), 1);
+                        eq += (uint64_t)__builtin_popcountll(em);
+                    }
+                }
+                __builtin_amdgcn_wave_barrier();  // (the wave has read the state that lane 0 changes)
+                if (lane == 0) {
+                    if (n_aln == 0) {
+                        F.best_score = b;
+                        F.best_diff = mm + go + ((mode & MODE_GAPE) ? ge : 0);
+                        if (!(mode & MODE_NONSTOP)) F.max_diff = (F.best_diff + 1 > F.md_read) ? F.md_read : F.best_diff + 1;
+                    }
+                    if (same) F.best_cnt = (int)(uint32_t)((uint64_t)(int64_t)F.best_cnt + (hl - hk + 1));
+                    if (stop_hits) {
+                        F.status = 1;
+                        F.result = n_aln;
+                    } else if (!dup) {
+                        if (n_aln == a.rec_cap) {
+                            F.status = 1;
+                            F.result = ERR_ALN;
+                        } else {
+                            const int ins = y_ins(hy), del = go + ge - ins;
+                            galn_aln_rec_t r;
+                            r.packed = ((uint64_t)(mm & 0xff)) | ((uint64_t)(go & 0xff) << 8) | ((uint64_t)(ge & 0xff) << 16) |
+                                       ((uint64_t)(b & 0xfffff) << 24) | ((uint64_t)(ins & 0x3ff) << 44) |
+                                       ((uint64_t)(del & 0x3ff) << 54);
+                            r.k = hk;
+                            r.l = hl;
+                            REC[n_aln] = r;
+                            F.n_aln = n_aln + 1;
+                        }
+                    }
+                }
+            }
+            if (tid == 0 && F.status == 0 && a.deep_pops && F.pops >= a.deep_pops) {
+                F.status = 1;
+                F.result = ERR_HEAVY;
             }
             __syncthreads();
         }
         // ---- the read's result ----
-        if (lane == 0) {
+        if (tid == 0) {
             int n = F.result;
-            const int rd = F.rid;
-            if (n > 0) {
-                const unsigned long long b0 = atomicAdd(a.out_top, (unsigned long long)n);
-                if (b0 + (unsigned long long)n > a.out_cap) {
-                    n = ERR_OUT;
-                } else {
-                    for (int j = 0; j < n; ++j) a.out_rec[b0 + j] = REC[j];
-                    a.out_off[rd] = b0;
-                }
-            }
-            if (n == ERR_STACK || n == ERR_ALN || n == ERR_OUT) {
-                const int f = atomicAdd(a.fail_n, 1);
-                a.fail_list[f] = rd;
-                atomicOr(a.fail_kind + (n == ERR_OUT ? 0 : n == ERR_ALN ? 1 : 2), 1);
+            if (n == ERR_HEAVY) {
+                a.deep_list[atomicAdd(a.deep_n, 1)] = pos;
             } else {
-                atomicAdd(a.algo_bytes, F.obytes);
+                if (n > 0) {
+                    const unsigned long long b0 = atomicAdd(a.out_top, (unsigned long long)n);
+                    if (b0 + (unsigned long long)n > a.out_cap) {
+                        n = ERR_OUT;
+                    } else {
+                        for (int j = 0; j < n; ++j) a.out_rec[b0 + j] = REC[j];
+                        a.out_off[rid] = b0;
+                    }
+                }
+                if (n == ERR_STACK || n == ERR_ALN || n == ERR_OUT) {
+                    const int f = atomicAdd(a.fail_n, 1);
+                    a.fail_list[f] = rid;
+                    atomicOr(a.fail_kind + (n == ERR_OUT ? 0 : n == ERR_ALN ? 1 : 2), 1);
+                } else {
+                    atomicAdd(a.algo_bytes, F.obytes);
+                }
+                a.out_n[rid] = n;
+                a.out_pops[rid] = F.pops;
+                if (TRACE) a.out_trace[rid] = F.trace;
+                if (a.out_bytes) a.out_bytes[rid] = F.obytes;
             }
-            a.out_n[rd] = n;
-            a.out_pops[rd] = F.pops;
-            if (TRACE) a.out_trace[rd] = F.trace;
-            if (a.out_bytes) a.out_bytes[rd] = F.obytes;
             // keep a few granules for the next read; the rest go back to the pool
             if (F.n_own > H_KEEP) {
                 gran_push(a.ghead, a.gnext, OWN, H_KEEP, F.n_own);
@@ -2178,7 +2393,7 @@ __global__ void __launch_bounds__(64) __attribute__((amdgpu_waves_per_eu(WPE))) 
         }
         __syncthreads();
     }
-    if (a.stats && lane < 16) atomicAdd(a.stats + lane, F.st[lane]);
+    if (a.stats && tid < 16) atomicAdd(a.stats + tid, F.st[tid]);
 }
 
 // A read's record count for the output offsets (error codes count none).
@@ -2266,6 +2481,7 @@ struct SearchCtx {
 struct galn_hip_index {
     int device = 0;
     uint32_t *d_bwt = nullptr;
+    uint64_t *d_ext = nullptr;  // per epoch: the bases' counts at its start (k_epochs)
     DMeta meta{};
     galn_bwt_meta_t hmeta{};
     int n_cu = 0;
@@ -2557,12 +2773,14 @@ int resident_slots(galn_hip_readset *rs, int block, bool trace, int waves_per_cu
     return nb * idx->n_cu * block;
 }
 
+constexpr int HEAVY_CPL = 4;  // chains per thread and round of the wave engine
+
 struct HLayout {
     uint64_t slot_bytes;
     uint32_t rec_off, own_off, plog_off, slog_off;
 };
 
-HLayout make_hlayout(int rec_cap, int own_cap)
+HLayout make_hlayout(int rec_cap, int own_cap, int nw, bool trace)
 {
     HLayout L{};
     size_t off = 0;
@@ -2571,21 +2789,40 @@ HLayout make_hlayout(int rec_cap, int own_cap)
     L.own_off = (uint32_t)off;
     off += align_up((size_t)own_cap * 4, 256);
     L.plog_off = (uint32_t)off;
-    off += (size_t)HW * H_PUSH * sizeof(Ent);
+    off += (size_t)3 * nw * HW * H_LOG * sizeof(Ent);
     L.slog_off = (uint32_t)off;
-    off += (size_t)HW * H_STEPS * sizeof(Ent);
+    if (trace) off += (size_t)nw * HW * H_SLOG * (sizeof(Ent) + 1);
+    off = align_up(off, 256);
     if ((off / 256) % 2 == 0) off += 256;
     L.slot_bytes = off;
     return L;
 }
 
-size_t heavy_lds_bytes(int buckets, int wlen, int swlen)
+// LDS of a workgroup of the wave engine, in the order k_heavy carves it up
+size_t heavy_lds_bytes(int buckets, int wlen, int swlen, int nw, int cpl)
 {
     size_t b = (sizeof(HShared) + 15) & ~(size_t)15;
-    b += (size_t)buckets * 12;
-    b = (b + 15) & ~(size_t)15;
-    b += (size_t)H_PIECES * 16 + (size_t)(wlen + swlen) * 8 + 2 * HW * 4 + (size_t)HW * H_STEPS * 2 + (size_t)wlen;
+    b += (size_t)H_PIECES * 16 + (size_t)nw * HW * cpl * heavy_chain_bytes;
+    b += (size_t)(wlen + 1 + swlen) * 8 + (size_t)buckets * 8 + H_STEPS * 2 + (size_t)wlen;
     return b;
+}
+
+size_t heavy_lds_of(const galn_hip_readset *rs, int nw, int cpl)
+{
+    const int swlen = (rs->seed_len > 0 && rs->seed_len < rs->max_len) ? rs->seed_len + 1 : 1;
+    return heavy_lds_bytes(buckets_of(rs), rs->max_len + 1, swlen, nw, cpl);
+}
+
+typedef void (*HeavyKernel)(HArgs);
+
+HeavyKernel heavy_kernel(const galn_hip_readset *rs, bool trace)
+{
+    const bool wide = rs->idx->meta.ext != nullptr;
+    if (rs->heavy_wpe == 5)
+        return trace ? (wide ? k_heavy<true, true, 1, HEAVY_CPL, 5> : k_heavy<true, false, 1, HEAVY_CPL, 5>)
+                     : (wide ? k_heavy<false, true, 1, HEAVY_CPL, 5> : k_heavy<false, false, 1, HEAVY_CPL, 5>);
+    return trace ? (wide ? k_heavy<true, true, 1, HEAVY_CPL, 4> : k_heavy<true, false, 1, HEAVY_CPL, 4>)
+                 : (wide ? k_heavy<false, true, 1, HEAVY_CPL, 4> : k_heavy<false, false, 1, HEAVY_CPL, 4>);
 }
 
 // the wave-per-read engine keeps each chain's pops in order only when every child scores above its parent
@@ -2647,7 +2884,7 @@ int prepare_tier(galn_hip_readset *rs, const Tier &t, int slots, int pool_lanes)
 }
 
 // The allocations of a wave-engine launch of `waves` waves.
-int prepare_heavy(galn_hip_readset *rs, int waves, int rec_cap)
+int prepare_heavy(galn_hip_readset *rs, int waves, int rec_cap, bool trace)
 {
     SearchCtx *cx = rs->ctx;
     // granules for the waves that can get reads, rounded up to a power of two
@@ -2656,7 +2893,7 @@ int prepare_heavy(galn_hip_readset *rs, int waves, int rec_cap)
     int r = ensure_pool(cx, p2);
     if (r) return r;
     const int own_cap = (int)std::min<uint64_t>(cx->n_gran, 32768);
-    const HLayout L = make_hlayout(rec_cap, own_cap);
+    const HLayout L = make_hlayout(rec_cap, own_cap, 1, trace);
     return grow_dev((void **)&rs->d_hscratch, rs->hscratch_bytes, (size_t)waves * L.slot_bytes, cx->stream);
 }
 
@@ -2725,7 +2962,7 @@ int reserve_search(galn_hip_readset *rs, int n, int max_len, uint32_t flags)
     uint64_t p2 = 1024;
     while (p2 < (uint64_t)waves * 256) p2 <<= 1;
     if (!soft(ensure_pool(cx, p2))) {
-        const HLayout L = make_hlayout(256, (int)std::min<uint64_t>(cx->n_gran, 32768));
+        const HLayout L = make_hlayout(256, (int)std::min<uint64_t>(cx->n_gran, 32768), 1, (flags & GALN_HIP_TRACE) != 0);
         soft(grow_dev((void **)&rs->d_hscratch, rs->hscratch_bytes, (size_t)waves * L.slot_bytes, s));
     }
     // the results: the record counts' scan over n reads and the staged records
@@ -2813,15 +3050,15 @@ int run_tier(galn_hip_readset *rs, uint32_t flags, const Tier &t, const int32_t 
     return 0;
 }
 
-// Pushes the wave engine commits per round: H_CAP, or a lower value (at least H_PUSH, so that a
-// round's first chain always fits) from GALN_HIP_TEST_PUSH_CAP, which the tests set to make the
+// Pushes the wave engine commits per round: H_CAP, or a lower value (at least H_MINCAP; a round's first
+// chain always fits) from GALN_HIP_TEST_PUSH_CAP, which the tests set to make the
 // cap cut rounds short and check that the results do not change.
 int heavy_push_cap()
 {
     const char *v = getenv("GALN_HIP_TEST_PUSH_CAP");
     if (!v || !*v) return H_CAP;
     const long c = strtol(v, nullptr, 10);
-    return (int)std::min<long>(H_CAP, std::max<long>(H_PUSH, c));
+    return (int)std::min<long>(H_CAP, std::max<long>(H_MINCAP, c));
 }
 
 // The wave-per-read engine over list[0..n): one wave per read, `waves` resident waves
@@ -2835,13 +3072,14 @@ int run_heavy(galn_hip_readset *rs, uint32_t flags, const int32_t *list, int n, 
     const bool dev_count = n < 0;  // the count is the heavy-list length k_search leaves on the device
     if (n == 0) return 0;
     waves = std::max(1, dev_count ? waves : std::min(waves, n));
-    int r = prepare_heavy(rs, waves, rec_cap);
+    const bool tr = (flags & GALN_HIP_TRACE) != 0;
+    int r = prepare_heavy(rs, waves, rec_cap, tr);
     if (r) return r;
     const int own_cap = (int)std::min<uint64_t>(cx->n_gran, 32768);
-    const HLayout L = make_hlayout(rec_cap, own_cap);
+    const HLayout L = make_hlayout(rec_cap, own_cap, 1, tr);
     const int wlen = rs->max_len + 1;
     const int swlen = (rs->seed_len > 0 && rs->seed_len < rs->max_len) ? rs->seed_len + 1 : 1;
-    const size_t lds = heavy_lds_bytes(buckets_of(rs), wlen, swlen);
+    const size_t lds = heavy_lds_of(rs, 1, HEAVY_CPL);
     if (lds > 65536) return fail(GALN_HIP_E_UNSUPPORTED, "wave engine: %zu bytes of LDS needed", lds);
     HArgs a{};
     a.bwt = idx->d_bwt;
@@ -2920,22 +3158,12 @@ int run_heavy(galn_hip_readset *rs, uint32_t flags, const int32_t *list, int n, 
         w.hand_cap = a.hand_cap;
         w.wlen = wlen;
         w.swlen = swlen;
+        w.check = 1;
         const int wgrid = dev_count ? idx->n_cu * 8 : std::max(1, std::min(idx->n_cu * 8, (n + 255) / 256));
         hipLaunchKernelGGL(k_widths, dim3(wgrid), dim3(256), 0, fst, w);
         HIP_OK(hipGetLastError());
     }
-    const bool tr = (flags & GALN_HIP_TRACE) != 0;
-    if (rs->heavy_wpe == 5) {
-        if (tr)
-            hipLaunchKernelGGL((k_heavy<true, 5>), dim3(waves), dim3(HW), lds, fst, a);
-        else
-            hipLaunchKernelGGL((k_heavy<false, 5>), dim3(waves), dim3(HW), lds, fst, a);
-    } else {
-        if (tr)
-            hipLaunchKernelGGL((k_heavy<true, 4>), dim3(waves), dim3(HW), lds, fst, a);
-        else
-            hipLaunchKernelGGL((k_heavy<false, 4>), dim3(waves), dim3(HW), lds, fst, a);
-    }
+    hipLaunchKernelGGL(heavy_kernel(rs, tr), dim3(waves), dim3(HW), lds, fst, a);
     HIP_OK(hipGetLastError());
     if (!rs->capturing) HIP_OK(hipEventRecord(rs->lev[2 * li + 1], fst));
     return 0;
@@ -2943,18 +3171,9 @@ int run_heavy(galn_hip_readset *rs, uint32_t flags, const int32_t *list, int n, 
 
 int heavy_waves(galn_hip_readset *rs, uint32_t flags)
 {
-    const int wlen = rs->max_len + 1;
-    const int swlen = (rs->seed_len > 0 && rs->seed_len < rs->max_len) ? rs->seed_len + 1 : 1;
-    const size_t lds = heavy_lds_bytes(buckets_of(rs), wlen, swlen);
     int nb = 0;
-    const bool tr = (flags & GALN_HIP_TRACE) != 0;
-    hipError_t e;
-    if (rs->heavy_wpe == 5)
-        e = tr ? hipOccupancyMaxActiveBlocksPerMultiprocessor(&nb, k_heavy<true, 5>, HW, lds)
-               : hipOccupancyMaxActiveBlocksPerMultiprocessor(&nb, k_heavy<false, 5>, HW, lds);
-    else
-        e = tr ? hipOccupancyMaxActiveBlocksPerMultiprocessor(&nb, k_heavy<true, 4>, HW, lds)
-               : hipOccupancyMaxActiveBlocksPerMultiprocessor(&nb, k_heavy<false, 4>, HW, lds);
+    const hipError_t e = hipOccupancyMaxActiveBlocksPerMultiprocessor(
+        &nb, reinterpret_cast<const void *>(heavy_kernel(rs, (flags & GALN_HIP_TRACE) != 0)), HW, heavy_lds_of(rs, 1, HEAVY_CPL));
     if (e != hipSuccess || nb < 1) nb = 1;
     return nb * rs->idx->n_cu;
 }
@@ -3089,7 +3308,7 @@ int readset_search(galn_hip_readset *rs, int form, uint32_t flags, const galn_hi
             key.push_cap = heavy_push_cap();
             key.heavy_wpe = rs->heavy_wpe;
             if ((r = prepare_tier(rs, t0, slots, std::min(slots, rs->n))) ||
-                (budget && (r = prepare_heavy(rs, hwaves, 256))))
+                (budget && (r = prepare_heavy(rs, hwaves, 256, trace))))
                 return r;
             while (rs->lev.size() < 4) {
                 hipEvent_t e;
@@ -3381,7 +3600,6 @@ int galn_hip_index_open(const uint32_t *bwt, const galn_bwt_meta_t *meta, int de
     idx->device = device;
     idx->hmeta = *meta;
     idx->meta.primary = meta->primary;
-    for (int i = 0; i < 5; ++i) idx->meta.L2[i] = meta->L2[i];
     idx->meta.seq_len = meta->seq_len;
     hipDeviceProp_t prop;
     if (hipGetDeviceProperties(&prop, device) != hipSuccess) {
@@ -3404,16 +3622,35 @@ int galn_hip_index_open(const uint32_t *bwt, const galn_bwt_meta_t *meta, int de
         delete idx;
         return fail(GALN_HIP_E_DEVICE, "index upload failed");
     }
+    // 32-bit counts reach 2^32 - 1 (row seq_len + 1 included); a larger index counts per epoch of 2^24
+    // blocks. GALN_HIP_TEST_EPOCH=n makes the epochs 2^n blocks on an index of any size (tests).
     const uint64_t n_blocks = ((uint64_t)meta->bwt_size + 15) / 16;
-    if (n_blocks > 0)
+    uint32_t eshift = 24;
+    bool wide = meta->seq_len >= 0xfffffffeull;
+    if (const char *v = getenv("GALN_HIP_TEST_EPOCH"); v && *v) {
+        eshift = (uint32_t)std::min(24L, std::max(1L, strtol(v, nullptr, 10)));
+        wide = true;
+    }
+    const uint32_t n_ep = wide ? (uint32_t)((n_blocks >> eshift) + 1) : 1u;
+    bool up = hipMalloc(&idx->d_ext, (size_t)n_ep * 32) == hipSuccess;
+    if (up && n_blocks > 0) {
+        const uint64_t *const L2 = meta->L2;
+        hipLaunchKernelGGL(k_epochs, dim3((4 * n_ep + 255) / 256), dim3(256), 0, idx->ctx0.stream, (const uint32_t *)idx->d_bwt, n_blocks,
+                           eshift, make_uint4((uint32_t)L2[0], (uint32_t)L2[1], (uint32_t)L2[2], (uint32_t)L2[3]),
+                           make_uint4((uint32_t)(L2[0] >> 32), (uint32_t)(L2[1] >> 32), (uint32_t)(L2[2] >> 32), (uint32_t)(L2[3] >> 32)),
+                           idx->d_ext, n_ep);
         hipLaunchKernelGGL(k_planes, dim3((unsigned)((n_blocks + 255) / 256)), dim3(256), 0, idx->ctx0.stream, idx->d_bwt,
-                           n_blocks);
-    if (hipGetLastError() != hipSuccess || hipStreamSynchronize(idx->ctx0.stream) != hipSuccess) {
+                           n_blocks, (const uint64_t *)idx->d_ext, eshift, wide ? 1 : 0);
+    }
+    if (!up || hipGetLastError() != hipSuccess || hipStreamSynchronize(idx->ctx0.stream) != hipSuccess) {
         (void)hipStreamDestroy(idx->ctx0.stream);
         (void)hipFree(idx->d_bwt);
+        if (idx->d_ext) (void)hipFree(idx->d_ext);
         delete idx;
         return fail(GALN_HIP_E_DEVICE, "index upload failed");
     }
+    idx->meta.ext = wide ? idx->d_ext : nullptr;
+    idx->meta.eshift = eshift;
     // device address of the no-allocation search's array on this device (once per device); a
     // failure here is reported by that entry point, which looks it up again
     if (noalloc_setup(device) != 0) g_err[0] = 0;
@@ -3430,6 +3667,7 @@ int galn_hip_index_close(galn_hip_index *idx)
     (void)hipSetDevice(idx->device);
     if (idx->ctx0.stream) (void)hipStreamSynchronize(idx->ctx0.stream);
     (void)hipFree(idx->d_bwt);
+    if (idx->d_ext) (void)hipFree(idx->d_ext);
     if (idx->d_sa) (void)hipFree(idx->d_sa);
     idx->ctx0.free_pool();
     if (idx->ctx0.stream) (void)hipStreamDestroy(idx->ctx0.stream);
