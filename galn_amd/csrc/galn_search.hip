@@ -1253,8 +1253,11 @@ __global__ void __launch_bounds__(256) k_sa_walk(const uint32_t *__restrict__ bw
 // hit, which changes the state and ends the commit. Chains after that hit are discarded and run again in
 // the next round. The result, the pop count and the trace are those of the sequential search.
 //
-// Buckets are LIFO lists of segments (a 16-byte header naming the segment below, then the entries) in
-// granules the workgroup takes from the stack pool.
+// A bucket is a LIFO list of granules of the stack pool, all full below the top one: entry 0 names the
+// granule below, 1023 entries follow. A round's heads come from the top two granules, its pushes fill the
+// top one up, and a granule that empties is the next one taken. (Buckets that took a piece of a shared
+// granule each round gave a round only the last piece, 91 heads of up to 256 on average, and a read's
+// memory grew with its pushes, not with its stack.)
 //
 // What bounds it: vector issue, then the lookups' latency on a round's longest chain. A wave pays a full
 // iteration while one lane has a lookup left, and the chains of a heavy read are 2.3 steps long on average,
@@ -1263,6 +1266,11 @@ __global__ void __launch_bounds__(256) k_sa_walk(const uint32_t *__restrict__ bw
 // one held the wave for the longest tail of every step), 32-bit intervals and packed fields kept in
 // registers below 2^32 symbols, and one log per bucket code (a placed push needs no ranks, ballots or score)
 // took 2M ancient DNA reads on 100 Mbp from 308 ms of this kernel to 238, and 262,144 from 130 to 80.
+//
+// The tail: a read's rounds follow each other, and when the last read has been taken the waves that are done
+// leave the ones still on a read of a million pops. Those reads are parked and gone on with by workgroups of
+// four waves, whose round takes 1024 chains: 4001 reads, the longest of 630k pops, 41 -> 15 ms; 262,144
+// reads 80 -> 44 ms.
 
 constexpr int HW = 64;         // lanes of a wave
 constexpr int H_STEPS = 32;    // chain steps per round
@@ -1273,7 +1281,10 @@ constexpr int H_CAP = 4096;    // pushes committed per round and wave
 constexpr int H_KEEP = 64;     // granules a workgroup keeps between reads
 constexpr int H_PIECES = 48;   // segment pieces one round may add (three buckets)
 constexpr int H_MINCAP = 128;  // the lowest push cap a test may set
-constexpr uint32_t GENT = (uint32_t)GRAN * CH;  // entries per granule
+constexpr uint32_t GENT = (uint32_t)GRAN * CH;  // entries per granule, its link included
+constexpr uint32_t GFULL = GENT - 1;
+constexpr int H_LOOK = 16;     // rounds between looks at the queue
+constexpr int H_FREE = 32;     // emptied granules kept in LDS
 static_assert(H_LOG <= 120 && H_LOG > 2 * H_SPUSH, "push counts and offsets are 7-bit fields");
 static_assert(H_SLOG >= 2 * H_STEPS, "a chain's steps fit the rest of a thread's step log");
 
@@ -1290,7 +1301,6 @@ struct HArgs {
     const galn_search_opt_t *bopts;
     const int32_t *nstacks;
     const int32_t *list;        // read ids by position, or null (the position)
-    const int32_t *poslist;     // positions to search, or null (0 .. n_list - 1)
     int32_t n_list;
     const int32_t *n_list_dev;  // when set, the number of reads is read here
     const uint64_t *hand;       // widths by position (k_search or k_widths), or null
@@ -1300,13 +1310,14 @@ struct HArgs {
     int32_t n_slots;
     uint8_t *scratch;
     uint64_t slot_bytes;
-    uint32_t rec_off, own_off, plog_off, slog_off;
+    uint32_t rec_off, own_off, spill_off, plog_off, slog_off;
     int32_t own_cap, rec_cap;
     Ent *pool;
     uint32_t *gnext;
     unsigned long long *ghead;
     uint32_t *gbump;
     uint32_t n_gran;
+    int32_t first_gran;         // granules each workgroup holds from the start (gbump begins after them)
     int32_t *out_n;
     uint64_t *out_off, *out_pops, *out_trace, *out_bytes;
     galn_aln_rec_t *out_rec;
@@ -1318,28 +1329,41 @@ struct HArgs {
     int32_t wlen;     // LDS widths: longest read + 1
     int32_t swlen;    // LDS seed widths
     int32_t push_cap; // pushes committed per round (H_CAP per wave unless a test lowers it)
-    uint32_t deep_pops;  // > 0: a read that has popped this many goes to deep_list (its position)
-    int32_t *deep_list, *deep_n;
+    // a read that is still running when no other is left to take, after park_pops pops (0: never), is parked:
+    // its workgroup writes its state to its scratch, lists itself in park_list and ends; a launch of
+    // workgroups of more waves goes on with it
+    uint32_t park_pops;
+    int32_t *park_list, *park_n;
+    uint32_t state_off;
+    uint8_t *park_scratch;          // that launch's: the scratch of the launch that parked, its layout
+    uint64_t park_slot_bytes;
+    uint32_t park_rec_off, park_own_off, park_spill_off, park_state_off;
     unsigned long long *stats;  // [16] engine counters (rounds, chains, steps, cycles)
 };
 
 struct HShared {
-    int len, n_stacks, md_read, seeding, seed_len;
+    int rid, len, n_stacks, md_read, seeding, seed_len;
     int s_mm, s_gapo, s_gape, mode, ies, mdo, max_entries, max_gapo, max_gape, msd, max_top2;
     int best_score, best_diff, max_diff, best_cnt, n_aln, n_entries;
     unsigned long long pops, trace, obytes;
     unsigned long long bm[4];
-    int has_pend, claim, status, result, K, b, n_piece, n_own, n_used, aleft, nN, bad;
-    uint32_t abase;
+    int has_pend, claim, status, result, K, b, n_piece, n_own, n_used, n_free, n_spill, nN, bad;
+    uint32_t own[H_KEEP], free_g[H_FREE];  // the first granules held; emptied ones (more of them in the spill list)
     int next, stop, lim, l_kind, cut;  // the round's claims, first stopping chain, commit limit
     uint32_t tot01, tot2s, totb;       // committed pushes (16 bits per bucket code), pops, index bytes / 64
     int fp[3];                         // first piece of each bucket code
     uint32_t wsum[3][16];              // per wave: scan totals
     int wlive[16];
-    unsigned long long st[16];
     uint64_t hk, hl;                   // the last committed chain's hit, or its pending child
     uint32_t hx, hy;
 };
+static_assert(sizeof(HShared) % 8 == 0, "the widths follow it in a parked read's state");
+
+// what a read's state is besides HShared: the widths, the buckets
+__host__ __device__ inline size_t heavy_state_bytes(int buckets, int wlen, int swlen)
+{
+    return sizeof(HShared) + (size_t)(wlen + 1 + swlen) * 8 + (size_t)buckets * 12;
+}
 
 __device__ __forceinline__ int hbm_low(const unsigned long long *bm)
 {
@@ -1519,9 +1543,9 @@ __global__ void __launch_bounds__(64 * NW) __attribute__((amdgpu_waves_per_eu(WP
     constexpr int T = 64 * NW, KMAX = T * CPL;
     static_assert(T <= 256, "a thread's index takes 8 bits of its chains' records");
     extern __shared__ __align__(16) uint8_t hlds[];
-    HShared &F = *reinterpret_cast<HShared *>(hlds);
-    uint8_t *lp = hlds + ((sizeof(HShared) + 15) & ~(size_t)15);
-    uint4 *const pieces = reinterpret_cast<uint4 *>(lp);  // {bucket code, rank0, len, base}
+    // the launch of NW > 1 waves goes on with reads that the launch of one wave parked
+    constexpr bool RESUME = NW > 1;
+    uint4 *const pieces = reinterpret_cast<uint4 *>(hlds);         // {bucket code, rank0, len, base}
     Ent *const hent = reinterpret_cast<Ent *>(pieces + H_PIECES);  // live chains' heads, in order
     uint16_t *const epre = reinterpret_cast<uint16_t *>(hent);     // after them: pushes before each chain, by code
     uint32_t *const cA = reinterpret_cast<uint32_t *>(hent + KMAX);  // pushes by code (8 bits each) | stop kind << 24
@@ -1529,19 +1553,23 @@ __global__ void __launch_bounds__(64 * NW) __attribute__((amdgpu_waves_per_eu(WP
     uint32_t *const cC = cB + KMAX;                                  // steps | index bytes / 64 << 6
     uint16_t *const hcid = reinterpret_cast<uint16_t *>(cC + KMAX);  // live chains' ids
     uint16_t *const cS = hcid + KMAX;                                // trace build: place in the thread's step log
-    uint64_t *const Wp = reinterpret_cast<uint64_t *>(cS + KMAX);    // Wp[i] = width of position i - 1
+    unsigned long long *const ST = reinterpret_cast<unsigned long long *>(cS + KMAX);  // [16] counters
+    HShared &F = *reinterpret_cast<HShared *>(ST + 16);
+    uint64_t *const Wp = reinterpret_cast<uint64_t *>(&F + 1);       // Wp[i] = width of position i - 1
     uint64_t *const SW = Wp + a.wlen + 1;
-    uint32_t *const seg_base = reinterpret_cast<uint32_t *>(SW + a.swlen);
-    uint32_t *const seg_cnt = seg_base + a.buckets;
-    uint16_t *const s0info = reinterpret_cast<uint16_t *>(seg_cnt + a.buckets);  // chain 0's steps: pushes | index bytes / 64 << 4
+    uint32_t *const seg_top = reinterpret_cast<uint32_t *>(SW + a.swlen);  // per bucket: its top granule,
+    uint32_t *const seg_cnt = seg_top + a.buckets;                         // that one's entries (0: empty bucket)
+    uint32_t *const seg_prev = seg_cnt + a.buckets;                        // and the granule below, or NIL
+    uint16_t *const s0info = reinterpret_cast<uint16_t *>(seg_prev + a.buckets);  // chain 0's steps: pushes | index bytes / 64 << 4
     uint8_t *const QL = reinterpret_cast<uint8_t *>(s0info + H_STEPS);           // the read's query
     static_assert(MAXLEN * 2 + 2 < 4096, "a step's index bytes fit the step info");
 
     const int tid = threadIdx.x, lane = tid & (HW - 1), wave = tid >> 6;
     if ((int)blockIdx.x >= a.n_slots) return;
     uint8_t *const base = a.scratch + (uint64_t)blockIdx.x * a.slot_bytes;
-    galn_aln_rec_t *const REC = reinterpret_cast<galn_aln_rec_t *>(base + a.rec_off);
-    uint32_t *const OWN = reinterpret_cast<uint32_t *>(base + a.own_off);
+    galn_aln_rec_t *REC = reinterpret_cast<galn_aln_rec_t *>(base + a.rec_off);
+    uint32_t *OWN = reinterpret_cast<uint32_t *>(base + a.own_off);
+    uint32_t *SPILL = reinterpret_cast<uint32_t *>(base + a.spill_off);
     Ent *const LOG = reinterpret_cast<Ent *>(base + a.plog_off);     // code c, thread t: [(c * T + t) * H_LOG]
     Ent *const SLOG = reinterpret_cast<Ent *>(base + a.slog_off);    // trace build: thread t's steps at t * H_SLOG
     uint8_t *const SINFO = reinterpret_cast<uint8_t *>(SLOG + T * H_SLOG);  // and their push counts
@@ -1550,9 +1578,10 @@ __global__ void __launch_bounds__(64 * NW) __attribute__((amdgpu_waves_per_eu(WP
     const K seq_len = (K)M.seq_len;
 
     if (tid == 0) {
-        for (int j = 0; j < 16; ++j) F.st[j] = 0;
-        F.n_own = 0;  // granules this workgroup holds; a read reuses them before taking more
+        for (int j = 0; j < 16; ++j) ST[j] = 0;
+        F.n_own = RESUME ? 0 : a.first_gran;  // granules this workgroup holds; a read reuses them before taking more
     }
+    if (!RESUME && tid < a.first_gran) OWN[tid] = F.own[tid] = blockIdx.x * (uint32_t)a.first_gran + (uint32_t)tid;
     const int n_list = a.n_list_dev ? *a.n_list_dev : a.n_list;
     for (;;) {
         const long long t_read = a.stats ? wall_clock64() : 0;
@@ -1561,107 +1590,139 @@ __global__ void __launch_bounds__(64 * NW) __attribute__((amdgpu_waves_per_eu(WP
         const int claim = F.claim;
         if (claim >= n_list) break;
         // ---- read set-up ----
-        const int pos = a.poslist ? a.poslist[claim] : claim;
-        const int rid = a.list ? a.list[pos] : pos;
-        const int len = a.qlen[rid];
-        const uint8_t *const qg = a.query + a.qoff[rid];
-        for (int j = tid; j < len && j < a.wlen; j += T) QL[j] = qg[j];
-        if (tid == 0) {
-            const int b0 = a.batch[rid];
-            const galn_search_opt_t o = a.bopts[b0];
-            F.len = len;
-            F.s_mm = o.s_mm;
-            F.s_gapo = o.s_gapo;
-            F.s_gape = o.s_gape;
-            F.mode = o.mode;
-            F.ies = o.indel_end_skip;
-            F.mdo = o.max_del_occ;
-            F.max_entries = o.max_entries;
-            F.max_gapo = o.max_gapo;
-            F.max_gape = o.max_gape;
-            F.msd = o.max_seed_diff;
-            F.max_top2 = o.max_top2;
-            F.n_stacks = a.nstacks[b0];
-            F.md_read = a.maxdiff[rid];
-            F.seed_len = o.seed_len;
-            F.seeding = o.seed_len < len;
-            F.nN = 0;
-            F.obytes = 0;
-            F.n_used = 0;
-            F.aleft = 0;
-            F.abase = 0;
-            F.status = 0;
-            F.bad = 0;
-        }
-        __syncthreads();
-        const bool unsup = len < 1 || len > MAXLEN || len + 1 > a.wlen || F.n_stacks > a.buckets || F.md_read > MAXDIFF ||
-                           F.max_gapo > MAXDIFF || F.max_gapo + F.max_gape > 255;
-        const uint64_t h0 = (!unsup && a.hand && pos < a.hand_cap) ? a.hand[(uint64_t)pos * a.hand_stride] : 0;
-        if (!unsup) {
-            if (h0 >> 63) {
-                // the widths computed for this read
-                const uint64_t *src = a.hand + (uint64_t)pos * a.hand_stride;
-                for (int j = tid; j <= len; j += T) Wp[1 + j] = lw_make<WIDE>(wval(src[1 + j]), (uint32_t)wbid(src[1 + j]));
-                if (F.seeding)
-                    for (int j = tid; j <= F.seed_len; j += T)
-                        SW[j] = lw_make<WIDE>(wval(src[2 + len + j]), (uint32_t)wbid(src[2 + len + j]));
-                if (tid == 0) F.obytes = h0 & ~(1ull << 63);
-            } else {
-                uint64_t wb = 0;
-                auto putw = [Wp](int i, uint64_t v, int bid) { Wp[1 + i] = lw_make<WIDE>(v, (uint32_t)bid); };
-                auto puts = [SW](int i, uint64_t v, int bid) { SW[i] = lw_make<WIDE>(v, (uint32_t)bid); };
-                if (tid == 0) wb = cal_width_one(a.bwt, M, len, QL, putw);
-                if (tid == 1 && F.seeding) wb = cal_width_one(a.bwt, M, F.seed_len, QL + (len - F.seed_len), puts);
-                if (wb) atomicAdd(&F.obytes, (unsigned long long)wb);
+        int rid, len;
+        if constexpr (RESUME) {
+            // a parked read: its state, and its records and granules where its workgroup kept them
+            uint8_t *const pb = a.park_scratch + (uint64_t)a.park_list[claim] * a.park_slot_bytes;
+            const uint32_t *const st = reinterpret_cast<const uint32_t *>(pb + a.park_state_off);
+            __syncthreads();  // (F.claim is part of it)
+            for (int j = tid; j < (int)(heavy_state_bytes(a.buckets, a.wlen, a.swlen) / 4); j += T)
+                reinterpret_cast<uint32_t *>(&F)[j] = st[j];
+            REC = reinterpret_cast<galn_aln_rec_t *>(pb + a.park_rec_off);
+            OWN = reinterpret_cast<uint32_t *>(pb + a.park_own_off);
+            SPILL = reinterpret_cast<uint32_t *>(pb + a.park_spill_off);
+            __syncthreads();
+            rid = F.rid;
+            len = F.len;
+            const uint8_t *const qg = a.query + a.qoff[rid];
+            for (int j = tid; j < len; j += T) QL[j] = qg[j];
+            __syncthreads();
+        } else {
+            const int pos = claim;
+            rid = a.list ? a.list[pos] : pos;
+            len = a.qlen[rid];
+            const uint8_t *const qg = a.query + a.qoff[rid];
+            for (int j = tid; j < len && j < a.wlen; j += T) QL[j] = qg[j];
+            if (tid == 0) {
+                const int b0 = a.batch[rid];
+                const galn_search_opt_t o = a.bopts[b0];
+                F.rid = rid;
+                F.len = len;
+                F.s_mm = o.s_mm;
+                F.s_gapo = o.s_gapo;
+                F.s_gape = o.s_gape;
+                F.mode = o.mode;
+                F.ies = o.indel_end_skip;
+                F.mdo = o.max_del_occ;
+                F.max_entries = o.max_entries;
+                F.max_gapo = o.max_gapo;
+                F.max_gape = o.max_gape;
+                F.msd = o.max_seed_diff;
+                F.max_top2 = o.max_top2;
+                F.n_stacks = a.nstacks[b0];
+                F.md_read = a.maxdiff[rid];
+                F.seed_len = o.seed_len;
+                F.seeding = o.seed_len < len;
+                F.nN = 0;
+                F.obytes = 0;
+                F.n_used = 0;
+                F.n_free = 0;
+                F.n_spill = 0;
+                F.status = 0;
+                F.bad = 0;
             }
-            int nN = 0;
-            for (int j = tid; j < len; j += T) nN += QL[j] > 3;
-            if (nN) atomicAdd(&F.nN, nN);
-        }
-        __syncthreads();
-        // ---- search set-up ----
-        if (tid == 0) {
-            F.best_score = (F.md_read + 1) * F.s_mm + (F.max_gapo + 1) * F.s_gapo + (F.max_gape + 1) * F.s_gape;
-            F.best_diff = F.md_read + 1;
-            F.max_diff = F.md_read;
-            F.best_cnt = 0;
-            F.n_aln = 0;
-            F.pops = 0;
-            F.trace = TR_INIT;
-            F.bm[0] = F.bm[1] = F.bm[2] = F.bm[3] = 0;
-            F.has_pend = 0;
-            F.n_entries = 0;
-            Wp[0] = 0;
-            if (unsup) {
-                F.status = 1;
-                F.result = ERR_UNSUP;
-            } else if (F.nN > F.md_read) {
-                F.status = 1;
-                F.result = 0;
-            } else if (F.n_stacks <= 0) {
-                F.status = 1;
-                F.result = ERR_SCORE;
-            } else {
-                F.has_pend = 1;
-                F.hk = 0;
-                F.hl = M.seq_len;
-                F.hx = (uint32_t)len;
-                F.hy = 0;
-                F.b = 0;
-                F.n_entries = 1;
+            __syncthreads();
+            const bool unsup = len < 1 || len > MAXLEN || len + 1 > a.wlen || F.n_stacks > a.buckets || F.md_read > MAXDIFF ||
+                               F.max_gapo > MAXDIFF || F.max_gapo + F.max_gape > 255;
+            const uint64_t h0 = (!unsup && a.hand && pos < a.hand_cap) ? a.hand[(uint64_t)pos * a.hand_stride] : 0;
+            if (!unsup) {
+                if (h0 >> 63) {
+                    // the widths computed for this read
+                    const uint64_t *src = a.hand + (uint64_t)pos * a.hand_stride;
+                    for (int j = tid; j <= len; j += T) Wp[1 + j] = lw_make<WIDE>(wval(src[1 + j]), (uint32_t)wbid(src[1 + j]));
+                    if (F.seeding)
+                        for (int j = tid; j <= F.seed_len; j += T)
+                            SW[j] = lw_make<WIDE>(wval(src[2 + len + j]), (uint32_t)wbid(src[2 + len + j]));
+                    if (tid == 0) F.obytes = h0 & ~(1ull << 63);
+                } else {
+                    uint64_t wb = 0;
+                    auto putw = [Wp](int i, uint64_t v, int bid) { Wp[1 + i] = lw_make<WIDE>(v, (uint32_t)bid); };
+                    auto puts = [SW](int i, uint64_t v, int bid) { SW[i] = lw_make<WIDE>(v, (uint32_t)bid); };
+                    if (tid == 0) wb = cal_width_one(a.bwt, M, len, QL, putw);
+                    if (tid == 1 && F.seeding) wb = cal_width_one(a.bwt, M, F.seed_len, QL + (len - F.seed_len), puts);
+                    if (wb) atomicAdd(&F.obytes, (unsigned long long)wb);
+                }
+                int nN = 0;
+                for (int j = tid; j < len; j += T) nN += QL[j] > 3;
+                if (nN) atomicAdd(&F.nN, nN);
             }
+            for (int j = tid; j < a.buckets; j += T) seg_cnt[j] = 0;
+            __syncthreads();
+            // ---- search set-up ----
+            if (tid == 0) {
+                F.best_score = (F.md_read + 1) * F.s_mm + (F.max_gapo + 1) * F.s_gapo + (F.max_gape + 1) * F.s_gape;
+                F.best_diff = F.md_read + 1;
+                F.max_diff = F.md_read;
+                F.best_cnt = 0;
+                F.n_aln = 0;
+                F.pops = 0;
+                F.trace = TR_INIT;
+                F.bm[0] = F.bm[1] = F.bm[2] = F.bm[3] = 0;
+                F.has_pend = 0;
+                F.n_entries = 0;
+                Wp[0] = 0;
+                if (unsup) {
+                    F.status = 1;
+                    F.result = ERR_UNSUP;
+                } else if (F.nN > F.md_read) {
+                    F.status = 1;
+                    F.result = 0;
+                } else if (F.n_stacks <= 0) {
+                    F.status = 1;
+                    F.result = ERR_SCORE;
+                } else {
+                    F.has_pend = 1;
+                    F.hk = 0;
+                    F.hl = M.seq_len;
+                    F.hx = (uint32_t)len;
+                    F.hy = 0;
+                    F.b = 0;
+                    F.n_entries = 1;
+                }
+            }
+            __syncthreads();
         }
-        __syncthreads();
         if (a.stats && tid == 0) {
-            F.st[12] += (unsigned long long)(wall_clock64() - t_read);
-            F.st[15] += 1;
+            ST[12] += (unsigned long long)(wall_clock64() - t_read);
+            if (!RESUME) ST[15] += 1;
         }
         // ---- rounds ----
+        int n_round = 0;
         long long t_round_end = 0;  // with stats: end of the last round's commit
         for (;;) {
             const long long t_round = a.stats ? wall_clock64() : 0;
-            if (a.stats && tid == 0 && t_round_end) F.st[14] += (unsigned long long)(t_round - t_round_end);
+            if (a.stats && tid == 0 && t_round_end) ST[14] += (unsigned long long)(t_round - t_round_end);
+            int taken_reads = 0;
             if (tid == 0 && F.status == 0) {  // (the others read the status after the barrier)
+                // reads taken so far, looked at when this round has been committed. One load in H_LOOK rounds:
+                // all workgroups loading this word every round made a round 50% longer. With a workgroup for
+                // every read each takes its own, whatever the others do.
+                if (!RESUME && a.park_pops && F.pops >= a.park_pops) {
+                    if (n_list <= a.n_slots)
+                        taken_reads = n_list;
+                    else if ((++n_round & (H_LOOK - 1)) == 0)
+                        taken_reads = __hip_atomic_load(a.qnext, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+                }
                 // a pending exact child is the top of the lowest bucket (the bucket it came from)
                 const int b = F.has_pend ? F.b : hbm_low(F.bm);
                 if (b < 0 || F.n_entries > F.max_entries) {
@@ -1669,8 +1730,8 @@ __global__ void __launch_bounds__(64 * NW) __attribute__((amdgpu_waves_per_eu(WP
                     F.result = F.n_aln;
                 } else {
                     F.b = b;
-                    const bool bit = (F.bm[b >> 6] >> (b & 63)) & 1ull;
-                    const uint32_t avail = (uint32_t)F.has_pend + (bit ? seg_cnt[b] : 0u);
+                    const uint32_t cb = seg_cnt[b];
+                    const uint32_t avail = (uint32_t)F.has_pend + cb + (cb && seg_prev[b] != NIL ? GFULL : 0u);
                     if (!(F.mode & MODE_NONSTOP) && (uint32_t)b > (uint32_t)(F.best_score + F.s_mm)) {
                         // this pop ends the search (src/bwtgap_hd.h:366)
                         F.pops += 1;
@@ -1683,7 +1744,7 @@ __global__ void __launch_bounds__(64 * NW) __attribute__((amdgpu_waves_per_eu(WP
                                 e.x = F.hx;
                                 e.y = F.hy;
                             } else {
-                                e = get_item<WIDE>(POOL + seg_base[b] + seg_cnt[b] - 1);
+                                e = get_item<WIDE>(POOL + seg_top[b] * GENT + seg_cnt[b]);
                             }
                             F.trace = trace_item(F.trace, b, e.k, e.l, e.x, e.y, F.n_entries);
                         }
@@ -1703,7 +1764,7 @@ __global__ void __launch_bounds__(64 * NW) __attribute__((amdgpu_waves_per_eu(WP
             if (F.status) break;
             const int b = F.b, nK = F.K, hp = F.has_pend;
             const long long t_spec = a.stats ? wall_clock64() : 0;
-            if (a.stats && tid == 0) F.st[13] += (unsigned long long)(t_spec - t_round);
+            if (a.stats && tid == 0) ST[13] += (unsigned long long)(t_spec - t_round);
             const int s_mm = F.s_mm, s_gapo = F.s_gapo, s_gape = F.s_gape, mode = F.mode, max_diff = F.max_diff;
             const int n_stacks = F.n_stacks, max_gapo = F.max_gapo, max_gape = F.max_gape, ies = F.ies, mdo = F.mdo;
             const int msd = F.msd, sofs = len - F.seed_len;
@@ -1719,7 +1780,7 @@ __global__ void __launch_bounds__(64 * NW) __attribute__((amdgpu_waves_per_eu(WP
             // ---- chain heads, from the top of bucket b; those that cannot go on end here. Wave w loads
             // heads w * 64 * CPL on; the live ones are listed in order ----
             {
-                const uint32_t top = hp ? 0u : 1u;  // head c is entry seg_cnt - top - c + ... of the top segment
+                const uint32_t tc = seg_cnt[b], tb = seg_top[b] * GENT, pb = seg_prev[b] * GENT;
                 uint64_t lm[CPL];
                 int cnt = 0;
                 Item<WIDE> h[CPL];
@@ -1733,7 +1794,9 @@ __global__ void __launch_bounds__(64 * NW) __attribute__((amdgpu_waves_per_eu(WP
                             h[r].x = F.hx;
                             h[r].y = F.hy;
                         } else {
-                            h[r] = get_item<WIDE>(POOL + seg_base[b] + seg_cnt[b] - top - (uint32_t)c);
+                            // entry d below the top one: in the top granule, or in the full one below it
+                            const uint32_t d = (uint32_t)(c - hp);
+                            h[r] = get_item<WIDE>(POOL + (d < tc ? tb + tc - d : pb + GFULL - (d - tc)));
                         }
                     }
                 }
@@ -2150,65 +2213,61 @@ __global__ void __launch_bounds__(64 * NW) __attribute__((amdgpu_waves_per_eu(WP
             const uint32_t tot01 = F.tot01, tot2s = F.tot2s;
             const int T0 = (int)(tot01 & 0xffffu), T1 = (int)(tot01 >> 16), T2 = (int)(tot2s & 0xffffu);
             if (tid == 0) {
-                // pieces of the workgroup's current granule for each bucket that receives pushes; a
-                // bucket's new piece links to its previous top segment
+                // where each bucket's pushes go: the rest of its top granule, then new ones
                 int np_ = 0;
                 bool oom = false;
-                uint32_t abase = F.abase;
-                int aleft = F.aleft;
                 for (int c = 0; c < 3 && !oom; ++c) {
                     // (selects: arrays indexed by c would live in scratch memory)
                     const int sbk = c == 0 ? tg0 : c == 1 ? tg1 : tg2;
-                    uint32_t rem = (uint32_t)(c == 0 ? T0 : c == 1 ? T1 : T2);
+                    uint32_t rem = (uint32_t)(c == 0 ? T0 : c == 1 ? T1 : T2), rk = 0;
                     if (!rem) continue;
-                    const bool bit = (F.bm[sbk >> 6] >> (sbk & 63)) & 1ull;
-                    uint32_t prev_base = bit ? seg_base[sbk] : NIL, prev_size = bit ? seg_cnt[sbk] : 0u, rk = 0;
+                    uint32_t cnt = seg_cnt[sbk], top = cnt ? seg_top[sbk] : NIL;
                     F.fp[c] = np_;
+                    if (cnt && cnt < GFULL) {
+                        rk = min(rem, GFULL - cnt);
+                        pieces[np_++] = make_uint4((uint32_t)c, 0u, rk, top * GENT + 1 + cnt);
+                        cnt += rk;
+                        rem -= rk;
+                    }
                     while (rem > 0) {
-                        if (aleft < 2) {
-                            uint32_t g;
-                            if (F.n_used < F.n_own) {
-                                g = OWN[F.n_used];
-                            } else {
-                                if (F.n_own >= a.own_cap) {
-                                    oom = true;
-                                    break;
-                                }
-                                g = gran_pop(a.ghead, a.gnext, a.gbump, a.n_gran);
-                                if (g == NIL) {
-                                    oom = true;
-                                    break;
-                                }
-                                if (a.stats) F.st[11] += 1;
-                                OWN[F.n_own++] = g;
-                            }
+                        uint32_t g;
+                        if (F.n_free > 0) {
+                            g = F.free_g[--F.n_free];
+                        } else if (F.n_spill > 0) {
+                            g = SPILL[--F.n_spill];
+                        } else if (F.n_used < F.n_own) {
+                            g = F.n_used < H_KEEP ? F.own[F.n_used] : OWN[F.n_used];
                             ++F.n_used;
-                            abase = g * GENT;
-                            aleft = (int)GENT;
+                        } else {
+                            g = F.n_own < a.own_cap ? gran_pop(a.ghead, a.gnext, a.gbump, a.n_gran) : NIL;
+                            if (g == NIL) {
+                                oom = true;
+                                break;
+                            }
+                            if (a.stats) ST[11] += 1;
+                            if (F.n_own < H_KEEP) F.own[F.n_own] = g;
+                            OWN[F.n_own++] = g;
+                            ++F.n_used;
                         }
-                        if (np_ == H_PIECES) {  // (not possible: the push cap spans fewer pieces)
+                        if (np_ == H_PIECES) {  // (not possible: the push cap spans fewer granules)
                             oom = true;
                             break;
                         }
-                        const uint32_t plen = min(rem, (uint32_t)aleft - 1);
-                        Ent hdr;
-                        hdr.w0 = (uint64_t)prev_base | (uint64_t)prev_size << 32;
-                        hdr.w1 = 0;
-                        POOL[abase] = hdr;
-                        pieces[np_++] = make_uint4((uint32_t)c, rk, plen, abase + 1);
-                        prev_base = abase + 1;
-                        prev_size = plen;
-                        abase += plen + 1;
-                        aleft -= (int)plen + 1;
-                        rem -= plen;
-                        rk += plen;
+                        Ent link;
+                        link.w0 = top;
+                        link.w1 = 0;
+                        POOL[g * GENT] = link;
+                        seg_prev[sbk] = top;
+                        top = g;
+                        cnt = min(rem, GFULL);
+                        pieces[np_++] = make_uint4((uint32_t)c, rk, cnt, g * GENT + 1);
+                        rem -= cnt;
+                        rk += cnt;
                     }
-                    seg_base[sbk] = prev_base;
-                    seg_cnt[sbk] = prev_size;
+                    seg_top[sbk] = top;
+                    seg_cnt[sbk] = cnt;
                     F.bm[sbk >> 6] |= 1ull << (sbk & 63);
                 }
-                F.abase = abase;
-                F.aleft = aleft;
                 F.n_piece = np_;
                 if (oom) {
                     F.status = 1;
@@ -2255,18 +2314,26 @@ __global__ void __launch_bounds__(64 * NW) __attribute__((amdgpu_waves_per_eu(WP
                 const int from_seg = taken - hp;
                 F.has_pend = 0;
                 if (from_seg > 0) {
-                    const uint32_t left_n = seg_cnt[b] - (uint32_t)from_seg;
-                    seg_cnt[b] = left_n;
-                    if (left_n == 0) {
-                        const Ent hdr = POOL[seg_base[b] - 1];
-                        const uint32_t pb = (uint32_t)hdr.w0, ps = (uint32_t)(hdr.w0 >> 32);
-                        if (pb == NIL) {
+                    uint32_t n = (uint32_t)from_seg, cnt = seg_cnt[b], top = seg_top[b], prev = seg_prev[b];
+                    while (n >= cnt) {
+                        // the top granule is empty: the next one taken, and the one below is the top
+                        n -= cnt;
+                        if (F.n_free < H_FREE)
+                            F.free_g[F.n_free++] = top;
+                        else
+                            SPILL[F.n_spill++] = top;
+                        if (prev == NIL) {
+                            cnt = 0;
                             F.bm[b >> 6] &= ~(1ull << (b & 63));
-                        } else {
-                            seg_base[b] = pb;
-                            seg_cnt[b] = ps;
+                            break;
                         }
+                        top = prev;
+                        cnt = GFULL;
+                        prev = (uint32_t)POOL[top * GENT].w0;
                     }
+                    seg_cnt[b] = cnt - n;
+                    seg_top[b] = top;
+                    seg_prev[b] = prev;
                 }
                 // entries: every chain's head left, its pushes came; a pending child is one more
                 int ne = F.n_entries + T0 + T1 + T2 - taken;
@@ -2280,19 +2347,19 @@ __global__ void __launch_bounds__(64 * NW) __attribute__((amdgpu_waves_per_eu(WP
                     F.result = F.bad ? ERR_INTERNAL : ERR_SCORE;
                 }
                 if (a.stats) {
-                    F.st[0] += 1;
-                    F.st[1] += (unsigned long long)nK;
-                    F.st[2] += (unsigned long long)taken;
-                    F.st[3] += tot2s >> 16;
-                    F.st[4] += (unsigned long long)its;
-                    F.st[5] += (unsigned long long)(t_commit - t_spec);
+                    ST[0] += 1;
+                    ST[1] += (unsigned long long)nK;
+                    ST[2] += (unsigned long long)taken;
+                    ST[3] += tot2s >> 16;
+                    ST[4] += (unsigned long long)its;
+                    ST[5] += (unsigned long long)(t_commit - t_spec);
                     const long long t_end = wall_clock64();
                     t_round_end = t_end;
-                    F.st[6] += (unsigned long long)(t_end - t_commit);
-                    F.st[7] += (unsigned long long)(t_c1 - t_commit);
-                    F.st[8] += (unsigned long long)(t_c2 - t_c1);
-                    F.st[9] += (unsigned long long)(t_c3 - t_c2);
-                    F.st[10] += (unsigned long long)(t_end - t_c3);
+                    ST[6] += (unsigned long long)(t_end - t_commit);
+                    ST[7] += (unsigned long long)(t_c1 - t_commit);
+                    ST[8] += (unsigned long long)(t_c2 - t_c1);
+                    ST[9] += (unsigned long long)(t_c3 - t_c2);
+                    ST[10] += (unsigned long long)(t_end - t_c3);
                 }
             }
             if (l_kind == K_HIT && wave == 0 && F.status == 0) {
@@ -2352,48 +2419,57 @@ __global__ void __launch_bounds__(64 * NW) __attribute__((amdgpu_waves_per_eu(WP
                     }
                 }
             }
-            if (tid == 0 && F.status == 0 && a.deep_pops && F.pops >= a.deep_pops) {
-                F.status = 1;
-                F.result = ERR_HEAVY;
-            }
+            if (!RESUME && tid == 0 && F.status == 0 && a.park_pops && taken_reads >= n_list) F.status = 2;
             __syncthreads();
+        }
+        if (!RESUME && F.status == 2) {
+            __syncthreads();
+            if (tid == 0) F.status = 0;
+            __syncthreads();
+            uint32_t *const st = reinterpret_cast<uint32_t *>(base + a.state_off);
+            for (int j = tid; j < (int)(heavy_state_bytes(a.buckets, a.wlen, a.swlen) / 4); j += T)
+                st[j] = reinterpret_cast<const uint32_t *>(&F)[j];
+            if (tid == 0) {
+                a.park_list[atomicAdd(a.park_n, 1)] = (int32_t)blockIdx.x;
+                F.n_own = 0;  // its granules stay with it
+            }
+            break;  // (no read is left to take)
         }
         // ---- the read's result ----
         if (tid == 0) {
             int n = F.result;
-            if (n == ERR_HEAVY) {
-                a.deep_list[atomicAdd(a.deep_n, 1)] = pos;
-            } else {
-                if (n > 0) {
-                    const unsigned long long b0 = atomicAdd(a.out_top, (unsigned long long)n);
-                    if (b0 + (unsigned long long)n > a.out_cap) {
-                        n = ERR_OUT;
-                    } else {
-                        for (int j = 0; j < n; ++j) a.out_rec[b0 + j] = REC[j];
-                        a.out_off[rid] = b0;
-                    }
-                }
-                if (n == ERR_STACK || n == ERR_ALN || n == ERR_OUT) {
-                    const int f = atomicAdd(a.fail_n, 1);
-                    a.fail_list[f] = rid;
-                    atomicOr(a.fail_kind + (n == ERR_OUT ? 0 : n == ERR_ALN ? 1 : 2), 1);
+            if (n > 0) {
+                const unsigned long long b0 = atomicAdd(a.out_top, (unsigned long long)n);
+                if (b0 + (unsigned long long)n > a.out_cap) {
+                    n = ERR_OUT;
                 } else {
-                    atomicAdd(a.algo_bytes, F.obytes);
+                    for (int j = 0; j < n; ++j) a.out_rec[b0 + j] = REC[j];
+                    a.out_off[rid] = b0;
                 }
-                a.out_n[rid] = n;
-                a.out_pops[rid] = F.pops;
-                if (TRACE) a.out_trace[rid] = F.trace;
-                if (a.out_bytes) a.out_bytes[rid] = F.obytes;
             }
-            // keep a few granules for the next read; the rest go back to the pool
-            if (F.n_own > H_KEEP) {
-                gran_push(a.ghead, a.gnext, OWN, H_KEEP, F.n_own);
-                F.n_own = H_KEEP;
+            if (n == ERR_STACK || n == ERR_ALN || n == ERR_OUT) {
+                const int f = atomicAdd(a.fail_n, 1);
+                a.fail_list[f] = rid;
+                atomicOr(a.fail_kind + (n == ERR_OUT ? 0 : n == ERR_ALN ? 1 : 2), 1);
+            } else {
+                atomicAdd(a.algo_bytes, F.obytes);
+            }
+            a.out_n[rid] = n;
+            a.out_pops[rid] = F.pops;
+            if (TRACE) a.out_trace[rid] = F.trace;
+            if (a.out_bytes) a.out_bytes[rid] = F.obytes;
+            // keep a few granules for the next read; the rest go back to the pool (a parked read's all)
+            const int keep = RESUME ? 0 : H_KEEP;
+            if (F.n_own > keep) {
+                gran_push(a.ghead, a.gnext, OWN, keep, F.n_own);
+                F.n_own = keep;
             }
         }
         __syncthreads();
     }
-    if (a.stats && tid < 16) atomicAdd(a.stats + tid, F.st[tid]);
+    // the granules this workgroup still holds are for the reads that were parked
+    if (tid == 0 && a.park_pops && F.n_own > 0) gran_push(a.ghead, a.gnext, OWN, 0, F.n_own);
+    if (a.stats && tid < 16) atomicAdd(a.stats + tid, ST[tid]);
 }
 
 // A read's record count for the output offsets (error codes count none).
@@ -2500,7 +2576,7 @@ struct GraphKey {
     uint64_t budget;
     uint32_t rec_cap, keep;
     const int32_t *list;
-    const void *ptr[20];
+    const void *ptr[21];
     uint64_t rec_cap_out, n_gran, scratch_bytes, hscratch_bytes;
     int32_t max_len, seed_len, max_stacks, max_entries;
     const void *hand;
@@ -2508,6 +2584,7 @@ struct GraphKey {
     uint32_t hand_stride;
     int32_t push_cap;
     int32_t heavy_wpe;
+    uint32_t park_pops;
 };
 
 struct galn_hip_readset {
@@ -2534,11 +2611,14 @@ struct galn_hip_readset {
     uint64_t rec_cap = 0;
     unsigned long long *d_top = nullptr;
     int32_t *d_fail[2] = {nullptr, nullptr};
-    int32_t *d_ctr = nullptr;      // [0],[1] failure counts, [2] queue head, [3] heavy count, [4..6] failure kinds
+    int32_t *d_ctr = nullptr;      // [0],[1] failure counts, [2] queue head, [3] heavy count, [4..6] failure kinds,
+                                   // [8] parked count, [9] parked queue head
     int32_t *d_heavy = nullptr;    // reads handed to the wave-per-read engine
     unsigned long long *d_stats = nullptr;  // wave-per-read engine counters of the last search
     uint8_t *d_hscratch = nullptr; // per-wave regions of the wave-per-read engine
     size_t hscratch_bytes = 0;
+    int32_t *d_park = nullptr;     // its workgroups that parked a read
+    size_t park_bytes = 0;
     // per-lane regions (grown on demand)
     uint8_t *d_scratch = nullptr;
     size_t scratch_bytes = 0;
@@ -2773,14 +2853,23 @@ int resident_slots(galn_hip_readset *rs, int block, bool trace, int waves_per_cu
     return nb * idx->n_cu * block;
 }
 
-constexpr int HEAVY_CPL = 4;  // chains per thread and round of the wave engine
+// Chains per thread and round of the wave engine: 2 (8.5 KB of LDS, 18 waves a CU) against 4 (12.6 KB, 12):
+// 2M ancient DNA reads 217 ms against 233, 100k reads of 100 bp 7.5 against 8.9; one wave alone on a read
+// runs faster with 4 (262,144 reads 83 ms against 77 without parking), which is what the workgroups that go
+// on with parked reads take.
+constexpr int HEAVY_CPL = 2;
+constexpr int DEEP_NW = 4, DEEP_CPL = 4;
+// A read may be parked after this many pops, where it can be expected to pop as many again: 100k pairs of
+// 150 bp 39 ms (45 after 8192, 52 after 32768, 42 after 512), 2M ancient DNA reads 222 ms at any of them.
+constexpr uint32_t PARK_POPS = 2048;
+constexpr int FIRST_GRAN = 8;  // granules a workgroup of it starts with
 
 struct HLayout {
     uint64_t slot_bytes;
-    uint32_t rec_off, own_off, plog_off, slog_off;
+    uint32_t rec_off, own_off, spill_off, state_off, plog_off, slog_off;
 };
 
-HLayout make_hlayout(int rec_cap, int own_cap, int nw, bool trace)
+HLayout make_hlayout(int rec_cap, int own_cap, int nw, bool trace, size_t state_bytes)
 {
     HLayout L{};
     size_t off = 0;
@@ -2788,6 +2877,10 @@ HLayout make_hlayout(int rec_cap, int own_cap, int nw, bool trace)
     off += align_up((size_t)rec_cap * sizeof(galn_aln_rec_t), 256);
     L.own_off = (uint32_t)off;
     off += align_up((size_t)own_cap * 4, 256);
+    L.spill_off = (uint32_t)off;
+    off += align_up((size_t)own_cap * 4, 256);
+    L.state_off = (uint32_t)off;
+    off += align_up(state_bytes, 256);
     L.plog_off = (uint32_t)off;
     off += (size_t)3 * nw * HW * H_LOG * sizeof(Ent);
     L.slog_off = (uint32_t)off;
@@ -2801,10 +2894,14 @@ HLayout make_hlayout(int rec_cap, int own_cap, int nw, bool trace)
 // LDS of a workgroup of the wave engine, in the order k_heavy carves it up
 size_t heavy_lds_bytes(int buckets, int wlen, int swlen, int nw, int cpl)
 {
-    size_t b = (sizeof(HShared) + 15) & ~(size_t)15;
-    b += (size_t)H_PIECES * 16 + (size_t)nw * HW * cpl * heavy_chain_bytes;
-    b += (size_t)(wlen + 1 + swlen) * 8 + (size_t)buckets * 8 + H_STEPS * 2 + (size_t)wlen;
-    return b;
+    return (size_t)H_PIECES * 16 + (size_t)nw * HW * cpl * heavy_chain_bytes + 16 * 8 + heavy_state_bytes(buckets, wlen, swlen) +
+           H_STEPS * 2 + (size_t)wlen;
+}
+
+size_t heavy_state_of(const galn_hip_readset *rs)
+{
+    const int swlen = (rs->seed_len > 0 && rs->seed_len < rs->max_len) ? rs->seed_len + 1 : 1;
+    return heavy_state_bytes(buckets_of(rs), rs->max_len + 1, swlen);
 }
 
 size_t heavy_lds_of(const galn_hip_readset *rs, int nw, int cpl)
@@ -2815,14 +2912,34 @@ size_t heavy_lds_of(const galn_hip_readset *rs, int nw, int cpl)
 
 typedef void (*HeavyKernel)(HArgs);
 
-HeavyKernel heavy_kernel(const galn_hip_readset *rs, bool trace)
+HeavyKernel heavy_kernel(const galn_hip_readset *rs, bool trace, bool deep)
 {
     const bool wide = rs->idx->meta.ext != nullptr;
+    if (deep)
+        return trace ? (wide ? k_heavy<true, true, DEEP_NW, DEEP_CPL, 4> : k_heavy<true, false, DEEP_NW, DEEP_CPL, 4>)
+                     : (wide ? k_heavy<false, true, DEEP_NW, DEEP_CPL, 4> : k_heavy<false, false, DEEP_NW, DEEP_CPL, 4>);
     if (rs->heavy_wpe == 5)
         return trace ? (wide ? k_heavy<true, true, 1, HEAVY_CPL, 5> : k_heavy<true, false, 1, HEAVY_CPL, 5>)
                      : (wide ? k_heavy<false, true, 1, HEAVY_CPL, 5> : k_heavy<false, false, 1, HEAVY_CPL, 5>);
     return trace ? (wide ? k_heavy<true, true, 1, HEAVY_CPL, 4> : k_heavy<true, false, 1, HEAVY_CPL, 4>)
                  : (wide ? k_heavy<false, true, 1, HEAVY_CPL, 4> : k_heavy<false, false, 1, HEAVY_CPL, 4>);
+}
+
+// Workgroups of the wave engine that are resident at once.
+int heavy_grid(galn_hip_readset *rs, uint32_t flags, bool deep)
+{
+    const int nw = deep ? DEEP_NW : 1, cpl = deep ? DEEP_CPL : HEAVY_CPL;
+    int nb = 0;
+    const hipError_t e = hipOccupancyMaxActiveBlocksPerMultiprocessor(
+        &nb, reinterpret_cast<const void *>(heavy_kernel(rs, (flags & GALN_HIP_TRACE) != 0, deep)), nw * HW, heavy_lds_of(rs, nw, cpl));
+    if (e != hipSuccess || nb < 1) nb = 1;
+    return nb * rs->idx->n_cu;
+}
+
+// A workgroup's first granules: FIRST_GRAN of them, fewer in a small pool (half of it is left to share).
+int first_gran(const SearchCtx *cx, int groups)
+{
+    return (int)std::min<uint64_t>(FIRST_GRAN, cx->n_gran / 2 / (uint64_t)std::max(groups, 1));
 }
 
 // the wave-per-read engine keeps each chain's pops in order only when every child scores above its parent
@@ -2883,8 +3000,18 @@ int prepare_tier(galn_hip_readset *rs, const Tier &t, int slots, int pool_lanes)
     return ensure_pool(rs->ctx, p2);
 }
 
+// Bytes of scratch for the wave engine: `waves` workgroups of one wave, then the workgroups that go on with
+// parked reads (which read the former's).
+size_t heavy_scratch(galn_hip_readset *rs, int waves, int rec_cap, uint32_t flags)
+{
+    const bool trace = (flags & GALN_HIP_TRACE) != 0;
+    const int own_cap = (int)std::min<uint64_t>(rs->ctx->n_gran, 32768);
+    const size_t one = (size_t)waves * make_hlayout(rec_cap, own_cap, 1, trace, heavy_state_of(rs)).slot_bytes;
+    return one + (size_t)std::min(waves, heavy_grid(rs, flags, true)) * make_hlayout(0, 0, DEEP_NW, trace, 0).slot_bytes;
+}
+
 // The allocations of a wave-engine launch of `waves` waves.
-int prepare_heavy(galn_hip_readset *rs, int waves, int rec_cap, bool trace)
+int prepare_heavy(galn_hip_readset *rs, int waves, int rec_cap, uint32_t flags)
 {
     SearchCtx *cx = rs->ctx;
     // granules for the waves that can get reads, rounded up to a power of two
@@ -2892,9 +3019,8 @@ int prepare_heavy(galn_hip_readset *rs, int waves, int rec_cap, bool trace)
     while (p2 < want) p2 <<= 1;
     int r = ensure_pool(cx, p2);
     if (r) return r;
-    const int own_cap = (int)std::min<uint64_t>(cx->n_gran, 32768);
-    const HLayout L = make_hlayout(rec_cap, own_cap, 1, trace);
-    return grow_dev((void **)&rs->d_hscratch, rs->hscratch_bytes, (size_t)waves * L.slot_bytes, cx->stream);
+    if ((r = grow_dev((void **)&rs->d_park, rs->park_bytes, (size_t)waves * 4, cx->stream))) return r;
+    return grow_dev((void **)&rs->d_hscratch, rs->hscratch_bytes, heavy_scratch(rs, waves, rec_cap, flags), cx->stream);
 }
 
 // Hand-off slots for the widths of reads moving to the wave engine: one per read, up to
@@ -2928,8 +3054,6 @@ int prepare_hand(galn_hip_readset *rs)
     return 0;
 }
 
-int heavy_waves(galn_hip_readset *rs, uint32_t flags);
-
 // The batched form's buffers sized for launches of up to n reads of up to max_len bases: the
 // hand-off slots, the stack pool and wave-engine scratch of min(grid, n) waves, the results' scan
 // space and two staged records per read. Without it these grow by doubling as launches get larger
@@ -2958,12 +3082,11 @@ int reserve_search(galn_hip_readset *rs, int n, int max_len, uint32_t flags)
         rs->hand_cap = 0;
     }
     // the stack pool and the wave engine's per-wave scratch, as prepare_heavy sizes them
-    const int waves = std::max(1, std::min(heavy_waves(rs, flags), n));
+    const int waves = std::max(1, std::min(heavy_grid(rs, flags, false), n));
     uint64_t p2 = 1024;
     while (p2 < (uint64_t)waves * 256) p2 <<= 1;
     if (!soft(ensure_pool(cx, p2))) {
-        const HLayout L = make_hlayout(256, (int)std::min<uint64_t>(cx->n_gran, 32768), 1, (flags & GALN_HIP_TRACE) != 0);
-        soft(grow_dev((void **)&rs->d_hscratch, rs->hscratch_bytes, (size_t)waves * L.slot_bytes, s));
+        soft(grow_dev((void **)&rs->d_hscratch, rs->hscratch_bytes, heavy_scratch(rs, waves, 256, flags), s));
     }
     // the results: the record counts' scan over n reads and the staged records
     size_t tmp = 0;
@@ -2979,7 +3102,7 @@ void fill_key_ptrs(const galn_hip_readset *rs, GraphKey &k)
 {
     const void *p[] = {rs->d_query, rs->d_qoff, rs->d_qlen, rs->d_maxdiff, rs->d_batch, rs->d_nstacks, rs->d_bopts,
                        rs->d_sorted, rs->d_out_n, rs->d_out_off, rs->d_pops, rs->d_trace, rs->d_bytes, rs->d_rec,
-                       rs->d_fail[0], rs->d_fail[1], rs->d_heavy, rs->d_scratch, rs->d_hscratch, rs->ctx->d_pool_chk};
+                       rs->d_fail[0], rs->d_fail[1], rs->d_heavy, rs->d_park, rs->d_scratch, rs->d_hscratch, rs->ctx->d_pool_chk};
     static_assert(sizeof(p) == sizeof(k.ptr), "graph key pointers");
     memcpy(k.ptr, p, sizeof p);
     k.rec_cap_out = rs->rec_cap;
@@ -3061,6 +3184,13 @@ int heavy_push_cap()
     return (int)std::min<long>(H_CAP, std::max<long>(H_MINCAP, c));
 }
 
+// Pops from which on a read may be parked (0: never).
+uint32_t heavy_park_pops()
+{
+    const char *v = getenv("GALN_HIP_TEST_PARK_POPS");
+    return v && *v ? (uint32_t)strtoul(v, nullptr, 10) : PARK_POPS;
+}
+
 // The wave-per-read engine over list[0..n): one wave per read, `waves` resident waves
 // claiming reads from a device counter; failures land in fail buffer `fo`.
 int run_heavy(galn_hip_readset *rs, uint32_t flags, const int32_t *list, int n, int rec_cap, int fo, int tier_id,
@@ -3073,14 +3203,17 @@ int run_heavy(galn_hip_readset *rs, uint32_t flags, const int32_t *list, int n, 
     if (n == 0) return 0;
     waves = std::max(1, dev_count ? waves : std::min(waves, n));
     const bool tr = (flags & GALN_HIP_TRACE) != 0;
-    int r = prepare_heavy(rs, waves, rec_cap, tr);
+    int r = prepare_heavy(rs, waves, rec_cap, flags);
     if (r) return r;
     const int own_cap = (int)std::min<uint64_t>(cx->n_gran, 32768);
-    const HLayout L = make_hlayout(rec_cap, own_cap, 1, tr);
+    const HLayout L = make_hlayout(rec_cap, own_cap, 1, tr, heavy_state_of(rs));
     const int wlen = rs->max_len + 1;
     const int swlen = (rs->seed_len > 0 && rs->seed_len < rs->max_len) ? rs->seed_len + 1 : 1;
     const size_t lds = heavy_lds_of(rs, 1, HEAVY_CPL);
-    if (lds > 65536) return fail(GALN_HIP_E_UNSUPPORTED, "wave engine: %zu bytes of LDS needed", lds);
+    const size_t lds_deep = heavy_lds_of(rs, DEEP_NW, DEEP_CPL);
+    if (std::max(lds, lds_deep) > 65536)
+        return fail(GALN_HIP_E_UNSUPPORTED, "wave engine: %zu bytes of LDS needed", std::max(lds, lds_deep));
+    const uint32_t park_pops = heavy_park_pops();
     HArgs a{};
     a.bwt = idx->d_bwt;
     a.meta = idx->meta;
@@ -3103,6 +3236,7 @@ int run_heavy(galn_hip_readset *rs, uint32_t flags, const int32_t *list, int n, 
     a.slot_bytes = L.slot_bytes;
     a.rec_off = L.rec_off;
     a.own_off = L.own_off;
+    a.spill_off = L.spill_off;
     a.plog_off = L.plog_off;
     a.slog_off = L.slog_off;
     a.own_cap = own_cap;
@@ -3128,9 +3262,15 @@ int run_heavy(galn_hip_readset *rs, uint32_t flags, const int32_t *list, int n, 
     a.push_cap = heavy_push_cap();
     a.swlen = swlen;
     a.stats = (flags & GALN_HIP_STATS) ? rs->d_stats : nullptr;
+    a.park_pops = park_pops;
+    a.park_list = rs->d_park;
+    a.park_n = rs->d_ctr + 8;
+    a.state_off = L.state_off;
+    a.first_gran = first_gran(cx, waves);
     FILL(rs->d_ctr + 2, 0, sizeof(int32_t));
+    FILL(rs->d_ctr + 8, 0, 2 * sizeof(int32_t));
     FILL(cx->d_ghead, 0xffffffffu, NSHARD * 8);
-    FILL(cx->d_gbump, 0, 4);
+    FILL(cx->d_gbump, (uint32_t)(a.first_gran * waves), 4);
     const int li = (int)rs->launches.size();
     if (li >= galn_hip_readset::MAX_LAUNCH) return fail(GALN_HIP_E_DEVICE, "too many launches in one search");
     while ((int)rs->lev.size() < 2 * (li + 1)) {
@@ -3163,19 +3303,34 @@ int run_heavy(galn_hip_readset *rs, uint32_t flags, const int32_t *list, int n, 
         hipLaunchKernelGGL(k_widths, dim3(wgrid), dim3(256), 0, fst, w);
         HIP_OK(hipGetLastError());
     }
-    hipLaunchKernelGGL(heavy_kernel(rs, tr), dim3(waves), dim3(HW), lds, fst, a);
+    hipLaunchKernelGGL(heavy_kernel(rs, tr, false), dim3(waves), dim3(HW), lds, fst, a);
+    if (park_pops) {
+        // the reads still running when the last one was taken, with more waves each (their count is read on
+        // the device; the workgroups end at once when there are none)
+        HIP_OK(hipGetLastError());
+        const int groups = std::min(waves, heavy_grid(rs, flags, true));
+        const HLayout D = make_hlayout(0, 0, DEEP_NW, tr, 0);
+        HArgs d = a;
+        d.n_list_dev = rs->d_ctr + 8;
+        d.qnext = rs->d_ctr + 9;
+        d.n_slots = groups;
+        d.scratch = a.scratch + (size_t)waves * L.slot_bytes;
+        d.slot_bytes = D.slot_bytes;
+        d.plog_off = D.plog_off;
+        d.slog_off = D.slog_off;
+        d.push_cap = a.push_cap == H_CAP ? H_CAP * DEEP_NW : a.push_cap;
+        d.park_pops = 0;
+        d.park_scratch = a.scratch;
+        d.park_slot_bytes = L.slot_bytes;
+        d.park_rec_off = L.rec_off;
+        d.park_own_off = L.own_off;
+        d.park_spill_off = L.spill_off;
+        d.park_state_off = L.state_off;
+        hipLaunchKernelGGL(heavy_kernel(rs, tr, true), dim3(groups), dim3(DEEP_NW * HW), lds_deep, fst, d);
+    }
     HIP_OK(hipGetLastError());
     if (!rs->capturing) HIP_OK(hipEventRecord(rs->lev[2 * li + 1], fst));
     return 0;
-}
-
-int heavy_waves(galn_hip_readset *rs, uint32_t flags)
-{
-    int nb = 0;
-    const hipError_t e = hipOccupancyMaxActiveBlocksPerMultiprocessor(
-        &nb, reinterpret_cast<const void *>(heavy_kernel(rs, (flags & GALN_HIP_TRACE) != 0)), HW, heavy_lds_of(rs, 1, HEAVY_CPL));
-    if (e != hipSuccess || nb < 1) nb = 1;
-    return nb * rs->idx->n_cu;
 }
 
 int read_ctr(galn_hip_readset *rs, int which, int32_t *v)
@@ -3295,7 +3450,7 @@ int readset_search(galn_hip_readset *rs, int form, uint32_t flags, const galn_hi
         const int hp = tune ? tune->heavy_pops : 0;
         rs->heavy_wpe = tune && tune->heavy_waves_per_simd == 5 ? 5 : 4;
         budget = (hp < 0 || !heavy_ok(rs)) ? 0 : (uint64_t)(hp > 0 ? hp : DEFAULT_HEAVY_POPS);
-        hwaves = heavy_waves(rs, flags);
+        hwaves = heavy_grid(rs, flags, false);
         if (budget && (r = prepare_hand(rs))) return r;
         const int32_t *list = sorted ? rs->d_sorted : nullptr;
         if (graph) {
@@ -3306,9 +3461,10 @@ int readset_search(galn_hip_readset *rs, int form, uint32_t flags, const galn_hi
             key.flags = flags, key.block = block, key.slots = slots, key.hwaves = hwaves, key.n = rs->n;
             key.budget = budget, key.rec_cap = (uint32_t)t0.rec_cap, key.keep = (uint32_t)t0.keep, key.list = list;
             key.push_cap = heavy_push_cap();
+            key.park_pops = heavy_park_pops();
             key.heavy_wpe = rs->heavy_wpe;
             if ((r = prepare_tier(rs, t0, slots, std::min(slots, rs->n))) ||
-                (budget && (r = prepare_heavy(rs, hwaves, 256, trace))))
+                (budget && (r = prepare_heavy(rs, hwaves, 256, flags))))
                 return r;
             while (rs->lev.size() < 4) {
                 hipEvent_t e;
@@ -3684,7 +3840,7 @@ int galn_hip_readset_free(galn_hip_readset *rs)
     (void)hipStreamSynchronize(rs->ctx->stream);
     void *ptrs[] = {rs->d_query, rs->d_qoff, rs->d_qlen, rs->d_maxdiff, rs->d_batch, rs->d_nstacks, rs->d_bopts,
                     rs->d_sorted, rs->d_out_n, rs->d_out_off, rs->d_pops, rs->d_trace, rs->d_bytes, rs->d_rec, rs->d_top,
-                    rs->d_fail[0], rs->d_fail[1], rs->d_ctr, rs->d_scratch, rs->d_algo, rs->d_heavy, rs->d_hscratch,
+                    rs->d_fail[0], rs->d_fail[1], rs->d_ctr, rs->d_scratch, rs->d_algo, rs->d_heavy, rs->d_park, rs->d_hscratch,
                     rs->d_stats, rs->d_incl, rs->d_roff, rs->d_stage, rs->d_scan_tmp, rs->d_hand};
     for (void *p : ptrs)
         if (p) (void)hipFree(p);
@@ -3716,7 +3872,7 @@ int galn_hip_readset_upload(galn_hip_index *idx, const galn_hip_reads *reads, ga
     rs->ctx = &idx->ctx0;
     idx->n_readsets.fetch_add(1);
     auto M = [&](void **p, size_t b) __attribute__((always_inline)) -> bool { return hipMalloc(p, b) == hipSuccess; };
-    bool ok = M((void **)&rs->d_top, 8) && M((void **)&rs->d_ctr, 8 * sizeof(int32_t)) && M((void **)&rs->d_stats, 16 * 8) &&
+    bool ok = M((void **)&rs->d_top, 8) && M((void **)&rs->d_ctr, 16 * sizeof(int32_t)) && M((void **)&rs->d_stats, 16 * 8) &&
               M((void **)&rs->d_algo, sizeof(unsigned long long) * galn_hip_readset::MAX_LAUNCH);
     if (!ok) {
         galn_hip_readset_free(rs);
