@@ -172,6 +172,9 @@ __device__ __forceinline__ T cold_ld(const __attribute__((address_space(4))) T *
 // (for r != primary), so the symbols at or before row k - 1 are P = k - (k > primary), k = 0 included, and
 // those at or before row l are P = l + (l < primary).
 
+// a value the compiler takes as it is
+#define OPAQUE(v) asm("" : "+v"(v))
+
 // what a position's count is computed from
 struct OccWord {
     uint4 C;
@@ -190,8 +193,10 @@ __device__ __forceinline__ void occ_load(const uint32_t *__restrict__ bwt, K P, 
     Sub sub;
     if constexpr (sizeof(K) == 4) {
         const uint32_t off = ((uint32_t)P >> 7) << 6;  // below 2^31
+        uint32_t so = off + (in - 16u);
+        OPAQUE(so);  // (one 32-bit offset from the scalar base, not a 64-bit address of its own)
         o.C = *reinterpret_cast<const uint4 *>(base + off);
-        sub = *reinterpret_cast<const Sub *>(base + (off + in));
+        sub = *reinterpret_cast<const Sub *>(base + 16 + so);
     } else {
         const uint64_t off = ((uint64_t)P >> 7) << 6;
         o.C = *reinterpret_cast<const uint4 *>(base + off);
@@ -1271,13 +1276,21 @@ __global__ void __launch_bounds__(256) k_sa_walk(const uint32_t *__restrict__ bw
 // leave the ones still on a read of a million pops. Those reads are parked and gone on with by workgroups of
 // four waves, whose round takes 1024 chains: 4001 reads, the longest of 630k pops, 41 -> 15 ms; 262,144
 // reads 80 -> 44 ms.
+//
+// The log: a thread's own (1 KB a bucket code) touched up to 400 half-filled lines a round, 4.2e9 write
+// requests past L2 for 2M reads; one log per wave in the order of the iterations is 16 bytes after 16 bytes
+// and stays in L2. Its stores are issued after the next step's lookups, which a pop needs the exact child's
+// interval for and nothing else. With choices written as arithmetic instead of branches (186 -> 142 scalar
+// instructions an iteration) and the kernel's cold arguments read where they are used (373 -> 87 static
+// readlanes of spilled scalars): 2M reads 225 -> 210 ms, 100k of 100 bp 7.75 -> 7.17, the 4001 15 -> 13,
+// 100,003 reads of a 700 Mbp repeat-rich genome 142 -> 125.
 
 constexpr int HW = 64;         // lanes of a wave
 constexpr int H_STEPS = 32;    // chain steps per round
-constexpr int H_LOG = 64;      // logged pushes per thread and bucket code
+constexpr int H_LOG = 8192;    // pushes logged per wave and round
 constexpr int H_SPUSH = 9;     // pushes of one step at most
+constexpr int H_CPUSH = 127;   // pushes of a chain and round to one bucket at most (7-bit ranks)
 constexpr int H_SLOG = 64;     // trace build: steps logged per thread
-constexpr int H_CAP = 4096;    // pushes committed per round and wave
 constexpr int H_KEEP = 64;     // granules a workgroup keeps between reads
 constexpr int H_PIECES = 48;   // segment pieces one round may add (three buckets)
 constexpr int H_MINCAP = 128;  // the lowest push cap a test may set
@@ -1285,7 +1298,7 @@ constexpr uint32_t GENT = (uint32_t)GRAN * CH;  // entries per granule, its link
 constexpr uint32_t GFULL = GENT - 1;
 constexpr int H_LOOK = 16;     // rounds between looks at the queue
 constexpr int H_FREE = 32;     // emptied granules kept in LDS
-static_assert(H_LOG <= 120 && H_LOG > 2 * H_SPUSH, "push counts and offsets are 7-bit fields");
+static_assert(H_LOG > 2 * HW * H_SPUSH, "every lane of a wave can log a step's pushes");
 static_assert(H_SLOG >= 2 * H_STEPS, "a chain's steps fit the rest of a thread's step log");
 
 enum : int { K_END = 0, K_HIT = 1, K_TRUNC = 2, K_ESCORE = 3 };
@@ -1328,7 +1341,7 @@ struct HArgs {
     int32_t buckets;  // LDS buckets: the largest n_stacks of the launch
     int32_t wlen;     // LDS widths: longest read + 1
     int32_t swlen;    // LDS seed widths
-    int32_t push_cap; // pushes committed per round (H_CAP per wave unless a test lowers it)
+    int32_t push_cap; // pushes committed per round (more than the logs hold unless a test lowers it)
     // a read that is still running when no other is left to take, after park_pops pops (0: never), is parked:
     // its workgroup writes its state to its scratch, lists itself in park_list and ends; a launch of
     // workgroups of more waves goes on with it
@@ -1362,7 +1375,7 @@ static_assert(sizeof(HShared) % 8 == 0, "the widths follow it in a parked read's
 // what a read's state is besides HShared: the widths, the buckets
 __host__ __device__ inline size_t heavy_state_bytes(int buckets, int wlen, int swlen)
 {
-    return sizeof(HShared) + (size_t)(wlen + 1 + swlen) * 8 + (size_t)buckets * 12;
+    return sizeof(HShared) + (size_t)(wlen + swlen + 2) * 8 + (size_t)buckets * 12;
 }
 
 __device__ __forceinline__ int hbm_low(const unsigned long long *bm)
@@ -1453,13 +1466,15 @@ __device__ __forceinline__ uint64_t trace_item(uint64_t t, int score, uint64_t k
 }
 
 // widths in LDS: the value in the low part, the bound above it (32 bits each below 2^32 symbols, so that
-// neither needs a shift; the 48 | 16 of the hand-off slots otherwise)
+// neither needs a shift; the 48 | 16 of the hand-off slots otherwise). A sentinel before position 0 bounds
+// nothing, so that the first positions need no case of their own.
+constexpr uint32_t NO_BOUND = 0xffffb000u;  // a bound below any number of differences, also as 16 bits
 template <bool WIDE>
-__device__ __forceinline__ uint32_t lw_bid(uint64_t v) { return WIDE ? (uint32_t)(v >> 48) : (uint32_t)(v >> 32); }
+__device__ __forceinline__ int lw_bid(uint64_t v) { return WIDE ? (int)((int64_t)v >> 48) : (int)(v >> 32); }
 template <bool WIDE>
 __device__ __forceinline__ uint64_t lw_val(uint64_t v) { return WIDE ? v & W48 : v & 0xffffffffull; }
 template <bool WIDE>
-__device__ __forceinline__ uint64_t lw_make(uint64_t w, uint32_t bid) { return WIDE ? w | (uint64_t)bid << 48 : w | (uint64_t)bid << 32; }
+__device__ __forceinline__ uint64_t lw_make(uint64_t w, uint32_t bid) { return w | (uint64_t)bid << (WIDE ? 48 : 32); }
 
 // bwt_cal_width by one thread (src/bwtgap_hd.h:216-242); returns the algorithmic bytes. put(i, w, bid)
 // stores position i's width.
@@ -1531,8 +1546,19 @@ __global__ void __launch_bounds__(256) k_widths(WArgs a)
     }
 }
 
+// A wave logs a round's pushes in the order it makes them, 16 bytes after 16 bytes. A logged push holds, beside
+// the entry, its chain, its rank among the chain's pushes to its bucket and the bucket's code, so that it can
+// be placed by itself. A pushed entry's last_diff_pos is its position i (every push is a difference there), so
+// its ten bits are free: rank in y[0:7), and below 2^32 symbols code in x[26:28), chain in y[26:32) and
+// x[28:32); a larger index keeps code and chain in a word per push after the log.
+constexpr int H_CHAIN_BITS = 10;
+constexpr size_t heavy_log_bytes(bool wide) { return (size_t)H_LOG * (sizeof(Ent) + (wide ? 4 : 0)); }
+
 // LDS of a workgroup of nw waves, cpl chains per thread (k_heavy carves it up in this order)
-constexpr size_t heavy_chain_bytes = 16 + 4 + 4 + 4 + 2 + 2;  // head | counts | log place | steps | id | trace place
+constexpr size_t heavy_chain_bytes = 16 + 4 + 4 + 2 + 2;  // head | counts | steps | id | trace place
+
+typedef const __attribute__((address_space(4))) HArgs HArgsC;
+#define HA(f) cold_ld(&((HArgsC *)__builtin_amdgcn_kernarg_segment_ptr())->f)
 
 // NW waves per read; WPE waves per SIMD: 4 at 128 VGPRs, or 5 (96 VGPRs) for indexes in HBM, where a wave
 // waits on its loads.
@@ -1541,7 +1567,7 @@ __global__ void __launch_bounds__(64 * NW) __attribute__((amdgpu_waves_per_eu(WP
 {
     using K = typename Item<WIDE>::K;
     constexpr int T = 64 * NW, KMAX = T * CPL;
-    static_assert(T <= 256, "a thread's index takes 8 bits of its chains' records");
+    static_assert(KMAX <= 1 << H_CHAIN_BITS, "a chain's id in its pushes");
     extern __shared__ __align__(16) uint8_t hlds[];
     // the launch of NW > 1 waves goes on with reads that the launch of one wave parked
     constexpr bool RESUME = NW > 1;
@@ -1549,43 +1575,49 @@ __global__ void __launch_bounds__(64 * NW) __attribute__((amdgpu_waves_per_eu(WP
     Ent *const hent = reinterpret_cast<Ent *>(pieces + H_PIECES);  // live chains' heads, in order
     uint16_t *const epre = reinterpret_cast<uint16_t *>(hent);     // after them: pushes before each chain, by code
     uint32_t *const cA = reinterpret_cast<uint32_t *>(hent + KMAX);  // pushes by code (8 bits each) | stop kind << 24
-    uint32_t *const cB = cA + KMAX;                                  // place in the thread's logs (8 bits each) | thread << 24
-    uint32_t *const cC = cB + KMAX;                                  // steps | index bytes / 64 << 6
+    uint32_t *const cC = cA + KMAX;                                  // steps | index bytes / 64 << 6
     uint16_t *const hcid = reinterpret_cast<uint16_t *>(cC + KMAX);  // live chains' ids
-    uint16_t *const cS = hcid + KMAX;                                // trace build: place in the thread's step log
+    uint16_t *const cS = hcid + KMAX;                                // trace build: place in the step logs
     unsigned long long *const ST = reinterpret_cast<unsigned long long *>(cS + KMAX);  // [16] counters
     HShared &F = *reinterpret_cast<HShared *>(ST + 16);
     uint64_t *const Wp = reinterpret_cast<uint64_t *>(&F + 1);       // Wp[i] = width of position i - 1
-    uint64_t *const SW = Wp + a.wlen + 1;
-    uint32_t *const seg_top = reinterpret_cast<uint32_t *>(SW + a.swlen);  // per bucket: its top granule,
-    uint32_t *const seg_cnt = seg_top + a.buckets;                         // that one's entries (0: empty bucket)
-    uint32_t *const seg_prev = seg_cnt + a.buckets;                        // and the granule below, or NIL
-    uint16_t *const s0info = reinterpret_cast<uint16_t *>(seg_prev + a.buckets);  // chain 0's steps: pushes | index bytes / 64 << 4
+    uint64_t *const SW = Wp + HA(wlen) + 1;                          // SW[i] = seed width of position i - 1
+    uint32_t *const seg_top = reinterpret_cast<uint32_t *>(SW + HA(swlen) + 1);  // per bucket: its top granule,
+    uint32_t *const seg_cnt = seg_top + HA(buckets);                         // that one's entries (0: empty bucket)
+    uint32_t *const seg_prev = seg_cnt + HA(buckets);                        // and the granule below, or NIL
+    uint16_t *const s0info = reinterpret_cast<uint16_t *>(seg_prev + HA(buckets));  // chain 0's steps: pushes | index bytes / 64 << 4
     uint8_t *const QL = reinterpret_cast<uint8_t *>(s0info + H_STEPS);           // the read's query
     static_assert(MAXLEN * 2 + 2 < 4096, "a step's index bytes fit the step info");
 
     const int tid = threadIdx.x, lane = tid & (HW - 1), wave = tid >> 6;
-    if ((int)blockIdx.x >= a.n_slots) return;
-    uint8_t *const base = a.scratch + (uint64_t)blockIdx.x * a.slot_bytes;
-    galn_aln_rec_t *REC = reinterpret_cast<galn_aln_rec_t *>(base + a.rec_off);
-    uint32_t *OWN = reinterpret_cast<uint32_t *>(base + a.own_off);
-    uint32_t *SPILL = reinterpret_cast<uint32_t *>(base + a.spill_off);
-    Ent *const LOG = reinterpret_cast<Ent *>(base + a.plog_off);     // code c, thread t: [(c * T + t) * H_LOG]
-    Ent *const SLOG = reinterpret_cast<Ent *>(base + a.slog_off);    // trace build: thread t's steps at t * H_SLOG
+    if ((int)blockIdx.x >= HA(n_slots)) return;
+    uint8_t *const base = HA(scratch) + (uint64_t)blockIdx.x * HA(slot_bytes);
+    galn_aln_rec_t *REC = reinterpret_cast<galn_aln_rec_t *>(base + HA(rec_off));
+    uint32_t *OWN = reinterpret_cast<uint32_t *>(base + HA(own_off));
+    uint32_t *SPILL = reinterpret_cast<uint32_t *>(base + HA(spill_off));
+    // this wave's pushes of the round (all waves' entries, then their words)
+    Ent *const LOG = reinterpret_cast<Ent *>(base + HA(plog_off)) + wave * H_LOG;
+    uint32_t *const LOGW = reinterpret_cast<uint32_t *>(reinterpret_cast<Ent *>(base + HA(plog_off)) + NW * H_LOG) + wave * H_LOG;
+    Ent *const SLOG = reinterpret_cast<Ent *>(base + HA(slog_off));    // trace build: thread t's steps at t * H_SLOG
     uint8_t *const SINFO = reinterpret_cast<uint8_t *>(SLOG + T * H_SLOG);  // and their push counts
     Ent *const POOL = a.pool;
     const DMeta &M = a.meta;
+    // (arguments not used in the lookups are read from the kernel argument segment where they are used: held
+    // in scalar registers for the whole kernel they spilled, and a fifth of the vector instructions were
+    // reads of spilled ones)
     const K seq_len = (K)M.seq_len;
 
     if (tid == 0) {
         for (int j = 0; j < 16; ++j) ST[j] = 0;
-        F.n_own = RESUME ? 0 : a.first_gran;  // granules this workgroup holds; a read reuses them before taking more
+        F.n_own = RESUME ? 0 : HA(first_gran);  // granules this workgroup holds; a read reuses them before taking more
     }
-    if (!RESUME && tid < a.first_gran) OWN[tid] = F.own[tid] = blockIdx.x * (uint32_t)a.first_gran + (uint32_t)tid;
-    const int n_list = a.n_list_dev ? *a.n_list_dev : a.n_list;
+    if (!RESUME && tid < HA(first_gran)) OWN[tid] = F.own[tid] = blockIdx.x * (uint32_t)HA(first_gran) + (uint32_t)tid;
+    const int n_list = HA(n_list_dev) ? *HA(n_list_dev) : HA(n_list);
+    const bool stats = HA(stats) != nullptr;
+    const int state_words = (int)(heavy_state_bytes(HA(buckets), HA(wlen), HA(swlen)) / 4);
     for (;;) {
-        const long long t_read = a.stats ? wall_clock64() : 0;
-        if (tid == 0) F.claim = atomicAdd(a.qnext, 1);
+        const long long t_read = stats ? wall_clock64() : 0;
+        if (tid == 0) F.claim = atomicAdd(HA(qnext), 1);
         __syncthreads();
         const int claim = F.claim;
         if (claim >= n_list) break;
@@ -1593,29 +1625,30 @@ __global__ void __launch_bounds__(64 * NW) __attribute__((amdgpu_waves_per_eu(WP
         int rid, len;
         if constexpr (RESUME) {
             // a parked read: its state, and its records and granules where its workgroup kept them
-            uint8_t *const pb = a.park_scratch + (uint64_t)a.park_list[claim] * a.park_slot_bytes;
-            const uint32_t *const st = reinterpret_cast<const uint32_t *>(pb + a.park_state_off);
+            uint8_t *const pb = HA(park_scratch) + (uint64_t)HA(park_list)[claim] * HA(park_slot_bytes);
+            const uint32_t *const st = reinterpret_cast<const uint32_t *>(pb + HA(park_state_off));
             __syncthreads();  // (F.claim is part of it)
-            for (int j = tid; j < (int)(heavy_state_bytes(a.buckets, a.wlen, a.swlen) / 4); j += T)
+            for (int j = tid; j < state_words; j += T)
                 reinterpret_cast<uint32_t *>(&F)[j] = st[j];
-            REC = reinterpret_cast<galn_aln_rec_t *>(pb + a.park_rec_off);
-            OWN = reinterpret_cast<uint32_t *>(pb + a.park_own_off);
-            SPILL = reinterpret_cast<uint32_t *>(pb + a.park_spill_off);
+            REC = reinterpret_cast<galn_aln_rec_t *>(pb + HA(park_rec_off));
+            OWN = reinterpret_cast<uint32_t *>(pb + HA(park_own_off));
+            SPILL = reinterpret_cast<uint32_t *>(pb + HA(park_spill_off));
             __syncthreads();
             rid = F.rid;
             len = F.len;
-            const uint8_t *const qg = a.query + a.qoff[rid];
+            const uint8_t *const qg = HA(query) + HA(qoff)[rid];
             for (int j = tid; j < len; j += T) QL[j] = qg[j];
             __syncthreads();
         } else {
             const int pos = claim;
-            rid = a.list ? a.list[pos] : pos;
-            len = a.qlen[rid];
-            const uint8_t *const qg = a.query + a.qoff[rid];
-            for (int j = tid; j < len && j < a.wlen; j += T) QL[j] = qg[j];
+            rid = HA(list) ? HA(list)[pos] : pos;
+            len = HA(qlen)[rid];
+            const uint8_t *const qg = HA(query) + HA(qoff)[rid];
+            const int qn = min(len, HA(wlen));
+            for (int j = tid; j < qn; j += T) QL[j] = qg[j];
             if (tid == 0) {
-                const int b0 = a.batch[rid];
-                const galn_search_opt_t o = a.bopts[b0];
+                const int b0 = HA(batch)[rid];
+                const galn_search_opt_t o = HA(bopts)[b0];
                 F.rid = rid;
                 F.len = len;
                 F.s_mm = o.s_mm;
@@ -1629,8 +1662,8 @@ __global__ void __launch_bounds__(64 * NW) __attribute__((amdgpu_waves_per_eu(WP
                 F.max_gape = o.max_gape;
                 F.msd = o.max_seed_diff;
                 F.max_top2 = o.max_top2;
-                F.n_stacks = a.nstacks[b0];
-                F.md_read = a.maxdiff[rid];
+                F.n_stacks = HA(nstacks)[b0];
+                F.md_read = HA(maxdiff)[rid];
                 F.seed_len = o.seed_len;
                 F.seeding = o.seed_len < len;
                 F.nN = 0;
@@ -1642,22 +1675,22 @@ __global__ void __launch_bounds__(64 * NW) __attribute__((amdgpu_waves_per_eu(WP
                 F.bad = 0;
             }
             __syncthreads();
-            const bool unsup = len < 1 || len > MAXLEN || len + 1 > a.wlen || F.n_stacks > a.buckets || F.md_read > MAXDIFF ||
+            const bool unsup = len < 1 || len > MAXLEN || len + 1 > HA(wlen) || F.n_stacks > HA(buckets) || F.md_read > MAXDIFF ||
                                F.max_gapo > MAXDIFF || F.max_gapo + F.max_gape > 255;
-            const uint64_t h0 = (!unsup && a.hand && pos < a.hand_cap) ? a.hand[(uint64_t)pos * a.hand_stride] : 0;
+            const uint64_t h0 = (!unsup && HA(hand) && pos < HA(hand_cap)) ? HA(hand)[(uint64_t)pos * HA(hand_stride)] : 0;
             if (!unsup) {
                 if (h0 >> 63) {
                     // the widths computed for this read
-                    const uint64_t *src = a.hand + (uint64_t)pos * a.hand_stride;
+                    const uint64_t *src = HA(hand) + (uint64_t)pos * HA(hand_stride);
                     for (int j = tid; j <= len; j += T) Wp[1 + j] = lw_make<WIDE>(wval(src[1 + j]), (uint32_t)wbid(src[1 + j]));
                     if (F.seeding)
                         for (int j = tid; j <= F.seed_len; j += T)
-                            SW[j] = lw_make<WIDE>(wval(src[2 + len + j]), (uint32_t)wbid(src[2 + len + j]));
+                            SW[1 + j] = lw_make<WIDE>(wval(src[2 + len + j]), (uint32_t)wbid(src[2 + len + j]));
                     if (tid == 0) F.obytes = h0 & ~(1ull << 63);
                 } else {
                     uint64_t wb = 0;
                     auto putw = [Wp](int i, uint64_t v, int bid) { Wp[1 + i] = lw_make<WIDE>(v, (uint32_t)bid); };
-                    auto puts = [SW](int i, uint64_t v, int bid) { SW[i] = lw_make<WIDE>(v, (uint32_t)bid); };
+                    auto puts = [SW](int i, uint64_t v, int bid) { SW[1 + i] = lw_make<WIDE>(v, (uint32_t)bid); };
                     if (tid == 0) wb = cal_width_one(a.bwt, M, len, QL, putw);
                     if (tid == 1 && F.seeding) wb = cal_width_one(a.bwt, M, F.seed_len, QL + (len - F.seed_len), puts);
                     if (wb) atomicAdd(&F.obytes, (unsigned long long)wb);
@@ -1666,7 +1699,8 @@ __global__ void __launch_bounds__(64 * NW) __attribute__((amdgpu_waves_per_eu(WP
                 for (int j = tid; j < len; j += T) nN += QL[j] > 3;
                 if (nN) atomicAdd(&F.nN, nN);
             }
-            for (int j = tid; j < a.buckets; j += T) seg_cnt[j] = 0;
+            const int nbk = HA(buckets);
+            for (int j = tid; j < nbk; j += T) seg_cnt[j] = 0;
             __syncthreads();
             // ---- search set-up ----
             if (tid == 0) {
@@ -1680,7 +1714,7 @@ __global__ void __launch_bounds__(64 * NW) __attribute__((amdgpu_waves_per_eu(WP
                 F.bm[0] = F.bm[1] = F.bm[2] = F.bm[3] = 0;
                 F.has_pend = 0;
                 F.n_entries = 0;
-                Wp[0] = 0;
+                Wp[0] = SW[0] = lw_make<WIDE>(0, NO_BOUND);
                 if (unsup) {
                     F.status = 1;
                     F.result = ERR_UNSUP;
@@ -1702,7 +1736,7 @@ __global__ void __launch_bounds__(64 * NW) __attribute__((amdgpu_waves_per_eu(WP
             }
             __syncthreads();
         }
-        if (a.stats && tid == 0) {
+        if (stats && tid == 0) {
             ST[12] += (unsigned long long)(wall_clock64() - t_read);
             if (!RESUME) ST[15] += 1;
         }
@@ -1710,18 +1744,18 @@ __global__ void __launch_bounds__(64 * NW) __attribute__((amdgpu_waves_per_eu(WP
         int n_round = 0;
         long long t_round_end = 0;  // with stats: end of the last round's commit
         for (;;) {
-            const long long t_round = a.stats ? wall_clock64() : 0;
-            if (a.stats && tid == 0 && t_round_end) ST[14] += (unsigned long long)(t_round - t_round_end);
+            const long long t_round = stats ? wall_clock64() : 0;
+            if (stats && tid == 0 && t_round_end) ST[14] += (unsigned long long)(t_round - t_round_end);
             int taken_reads = 0;
             if (tid == 0 && F.status == 0) {  // (the others read the status after the barrier)
                 // reads taken so far, looked at when this round has been committed. One load in H_LOOK rounds:
                 // all workgroups loading this word every round made a round 50% longer. With a workgroup for
                 // every read each takes its own, whatever the others do.
-                if (!RESUME && a.park_pops && F.pops >= a.park_pops) {
-                    if (n_list <= a.n_slots)
+                if (!RESUME && HA(park_pops) && F.pops >= HA(park_pops)) {
+                    if (n_list <= HA(n_slots))
                         taken_reads = n_list;
                     else if ((++n_round & (H_LOOK - 1)) == 0)
-                        taken_reads = __hip_atomic_load(a.qnext, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+                        taken_reads = __hip_atomic_load(HA(qnext), __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
                 }
                 // a pending exact child is the top of the lowest bucket (the bucket it came from)
                 const int b = F.has_pend ? F.b : hbm_low(F.bm);
@@ -1763,8 +1797,8 @@ __global__ void __launch_bounds__(64 * NW) __attribute__((amdgpu_waves_per_eu(WP
             __syncthreads();
             if (F.status) break;
             const int b = F.b, nK = F.K, hp = F.has_pend;
-            const long long t_spec = a.stats ? wall_clock64() : 0;
-            if (a.stats && tid == 0) ST[13] += (unsigned long long)(t_spec - t_round);
+            const long long t_spec = stats ? wall_clock64() : 0;
+            if (stats && tid == 0) ST[13] += (unsigned long long)(t_spec - t_round);
             const int s_mm = F.s_mm, s_gapo = F.s_gapo, s_gape = F.s_gape, mode = F.mode, max_diff = F.max_diff;
             const int n_stacks = F.n_stacks, max_gapo = F.max_gapo, max_gape = F.max_gape, ies = F.ies, mdo = F.mdo;
             const int msd = F.msd, sofs = len - F.seed_len;
@@ -1807,10 +1841,9 @@ __global__ void __launch_bounds__(64 * NW) __attribute__((amdgpu_waves_per_eu(WP
                     if (!TRACE && live) {
                         const int m = left(max_diff, h[r].x, h[r].y);
                         const uint32_t i0 = h[r].x & X_I;
-                        if (m < 0 || (i0 > 0 && m < (int)lw_bid<WIDE>(Wp[i0]))) {
+                        if (m < 0 || (i0 > 0 && m < lw_bid<WIDE>(Wp[i0]))) {
                             live = false;
                             cA[c] = 0;
-                            cB[c] = 0;
                             cC[c] = 1;  // one pop, no lookup
                             if (c == 0) s0info[0] = 0;
                         }
@@ -1841,245 +1874,272 @@ __global__ void __launch_bounds__(64 * NW) __attribute__((amdgpu_waves_per_eu(WP
 #pragma unroll
             for (int w = 0; w < NW; ++w) nlive += F.wlive[w];
             // ---- speculation: every thread runs chains, one lookup an iteration, and takes the next live
-            // one when its own has ended ----
+            // one when its own has ended. A step's children are logged while the next step's lookups are on
+            // their way ----
             int next = T, stop = 0x7fffffff, its = 0;  // (NW > 1: the claims and the stop are F.next, F.stop)
-            uint32_t np3 = 0, o3 = 0;                  // logged pushes by code, 8 bits each; at the chain's start
+            uint32_t wl = 0;                           // pushes this wave has logged
+            uint64_t stopped = 0;                      // lanes whose chain has stopped
+            bool more = true;                          // (uniform) chains are left to take
+            // the chain: its pushes by bucket code (8 bits each), pops, index bytes / 64
+            uint32_t np3 = 0, sby = 0;
             int cid = -1, kind = K_END, steps = 0, m = 0, m_seed = 0, so = 0, sl = 0;
-            uint32_t sby = 0, sp = 0, spb = 0;  // index bytes / 64 of the chain; pushes, bytes of its last pop
-            bool busy = false, fin = false, tail = false;
+            bool busy = false, tail = false;
             K k = 0, l = 0;
             uint32_t x = 0, y = 0;
-            constexpr uint32_t ROOM = 0x010101u * (uint32_t)(127 - (H_LOG - H_SPUSH));  // sets bit 7 of a full log's count
-            bool first = true;
+            // children not yet logged: bit 0 an insertion, bits 1-4 deletions by base, bits 5-8 mismatches in
+            // their order, bits 9-10 the query's base, bit 11 the gap is opened; their chain, its pushes before
+            // them, and what they are made of
+            uint32_t ch = 0, p_np3, p_x, p_y;
+            int p_cid;
+            K pk, pl, ca[4], cb[4];
+            constexpr uint32_t ROOM = 0x010101u * (uint32_t)(127 - (H_CPUSH - H_SPUSH));  // sets bit 7 of a full count
+            constexpr uint32_t LOG_FULL = H_LOG - 2 * HW * H_SPUSH;
+            const bool near = F.n_entries + H_STEPS * H_SPUSH > F.max_entries;  // chain 0 may cross the limit
+            auto finish = [&]() __attribute__((always_inline)) {
+                cA[cid] = np3 | (uint32_t)kind << 24;
+                cC[cid] = (uint32_t)steps | sby << 6;
+                if (TRACE) cS[cid] = (uint16_t)(tid * H_SLOG + so);
+                if (NW > 1 && kind != K_END) atomicMin(&F.stop, cid);
+                busy = false;
+            };
+            // pop the entry in k, l, x, y (w: the width of the position before its own): it dies, is a hit, or
+            // needs a lookup (src/bwtgap_hd.h:369-396)
+            auto pop = [&](uint64_t w) __attribute__((always_inline)) {
+                if (TRACE) {
+                    put_item<WIDE>(SLOG + tid * H_SLOG + sl, k, l, x, y);
+                    SINFO[tid * H_SLOG + sl] = 0;
+                    ++sl;
+                }
+                if (near && cid == 0) s0info[steps] = 0;
+                ++steps;
+                tail = m == 0 && ((x & X_ST) == 0 || (mode & MODE_GAPE) || y_ge(y) == max_gape);
+                const bool dead = m < max(lw_bid<WIDE>(w), 0);
+                if (dead || (x & X_I) == 0) {
+                    kind = dead ? K_END : K_HIT;
+                    finish();
+                }
+            };
+            auto take = [&](int p) __attribute__((always_inline)) {
+                const Item<WIDE> e = get_item<WIDE>(hent + p);
+                cid = hcid[p];
+                k = e.k;
+                l = e.l;
+                x = e.x;
+                y = e.y;
+                m = left(max_diff, x, y);
+                m_seed = left(msd, x, y);
+                steps = 0;
+                sby = 0;
+                np3 = 0;
+                so = sl;
+                busy = true;
+                pop(Wp[x & X_I]);
+            };
+            if (tid < nlive) take(tid);
             for (;;) {
-                const bool want = !busy && !fin && ((np3 + ROOM) & 0x808080u) == 0 && (!TRACE || sl <= H_SLOG - H_STEPS);
-                if (!busy && !want) fin = true;
-                const uint64_t wm = __ballot(want);
-                if (wm) {
-                    int p;
-                    if (first) {
-                        p = tid;
-                    } else if (NW == 1) {
-                        p = next + lanes_below(wm);
-                        next += __builtin_popcountll(wm);
-                    } else {
-                        int g = 0;
-                        const int leader = __builtin_ctzll(wm);
-                        if (lane == leader) g = atomicAdd(&F.next, __builtin_popcountll(wm));
-                        p = __shfl(g, leader) + lanes_below(wm);
-                    }
-                    if (want) {
-                        fin = true;
-                        if (p < nlive) {
-                            const int c = hcid[p];
-                            if (c < (NW == 1 ? stop : __hip_atomic_load(&F.stop, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_WORKGROUP))) {
-                                const Item<WIDE> e = get_item<WIDE>(hent + p);
-                                fin = false;
-                                busy = true;
-                                tail = false;
-                                cid = c;
-                                k = e.k;
-                                l = e.l;
-                                x = e.x;
-                                y = e.y;
-                                m = left(max_diff, x, y);
-                                m_seed = left(msd, x, y);
-                                steps = 0;
-                                sby = 0;
-                                o3 = np3;
-                                so = sl;
+                if (more) {
+                    const uint64_t wm = __ballot(!busy && kind == K_END && (!TRACE || sl <= H_SLOG - H_STEPS));
+                    if (wm) {
+                        int g;
+                        if (NW == 1) {
+                            g = next;
+                            next += __builtin_popcountll(wm);
+                            more = next < nlive;
+                        } else {
+                            g = 0;
+                            if (lane == 0) {
+                                if (__hip_atomic_load(&F.stop, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_WORKGROUP) == 0x7fffffff)
+                                    g = atomicAdd(&F.next, __builtin_popcountll(wm));
+                                else
+                                    g = nlive;
                             }
+                            g = __builtin_amdgcn_readlane(g, 0);
+                            more = g + __builtin_popcountll(wm) < nlive;
                         }
+                        const int p = g + lanes_below(wm);
+                        if ((wm >> lane & 1ull) && p < nlive) take(p);
                     }
                 }
-                first = false;
-                if (!__ballot(busy)) break;
-                ++its;
-                bool ended = false;
+                const uint64_t run_m = __ballot(busy);
+                uint32_t qb = 0, i0 = 0;
+                uint64_t wA = 0, wB = 0;
+                K Pk = 0, Pl = 0;
+                OccWord A, B;
                 if (busy) {
-                    const uint32_t i0 = x & X_I;
-                    uint64_t wB = 0;
-                    if (!tail) {
-                        // a pop
-                        if (TRACE) {
-                            put_item<WIDE>(SLOG + tid * H_SLOG + sl, k, l, x, y);
-                            ++sl;
+                    i0 = x & X_I;
+                    Pk = pos_k<K>(M, k);
+                    Pl = pos_l<K>(M, l);
+                    occ_load<K>(a.bwt, Pk, A);
+                    occ_load<K>(a.bwt, Pl, B);
+                    qb = QL[i0 - 1];
+                    wA = Wp[i0 - 1];
+                    wB = Wp[i0];
+                }
+                // ---- the last step's children to the log, each lane's after those of the lanes before it ----
+                if (__ballot((ch & 511u) != 0)) {
+                    const uint32_t nch = __builtin_popcount(ch & 511u);
+                    const uint32_t incl = wave_incl_scan(nch);
+                    if (nch) {
+                        uint32_t at = wl + incl - nch;
+                        const uint32_t tag_x = (uint32_t)p_cid >> 6 << 28, tag_y = (uint32_t)p_cid << 26;
+                        auto put = [&](K ck, K cl, uint32_t cx, uint32_t cy, uint32_t code, uint32_t rank) __attribute__((always_inline)) {
+                            if constexpr (WIDE) {
+                                put_item<WIDE>(LOG + at, ck, cl, cx, cy | rank);
+                                LOGW[at] = (uint32_t)p_cid | code << H_CHAIN_BITS;
+                            } else {
+                                put_item<WIDE>(LOG + at, ck, cl, cx, cy + rank);
+                            }
+                            ++at;
+                        };
+                        if (ch & 31u) {
+                            const bool open = (ch >> 11 & 1u) != 0;
+                            const uint32_t sh = open ? (uint32_t)sh1 : (uint32_t)sh2, code = sh >> 3;
+                            uint32_t xg = p_x + (open ? X_GO : 0u), yg = p_y + (open ? 0u : Y_GE), rank = (p_np3 >> sh) & 127u;
+                            if (!WIDE) {
+                                xg |= code << 26 | tag_x;
+                                yg |= tag_y;
+                            }
+                            if (ch & 1u) put(pk, pl, (xg - 1) | X_INS, yg + Y_IN, code, rank++);
+#pragma unroll
+                            for (int j = 0; j < 4; ++j)
+                                if (ch >> (1 + j) & 1u) put(ca[j] + 1, cb[j], xg | X_DEL, yg, code, rank++);
+                            p_np3 += (uint32_t)__builtin_popcount(ch & 31u) << sh;
                         }
-                        ++steps;
-                        sp = 0;
-                        spb = 0;
-                        wB = Wp[i0];
-                        if (i0 == 0 && m >= 0) {
-                            ended = true;
-                            kind = K_HIT;
-                        } else if (m < 0 || m < (int)lw_bid<WIDE>(wB)) {
-                            ended = true;  // pruned
-                        } else if (m == 0 && ((x & X_ST) == 0 || (mode & MODE_GAPE) || y_ge(y) == max_gape)) {
-                            tail = true;
+                        if (ch >> 5 & 15u) {
+                            // slot t of the rotated intervals holds base (query base + t) & 3, the mismatches' order
+                            const bool r1 = (ch >> 9 & 1u) != 0, r2 = (ch >> 10 & 1u) != 0;
+                            const K k0 = r1 ? ca[1] : ca[0], k1 = r1 ? ca[2] : ca[1], k2 = r1 ? ca[3] : ca[2], k3 = r1 ? ca[0] : ca[3];
+                            const K l0 = r1 ? cb[1] : cb[0], l1 = r1 ? cb[2] : cb[1], l2 = r1 ? cb[3] : cb[2], l3 = r1 ? cb[0] : cb[3];
+                            uint32_t rank = p_np3 & 127u, xm = p_x - 1 + X_MM, ym = p_y;
+                            if (!WIDE) {
+                                xm |= tag_x;
+                                ym |= tag_y;
+                            }
+                            if (ch & 32u) put((r2 ? k3 : k1) + 1, r2 ? l3 : l1, xm, ym, 0u, rank++);
+                            if (ch & 64u) put((r2 ? k0 : k2) + 1, r2 ? l0 : l2, xm, ym, 0u, rank++);
+                            if (ch & 128u) put((r2 ? k1 : k3) + 1, r2 ? l1 : l3, xm, ym, 0u, rank++);
+                            if (ch & 256u) put((r2 ? k2 : k0) + 1, r2 ? l2 : l0, xm, ym, 0u, rank++);
                         }
+                        ch = 0;
                     }
-                    if (!ended) {
-                        const uint32_t qb = QL[i0 - 1];
-                        const K Pk = pos_k<K>(M, k), Pl = pos_l<K>(M, l);
-                        OccWord A, B;
-                        occ_load<K>(a.bwt, Pk, A);
-                        occ_load<K>(a.bwt, Pl, B);
-                        const uint64_t wA = Wp[i0 - 1];
-                        const uint32_t units = occ_units<K>(Pk, Pl);
-                        K ca[4], cb[4];
-                        occ_count<K>(M, WIDE, A, Pk, ca);
-                        occ_count<K>(M, WIDE, B, Pl, cb);
-                        if (tail) {
-                            // exact tail: bwt_match_exact_alt, src/bwtgap_hd.h:195-211
-                            ended = true;
-                            if (qb <= 3) {
-                                spb += units;
-                                const K kk = pick4(ca, (int)qb) + 1, ll = pick4(cb, (int)qb);
-                                if (kk <= ll) {
-                                    k = kk;
-                                    l = ll;
-                                    x -= 1;
-                                    if (i0 > 1)
-                                        ended = false;
-                                    else if ((uint32_t)(ll - kk + 1) != 0)
-                                        kind = K_HIT;
-                                }
+                    wl += (uint32_t)__builtin_amdgcn_readlane((int)incl, HW - 1);
+                    if (wl > LOG_FULL) more = false;
+                }
+                if (!run_m) break;
+                ++its;
+                if (busy) {
+                    const uint32_t units = occ_units<K>(Pk, Pl);
+                    occ_count<K>(M, WIDE, A, Pk, ca);
+                    occ_count<K>(M, WIDE, B, Pl, cb);
+                    const bool at0 = near && cid == 0;
+                    // the exact child's interval
+                    const K xk = pick4(ca, (int)qb) + 1, xl = pick4(cb, (int)qb);
+                    const bool ex = qb <= 3 && xk <= xl;
+                    if (tail) {
+                        // exact tail: bwt_match_exact_alt, src/bwtgap_hd.h:195-211
+                        if (qb <= 3) {
+                            sby += units;
+                            if (at0) s0info[steps - 1] += (uint16_t)(units << 4);
+                        }
+                        if (ex && i0 > 1) {
+                            k = xk;
+                            l = xl;
+                            x -= 1;
+                        } else {
+                            if (ex && (uint32_t)(xl - xk + 1) != 0) {
+                                kind = K_HIT;
+                                k = xk;
+                                l = xl;
+                            }
+                            finish();
+                        }
+                    } else {
+                        // expansion: src/bwtgap_hd.h:412-470. The widths before position 0 (and before the seed)
+                        // bound nothing.
+                        sby += units;
+                        const int i = (int)i0 - 1, ge = y_ge(y), go = x_go(x);
+                        const int bA = lw_bid<WIDE>(wA);
+                        bool allow_diff = bA < m;
+                        bool allow_M = !(bA == m - 1 && wA == wB);
+                        if (seeding) {
+                            const uint64_t *const s = SW + max(i - sofs, 0);
+                            const uint64_t sA = s[0], sB = s[1];
+                            const int bS = lw_bid<WIDE>(sA);
+                            allow_diff = allow_diff && bS < m_seed;
+                            allow_M = allow_M && !(bS == m_seed - 1 && sA == sB);
+                        }
+                        const uint32_t st = x & X_ST;
+                        const bool open = st == 0;
+                        // bases that occur, and in the mismatches' order: bit t base (qb + t) & 3
+                        const uint32_t e4 = (ca[0] < cb[0] ? 1u : 0u) | (ca[1] < cb[1] ? 2u : 0u) | (ca[2] < cb[2] ? 4u : 0u) |
+                                            (ca[3] < cb[3] ? 8u : 0u);
+                        const uint32_t rot = (e4 * 17u) >> (qb & 3u);
+                        // gap children: opened by an entry that ends in a match, or extended
+                        const int tmp = (mode & MODE_LOGGAP) ? int_log2((uint32_t)(ge + go)) / 2 + 1 : go + ge;
+                        const bool gap = allow_diff && min(i, len - i) >= ies + tmp && (open ? go < max_gapo : ge < max_gape);
+                        const bool del = st != X_INS && (open || ge + go < max_diff || (uint64_t)(K)(l - k + 1) < (uint64_t)(int64_t)mdo);
+                        ch = gap ? (st != X_DEL ? 1u : 0u) | (del ? e4 << 1 : 0u) : 0u;
+                        const int tg = open ? tg1 : tg2;
+                        if (ch && (tg < 0 || tg >= n_stacks)) {
+                            kind = K_ESCORE;
+                            ch = 0;
+                        } else if (allow_diff && allow_M) {
+                            // mismatches, all four bases at an N
+                            const uint32_t mm = (rot >> 1 & 7u) | (qb > 3 ? (rot & 1u) << 3 : 0u);
+                            if (mm && (tg0 < 0 || tg0 >= n_stacks))
+                                kind = K_ESCORE;
+                            else
+                                ch |= mm << 5;
+                        }
+                        p_np3 = np3;
+                        p_x = x & ~X_ST;
+                        p_y = y & ~Y_LDP;
+                        p_cid = cid;
+                        pk = k;
+                        pl = l;
+                        np3 += (uint32_t)__builtin_popcount(ch & 31u) << (open ? sh1 : sh2);
+                        np3 += (uint32_t)__builtin_popcount(ch >> 5);
+                        if (at0) s0info[steps - 1] = (uint16_t)(__builtin_popcount(ch) | units << 4);
+                        if (TRACE) SINFO[tid * H_SLOG + sl - 1] = (uint8_t)__builtin_popcount(ch);
+                        ch |= qb << 9 & 0x600u;
+                        ch |= open ? 0x800u : 0u;
+                        if (kind == K_END && ex) {
+                            // the exact child is popped next, or (the round's steps or the log used up) in the
+                            // next round
+                            k = xk;
+                            l = xl;
+                            x = p_x - 1;
+                            y = p_y;
+                            if (steps == H_STEPS || wl > LOG_FULL || ((np3 + ROOM) & 0x808080u) != 0) {
+                                kind = K_TRUNC;
+                                finish();
+                            } else {
+                                pop(wA);
                             }
                         } else {
-                            // expansion: src/bwtgap_hd.h:412-470
-                            spb = units;
-                            const int i = (int)i0 - 1;
-                            bool allow_diff = true, allow_M = true;
-                            if (i > 0) {
-                                const int bA = (int)lw_bid<WIDE>(wA);
-                                if (bA > m - 1)
-                                    allow_diff = false;
-                                else if (bA == m - 1 && wA == wB)
-                                    allow_M = false;
-                                if (seeding) {
-                                    const int ii = i - sofs;
-                                    if (ii > 0) {
-                                        const uint64_t sA = SW[ii - 1], sB = SW[ii];
-                                        const int b_s = (int)lw_bid<WIDE>(sA);
-                                        if (b_s > m_seed - 1)
-                                            allow_diff = false;
-                                        else if (b_s == m_seed - 1 && sA == sB)
-                                            allow_M = false;
-                                    }
-                                }
-                            }
-                            const int ge = y_ge(y), go = x_go(x);
-                            const uint32_t st = x & X_ST, xb = x & ~X_ST, yb = y & ~Y_LDP;
-                            if (allow_diff) {
-                                const int tmp = (mode & MODE_LOGGAP) ? int_log2((uint32_t)(ge + go)) / 2 + 1 : go + ge;
-                                if (i >= ies + tmp && len - i >= ies + tmp) {
-                                    // gap children: opened by an entry that ends in a match, or extended
-                                    const bool open = st == 0;
-                                    const bool may = open ? go < max_gapo : ge < max_gape;
-                                    const bool ins = may && st != X_DEL;
-                                    const bool del = may && st != X_INS &&
-                                                     (open || ge + go < max_diff || (uint64_t)(K)(l - k + 1) < (uint64_t)(int64_t)mdo);
-                                    const uint32_t dm = !del ? 0u
-                                                             : (ca[0] < cb[0] ? 1u : 0u) | (ca[1] < cb[1] ? 2u : 0u) |
-                                                                   (ca[2] < cb[2] ? 4u : 0u) | (ca[3] < cb[3] ? 8u : 0u);
-                                    if (ins || dm) {
-                                        const int tg = open ? tg1 : tg2, sh = open ? sh1 : sh2;
-                                        if (tg < 0 || tg >= n_stacks) {
-                                            kind = K_ESCORE;
-                                        } else {
-                                            Ent *d = LOG + ((sh >> 3) * T + tid) * H_LOG + ((np3 >> sh) & 127u);
-                                            const uint32_t xg = xb + (open ? X_GO : 0u), yg = yb + (open ? 0u : Y_GE);
-                                            if (ins) put_item<WIDE>(d++, k, l, (xg - 1) | X_INS, (yg + Y_IN) | (uint32_t)i);
-#pragma unroll
-                                            for (int j = 0; j < 4; ++j)
-                                                if (dm >> j & 1u) put_item<WIDE>(d++, ca[j] + 1, cb[j], xg | X_DEL, yg | i0);
-                                            const uint32_t n = (ins ? 1u : 0u) + __builtin_popcount(dm);
-                                            np3 += n << sh;
-                                            sp += n;
-                                        }
-                                    }
-                                }
-                            }
-                            ended = true;
-                            if (kind == K_END) {
-                                // the intervals rotated so that slot t holds base (qb + t) & 3, the order of the
-                                // mismatch loop
-                                const bool r1 = (qb & 1u) != 0, r2 = (qb & 2u) != 0;
-                                K RK[4], RL[4], TK[4], TL[4];
-#pragma unroll
-                                for (int t = 0; t < 4; ++t) {
-                                    TK[t] = r1 ? ca[(t + 1) & 3] : ca[t];
-                                    TL[t] = r1 ? cb[(t + 1) & 3] : cb[t];
-                                }
-#pragma unroll
-                                for (int t = 0; t < 4; ++t) {
-                                    RK[t] = r2 ? TK[(t + 2) & 3] : TK[t];
-                                    RL[t] = r2 ? TL[(t + 2) & 3] : TL[t];
-                                }
-                                const bool x0 = RK[0] < RL[0];
-                                if (allow_diff && allow_M) {
-                                    // mismatches: the other bases in order, and all four of them at an N
-                                    const uint32_t mmk = (RK[1] < RL[1] ? 1u : 0u) | (RK[2] < RL[2] ? 2u : 0u) |
-                                                         (RK[3] < RL[3] ? 4u : 0u) | (qb > 3 && x0 ? 8u : 0u);
-                                    if (mmk) {
-                                        if (tg0 < 0 || tg0 >= n_stacks) {
-                                            kind = K_ESCORE;
-                                        } else {
-                                            Ent *d = LOG + tid * H_LOG + (np3 & 127u);
-                                            const uint32_t xm = xb - 1 + X_MM, ym = yb | (uint32_t)i;
-#pragma unroll
-                                            for (int t = 1; t <= 4; ++t)
-                                                if (mmk >> (t - 1) & 1u) put_item<WIDE>(d++, RK[t & 3] + 1, RL[t & 3], xm, ym);
-                                            const uint32_t n = __builtin_popcount(mmk);
-                                            np3 += n;
-                                            sp += n;
-                                        }
-                                    }
-                                }
-                                if (kind == K_END && qb <= 3 && x0) {
-                                    // the exact child, popped next
-                                    k = RK[0] + 1;
-                                    l = RL[0];
-                                    x = xb - 1;
-                                    y = yb;
-                                    ended = false;
-                                    if (steps == H_STEPS || ((np3 + ROOM) & 0x808080u) != 0) {
-                                        ended = true;
-                                        kind = K_TRUNC;  // it goes on in the next round
-                                    }
-                                }
-                            }
-                            sby += spb;
+                            finish();
                         }
-                    }
-                    if (tail && ended) sby += spb;
-                    if (cid == 0) s0info[steps - 1] = (uint16_t)(sp | spb << 4);
-                    if (TRACE) SINFO[tid * H_SLOG + sl - 1] = (uint8_t)sp;
-                    if (ended) {
-                        cA[cid] = (np3 - o3) | (uint32_t)kind << 24;
-                        cB[cid] = o3 | (uint32_t)tid << 24;
-                        cC[cid] = (uint32_t)steps | sby << 6;
-                        if (TRACE) cS[cid] = (uint16_t)so;
-                        busy = false;
-                        if (kind != K_END) fin = true;  // what it stopped with stays in its registers
                     }
                 }
                 // the first chain that stops (a hit, a truncation, a score error): those after it run again
                 // in the next round
-                const uint64_t sm = __ballot(ended && kind != K_END);
-                if (sm) {
+                const uint64_t sm = __ballot(kind != K_END);
+                if (sm != stopped) {
+                    stopped = sm;
+                    more = false;
                     if (NW == 1) {
                         for (uint64_t t = sm; t; t &= t - 1) stop = min(stop, __builtin_amdgcn_readlane(cid, __builtin_ctzll(t)));
-                    } else if (ended && kind != K_END) {
-                        atomicMin(&F.stop, cid);
+                    } else {
+                        stop = __hip_atomic_load(&F.stop, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_WORKGROUP);
                     }
-                }
-                if (busy && cid > (NW == 1 ? stop : __hip_atomic_load(&F.stop, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_WORKGROUP))) {
-                    busy = false;
-                    fin = true;
+                    if (cid > stop) busy = false;
                 }
             }
-            const long long t_commit = a.stats ? wall_clock64() : 0;
+            if (NW == 1 && stopped == 0) {  // (a chain that stopped when it was taken last)
+                for (uint64_t t = __ballot(kind != K_END); t; t &= t - 1)
+                    stop = min(stop, __builtin_amdgcn_readlane(cid, __builtin_ctzll(t)));
+            }
+            const long long t_commit = stats ? wall_clock64() : 0;
             __syncthreads();
             // ---- commit plan, by scans over the chains (thread t: chains t * CPL on) ----
             if (NW > 1) {
@@ -2088,6 +2148,7 @@ __global__ void __launch_bounds__(64 * NW) __attribute__((amdgpu_waves_per_eu(WP
             }
             const int run = next < nlive ? (int)hcid[next] : nK;  // chains before the first one not taken
             const int J = min(stop, run - 1);
+            const int push_cap = HA(push_cap);
             uint32_t v01[CPL], v2s[CPL], vb[CPL];
             uint32_t s01 = 0, s2s = 0, sb = 0;
 #pragma unroll
@@ -2139,7 +2200,7 @@ __global__ void __launch_bounds__(64 * NW) __attribute__((amdgpu_waves_per_eu(WP
                         const bool over = (long)F.n_entries + pex - c + np > (long)F.max_entries;
                         if (c == 0)
                             walk0 = over;
-                        else if ((over || pex + np > a.push_cap) && wait == 0x7fffffff)
+                        else if ((over || pex + np > push_cap) && wait == 0x7fffffff)
                             wait = c;
                         p01 += v01[r];
                         p2s += v2s[r];
@@ -2177,7 +2238,7 @@ __global__ void __launch_bounds__(64 * NW) __attribute__((amdgpu_waves_per_eu(WP
                 int nb = F.n_entries;
                 const int cut = F.cut;
                 for (int j = 0; j <= (cut >= 0 ? 0 : last); ++j) {
-                    const int t0 = (int)(cB[j] >> 24) * H_SLOG + (int)cS[j], n = cut >= 0 ? cut : (int)(cC[j] & 63u);
+                    const int t0 = (int)cS[j], n = cut >= 0 ? cut : (int)(cC[j] & 63u);
                     for (int t = 0; t < n; ++t) {
                         const Item<WIDE> e = get_item<WIDE>(SLOG + t0 + t);
                         nb -= 1;
@@ -2209,7 +2270,7 @@ __global__ void __launch_bounds__(64 * NW) __attribute__((amdgpu_waves_per_eu(WP
                 F.hy = y;
             }
             __syncthreads();
-            const long long t_c1 = a.stats ? wall_clock64() : 0;
+            const long long t_c1 = stats ? wall_clock64() : 0;
             const uint32_t tot01 = F.tot01, tot2s = F.tot2s;
             const int T0 = (int)(tot01 & 0xffffu), T1 = (int)(tot01 >> 16), T2 = (int)(tot2s & 0xffffu);
             if (tid == 0) {
@@ -2239,12 +2300,12 @@ __global__ void __launch_bounds__(64 * NW) __attribute__((amdgpu_waves_per_eu(WP
                             g = F.n_used < H_KEEP ? F.own[F.n_used] : OWN[F.n_used];
                             ++F.n_used;
                         } else {
-                            g = F.n_own < a.own_cap ? gran_pop(a.ghead, a.gnext, a.gbump, a.n_gran) : NIL;
+                            g = F.n_own < HA(own_cap) ? gran_pop(HA(ghead), HA(gnext), HA(gbump), HA(n_gran)) : NIL;
                             if (g == NIL) {
                                 oom = true;
                                 break;
                             }
-                            if (a.stats) ST[11] += 1;
+                            if (stats) ST[11] += 1;
                             if (F.n_own < H_KEEP) F.own[F.n_own] = g;
                             OWN[F.n_own++] = g;
                             ++F.n_used;
@@ -2278,35 +2339,38 @@ __global__ void __launch_bounds__(64 * NW) __attribute__((amdgpu_waves_per_eu(WP
             }
             __syncthreads();
             if (F.status) break;
-            const long long t_c2 = a.stats ? wall_clock64() : 0;
-            // ---- placement: a bucket's push g of the round comes from the last chain with at most g pushes
-            // to the bucket before it, at its place in that chain's log ----
+            const long long t_c2 = stats ? wall_clock64() : 0;
+            // ---- placement: every logged push of a committed chain to its place among its bucket's pushes of
+            // the round ----
             {
                 const int npieces = F.n_piece;
-#pragma unroll
-                for (int c = 0; c < 3; ++c) {
-                    const int Tc = c == 0 ? T0 : c == 1 ? T1 : T2;
-                    const uint16_t *const ep = epre + c * KMAX;
-                    for (int g = tid; g < Tc; g += T) {
-                        int lo = 0;
-#pragma unroll
-                        for (int step = KMAX / 2; step > 0; step >>= 1)
-                            if (lo + step <= last && (int)ep[lo + step] <= g) lo += step;
-                        const uint32_t B = cB[lo];
-                        const int u = (int)((B >> (8 * c)) & 127u) + (g - (int)ep[lo]);
-                        int p = F.fp[c];
-                        while (p + 1 < npieces && (uint32_t)g >= pieces[p].y + pieces[p].z) ++p;
-                        const uint4 pc = pieces[p];
-                        if (u < H_LOG && pc.x == (uint32_t)c && (uint32_t)g - pc.y < pc.z) {
-                            POOL[pc.w + ((uint32_t)g - pc.y)] = LOG[(c * T + (int)(B >> 24)) * H_LOG + u];
-                        } else {
-                            F.bad = 1;  // a rank outside this round's pieces: not possible
-                        }
+                for (uint32_t g = lane; g < wl; g += HW) {
+                    Item<WIDE> e = get_item<WIDE>(LOG + g);
+                    uint32_t code, chain;
+                    if constexpr (WIDE) {
+                        const uint32_t w = LOGW[g];
+                        chain = w & ((1u << H_CHAIN_BITS) - 1);
+                        code = w >> H_CHAIN_BITS;
+                    } else {
+                        chain = e.x >> 28 << 6 | e.y >> 26;
+                        code = (e.x >> 26) & 3u;
+                        e.x &= (1u << 26) - 1;
+                        e.y &= (1u << 26) - 1;
                     }
+                    if ((int)chain > last) continue;
+                    const uint32_t R = epre[code * KMAX + chain] + (e.y & 127u);
+                    e.y = (e.y & ~Y_LDP) | (e.x & X_I);
+                    int p = F.fp[code];
+                    uint4 pc = pieces[p];
+                    while (R - pc.y >= pc.z && p + 1 < npieces) pc = pieces[++p];
+                    if (pc.x == code && R - pc.y < pc.z)
+                        put_item<WIDE>(POOL + pc.w + (R - pc.y), e.k, e.l, e.x, e.y);
+                    else
+                        F.bad = 1;  // a rank outside this round's pieces: not possible
                 }
             }
             __syncthreads();
-            const long long t_c3 = a.stats ? wall_clock64() : 0;
+            const long long t_c3 = stats ? wall_clock64() : 0;
             // ---- bucket b: the committed start entries leave its top; the state moves on ----
             const int l_kind = F.l_kind;
             if (tid == 0) {
@@ -2346,7 +2410,7 @@ __global__ void __launch_bounds__(64 * NW) __attribute__((amdgpu_waves_per_eu(WP
                     F.status = 1;
                     F.result = F.bad ? ERR_INTERNAL : ERR_SCORE;
                 }
-                if (a.stats) {
+                if (stats) {
                     ST[0] += 1;
                     ST[1] += (unsigned long long)nK;
                     ST[2] += (unsigned long long)taken;
@@ -2385,7 +2449,7 @@ __global__ void __launch_bounds__(64 * NW) __attribute__((amdgpu_waves_per_eu(WP
                         const int j = j0 + lane;
                         const uint64_t v = j < ldp ? Wp[1 + j] : 0, w = lw_val<WIDE>(v);
                         const uint64_t em = __ballot(j < ldp && w == ux);
-                        if (j < ldp && w > ux) Wp[1 + j] = lw_make<WIDE>(w - ux, lw_bid<WIDE>(v));
+                        if (j < ldp && w > ux) Wp[1 + j] = lw_make<WIDE>(w - ux, (uint32_t)lw_bid<WIDE>(v));
                         if (j < ldp && w == ux) Wp[1 + j] = lw_make<WIDE>(M.seq_len - (eq + (uint64_t)lanes_below(em) + 1), 1);
                         eq += (uint64_t)__builtin_popcountll(em);
                     }
@@ -2402,7 +2466,7 @@ __global__ void __launch_bounds__(64 * NW) __attribute__((amdgpu_waves_per_eu(WP
                         F.status = 1;
                         F.result = n_aln;
                     } else if (!dup) {
-                        if (n_aln == a.rec_cap) {
+                        if (n_aln == HA(rec_cap)) {
                             F.status = 1;
                             F.result = ERR_ALN;
                         } else {
@@ -2419,18 +2483,18 @@ __global__ void __launch_bounds__(64 * NW) __attribute__((amdgpu_waves_per_eu(WP
                     }
                 }
             }
-            if (!RESUME && tid == 0 && F.status == 0 && a.park_pops && taken_reads >= n_list) F.status = 2;
+            if (!RESUME && tid == 0 && F.status == 0 && HA(park_pops) && taken_reads >= n_list) F.status = 2;
             __syncthreads();
         }
         if (!RESUME && F.status == 2) {
             __syncthreads();
             if (tid == 0) F.status = 0;
             __syncthreads();
-            uint32_t *const st = reinterpret_cast<uint32_t *>(base + a.state_off);
-            for (int j = tid; j < (int)(heavy_state_bytes(a.buckets, a.wlen, a.swlen) / 4); j += T)
+            uint32_t *const st = reinterpret_cast<uint32_t *>(base + HA(state_off));
+            for (int j = tid; j < state_words; j += T)
                 st[j] = reinterpret_cast<const uint32_t *>(&F)[j];
             if (tid == 0) {
-                a.park_list[atomicAdd(a.park_n, 1)] = (int32_t)blockIdx.x;
+                HA(park_list)[atomicAdd(HA(park_n), 1)] = (int32_t)blockIdx.x;
                 F.n_own = 0;  // its granules stay with it
             }
             break;  // (no read is left to take)
@@ -2439,37 +2503,37 @@ __global__ void __launch_bounds__(64 * NW) __attribute__((amdgpu_waves_per_eu(WP
         if (tid == 0) {
             int n = F.result;
             if (n > 0) {
-                const unsigned long long b0 = atomicAdd(a.out_top, (unsigned long long)n);
-                if (b0 + (unsigned long long)n > a.out_cap) {
+                const unsigned long long b0 = atomicAdd(HA(out_top), (unsigned long long)n);
+                if (b0 + (unsigned long long)n > HA(out_cap)) {
                     n = ERR_OUT;
                 } else {
-                    for (int j = 0; j < n; ++j) a.out_rec[b0 + j] = REC[j];
-                    a.out_off[rid] = b0;
+                    for (int j = 0; j < n; ++j) HA(out_rec)[b0 + j] = REC[j];
+                    HA(out_off)[rid] = b0;
                 }
             }
             if (n == ERR_STACK || n == ERR_ALN || n == ERR_OUT) {
-                const int f = atomicAdd(a.fail_n, 1);
-                a.fail_list[f] = rid;
-                atomicOr(a.fail_kind + (n == ERR_OUT ? 0 : n == ERR_ALN ? 1 : 2), 1);
+                const int f = atomicAdd(HA(fail_n), 1);
+                HA(fail_list)[f] = rid;
+                atomicOr(HA(fail_kind) + (n == ERR_OUT ? 0 : n == ERR_ALN ? 1 : 2), 1);
             } else {
-                atomicAdd(a.algo_bytes, F.obytes);
+                atomicAdd(HA(algo_bytes), F.obytes);
             }
-            a.out_n[rid] = n;
-            a.out_pops[rid] = F.pops;
-            if (TRACE) a.out_trace[rid] = F.trace;
-            if (a.out_bytes) a.out_bytes[rid] = F.obytes;
+            HA(out_n)[rid] = n;
+            HA(out_pops)[rid] = F.pops;
+            if (TRACE) HA(out_trace)[rid] = F.trace;
+            if (HA(out_bytes)) HA(out_bytes)[rid] = F.obytes;
             // keep a few granules for the next read; the rest go back to the pool (a parked read's all)
             const int keep = RESUME ? 0 : H_KEEP;
             if (F.n_own > keep) {
-                gran_push(a.ghead, a.gnext, OWN, keep, F.n_own);
+                gran_push(HA(ghead), HA(gnext), OWN, keep, F.n_own);
                 F.n_own = keep;
             }
         }
         __syncthreads();
     }
     // the granules this workgroup still holds are for the reads that were parked
-    if (tid == 0 && a.park_pops && F.n_own > 0) gran_push(a.ghead, a.gnext, OWN, 0, F.n_own);
-    if (a.stats && tid < 16) atomicAdd(a.stats + tid, ST[tid]);
+    if (tid == 0 && HA(park_pops) && F.n_own > 0) gran_push(HA(ghead), HA(gnext), OWN, 0, F.n_own);
+    if (stats && tid < 16) atomicAdd(HA(stats) + tid, ST[tid]);
 }
 
 // A read's record count for the output offsets (error codes count none).
@@ -2869,7 +2933,7 @@ struct HLayout {
     uint32_t rec_off, own_off, spill_off, state_off, plog_off, slog_off;
 };
 
-HLayout make_hlayout(int rec_cap, int own_cap, int nw, bool trace, size_t state_bytes)
+HLayout make_hlayout(int rec_cap, int own_cap, int nw, bool trace, bool wide, size_t state_bytes)
 {
     HLayout L{};
     size_t off = 0;
@@ -2882,7 +2946,8 @@ HLayout make_hlayout(int rec_cap, int own_cap, int nw, bool trace, size_t state_
     L.state_off = (uint32_t)off;
     off += align_up(state_bytes, 256);
     L.plog_off = (uint32_t)off;
-    off += (size_t)3 * nw * HW * H_LOG * sizeof(Ent);
+    off += nw * heavy_log_bytes(wide);
+    off = align_up(off, 16);
     L.slog_off = (uint32_t)off;
     if (trace) off += (size_t)nw * HW * H_SLOG * (sizeof(Ent) + 1);
     off = align_up(off, 256);
@@ -3004,10 +3069,10 @@ int prepare_tier(galn_hip_readset *rs, const Tier &t, int slots, int pool_lanes)
 // parked reads (which read the former's).
 size_t heavy_scratch(galn_hip_readset *rs, int waves, int rec_cap, uint32_t flags)
 {
-    const bool trace = (flags & GALN_HIP_TRACE) != 0;
+    const bool trace = (flags & GALN_HIP_TRACE) != 0, wide = rs->idx->meta.ext != nullptr;
     const int own_cap = (int)std::min<uint64_t>(rs->ctx->n_gran, 32768);
-    const size_t one = (size_t)waves * make_hlayout(rec_cap, own_cap, 1, trace, heavy_state_of(rs)).slot_bytes;
-    return one + (size_t)std::min(waves, heavy_grid(rs, flags, true)) * make_hlayout(0, 0, DEEP_NW, trace, 0).slot_bytes;
+    const size_t one = (size_t)waves * make_hlayout(rec_cap, own_cap, 1, trace, wide, heavy_state_of(rs)).slot_bytes;
+    return one + (size_t)std::min(waves, heavy_grid(rs, flags, true)) * make_hlayout(0, 0, DEEP_NW, trace, wide, 0).slot_bytes;
 }
 
 // The allocations of a wave-engine launch of `waves` waves.
@@ -3173,15 +3238,15 @@ int run_tier(galn_hip_readset *rs, uint32_t flags, const Tier &t, const int32_t 
     return 0;
 }
 
-// Pushes the wave engine commits per round: H_CAP, or a lower value (at least H_MINCAP; a round's first
-// chain always fits) from GALN_HIP_TEST_PUSH_CAP, which the tests set to make the
-// cap cut rounds short and check that the results do not change.
+// Pushes the wave engine commits per round at most: what the logs hold, or a lower value (at least H_MINCAP;
+// a round's first chain always fits) from GALN_HIP_TEST_PUSH_CAP, which the tests set to make the cap cut
+// rounds short and check that the results do not change.
 int heavy_push_cap()
 {
     const char *v = getenv("GALN_HIP_TEST_PUSH_CAP");
-    if (!v || !*v) return H_CAP;
+    if (!v || !*v) return DEEP_NW * H_LOG;
     const long c = strtol(v, nullptr, 10);
-    return (int)std::min<long>(H_CAP, std::max<long>(H_MINCAP, c));
+    return (int)std::min<long>(DEEP_NW * H_LOG, std::max<long>(H_MINCAP, c));
 }
 
 // Pops from which on a read may be parked (0: never).
@@ -3202,11 +3267,11 @@ int run_heavy(galn_hip_readset *rs, uint32_t flags, const int32_t *list, int n, 
     const bool dev_count = n < 0;  // the count is the heavy-list length k_search leaves on the device
     if (n == 0) return 0;
     waves = std::max(1, dev_count ? waves : std::min(waves, n));
-    const bool tr = (flags & GALN_HIP_TRACE) != 0;
+    const bool tr = (flags & GALN_HIP_TRACE) != 0, wide = idx->meta.ext != nullptr;
     int r = prepare_heavy(rs, waves, rec_cap, flags);
     if (r) return r;
     const int own_cap = (int)std::min<uint64_t>(cx->n_gran, 32768);
-    const HLayout L = make_hlayout(rec_cap, own_cap, 1, tr, heavy_state_of(rs));
+    const HLayout L = make_hlayout(rec_cap, own_cap, 1, tr, wide, heavy_state_of(rs));
     const int wlen = rs->max_len + 1;
     const int swlen = (rs->seed_len > 0 && rs->seed_len < rs->max_len) ? rs->seed_len + 1 : 1;
     const size_t lds = heavy_lds_of(rs, 1, HEAVY_CPL);
@@ -3309,7 +3374,7 @@ int run_heavy(galn_hip_readset *rs, uint32_t flags, const int32_t *list, int n, 
         // the device; the workgroups end at once when there are none)
         HIP_OK(hipGetLastError());
         const int groups = std::min(waves, heavy_grid(rs, flags, true));
-        const HLayout D = make_hlayout(0, 0, DEEP_NW, tr, 0);
+        const HLayout D = make_hlayout(0, 0, DEEP_NW, tr, wide, 0);
         HArgs d = a;
         d.n_list_dev = rs->d_ctr + 8;
         d.qnext = rs->d_ctr + 9;
@@ -3318,7 +3383,6 @@ int run_heavy(galn_hip_readset *rs, uint32_t flags, const int32_t *list, int n, 
         d.slot_bytes = D.slot_bytes;
         d.plog_off = D.plog_off;
         d.slog_off = D.slog_off;
-        d.push_cap = a.push_cap == H_CAP ? H_CAP * DEEP_NW : a.push_cap;
         d.park_pops = 0;
         d.park_scratch = a.scratch;
         d.park_slot_bytes = L.slot_bytes;
