@@ -140,7 +140,7 @@ struct KArgs {
     int32_t *heavy_list;
     int32_t *heavy_n;
     // hand-off of a heavy read's widths: slot h (its place in heavy_list) holds
-    // [bytes | 1 << 63][W[0..len]][SW[0..seed_len]], or 0 when the widths were not kept
+    // [bytes | 3 << 62][W[0..len]][SW[0..seed_len]] ... [0], or 0 when the widths were not kept
     uint64_t *hand;
     uint32_t hand_stride;    // u64 words per slot
     int32_t hand_cap;        // slots
@@ -610,7 +610,8 @@ __global__ void __launch_bounds__(128) k_search(KArgs a)
                     for (int j = 0; j <= len; ++j) dst[1 + j] = W[j];
                     if (seeding)
                         for (int j = 0; j <= seed_len; ++j) dst[2 + len + j] = SW[j];
-                    dst[0] = wbytes | (1ull << 63);
+                    dst[CA(hand_stride) - 1] = 0;  // (the seed's bytes are among them)
+                    dst[0] = wbytes | (3ull << 62);
                 } else {
                     dst[0] = 0;
                 }
@@ -1478,33 +1479,41 @@ __device__ __forceinline__ uint64_t lw_make(uint64_t w, uint32_t bid) { return w
 
 // bwt_cal_width by one thread (src/bwtgap_hd.h:216-242); returns the algorithmic bytes. put(i, w, bid)
 // stores position i's width.
-template <class Put>
+template <class K, class Put>
 __device__ __forceinline__ uint64_t cal_width_one(const uint32_t *bwt, const DMeta &M, int len, const uint8_t *str, Put put)
 {
-    uint64_t k = 0, l = M.seq_len, bytes = 0;
+    K k = 0, l = (K)M.seq_len;
+    uint32_t units = 0;
     int bid = 0;
     for (int i = 0; i < len; ++i) {
         const int c0 = str[i];
         if (c0 <= 3) {
-            uint64_t ca[4], cb[4];
-            bytes += lf_pair(bwt, M, k, l, ca, cb);
+            const K Pk = pos_k<K>(M, k), Pl = pos_l<K>(M, l);
+            OccWord A, B;
+            occ_load<K>(bwt, Pk, A);
+            occ_load<K>(bwt, Pl, B);
+            K ca[4], cb[4];
+            occ_count<K>(M, sizeof(K) == 8, A, Pk, ca);
+            occ_count<K>(M, sizeof(K) == 8, B, Pl, cb);
+            units += occ_units<K>(Pk, Pl);
             k = pick4(ca, 3 - c0) + 1;
             l = pick4(cb, 3 - c0);
         }
         if (k > l || c0 > 3) {
             k = 0;
-            l = M.seq_len;
+            l = (K)M.seq_len;
             ++bid;
         }
-        put(i, l - k + 1, bid);
+        put(i, (uint64_t)l - k + 1, bid);
     }
     put(len, 0, ++bid);
-    return bytes;
+    return (uint64_t)units << 6;
 }
 
 // Widths of the reads given to the wave engine, into their hand-off slots (those that k_search has not
-// filled): one thread per read, all reads at once, so that the wave engine does not hold 64 lanes while one
-// of them walks a read's sequential width pass.
+// filled): two threads per read, one for the read's widths and one for its seed's (each a walk of as many
+// dependent lookups as it has positions), all reads at once, so that the wave engine does not hold 64 lanes
+// while one of them walks. A slot: [bytes | flags][W[0..len]][SW[0..seed_len]] ... [bytes of the seed's].
 struct WArgs {
     const uint32_t *bwt;
     DMeta meta;
@@ -1522,27 +1531,31 @@ struct WArgs {
     int32_t wlen, swlen;
     int32_t check;  // slots may hold widths already
 };
+constexpr uint64_t HAND_OK = 1ull << 63, HAND_SEARCH = 1ull << 62;  // a slot's flags: filled; by k_search
 
+template <bool WIDE>
 __global__ void __launch_bounds__(256) k_widths(WArgs a)
 {
+    using K = typename Item<WIDE>::K;
     const int n = min(a.n_list_dev ? *a.n_list_dev : a.n_list, a.hand_cap);
-    for (int pos = blockIdx.x * blockDim.x + threadIdx.x; pos < n; pos += gridDim.x * blockDim.x) {
+    for (int64_t t = (int64_t)blockIdx.x * blockDim.x + threadIdx.x; t < 2 * (int64_t)n; t += (int64_t)gridDim.x * blockDim.x) {
+        const int pos = (int)(t >> 1);
         uint64_t *const dst = a.hand + (uint64_t)pos * a.hand_stride;
-        if (a.check && (dst[0] >> 63)) continue;  // handed over by k_search
+        if (a.check && (dst[0] & HAND_SEARCH)) continue;
         const int rid = a.list ? a.list[pos] : pos;
         const int len = a.qlen[rid];
         const int sl = a.bopts[a.batch[rid]].seed_len;
         // (a read the wave engine rejects, or a seed it has no room for: no widths)
-        if (len < 1 || len + 1 > a.wlen || (sl < len && sl + 1 > a.swlen)) {
-            dst[0] = 0;
-            continue;
-        }
+        const bool none = len < 1 || len + 1 > a.wlen || (sl < len && sl + 1 > a.swlen);
         const uint8_t *const q = a.query + a.qoff[rid];
-        uint64_t *w = dst + 1;
-        uint64_t wb = cal_width_one(a.bwt, a.meta, len, q, [w](int i, uint64_t v, int bid) { w[i] = wpack(v, bid); });
-        w = dst + 2 + len;
-        if (sl < len) wb += cal_width_one(a.bwt, a.meta, sl, q + (len - sl), [w](int i, uint64_t v, int bid) { w[i] = wpack(v, bid); });
-        dst[0] = wb | (1ull << 63);
+        if (t & 1) {
+            if (none || sl >= len) continue;
+            uint64_t *const w = dst + 2 + len;
+            dst[a.hand_stride - 1] = cal_width_one<K>(a.bwt, a.meta, sl, q + (len - sl), [w](int i, uint64_t v, int bid) { w[i] = wpack(v, bid); });
+        } else {
+            uint64_t *const w = dst + 1;
+            dst[0] = none ? 0 : cal_width_one<K>(a.bwt, a.meta, len, q, [w](int i, uint64_t v, int bid) { w[i] = wpack(v, bid); }) | HAND_OK;
+        }
     }
 }
 
@@ -1686,13 +1699,13 @@ __global__ void __launch_bounds__(64 * NW) __attribute__((amdgpu_waves_per_eu(WP
                     if (F.seeding)
                         for (int j = tid; j <= F.seed_len; j += T)
                             SW[1 + j] = lw_make<WIDE>(wval(src[2 + len + j]), (uint32_t)wbid(src[2 + len + j]));
-                    if (tid == 0) F.obytes = h0 & ~(1ull << 63);
+                    if (tid == 0) F.obytes = (h0 & ~(HAND_OK | HAND_SEARCH)) + (F.seeding ? HA(hand)[(uint64_t)(pos + 1) * HA(hand_stride) - 1] : 0);
                 } else {
                     uint64_t wb = 0;
                     auto putw = [Wp](int i, uint64_t v, int bid) { Wp[1 + i] = lw_make<WIDE>(v, (uint32_t)bid); };
                     auto puts = [SW](int i, uint64_t v, int bid) { SW[1 + i] = lw_make<WIDE>(v, (uint32_t)bid); };
-                    if (tid == 0) wb = cal_width_one(a.bwt, M, len, QL, putw);
-                    if (tid == 1 && F.seeding) wb = cal_width_one(a.bwt, M, F.seed_len, QL + (len - F.seed_len), puts);
+                    if (tid == 0) wb = cal_width_one<K>(a.bwt, M, len, QL, putw);
+                    if (tid == 1 && F.seeding) wb = cal_width_one<K>(a.bwt, M, F.seed_len, QL + (len - F.seed_len), puts);
                     if (wb) atomicAdd(&F.obytes, (unsigned long long)wb);
                 }
                 int nN = 0;
@@ -3097,7 +3110,7 @@ constexpr uint64_t HAND_BYTES = 32ull << 30;
 int prepare_hand(galn_hip_readset *rs)
 {
     const int sl = (rs->seed_len > 0 && rs->seed_len < rs->max_len) ? rs->seed_len : 0;
-    const uint32_t stride = (uint32_t)(1 + (rs->max_len + 1) + (sl + 1));
+    const uint32_t stride = (uint32_t)(1 + (rs->max_len + 1) + (sl + 1) + 1);
     size_t freeb = 0, totalb = 0;
     HIP_OK(hipMemGetInfo(&freeb, &totalb));
     const uint64_t limit = std::min<uint64_t>(HAND_BYTES, (uint64_t)(freeb + rs->hand_bytes) / 4);
@@ -3136,7 +3149,7 @@ int reserve_search(galn_hip_readset *rs, int n, int max_len, uint32_t flags)
         return r;
     };
     // hand-off slots (seed widths of seeds up to 32 bases included), within prepare_hand's limit
-    const uint64_t stride = (uint64_t)(1 + (max_len + 1) + 33);
+    const uint64_t stride = (uint64_t)(1 + (max_len + 1) + 33 + 1);
     size_t freeb = 0, totalb = 0;
     HIP_OK(hipMemGetInfo(&freeb, &totalb));
     const uint64_t limit = std::min<uint64_t>(HAND_BYTES, (uint64_t)(freeb + rs->hand_bytes) / 4);
@@ -3176,6 +3189,21 @@ void fill_key_ptrs(const galn_hip_readset *rs, GraphKey &k)
     k.hscratch_bytes = rs->hscratch_bytes;
     k.max_len = rs->max_len, k.seed_len = rs->seed_len, k.max_stacks = rs->max_stacks, k.max_entries = rs->max_entries;
     k.hand = rs->d_hand, k.hand_cap = rs->hand_cap, k.hand_stride = rs->hand_stride;
+}
+
+// A launch record of this search, its byte counter cleared, its two events ready.
+int new_launch(galn_hip_readset *rs, int tier_id, int *li_out)
+{
+    const int li = (int)rs->launches.size();
+    if (li >= galn_hip_readset::MAX_LAUNCH) return fail(GALN_HIP_E_DEVICE, "too many launches in one search");
+    while ((int)rs->lev.size() < 2 * (li + 1)) {
+        hipEvent_t e;
+        HIP_OK(hipEventCreate(&e));
+        rs->lev.push_back(e);
+    }
+    rs->launches.push_back({tier_id, li, 0.0, 0});
+    *li_out = li;
+    return 0;
 }
 
 int run_tier(galn_hip_readset *rs, uint32_t flags, const Tier &t, const int32_t *list, int list_base, int n_list,
@@ -3221,15 +3249,9 @@ int run_tier(galn_hip_readset *rs, uint32_t flags, const Tier &t, const int32_t 
     // an empty free stack (tag and granule all ones) and no granule handed out yet
     FILL(cx->d_ghead, 0xffffffffu, NSHARD * 8);
     FILL(cx->d_gbump, 0, 4);
-    const int li = (int)rs->launches.size();
-    if (li >= galn_hip_readset::MAX_LAUNCH) return fail(GALN_HIP_E_DEVICE, "too many launches in one search");
-    while ((int)rs->lev.size() < 2 * (li + 1)) {
-        hipEvent_t e;
-        HIP_OK(hipEventCreate(&e));
-        rs->lev.push_back(e);
-    }
+    int li = 0;
+    if ((r = new_launch(rs, tier_id, &li))) return r;
     a.algo_bytes = rs->d_algo + li;
-    rs->launches.push_back({tier_id, li, 0.0, 0});
     const int grid = (slots + block - 1) / block;
     if (!rs->capturing) HIP_OK(hipEventRecord(rs->lev[2 * li], fst));
     r = launch(fst, a, block, grid, persist, (flags & GALN_HIP_TRACE) != 0, buckets_of(rs));
@@ -3256,10 +3278,41 @@ uint32_t heavy_park_pops()
     return v && *v ? (uint32_t)strtoul(v, nullptr, 10) : PARK_POPS;
 }
 
+// The widths of list[0..n) (n < 0: as many as k_search handed over) into the hand-off slots; `check`:
+// those that k_search filled stay.
+int launch_widths(galn_hip_readset *rs, const int32_t *list, int n, bool check)
+{
+    galn_hip_index *idx = rs->idx;
+    WArgs w{};
+    w.bwt = idx->d_bwt;
+    w.meta = idx->meta;
+    w.query = rs->d_query;
+    w.qoff = rs->d_qoff;
+    w.qlen = rs->d_qlen;
+    w.batch = rs->d_batch;
+    w.bopts = rs->d_bopts;
+    w.list = list;
+    w.n_list = std::max(n, 0);
+    w.n_list_dev = n < 0 ? rs->d_ctr + 3 : nullptr;
+    w.hand = rs->d_hand;
+    w.hand_stride = rs->hand_stride;
+    w.hand_cap = rs->hand_cap;
+    w.wlen = rs->max_len + 1;
+    w.swlen = (rs->seed_len > 0 && rs->seed_len < rs->max_len) ? rs->seed_len + 1 : 1;
+    w.check = check ? 1 : 0;
+    const int grid = n < 0 ? idx->n_cu * 8 : (int)std::max<int64_t>(1, std::min<int64_t>(idx->n_cu * 8, (2 * (int64_t)n + 255) / 256));
+    if (idx->meta.ext)
+        hipLaunchKernelGGL(k_widths<true>, dim3(grid), dim3(256), 0, rs->ctx->stream, w);
+    else
+        hipLaunchKernelGGL(k_widths<false>, dim3(grid), dim3(256), 0, rs->ctx->stream, w);
+    HIP_OK(hipGetLastError());
+    return 0;
+}
+
 // The wave-per-read engine over list[0..n): one wave per read, `waves` resident waves
 // claiming reads from a device counter; failures land in fail buffer `fo`.
 int run_heavy(galn_hip_readset *rs, uint32_t flags, const int32_t *list, int n, int rec_cap, int fo, int tier_id,
-              int waves)
+              int waves, bool widths_done = false)
 {
     galn_hip_index *idx = rs->idx;
     SearchCtx *cx = rs->ctx;
@@ -3336,38 +3389,11 @@ int run_heavy(galn_hip_readset *rs, uint32_t flags, const int32_t *list, int n, 
     FILL(rs->d_ctr + 8, 0, 2 * sizeof(int32_t));
     FILL(cx->d_ghead, 0xffffffffu, NSHARD * 8);
     FILL(cx->d_gbump, (uint32_t)(a.first_gran * waves), 4);
-    const int li = (int)rs->launches.size();
-    if (li >= galn_hip_readset::MAX_LAUNCH) return fail(GALN_HIP_E_DEVICE, "too many launches in one search");
-    while ((int)rs->lev.size() < 2 * (li + 1)) {
-        hipEvent_t e;
-        HIP_OK(hipEventCreate(&e));
-        rs->lev.push_back(e);
-    }
+    int li = 0;
+    if ((r = new_launch(rs, tier_id, &li))) return r;
     a.algo_bytes = rs->d_algo + li;
-    rs->launches.push_back({tier_id, li, 0.0, 0});
     if (!rs->capturing) HIP_OK(hipEventRecord(rs->lev[2 * li], fst));
-    if (a.hand && a.hand_cap > 0) {
-        WArgs w{};
-        w.bwt = a.bwt;
-        w.meta = a.meta;
-        w.query = a.query;
-        w.qoff = a.qoff;
-        w.qlen = a.qlen;
-        w.batch = a.batch;
-        w.bopts = a.bopts;
-        w.list = list;
-        w.n_list = a.n_list;
-        w.n_list_dev = a.n_list_dev;
-        w.hand = rs->d_hand;
-        w.hand_stride = a.hand_stride;
-        w.hand_cap = a.hand_cap;
-        w.wlen = wlen;
-        w.swlen = swlen;
-        w.check = 1;
-        const int wgrid = dev_count ? idx->n_cu * 8 : std::max(1, std::min(idx->n_cu * 8, (n + 255) / 256));
-        hipLaunchKernelGGL(k_widths, dim3(wgrid), dim3(256), 0, fst, w);
-        HIP_OK(hipGetLastError());
-    }
+    if (a.hand && a.hand_cap > 0 && !widths_done && (r = launch_widths(rs, list, n, true))) return r;
     hipLaunchKernelGGL(heavy_kernel(rs, tr, false), dim3(waves), dim3(HW), lds, fst, a);
     if (park_pops) {
         // the reads still running when the last one was taken, with more waves each (their count is read on
@@ -3465,9 +3491,12 @@ int run_retries(galn_hip_readset *rs, uint32_t flags, int fi, int32_t n, Tier t,
     return 0;
 }
 
-// Pops after which the batched form hands a read to the wave-per-read engine when no tuning is
-// given: measured best on the 10M-read aDNA workload (512: 2.67 s, 1024: 2.85 s, 4096: 3.34 s).
-constexpr int DEFAULT_HEAVY_POPS = 512;
+// Pops after which the batched form hands a read to the wave-per-read engine when no tuning is given: 1,
+// every read from the start, with its widths from k_widths. k_search's lanes take 6 us a pop on a read that is
+// searched alone (16 reads of 100 bp: 3.0 ms to 512 pops, 0.5 ms in the wave engine) and its waves
+// keep every lane until the last one is done (100k reads of 100 bp: 7.4 ms + 3.1 for the reads past 512
+// pops, 7.2 ms in the wave engine; 262,144 ancient DNA reads: 20 ms + 39 against 39).
+constexpr int DEFAULT_HEAVY_POPS = 1;
 
 int readset_search(galn_hip_readset *rs, int form, uint32_t flags, const galn_hip_tune_t *tune)
 {
@@ -3517,6 +3546,20 @@ int readset_search(galn_hip_readset *rs, int form, uint32_t flags, const galn_hi
         hwaves = heavy_grid(rs, flags, false);
         if (budget && (r = prepare_hand(rs))) return r;
         const int32_t *list = sorted ? rs->d_sorted : nullptr;
+        // every read to the wave engine: the widths launch stands in the place of k_search's
+        const bool direct = budget == 1;
+        auto first_tier = [&]() -> int {
+            if (!direct) return run_tier(rs, flags, t0, list, 0, rs->n, true, slots, 0, block, 0, budget);
+            int li = 0, rc = new_launch(rs, 0, &li);
+            if (rc) return rc;
+            if (!rs->capturing) HIP_OK(hipEventRecord(rs->lev[2 * li], fst));
+            if (rs->d_hand && rs->hand_cap > 0 && (rc = launch_widths(rs, list, rs->n, false))) return rc;
+            if (!rs->capturing) HIP_OK(hipEventRecord(rs->lev[2 * li + 1], fst));
+            return 0;
+        };
+        auto wave_tier = [&](int n) -> int {
+            return direct ? run_heavy(rs, flags, list, rs->n, 256, 0, 10, hwaves, true) : run_heavy(rs, flags, rs->d_heavy, n, 256, 0, 10, hwaves);
+        };
         if (graph) {
             // the prologue, the persistent launch and the wave-engine launch (its read count read
             // on the device) as one captured graph, replayed while nothing it holds has changed
@@ -3527,7 +3570,7 @@ int readset_search(galn_hip_readset *rs, int form, uint32_t flags, const galn_hi
             key.push_cap = heavy_push_cap();
             key.park_pops = heavy_park_pops();
             key.heavy_wpe = rs->heavy_wpe;
-            if ((r = prepare_tier(rs, t0, slots, std::min(slots, rs->n))) ||
+            if ((!direct && (r = prepare_tier(rs, t0, slots, std::min(slots, rs->n)))) ||
                 (budget && (r = prepare_heavy(rs, hwaves, 256, flags))))
                 return r;
             while (rs->lev.size() < 4) {
@@ -3548,9 +3591,9 @@ int readset_search(galn_hip_readset *rs, int form, uint32_t flags, const galn_hi
                     int rc = 0;
                     if (part == 0) {
                         rc = prologue();
-                        if (!rc) rc = run_tier(rs, flags, t0, list, 0, rs->n, true, slots, 0, block, 0, budget);
+                        if (!rc) rc = first_tier();
                     } else {
-                        rc = run_heavy(rs, flags, rs->d_heavy, -1, 256, 0, 10, hwaves);
+                        rc = wave_tier(-1);
                     }
                     rs->capturing = false;
                     hipGraph_t g = nullptr;
@@ -3583,10 +3626,12 @@ int readset_search(galn_hip_readset *rs, int form, uint32_t flags, const galn_hi
                 HIP_OK(hipEventRecord(rs->lev[3], fst));
             }
         } else {
-            r = run_tier(rs, flags, t0, list, 0, rs->n, true, slots, 0, block, 0, budget);
+            r = first_tier();
             int32_t nh = 0;
-            if (!r && budget && !(r = read_ctr(rs, 3, &nh)) && nh > 0)
-                r = run_heavy(rs, flags, rs->d_heavy, nh, 256, 0, 10, hwaves);
+            if (!r && direct)
+                r = wave_tier(rs->n);
+            else if (!r && budget && !(r = read_ctr(rs, 3, &nh)) && nh > 0)
+                r = wave_tier(nh);
         }
     }
     if (r) return r;

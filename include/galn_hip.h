@@ -123,7 +123,7 @@ typedef struct {
     int32_t rec_per_lane;      /* record slots per lane in the first tier */
     int32_t sort_by_cost;      /* 1: claim reads longest-first */
     int32_t heavy_pops;        /* pops after which a read moves to the wave-per-read engine
-                                  (0: default 512, -1: never) */
+                                  (0: the default, every read from its first pop; -1: never) */
     int32_t heavy_waves_per_simd; /* wave-per-read engine occupancy: 4 (0: default) or 5 (fewer
                                   registers, more of them spilled; more loads in flight, which pays
                                   for indexes in HBM) */
