@@ -37,6 +37,8 @@
 #include <cstdint>
 #include <cstdio>
 #include <cstring>
+#include <mutex>
+#include <utility>
 #include <vector>
 
 #include "galn_hip.h"
@@ -161,23 +163,24 @@ __global__ void k_collect(const uint64_t *P, uint64_t n, uint32_t b0, uint32_t b
     }
 }
 
-__global__ void k_keys(const uint64_t *P, uint64_t n, const uint64_t *pos, uint64_t m, uint64_t depth, uint64_t *key)
+// first keys of a chunk's suffixes, or (`all`) of every suffix, with its position
+__global__ void k_keys(const uint64_t *P, uint64_t n, uint64_t *pos, uint64_t m, int all, uint64_t *key)
 {
-    for (uint64_t j = blockIdx.x * (uint64_t)blockDim.x + threadIdx.x; j < m; j += (uint64_t)gridDim.x * blockDim.x)
-        key[j] = key_at(P, n, pos[j] + depth, KD);
+    for (uint64_t j = blockIdx.x * (uint64_t)blockDim.x + threadIdx.x; j < m; j += (uint64_t)gridDim.x * blockDim.x) {
+        if (all) pos[j] = j;
+        key[j] = key_at(P, n, all ? j : pos[j], KD);
+    }
 }
 
-// after the first sort: run heads, then the unresolved flags (members of runs of two or more)
-__global__ void k_heads(const uint64_t *K, uint64_t m, uint8_t *H)
+// after the first sort: run heads, and the unresolved flags (members of runs of two or more)
+__global__ void k_heads(const uint64_t *K, uint64_t m, uint8_t *H, uint8_t *U)
 {
-    for (uint64_t j = blockIdx.x * (uint64_t)blockDim.x + threadIdx.x; j < m; j += (uint64_t)gridDim.x * blockDim.x)
-        H[j] = (j == 0 || K[j] != K[j - 1]) ? 1 : 0;
-}
-
-__global__ void k_unres_all(const uint8_t *H, uint64_t m, uint8_t *U)
-{
-    for (uint64_t j = blockIdx.x * (uint64_t)blockDim.x + threadIdx.x; j < m; j += (uint64_t)gridDim.x * blockDim.x)
-        U[j] = (H[j] && (j + 1 == m || H[j + 1])) ? 0 : 1;
+    for (uint64_t j = blockIdx.x * (uint64_t)blockDim.x + threadIdx.x; j < m; j += (uint64_t)gridDim.x * blockDim.x) {
+        const uint64_t k = K[j];
+        const bool h = j == 0 || K[j - 1] != k;
+        H[j] = h ? 1 : 0;
+        U[j] = h && (j + 1 == m || K[j + 1] != k) ? 0 : 1;
+    }
 }
 
 // refinement: element t of the unresolved list (chunk slot idx[t]) gets its key at `depth`
@@ -230,26 +233,33 @@ struct HeadSlot {
 
 // BWT symbols by row for a finished chunk (rows r0 .. r0 + m - 1): the symbol before each
 // suffix, 0 as a stand-in for the $ at the row of suffix 0 (whose row becomes `primary`), and the
-// SA samples of rows 32, 64, ...
+// SA samples of rows 32, 64, ... One thread per row, so that a wave reads 64 positions in a row (a thread
+// per word of 32 rows read them 256 bytes apart: 229 us on 1e7 rows); 32 lanes put their word together.
 __global__ void k_emit(const uint64_t *P, const uint64_t *V, uint64_t m, uint64_t r0, uint64_t *R,
                        unsigned long long *primary, uint64_t *samples, uint64_t n_samples)
 {
-    const uint64_t w0 = r0 >> 5, w1 = (r0 + m - 1) >> 5;
-    for (uint64_t w = w0 + blockIdx.x * (uint64_t)blockDim.x + threadIdx.x; w <= w1; w += (uint64_t)gridDim.x * blockDim.x) {
-        const uint64_t lo = std::max(r0, w * 32), hi = std::min(r0 + m, w * 32 + 32);
+    const uint64_t first = r0 & ~31ull, end = (r0 + m + 31) & ~31ull;  // whole words
+    const uint64_t stride = (uint64_t)gridDim.x * blockDim.x;
+    for (uint64_t base = first + blockIdx.x * (uint64_t)blockDim.x; base < end; base += stride) {
+        const uint64_t r = base + threadIdx.x;
+        const bool in = r >= r0 && r < r0 + m;
         uint64_t v = 0;
-        for (uint64_t r = lo; r < hi; ++r) {
+        if (in) {
             const uint64_t pos = V[r - r0];
             if (pos == 0)
                 *primary = r;
             else
-                v |= (uint64_t)tsym(P, pos - 1) << (62 - 2 * (r & 31));
+                v = (uint64_t)tsym(P, pos - 1) << (62 - 2 * (r & 31));
             if (samples && (r & 31) == 0 && r >= 32 && (r >> 5) - 1 < n_samples) samples[(r >> 5) - 1] = pos;
         }
-        if (hi - lo == 32)
-            R[w] = v;
-        else if (v)
-            atomicOr(reinterpret_cast<unsigned long long *>(R + w), (unsigned long long)v);
+        for (int d = 16; d > 0; d >>= 1) v |= __shfl_xor((unsigned long long)v, d, 32);
+        if ((r & 31) == 0 && r < end) {
+            const uint64_t w = r >> 5;
+            if (r >= r0 && r + 32 <= r0 + m)
+                R[w] = v;
+            else if (v)
+                atomicOr(reinterpret_cast<unsigned long long *>(R + w), (unsigned long long)v);
+        }
     }
 }
 
@@ -352,55 +362,110 @@ struct Work {
     }
 };
 
-// Sorts one chunk's suffixes (pos[0..m), collected) into suffix order in V.
-struct ChunkBufs {
-    DevBuf pos_in, key_in, key_out, V, nv, H, idx, idx2, gid, tA, tAo, gA, gB, tB, flag, cnt;
-    uint64_t cap = 0;
+// A chunk's arrays, all in one allocation: positions and keys twice (the sort goes from one to the other
+// and back), head and tie flags. Freeing is what it costs: once the card's memory has been handed out, a
+// free of 0.9 GB takes 26 ms, ten times a 5 Mbp build's kernels (64 MB and less: 0.02 ms). So the arrays of
+// the tied suffixes lie in the keys' place, or in an allocation of their own where many are tied, which
+// takes 34 bytes a suffix where 90 were taken before, and a freed arena of up to ARENA_KEPT bytes (builds
+// of up to 15 Mbp) waits for the next build, until an index is opened: 5 Mbp take 3.0 ms (30.4 before).
+struct Arena {
+    void *p = nullptr;
+    size_t bytes = 0;
+    int device = -1;
 };
+constexpr size_t ARENA_KEPT = (size_t)1 << 30;
+std::mutex g_arena_mu;
+Arena g_arena;
 
-int chunk_alloc(ChunkBufs &c, uint64_t m)
+void arena_drop(Arena &a)
 {
-    if (m <= c.cap) return 0;
-    int r;
-    if ((r = dalloc(c.pos_in, m * 8)) || (r = dalloc(c.key_in, m * 8)) || (r = dalloc(c.key_out, m * 8)) ||
-        (r = dalloc(c.V, m * 8)) || (r = dalloc(c.nv, m * 8)) || (r = dalloc(c.H, m)) || (r = dalloc(c.idx, m * 4)) ||
-        (r = dalloc(c.idx2, m * 4)) || (r = dalloc(c.gid, m * 4)) || (r = dalloc(c.tA, m * 4)) ||
-        (r = dalloc(c.tAo, m * 4)) || (r = dalloc(c.gA, m * 4)) || (r = dalloc(c.gB, m * 4)) || (r = dalloc(c.tB, m * 4)) ||
-        (r = dalloc(c.flag, m)) || (r = dalloc(c.cnt, 16)))
-        return r;
-    c.cap = m;
-    return 0;
+    if (a.p) (void)hipFree(a.p);
+    a = Arena{};
 }
-// the chunk buffers, plus the radix sort's own copy of keys and values
-constexpr uint64_t CHUNK_BYTES_PER_SUFFIX = 8 * 5 + 1 + 4 * 8 + 1 + 16;
 
-int sort_chunk(Work &W, ChunkBufs &c, const uint64_t *P, uint64_t n, uint64_t m, int *rounds)
+struct ChunkBufs {
+    Arena a;
+    hipStream_t st;
+    uint64_t m;
+    uint64_t *pos[2], *key[2];
+    uint8_t *H, *flag;
+    uint64_t *cnt;
+    explicit ChunkBufs(hipStream_t s) : st(s) {}
+    ~ChunkBufs()
+    {
+        if (!a.p) return;
+        const bool idle = hipStreamSynchronize(st) == hipSuccess;
+        std::lock_guard<std::mutex> g(g_arena_mu);
+        if (idle && a.bytes <= ARENA_KEPT && a.bytes > g_arena.bytes) std::swap(a, g_arena);
+        arena_drop(a);
+    }
+    int alloc(int device, uint64_t m_)
+    {
+        m = m_;
+        const size_t col = (m * 8 + 255) / 256 * 256, need = 256 + 4 * col + 2 * ((m + 255) / 256 * 256);
+        {
+            std::lock_guard<std::mutex> g(g_arena_mu);
+            std::swap(a, g_arena);
+        }
+        if (a.device != device || a.bytes < need) {
+            arena_drop(a);
+            IHIP(hipMalloc(&a.p, need));
+            a.bytes = need;
+            a.device = device;
+        }
+        uint8_t *at = (uint8_t *)a.p;
+        cnt = (uint64_t *)at;
+        at += 256;
+        for (uint64_t **q : {&pos[0], &pos[1], &key[0], &key[1]}) {
+            *q = (uint64_t *)at;
+            at += col;
+        }
+        H = at;
+        flag = at + (m + 255) / 256 * 256;
+        return 0;
+    }
+};
+// per suffix: two positions, two keys and the flags; the tied suffixes' eight columns when all are tied;
+// their sort's own copy of keys and values
+constexpr uint64_t CHUNK_BYTES_PER_SUFFIX = 8 * 4 + 2 + 40 + 16;
+
+// Sorts one chunk's suffixes (pos[0][0..m), collected; `all`: every suffix) into suffix order in *Vout.
+int sort_chunk(Work &W, ChunkBufs &c, const uint64_t *P, uint64_t n, uint64_t m, bool all, int *rounds, const uint64_t **Vout)
 {
     hipStream_t st = W.st;
-    uint64_t *V = c.V.as<uint64_t>();
     // first key, first sort
-    hipLaunchKernelGGL(k_keys, dim3(grid_for(m)), dim3(256), 0, st, P, n, c.pos_in.as<uint64_t>(), m, (uint64_t)0,
-                       c.key_in.as<uint64_t>());
+    hipLaunchKernelGGL(k_keys, dim3(grid_for(m)), dim3(256), 0, st, P, n, c.pos[0], m, all ? 1 : 0, c.key[0]);
     IHIP(hipGetLastError());
     size_t tb = 0;
-    IHIP(rocprim::radix_sort_pairs(nullptr, tb, c.key_in.as<uint64_t>(), c.key_out.as<uint64_t>(), c.pos_in.as<uint64_t>(),
-                                   V, (size_t)m, 0, 63, st));
+    rocprim::double_buffer<uint64_t> dk(c.key[0], c.key[1]), dv(c.pos[0], c.pos[1]);
+    IHIP(rocprim::radix_sort_pairs(nullptr, tb, dk, dv, (size_t)m, 0, 63, st));
     if (int r = W.need(tb)) return r;
-    IHIP(rocprim::radix_sort_pairs(W.tmp.p, tb, c.key_in.as<uint64_t>(), c.key_out.as<uint64_t>(), c.pos_in.as<uint64_t>(),
-                                   V, (size_t)m, 0, 63, st));
-    uint8_t *H = c.H.as<uint8_t>();
-    hipLaunchKernelGGL(k_heads, dim3(grid_for(m)), dim3(256), 0, st, c.key_out.as<const uint64_t>(), m, H);
-    hipLaunchKernelGGL(k_unres_all, dim3(grid_for(m)), dim3(256), 0, st, (const uint8_t *)H, m, c.flag.as<uint8_t>());
+    IHIP(rocprim::radix_sort_pairs(W.tmp.p, tb, dk, dv, (size_t)m, 0, 63, st));
+    uint64_t *const V = dv.current(), *const nv = dv.alternate();
+    *Vout = V;
+    uint8_t *H = c.H;
+    hipLaunchKernelGGL(k_heads, dim3(grid_for(m)), dim3(256), 0, st, (const uint64_t *)dk.current(), m, H, c.flag);
     IHIP(hipGetLastError());
-    uint32_t *idx = c.idx.as<uint32_t>(), *idx2 = c.idx2.as<uint32_t>();
-    uint64_t *cnt = c.cnt.as<uint64_t>();
+    // (the keys are not read again: their place holds the tied suffixes' lists)
+    uint32_t *idx = (uint32_t *)c.key[0], *idx2 = idx + c.m;
+    uint64_t *cnt = c.cnt;
     rocprim::counting_iterator<uint32_t> ci(0u);
-    IHIP(rocprim::select(nullptr, tb, ci, c.flag.as<uint8_t>(), idx, cnt, (size_t)m, st));
+    IHIP(rocprim::select(nullptr, tb, ci, c.flag, idx, cnt, (size_t)m, st));
     if (int r = W.need(tb)) return r;
-    IHIP(rocprim::select(W.tmp.p, tb, ci, c.flag.as<uint8_t>(), idx, cnt, (size_t)m, st));
+    IHIP(rocprim::select(W.tmp.p, tb, ci, c.flag, idx, cnt, (size_t)m, st));
     uint64_t u = 0;
     IHIP(hipMemcpyAsync(&u, cnt, 8, hipMemcpyDeviceToHost, st));
     IHIP(hipStreamSynchronize(st));
+    const uint64_t u0 = (u + 63) / 64 * 64;
+    DevBuf tied;
+    uint64_t *nk = c.key[1];
+    if (40 * u0 > 8 * c.m) {
+        if (int r = dalloc(tied, 40 * u0)) return r;
+        nk = tied.as<uint64_t>();
+    }
+    uint64_t *const nkA = nk + u0;
+    uint32_t *const tA = (uint32_t *)(nkA + u0), *const tAo = tA + u0, *const gid = tAo + u0, *const gA = gid + u0,
+             *const gB = gA + u0, *const tB = gB + u0;
     uint64_t depth = 0;
     *rounds = 0;
     while (u > 0) {
@@ -409,9 +474,6 @@ int sort_chunk(Work &W, ChunkBufs &c, const uint64_t *P, uint64_t n, uint64_t m,
         ++*rounds;
         const uint32_t uu = (uint32_t)u;
         const unsigned g = grid_for(u);
-        uint64_t *nk = c.key_in.as<uint64_t>(), *nkA = c.key_out.as<uint64_t>();
-        uint32_t *tA = c.tA.as<uint32_t>(), *tAo = c.tAo.as<uint32_t>(), *gid = c.gid.as<uint32_t>();
-        uint32_t *gA = c.gA.as<uint32_t>(), *gB = c.gB.as<uint32_t>(), *tB = c.tB.as<uint32_t>();
         // groups: the slot of each element's run head (max scan over head slots)
         rocprim::transform_iterator<rocprim::counting_iterator<uint32_t>, HeadSlot, uint32_t> hs(ci, HeadSlot{H, idx});
         IHIP(rocprim::inclusive_scan(nullptr, tb, hs, gid, (size_t)u, rocprim::maximum<uint32_t>(), st));
@@ -430,20 +492,18 @@ int sort_chunk(Work &W, ChunkBufs &c, const uint64_t *P, uint64_t n, uint64_t m,
         if (int r = W.need(tb)) return r;
         IHIP(rocprim::radix_sort_pairs(W.tmp.p, tb, gA, gB, tAo, tB, (size_t)u, 0, 32, st));
         hipLaunchKernelGGL(k_gather_pos, dim3(g), dim3(256), 0, st, (const uint64_t *)V, (const uint32_t *)idx,
-                           (const uint32_t *)tB, uu, c.nv.as<uint64_t>());
-        hipLaunchKernelGGL(k_scatter_pos, dim3(g), dim3(256), 0, st, V, (const uint32_t *)idx, c.nv.as<const uint64_t>(),
+                           (const uint32_t *)tB, uu, nv);
+        hipLaunchKernelGGL(k_scatter_pos, dim3(g), dim3(256), 0, st, V, (const uint32_t *)idx, (const uint64_t *)nv,
                            (const uint32_t *)gB, (const uint64_t *)nk, (const uint32_t *)tB, uu, H);
         hipLaunchKernelGGL(k_unres, dim3(g), dim3(256), 0, st, (const uint8_t *)H, m, (const uint32_t *)idx, uu,
-                           c.flag.as<uint8_t>());
+                           c.flag);
         IHIP(hipGetLastError());
-        IHIP(rocprim::select(nullptr, tb, idx, c.flag.as<uint8_t>(), idx2, cnt, (size_t)u, st));
+        IHIP(rocprim::select(nullptr, tb, idx, c.flag, idx2, cnt, (size_t)u, st));
         if (int r = W.need(tb)) return r;
-        IHIP(rocprim::select(W.tmp.p, tb, idx, c.flag.as<uint8_t>(), idx2, cnt, (size_t)u, st));
+        IHIP(rocprim::select(W.tmp.p, tb, idx, c.flag, idx2, cnt, (size_t)u, st));
         IHIP(hipMemcpyAsync(&u, cnt, 8, hipMemcpyDeviceToHost, st));
         IHIP(hipStreamSynchronize(st));
-        std::swap(c.idx.p, c.idx2.p);
-        idx = c.idx.as<uint32_t>();
-        idx2 = c.idx2.as<uint32_t>();
+        std::swap(idx, idx2);
     }
     return 0;
 }
@@ -482,37 +542,49 @@ int build(const uint8_t *fwd, uint64_t len, int device, galn_bwt_meta_t *meta, u
         }
     }
     const uint64_t *Pc = P.as<const uint64_t>();
-    if ((r = dalloc(hist, (size_t)NBUCKET * 8))) return r;
-    IHIP(hipMemsetAsync(hist.p, 0, (size_t)NBUCKET * 8, st));
-    hipLaunchKernelGGL(k_hist, dim3(grid_for(n)), dim3(256), 0, st, Pc, n, hist.as<unsigned long long>());
-    IHIP(hipGetLastError());
-    std::vector<uint64_t> h(NBUCKET);
-    IHIP(hipMemcpyAsync(h.data(), hist.p, (size_t)NBUCKET * 8, hipMemcpyDeviceToHost, st));
-    IHIP(hipStreamSynchronize(st));
     // chunk capacity from the free memory (the packed body, n/2 bytes, comes after the chunks)
     size_t freeb = 0, totalb = 0;
     IHIP(hipMemGetInfo(&freeb, &totalb));
+    {
+        std::lock_guard<std::mutex> g(g_arena_mu);  // this build's to use, or freed before it allocates
+        if (g_arena.device == device) freeb += g_arena.bytes;
+    }
     const uint64_t reserve = (uint64_t)1 << 30;
     uint64_t cap = freeb > reserve ? (freeb - reserve) / (CHUNK_BYTES_PER_SUFFIX + 8) : 0;
     cap = std::min(cap, CHUNK_MAX);
     if (const char *e = getenv("GALN_HIP_TEST_BUILD_CHUNK")) cap = std::min<uint64_t>(cap, std::max(1L, strtol(e, nullptr, 10)));
-    // chunks: runs of consecutive buckets of at most `cap` suffixes
+    // chunks: one of all suffixes when they fit, else runs of consecutive buckets of at most `cap` suffixes
     struct Chunk {
         uint32_t b0, b1;
         uint64_t m, r0;
     };
     std::vector<Chunk> chunks;
     uint64_t row = 1, maxm = 0;
-    for (uint32_t b = 0; b < NBUCKET;) {
-        if (h[b] > cap)
-            return ifail(GALN_HIP_E_NOMEM, "build_bwt: %llu suffixes share a 10-symbol prefix; at most %llu fit a chunk",
-                         (unsigned long long)h[b], (unsigned long long)cap);
-        Chunk c{b, b, 0, row};
-        while (b < NBUCKET && c.m + h[b] <= cap) c.m += h[b++];
-        c.b1 = b;
-        row += c.m;
-        maxm = std::max(maxm, c.m);
-        if (c.m) chunks.push_back(c);
+    const bool one = n <= cap;
+    if (one) {
+        // (no histogram: its 78 MB to the host and the walk over them were 5 ms of a 5 Mbp build)
+        chunks.push_back({0, NBUCKET, n, 1});
+        row += n;
+        maxm = n;
+    } else {
+        if ((r = dalloc(hist, (size_t)NBUCKET * 8))) return r;
+        IHIP(hipMemsetAsync(hist.p, 0, (size_t)NBUCKET * 8, st));
+        hipLaunchKernelGGL(k_hist, dim3(grid_for(n)), dim3(256), 0, st, Pc, n, hist.as<unsigned long long>());
+        IHIP(hipGetLastError());
+        std::vector<uint64_t> h(NBUCKET);
+        IHIP(hipMemcpyAsync(h.data(), hist.p, (size_t)NBUCKET * 8, hipMemcpyDeviceToHost, st));
+        IHIP(hipStreamSynchronize(st));
+        for (uint32_t b = 0; b < NBUCKET;) {
+            if (h[b] > cap)
+                return ifail(GALN_HIP_E_NOMEM, "build_bwt: %llu suffixes share a 10-symbol prefix; at most %llu fit a chunk",
+                             (unsigned long long)h[b], (unsigned long long)cap);
+            Chunk c{b, b, 0, row};
+            while (b < NBUCKET && c.m + h[b] <= cap) c.m += h[b++];
+            c.b1 = b;
+            row += c.m;
+            maxm = std::max(maxm, c.m);
+            if (c.m) chunks.push_back(c);
+        }
     }
     if (row != n + 1) return ifail(GALN_HIP_E_DEVICE, "build_bwt: bucket counts sum to %llu, not %llu",
                                    (unsigned long long)(row - 1), (unsigned long long)n);
@@ -525,27 +597,29 @@ int build(const uint8_t *fwd, uint64_t len, int device, galn_bwt_meta_t *meta, u
     const char *vb = getenv("GALN_HIP_VERBOSE");
     const bool verbose = vb && *vb && strcmp(vb, "0") != 0;
     {
-        ChunkBufs cb;
-        if ((r = chunk_alloc(cb, maxm))) return r;
+        ChunkBufs cb(st);
+        if ((r = cb.alloc(device, maxm))) return r;
         int max_rounds = 0;
         for (const Chunk &c : chunks) {
-            IHIP(hipMemsetAsync(cb.cnt.p, 0, 8, st));
-            hipLaunchKernelGGL(k_collect, dim3(grid_for(n)), dim3(256), 0, st, Pc, n, c.b0, c.b1, cb.pos_in.as<uint64_t>(),
-                               cb.cnt.as<unsigned long long>());
-            IHIP(hipGetLastError());
-            uint64_t got = 0;
-            IHIP(hipMemcpyAsync(&got, cb.cnt.p, 8, hipMemcpyDeviceToHost, st));
-            IHIP(hipStreamSynchronize(st));
-            if (got != c.m) return ifail(GALN_HIP_E_DEVICE, "build_bwt: chunk collected %llu of %llu suffixes",
-                                         (unsigned long long)got, (unsigned long long)c.m);
+            if (!one) {
+                IHIP(hipMemsetAsync(cb.cnt, 0, 8, st));
+                hipLaunchKernelGGL(k_collect, dim3(grid_for(n)), dim3(256), 0, st, Pc, n, c.b0, c.b1, cb.pos[0],
+                                   (unsigned long long *)cb.cnt);
+                IHIP(hipGetLastError());
+                uint64_t got = 0;
+                IHIP(hipMemcpyAsync(&got, cb.cnt, 8, hipMemcpyDeviceToHost, st));
+                IHIP(hipStreamSynchronize(st));
+                if (got != c.m) return ifail(GALN_HIP_E_DEVICE, "build_bwt: chunk collected %llu of %llu suffixes",
+                                             (unsigned long long)got, (unsigned long long)c.m);
+            }
             int rounds = 0;
-            if ((r = sort_chunk(W, cb, Pc, n, c.m, &rounds))) return r;
+            const uint64_t *V = nullptr;
+            if ((r = sort_chunk(W, cb, Pc, n, c.m, one, &rounds, &V))) return r;
             max_rounds = std::max(max_rounds, rounds);
             if (verbose)
                 fprintf(stderr, "[galn_hip] build_bwt: chunk %zu of %zu: %llu suffixes sorted, %d refinement rounds\n",
                         (size_t)(&c - chunks.data()) + 1, chunks.size(), (unsigned long long)c.m, rounds);
-            const uint64_t words = ((c.r0 + c.m - 1) >> 5) - (c.r0 >> 5) + 1;
-            hipLaunchKernelGGL(k_emit, dim3(grid_for(words)), dim3(256), 0, st, Pc, cb.V.as<const uint64_t>(), c.m, c.r0,
+            hipLaunchKernelGGL(k_emit, dim3(grid_for(c.m + 64)), dim3(256), 0, st, Pc, V, c.m, c.r0,
                                R.as<uint64_t>(), primary.as<unsigned long long>(), samples_out ? S.as<uint64_t>() : nullptr,
                                n_samples);
             IHIP(hipGetLastError());
@@ -572,7 +646,9 @@ int build(const uint8_t *fwd, uint64_t len, int device, galn_bwt_meta_t *meta, u
     hipLaunchKernelGGL(k_block_counts, dim3(grid_for(nb)), dim3(256), 0, st, R.as<const uint64_t>(), n, prim, nb,
                        bc.as<uint32_t>());
     IHIP(hipGetLastError());
-    uint64_t totals[4] = {0, 0, 0, 0};
+    uint64_t totals[4] = {0, 0, 0, 0}, last[4] = {0, 0, 0, 0};
+    uint32_t lastc = 0;
+    IHIP(hipMemcpyAsync(&lastc, bc.as<uint32_t>() + nb - 1, 4, hipMemcpyDeviceToHost, st));
     for (int c = 0; c < 4; ++c) {
         rocprim::transform_iterator<const uint32_t *, Field, uint64_t> it(bc.as<const uint32_t>(), Field{c});
         size_t tb = 0;
@@ -581,12 +657,7 @@ int build(const uint8_t *fwd, uint64_t len, int device, galn_bwt_meta_t *meta, u
         if ((r = W.need(tb))) return r;
         IHIP(rocprim::exclusive_scan(W.tmp.p, tb, it, ex[c].as<uint64_t>(), (uint64_t)0, (size_t)nb,
                                      rocprim::plus<uint64_t>(), st));
-        uint64_t last = 0;
-        uint32_t lastc = 0;
-        IHIP(hipMemcpyAsync(&last, ex[c].as<uint64_t>() + nb - 1, 8, hipMemcpyDeviceToHost, st));
-        IHIP(hipMemcpyAsync(&lastc, bc.as<uint32_t>() + nb - 1, 4, hipMemcpyDeviceToHost, st));
-        IHIP(hipStreamSynchronize(st));
-        totals[c] = last + ((lastc >> (8 * c)) & 0xffu);
+        IHIP(hipMemcpyAsync(&last[c], ex[c].as<uint64_t>() + nb - 1, 8, hipMemcpyDeviceToHost, st));
     }
     hipLaunchKernelGGL(k_body, dim3(grid_for(nb * 16)), dim3(256), 0, st, R.as<const uint64_t>(), n, prim, nb,
                        ex[0].as<const uint64_t>(), ex[1].as<const uint64_t>(), ex[2].as<const uint64_t>(),
@@ -597,6 +668,7 @@ int build(const uint8_t *fwd, uint64_t len, int device, galn_bwt_meta_t *meta, u
     IHIP(hipMemcpyAsync(bwt, body.p, head * 4, hipMemcpyDeviceToHost, st));
     if (samples_out && n_samples) IHIP(hipMemcpyAsync(samples_out, S.p, n_samples * 8, hipMemcpyDeviceToHost, st));
     IHIP(hipStreamSynchronize(st));
+    for (int c = 0; c < 4; ++c) totals[c] = last[c] + ((lastc >> (8 * c)) & 0xffu);
     memcpy(bwt + head, totals, sizeof totals);
     meta->primary = prim;
     meta->L2[0] = 0;
@@ -609,6 +681,13 @@ int build(const uint8_t *fwd, uint64_t len, int device, galn_bwt_meta_t *meta, u
 }
 
 }  // namespace
+
+// Frees the chunk arena kept by earlier builds: an index is opened, the building is over (galn_search.hip).
+__attribute__((visibility("hidden"))) void galn_hip_build_trim()
+{
+    std::lock_guard<std::mutex> g(g_arena_mu);
+    arena_drop(g_arena);
+}
 
 extern "C" {
 

@@ -50,6 +50,8 @@
 
 #include "galn_hip.h"
 
+__attribute__((visibility("hidden"))) void galn_hip_build_trim();  // galn_index.hip
+
 namespace {
 
 constexpr int CH = 16;                       // entries per stack chunk
@@ -3861,6 +3863,7 @@ int galn_hip_index_open(const uint32_t *bwt, const galn_bwt_meta_t *meta, int de
     if (hipGetDeviceCount(&ndev) != hipSuccess || ndev == 0) return fail(GALN_HIP_E_DEVICE, "no HIP device");
     if (device < 0 || device >= ndev) return fail(GALN_HIP_E_DEVICE, "no HIP device %d (%d visible)", device, ndev);
     HIP_OK(hipSetDevice(device));
+    galn_hip_build_trim();
     galn_hip_index *idx = new galn_hip_index;
     idx->device = device;
     idx->hmeta = *meta;
