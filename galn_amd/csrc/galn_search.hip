@@ -1289,11 +1289,12 @@ __global__ void __launch_bounds__(256) k_sa_walk(const uint32_t *__restrict__ bw
 // 100,003 reads of a 700 Mbp repeat-rich genome 142 -> 125.
 
 constexpr int HW = 64;         // lanes of a wave
-constexpr int H_STEPS = 32;    // chain steps per round
+constexpr int H_STEPS = 60;    // chain steps per round
+constexpr int H_STEPS_PLAIN = 32;  // and where lone descents are not walked ahead
 constexpr int H_LOG = 8192;    // pushes logged per wave and round
 constexpr int H_SPUSH = 9;     // pushes of one step at most
 constexpr int H_CPUSH = 127;   // pushes of a chain and round to one bucket at most (7-bit ranks)
-constexpr int H_SLOG = 64;     // trace build: steps logged per thread
+constexpr int H_SLOG = 64;    // trace build: steps logged per thread
 constexpr int H_KEEP = 64;     // granules a workgroup keeps between reads
 constexpr int H_PIECES = 48;   // segment pieces one round may add (three buckets)
 constexpr int H_MINCAP = 128;  // the lowest push cap a test may set
@@ -1302,9 +1303,10 @@ constexpr uint32_t GFULL = GENT - 1;
 constexpr int H_LOOK = 16;     // rounds between looks at the queue
 constexpr int H_FREE = 32;     // emptied granules kept in LDS
 static_assert(H_LOG > 2 * HW * H_SPUSH, "every lane of a wave can log a step's pushes");
-static_assert(H_SLOG >= 2 * H_STEPS, "a chain's steps fit the rest of a thread's step log");
+static_assert(H_SLOG >= 2 * H_STEPS_PLAIN, "a chain's steps fit the rest of a thread's step log");
 
-enum : int { K_END = 0, K_HIT = 1, K_TRUNC = 2, K_ESCORE = 3 };
+enum : int { K_END = 0, K_HIT = 1, K_TRUNC = 2, K_ESCORE = 3, K_TAIL = 4, K_DEAD = 5 };  // (the last two only while walking ahead)
+constexpr int H_ALONE = 2;  // iterations with one lane at work after which it walks ahead
 
 struct HArgs {
     const uint32_t *bwt;
@@ -1364,6 +1366,7 @@ struct HShared {
     unsigned long long pops, trace, obytes;
     unsigned long long bm[4];
     int has_pend, claim, status, result, K, b, n_piece, n_own, n_used, n_free, n_spill, nN, bad;
+    int root, root_unused;  // steps of the root chain known beyond the root, until the first round's commit
     uint32_t own[H_KEEP], free_g[H_FREE];  // the first granules held; emptied ones (more of them in the spill list)
     int next, stop, lim, l_kind, cut;  // the round's claims, first stopping chain, commit limit
     uint32_t tot01, tot2s, totb;       // committed pushes (16 bits per bucket code), pops, index bytes / 64
@@ -1372,6 +1375,10 @@ struct HShared {
     int wlive[16];
     uint64_t hk, hl;                   // the last committed chain's hit, or its pending child
     uint32_t hx, hy;
+    struct {                           // per wave, a descent walked ahead: the entry after its steps, their number,
+        uint64_t k, l;                 // how it ended, and the chain's pops, index bytes / 64 and pushes before it
+        uint32_t n, end, steps, sby, np3, unused;
+    } ahead[4];
 };
 static_assert(sizeof(HShared) % 8 == 0, "the widths follow it in a parked read's state");
 
@@ -1403,6 +1410,15 @@ __device__ __forceinline__ uint32_t wave_incl_scan(uint32_t x)
     x += (uint32_t)__builtin_amdgcn_update_dpp(0, (int)x, 0x142, 0xa, 0xf, false);  // row_bcast:15
     x += (uint32_t)__builtin_amdgcn_update_dpp(0, (int)x, 0x143, 0xc, 0xf, false);  // row_bcast:31
     return x;
+}
+
+template <class K>
+__device__ __forceinline__ K lane_value(K v, int lane)
+{
+    if constexpr (sizeof(K) == 8)
+        return (K)(uint32_t)__builtin_amdgcn_readlane((int)(uint32_t)(v >> 32), lane) << 32 | (uint32_t)__builtin_amdgcn_readlane((int)(uint32_t)v, lane);
+    else
+        return (K)__builtin_amdgcn_readlane((int)v, lane);
 }
 
 // A stack entry in registers: the interval, x = i | n_mm << 10 | n_gapo << 17 | state << 24 and
@@ -1512,10 +1528,14 @@ __device__ __forceinline__ uint64_t cal_width_one(const uint32_t *bwt, const DMe
     return (uint64_t)units << 6;
 }
 
-// Widths of the reads given to the wave engine, into their hand-off slots (those that k_search has not
-// filled): two threads per read, one for the read's widths and one for its seed's (each a walk of as many
-// dependent lookups as it has positions), all reads at once, so that the wave engine does not hold 64 lanes
-// while one of them walks. A slot: [bytes | flags][W[0..len]][SW[0..seed_len]] ... [bytes of the seed's].
+// Widths and root chains of the reads given to the wave engine, into their hand-off slots (those that k_search
+// has filled keep their widths): three threads per read, one for the read's widths, one for its seed's and one
+// for the intervals of its exact descent, each a walk of as many dependent lookups as it has positions, all
+// reads at once, so that the wave engine does not hold 64 lanes while one of them walks. A slot:
+// [bytes | flags][W[0..len]][SW[0..seed_len]] ... [root steps 1 ..][their number][bytes of the seed's].
+// The descent from the root is a read's first chain and, for a read of a few hundred pops, four fifths of its
+// iterations with one lane at work: with its intervals known, the engine's first round has a lane for each of
+// its steps (100k reads of 100 bp 7.2 -> 4.9 ms, this kernel 0.47 -> 0.72).
 struct WArgs {
     const uint32_t *bwt;
     DMeta meta;
@@ -1533,6 +1553,7 @@ struct WArgs {
     int32_t wlen, swlen;
     int32_t check;  // slots may hold widths already
 };
+constexpr int H_ROOT = 127;  // steps of the root chain kept at most (one round's chains with the root itself)
 constexpr uint64_t HAND_OK = 1ull << 63, HAND_SEARCH = 1ull << 62;  // a slot's flags: filled; by k_search
 
 template <bool WIDE>
@@ -1540,25 +1561,57 @@ __global__ void __launch_bounds__(256) k_widths(WArgs a)
 {
     using K = typename Item<WIDE>::K;
     const int n = min(a.n_list_dev ? *a.n_list_dev : a.n_list, a.hand_cap);
-    for (int64_t t = (int64_t)blockIdx.x * blockDim.x + threadIdx.x; t < 2 * (int64_t)n; t += (int64_t)gridDim.x * blockDim.x) {
-        const int pos = (int)(t >> 1);
+    // a wave's threads do the same work for 64 reads (three walks in one wave follow each other)
+    const int64_t span = ((int64_t)n + HW - 1) / HW * HW;
+    for (int64_t t = (int64_t)blockIdx.x * blockDim.x + threadIdx.x; t < (WIDE ? 2 : 3) * span; t += (int64_t)gridDim.x * blockDim.x) {
+        const int role = t < span ? 0 : t < 2 * span ? 1 : 2;
+        const int pos = (int)(t - role * span);
+        if (pos >= n) continue;
         uint64_t *const dst = a.hand + (uint64_t)pos * a.hand_stride;
-        if (a.check && (dst[0] & HAND_SEARCH)) continue;
+        if (role < 2 && a.check && (dst[0] & HAND_SEARCH)) continue;
         const int rid = a.list ? a.list[pos] : pos;
         const int len = a.qlen[rid];
         const int sl = a.bopts[a.batch[rid]].seed_len;
         // (a read the wave engine rejects, or a seed it has no room for: no widths)
         const bool none = len < 1 || len + 1 > a.wlen || (sl < len && sl + 1 > a.swlen);
         const uint8_t *const q = a.query + a.qoff[rid];
-        if (t & 1) {
+        if (role == 0) {
+            uint64_t *const w = dst + 1;
+            dst[0] = none ? 0 : cal_width_one<K>(a.bwt, a.meta, len, q, [w](int i, uint64_t v, int bid) { w[i] = wpack(v, bid); }) | HAND_OK;
+        } else if (role == 1) {
             if (none || sl >= len) continue;
             uint64_t *const w = dst + 2 + len;
             dst[a.hand_stride - 1] = cal_width_one<K>(a.bwt, a.meta, sl, q + (len - sl), [w](int i, uint64_t v, int bid) { w[i] = wpack(v, bid); });
-        } else {
-            uint64_t *const w = dst + 1;
-            dst[0] = none ? 0 : cal_width_one<K>(a.bwt, a.meta, len, q, [w](int i, uint64_t v, int bid) { w[i] = wpack(v, bid); }) | HAND_OK;
+        } else if constexpr (!WIDE) {
+            uint64_t *const at = dst + 1 + a.wlen + a.swlen;
+            const int most = none ? 0 : min(len, min(a.wlen - 1, H_ROOT));
+            uint32_t k = 0, l = (uint32_t)a.meta.seq_len;
+            int s = 0;
+            while (s < most) {
+                const int c = q[len - 1 - s];
+                if (c > 3) break;
+                const uint32_t Pk = pos_k<uint32_t>(a.meta, k), Pl = pos_l<uint32_t>(a.meta, l);
+                OccWord A, B;
+                occ_load<uint32_t>(a.bwt, Pk, A);
+                occ_load<uint32_t>(a.bwt, Pl, B);
+                uint32_t ca[4], cb[4];
+                occ_count<uint32_t>(a.meta, false, A, Pk, ca);
+                occ_count<uint32_t>(a.meta, false, B, Pl, cb);
+                k = pick4(ca, c) + 1;
+                l = pick4(cb, c);
+                if (k > l) break;
+                at[s] = (uint64_t)l << 32 | k;
+                ++s;
+            }
+            dst[a.hand_stride - 2] = (uint64_t)s;
         }
     }
+}
+
+// words of a hand-off slot
+inline uint32_t hand_words(int wlen, int swlen, bool wide)
+{
+    return (uint32_t)(1 + wlen + swlen + (wide ? 0 : std::min(wlen - 1, H_ROOT)) + 2);
 }
 
 // A wave logs a round's pushes in the order it makes them, 16 bytes after 16 bytes. A logged push holds, beside
@@ -1575,17 +1628,24 @@ constexpr size_t heavy_chain_bytes = 16 + 4 + 4 + 2 + 2;  // head | counts | ste
 typedef const __attribute__((address_space(4))) HArgs HArgsC;
 #define HA(f) cold_ld(&((HArgsC *)__builtin_amdgcn_kernarg_segment_ptr())->f)
 
-// NW waves per read; WPE waves per SIMD: 4 at 128 VGPRs, or 5 (96 VGPRs) for indexes in HBM, where a wave
-// waits on its loads.
-template <bool TRACE, bool WIDE, int NW, int CPL, int WPE>
-__global__ void __launch_bounds__(64 * NW) __attribute__((amdgpu_waves_per_eu(WPE))) k_heavy(HArgs a)
+// NW waves per read, at four waves per SIMD (128 VGPRs): a variant of five (96) was 4% faster on light reads, 2%
+// slower on heavy ones, before the light reads' descents were taken out of the loop.
+template <bool TRACE, bool WIDE, int NW, int CPL>
+__global__ void __launch_bounds__(64 * NW) __attribute__((amdgpu_waves_per_eu(4, (TRACE || WIDE) ? 8 : 4))) k_heavy(HArgs a)
 {
     using K = typename Item<WIDE>::K;
     constexpr int T = 64 * NW, KMAX = T * CPL;
+    static_assert(NW > 1 || H_ROOT < KMAX, "the root's round");
     static_assert(KMAX <= 1 << H_CHAIN_BITS, "a chain's id in its pushes");
     extern __shared__ __align__(16) uint8_t hlds[];
     // the launch of NW > 1 waves goes on with reads that the launch of one wave parked
     constexpr bool RESUME = NW > 1;
+    // Steps of exact descents side by side (the root's round, a lone lane's descent), not in the trace build and
+    // not above 2^32 symbols: those variants spill most, and the code compiled for one of them with this in it
+    // read out of range, as a variant for five waves per SIMD (96 registers) gave wrong records, while the same
+    // source is right in the others and on the CPU.
+    constexpr bool AHEAD = !TRACE && !WIDE;
+    constexpr int STEPS = AHEAD ? H_STEPS : H_STEPS_PLAIN;
     uint4 *const pieces = reinterpret_cast<uint4 *>(hlds);         // {bucket code, rank0, len, base}
     Ent *const hent = reinterpret_cast<Ent *>(pieces + H_PIECES);  // live chains' heads, in order
     uint16_t *const epre = reinterpret_cast<uint16_t *>(hent);     // after them: pushes before each chain, by code
@@ -1688,6 +1748,7 @@ __global__ void __launch_bounds__(64 * NW) __attribute__((amdgpu_waves_per_eu(WP
                 F.n_spill = 0;
                 F.status = 0;
                 F.bad = 0;
+                F.root = 0;
             }
             __syncthreads();
             const bool unsup = len < 1 || len > MAXLEN || len + 1 > HA(wlen) || F.n_stacks > HA(buckets) || F.md_read > MAXDIFF ||
@@ -1701,7 +1762,10 @@ __global__ void __launch_bounds__(64 * NW) __attribute__((amdgpu_waves_per_eu(WP
                     if (F.seeding)
                         for (int j = tid; j <= F.seed_len; j += T)
                             SW[1 + j] = lw_make<WIDE>(wval(src[2 + len + j]), (uint32_t)wbid(src[2 + len + j]));
-                    if (tid == 0) F.obytes = (h0 & ~(HAND_OK | HAND_SEARCH)) + (F.seeding ? HA(hand)[(uint64_t)(pos + 1) * HA(hand_stride) - 1] : 0);
+                    if (tid == 0) {
+                        F.obytes = (h0 & ~(HAND_OK | HAND_SEARCH)) + (F.seeding ? src[HA(hand_stride) - 1] : 0);
+                        if (AHEAD) F.root = (int)src[HA(hand_stride) - 2];
+                    }
                 } else {
                     uint64_t wb = 0;
                     auto putw = [Wp](int i, uint64_t v, int bid) { Wp[1 + i] = lw_make<WIDE>(v, (uint32_t)bid); };
@@ -1748,6 +1812,9 @@ __global__ void __launch_bounds__(64 * NW) __attribute__((amdgpu_waves_per_eu(WP
                     F.b = 0;
                     F.n_entries = 1;
                 }
+                // (the widths' bounds fall towards the read's start: a root that is not dead has no dead step; with
+                // no difference allowed the whole descent is one pop)
+                if (AHEAD && (F.md_read <= 0 || F.status || F.md_read < lw_bid<WIDE>(Wp[len]))) F.root = 0;
             }
             __syncthreads();
         }
@@ -1800,7 +1867,7 @@ __global__ void __launch_bounds__(64 * NW) __attribute__((amdgpu_waves_per_eu(WP
                         F.status = 1;
                         F.result = F.n_aln;
                     } else {
-                        F.K = (int)min(avail, (uint32_t)KMAX);
+                        F.K = AHEAD && !RESUME && F.root ? F.root + 1 : (int)min(avail, (uint32_t)KMAX);
                         F.next = T;
                         F.stop = 0x7fffffff;
                         F.lim = 0x7fffffff;
@@ -1812,6 +1879,10 @@ __global__ void __launch_bounds__(64 * NW) __attribute__((amdgpu_waves_per_eu(WP
             __syncthreads();
             if (F.status) break;
             const int b = F.b, nK = F.K, hp = F.has_pend;
+            // the first round: a chain for every known step of the root chain, of that one pop (the last one goes
+            // on as any chain)
+            const bool root = AHEAD && !RESUME && F.root != 0;
+            const int solo = root ? nK - 1 : 0;
             const long long t_spec = stats ? wall_clock64() : 0;
             if (stats && tid == 0) ST[13] += (unsigned long long)(t_spec - t_round);
             const int s_mm = F.s_mm, s_gapo = F.s_gapo, s_gape = F.s_gape, mode = F.mode, max_diff = F.max_diff;
@@ -1822,6 +1893,15 @@ __global__ void __launch_bounds__(64 * NW) __attribute__((amdgpu_waves_per_eu(WP
             // extension, or the lower code of the same bucket (one log, so that its order is kept)
             const int tg0 = b + s_mm, tg1 = b + s_gapo, tg2 = b + s_gape;
             const int sh1 = s_gapo == s_mm ? 0 : 8, sh2 = s_gape == s_mm ? 0 : s_gape == s_gapo ? 8 : 16;
+            auto root_step = [&](int c) __attribute__((always_inline)) {
+                const uint64_t *const at = HA(hand) + (uint64_t)claim * HA(hand_stride) + 1 + HA(wlen) + HA(swlen) + (c - 1);
+                Item<WIDE> e;
+                e.k = (K)(uint32_t)at[0];
+                e.l = (K)(at[0] >> 32);
+                e.x = (uint32_t)(len - c);
+                e.y = 0;
+                return e;
+            };
             // differences still allowed to a chain (constant along it)
             auto left = [&](int lim, uint32_t x, uint32_t y) __attribute__((always_inline)) {
                 return lim - x_mm(x) - x_go(x) - ((mode & MODE_GAPE) ? y_ge(y) : 0);
@@ -1842,6 +1922,8 @@ __global__ void __launch_bounds__(64 * NW) __attribute__((amdgpu_waves_per_eu(WP
                             h[r].l = (K)F.hl;
                             h[r].x = F.hx;
                             h[r].y = F.hy;
+                        } else if (root) {
+                            h[r] = root_step(c);
                         } else {
                             // entry d below the top one: in the top granule, or in the full one below it
                             const uint32_t d = (uint32_t)(c - hp);
@@ -1891,7 +1973,7 @@ __global__ void __launch_bounds__(64 * NW) __attribute__((amdgpu_waves_per_eu(WP
             // ---- speculation: every thread runs chains, one lookup an iteration, and takes the next live
             // one when its own has ended. A step's children are logged while the next step's lookups are on
             // their way ----
-            int next = T, stop = 0x7fffffff, its = 0;  // (NW > 1: the claims and the stop are F.next, F.stop)
+            int next = T, stop = 0x7fffffff, its = 0, alone = 0;  // (NW > 1: the claims and the stop are F.next, F.stop)
             uint32_t wl = 0;                           // pushes this wave has logged
             uint64_t stopped = 0;                      // lanes whose chain has stopped
             bool more = true;                          // (uniform) chains are left to take
@@ -1909,7 +1991,7 @@ __global__ void __launch_bounds__(64 * NW) __attribute__((amdgpu_waves_per_eu(WP
             K pk, pl, ca[4], cb[4];
             constexpr uint32_t ROOM = 0x010101u * (uint32_t)(127 - (H_CPUSH - H_SPUSH));  // sets bit 7 of a full count
             constexpr uint32_t LOG_FULL = H_LOG - 2 * HW * H_SPUSH;
-            const bool near = F.n_entries + H_STEPS * H_SPUSH > F.max_entries;  // chain 0 may cross the limit
+            const bool near = F.n_entries + STEPS * H_SPUSH > F.max_entries;  // chain 0 may cross the limit
             auto finish = [&]() __attribute__((always_inline)) {
                 cA[cid] = np3 | (uint32_t)kind << 24;
                 cC[cid] = (uint32_t)steps | sby << 6;
@@ -1953,7 +2035,7 @@ __global__ void __launch_bounds__(64 * NW) __attribute__((amdgpu_waves_per_eu(WP
             if (tid < nlive) take(tid);
             for (;;) {
                 if (more) {
-                    const uint64_t wm = __ballot(!busy && kind == K_END && (!TRACE || sl <= H_SLOG - H_STEPS));
+                    const uint64_t wm = __ballot(!busy && kind == K_END && (!TRACE || sl <= H_SLOG - STEPS));
                     if (wm) {
                         int g;
                         if (NW == 1) {
@@ -1975,7 +2057,93 @@ __global__ void __launch_bounds__(64 * NW) __attribute__((amdgpu_waves_per_eu(WP
                         if ((wm >> lane & 1ull) && p < nlive) take(p);
                     }
                 }
-                const uint64_t run_m = __ballot(busy);
+                uint64_t run_m = __ballot(busy);
+                // ---- one lane is left: its exact descent is walked ahead by the wave (a lookup and little more
+                // per step), then each of its steps gets a lane of its own in one iteration. With the root's round
+                // two thirds of a light read's iterations still had one lane (13 a round of 95 pops; 8
+                // now), and a round takes 60 steps of a chain instead of 32: 100k reads of 100 bp 4.9 -> 4.1 ms, 100k pairs of 150 bp
+                // 43 -> 34, 100,003 repeat-rich reads 118 -> 105 ----
+                bool fan = false;
+                if (AHEAD && !more && !near && run_m != 0 && (run_m & (run_m - 1)) == 0 && wl <= LOG_FULL && __ballot(kind != K_END) == 0) {
+                    const int L = __builtin_ctzll(run_m);
+                    const int wcid = __builtin_amdgcn_readlane(cid, L);
+                    if (++alone >= H_ALONE && wcid >= solo) {
+                        const bool wtail = (__ballot(tail) >> L & 1ull) != 0;
+                        const uint32_t wx = (uint32_t)__builtin_amdgcn_readlane((int)x, L), wy = (uint32_t)__builtin_amdgcn_readlane((int)y, L);
+                        const int wm = __builtin_amdgcn_readlane(m, L), ws = __builtin_amdgcn_readlane(steps, L);
+                        K wk = lane_value<K>(k, L), wl_ = lane_value<K>(l, L);
+                        uint32_t i = wx & X_I, units = 0;
+                        int n = 0, end = K_END;
+                        for (;;) {
+                            if (!wtail && lane == n) {
+                                k = wk;
+                                l = wl_;
+                            }
+                            const uint32_t c = (uint32_t)__builtin_amdgcn_readlane((int)QL[i - 1], 0);
+                            ++n;
+                            if (c > 3) break;
+                            const K Pk = pos_k<K>(M, wk), Pl = pos_l<K>(M, wl_), P = (lane & 1) ? Pl : Pk;
+                            OccWord o;
+                            occ_load<K>(a.bwt, P, o);
+                            K cn[4];
+                            occ_count<K>(M, WIDE, o, P, cn);
+                            const K v = pick4(cn, (int)c);
+                            const K xk = lane_value<K>(v, 0) + 1, xl = lane_value<K>(v, 1);
+                            units += occ_units<K>(Pk, Pl);
+                            if (xk > xl) break;
+                            wk = xk;
+                            wl_ = xl;
+                            --i;
+                            if (wtail) {
+                                if (i > 0) continue;
+                                if ((uint32_t)(xl - xk + 1) != 0) end = K_HIT;
+                                break;
+                            }
+                            if (ws + n - 1 == STEPS) {
+                                end = K_TRUNC;
+                                break;
+                            }
+                            const bool dead = wm < max(__builtin_amdgcn_readlane(lw_bid<WIDE>(Wp[i]), 0), 0);
+                            if (dead || i == 0 || wm == 0) {
+                                end = dead ? K_DEAD : i == 0 ? K_HIT : K_TAIL;
+                                break;
+                            }
+                        }
+                        if (wtail) {
+                            if (busy) {
+                                sby += units;
+                                if (end == K_HIT) {
+                                    kind = K_HIT;
+                                    k = wk;
+                                    l = wl_;
+                                }
+                                finish();
+                            }
+                            run_m = 0;
+                        } else {
+                            if (busy) {
+                                F.ahead[wave].k = wk;
+                                F.ahead[wave].l = wl_;
+                                F.ahead[wave].n = (uint32_t)n;
+                                F.ahead[wave].end = (uint32_t)end;
+                                F.ahead[wave].steps = (uint32_t)steps;
+                                F.ahead[wave].sby = sby;
+                                F.ahead[wave].np3 = np3;
+                            }
+                            __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");  // (all lanes read it below)
+                            m_seed = __builtin_amdgcn_readlane(m_seed, L);
+                            m = wm;
+                            cid = wcid;
+                            x = lane ? (wx & ~X_ST) - (uint32_t)lane : wx;
+                            y = lane ? wy & ~Y_LDP : wy;
+                            np3 = 0;
+                            sby = 0;
+                            tail = false;
+                            busy = lane < n;
+                            fan = true;
+                        }
+                    }
+                }
                 uint32_t qb = 0, i0 = 0;
                 uint64_t wA = 0, wB = 0;
                 K Pk = 0, Pl = 0;
@@ -2118,19 +2286,64 @@ __global__ void __launch_bounds__(64 * NW) __attribute__((amdgpu_waves_per_eu(WP
                         if (TRACE) SINFO[tid * H_SLOG + sl - 1] = (uint8_t)__builtin_popcount(ch);
                         ch |= qb << 9 & 0x600u;
                         ch |= open ? 0x800u : 0u;
-                        if (kind == K_END && ex) {
+                        if (fan) {
+                        } else if (kind == K_END && ex && cid >= solo) {
                             // the exact child is popped next, or (the round's steps or the log used up) in the
                             // next round
                             k = xk;
                             l = xl;
                             x = p_x - 1;
                             y = p_y;
-                            if (steps == H_STEPS || wl > LOG_FULL || ((np3 + ROOM) & 0x808080u) != 0) {
+                            if (steps == STEPS || wl > LOG_FULL || ((np3 + ROOM) & 0x808080u) != 0) {
                                 kind = K_TRUNC;
                                 finish();
                             } else {
                                 pop(wA);
                             }
+                        } else {
+                            finish();
+                        }
+                    }
+                }
+                if (fan) {
+                    // the steps' pushes are ranked in their order (10 bits a bucket code); the chain ends at the step
+                    // whose pushes fill a code's ranks, or that met a score error; lane 0 goes on with it
+                    const auto &W = F.ahead[wave];
+                    const uint32_t base = W.np3, own = (np3 & 255u) | (np3 >> 8 & 255u) << 10 | (np3 >> 16 & 255u) << 20;
+                    const uint32_t incl = wave_incl_scan(own) + ((base & 255u) | (base >> 8 & 255u) << 10 | (base >> 16 & 255u) << 20);
+                    const int n = __builtin_amdgcn_readlane((int)W.n, 0);
+                    int end = __builtin_amdgcn_readlane((int)W.end, 0), fin = n - 1;
+                    const uint32_t most = max(max(incl & 1023u, incl >> 10 & 1023u), incl >> 20);
+                    const uint64_t full = __ballot(busy && most > (uint32_t)(H_CPUSH - H_SPUSH) && lane < n - 1), bad = __ballot(busy && kind == K_ESCORE);
+                    if (full) {
+                        fin = __builtin_ctzll(full);
+                        end = K_TRUNC;
+                    }
+                    if (bad && __builtin_ctzll(bad) <= fin) {
+                        fin = __builtin_ctzll(bad);
+                        end = K_ESCORE;
+                    }
+                    const uint64_t in = ~0ull >> (63 - fin);
+                    const uint32_t units = (uint32_t)(__builtin_popcountll(in & __ballot(sby != 0)) + __builtin_popcountll(in & __ballot(sby == 2)));
+                    const uint32_t pre = incl - own, tot = (uint32_t)__builtin_amdgcn_readlane((int)incl, fin);
+                    p_np3 = (pre & 255u) | (pre >> 10 & 255u) << 8 | (pre >> 20) << 16;
+                    const K nk = lane_value<K>(k, (fin + 1) & 63), nl = lane_value<K>(l, (fin + 1) & 63);
+                    if (lane > fin) ch = 0;
+                    kind = K_END;
+                    busy = false;
+                    if (lane == 0) {
+                        const bool inner = fin < n - 1;
+                        k = inner ? nk : (K)W.k;
+                        l = inner ? nl : (K)W.l;
+                        x = (x & ~X_ST) - (uint32_t)(fin + 1);
+                        y &= ~Y_LDP;
+                        np3 = (tot & 255u) | (tot >> 10 & 255u) << 8 | (tot >> 20) << 16;
+                        sby = W.sby + units;
+                        steps = (int)W.steps + fin + (end == K_DEAD || end == K_HIT || end == K_TAIL ? 1 : 0);
+                        kind = end == K_DEAD || end == K_TAIL ? K_END : end;
+                        if (end == K_TAIL) {
+                            busy = true;
+                            tail = true;
                         } else {
                             finish();
                         }
@@ -2211,8 +2424,9 @@ __global__ void __launch_bounds__(64 * NW) __attribute__((amdgpu_waves_per_eu(WP
                         epre[2 * KMAX + c] = (uint16_t)p2s;
                         const int pex = (int)((p01 & 0xffffu) + (p01 >> 16) + (p2s & 0xffffu));
                         const int np = (int)((v01[r] & 0xffffu) + (v01[r] >> 16) + (v2s[r] & 0xffffu));
-                        // each chain before this one popped its head and left its pushes
-                        const bool over = (long)F.n_entries + pex - c + np > (long)F.max_entries;
+                        // each chain before this one popped its head and left its pushes (in the root's round,
+                        // and the next step of the root chain)
+                        const bool over = (long)F.n_entries + pex - (root ? 0 : c) + np > (long)F.max_entries;
                         if (c == 0)
                             walk0 = over;
                         else if ((over || pex + np > push_cap) && wait == 0x7fffffff)
@@ -2258,7 +2472,7 @@ __global__ void __launch_bounds__(64 * NW) __attribute__((amdgpu_waves_per_eu(WP
                         const Item<WIDE> e = get_item<WIDE>(SLOG + t0 + t);
                         nb -= 1;
                         tr = trace_item(tr, b, e.k, e.l, e.x, e.y, nb);
-                        nb += (int)SINFO[t0 + t] + (t + 1 < n ? 1 : 0);  // its pushes, and its exact child
+                        nb += (int)SINFO[t0 + t] + (t + 1 < n || root ? 1 : 0);  // its pushes, and its exact child
                     }
                 }
                 F.trace = tr;
@@ -2390,8 +2604,9 @@ __global__ void __launch_bounds__(64 * NW) __attribute__((amdgpu_waves_per_eu(WP
             const int l_kind = F.l_kind;
             if (tid == 0) {
                 const int taken = last + 1;
-                const int from_seg = taken - hp;
+                const int from_seg = root ? 0 : taken - hp;
                 F.has_pend = 0;
+                F.root = 0;
                 if (from_seg > 0) {
                     uint32_t n = (uint32_t)from_seg, cnt = seg_cnt[b], top = seg_top[b], prev = seg_prev[b];
                     while (n >= cnt) {
@@ -2415,7 +2630,17 @@ __global__ void __launch_bounds__(64 * NW) __attribute__((amdgpu_waves_per_eu(WP
                     seg_prev[b] = prev;
                 }
                 // entries: every chain's head left, its pushes came; a pending child is one more
-                int ne = F.n_entries + T0 + T1 + T2 - taken;
+                int ne = F.n_entries + T0 + T1 + T2 - (root ? 1 : taken);
+                if (root && last < solo && l_kind == K_END) {
+                    // (cut short: the next step of the root chain waits)
+                    const Item<WIDE> e = root_step(last + 1);
+                    F.has_pend = 1;
+                    F.hk = e.k;
+                    F.hl = e.l;
+                    F.hx = e.x;
+                    F.hy = e.y;
+                    ne += 1;
+                }
                 if (l_kind == K_TRUNC) {
                     F.has_pend = 1;
                     ne += 1;
@@ -2662,7 +2887,6 @@ struct GraphKey {
     int32_t hand_cap;
     uint32_t hand_stride;
     int32_t push_cap;
-    int32_t heavy_wpe;
     uint32_t park_pops;
 };
 
@@ -2723,7 +2947,6 @@ struct galn_hip_readset {
     bool has_tuned = false;
     galn_hip_tune_t tuned{};
     uint32_t last_flags = 0;
-    int heavy_wpe = 4;  // waves per SIMD of the wave engine in the current search (4 or 5)
     hipEvent_t ev[4] = {nullptr, nullptr, nullptr, nullptr};
     struct Launch {
         int tier;
@@ -2996,13 +3219,10 @@ HeavyKernel heavy_kernel(const galn_hip_readset *rs, bool trace, bool deep)
 {
     const bool wide = rs->idx->meta.ext != nullptr;
     if (deep)
-        return trace ? (wide ? k_heavy<true, true, DEEP_NW, DEEP_CPL, 4> : k_heavy<true, false, DEEP_NW, DEEP_CPL, 4>)
-                     : (wide ? k_heavy<false, true, DEEP_NW, DEEP_CPL, 4> : k_heavy<false, false, DEEP_NW, DEEP_CPL, 4>);
-    if (rs->heavy_wpe == 5)
-        return trace ? (wide ? k_heavy<true, true, 1, HEAVY_CPL, 5> : k_heavy<true, false, 1, HEAVY_CPL, 5>)
-                     : (wide ? k_heavy<false, true, 1, HEAVY_CPL, 5> : k_heavy<false, false, 1, HEAVY_CPL, 5>);
-    return trace ? (wide ? k_heavy<true, true, 1, HEAVY_CPL, 4> : k_heavy<true, false, 1, HEAVY_CPL, 4>)
-                 : (wide ? k_heavy<false, true, 1, HEAVY_CPL, 4> : k_heavy<false, false, 1, HEAVY_CPL, 4>);
+        return trace ? (wide ? k_heavy<true, true, DEEP_NW, DEEP_CPL> : k_heavy<true, false, DEEP_NW, DEEP_CPL>)
+                     : (wide ? k_heavy<false, true, DEEP_NW, DEEP_CPL> : k_heavy<false, false, DEEP_NW, DEEP_CPL>);
+    return trace ? (wide ? k_heavy<true, true, 1, HEAVY_CPL> : k_heavy<true, false, 1, HEAVY_CPL>)
+                 : (wide ? k_heavy<false, true, 1, HEAVY_CPL> : k_heavy<false, false, 1, HEAVY_CPL>);
 }
 
 // Workgroups of the wave engine that are resident at once.
@@ -3112,7 +3332,7 @@ constexpr uint64_t HAND_BYTES = 32ull << 30;
 int prepare_hand(galn_hip_readset *rs)
 {
     const int sl = (rs->seed_len > 0 && rs->seed_len < rs->max_len) ? rs->seed_len : 0;
-    const uint32_t stride = (uint32_t)(1 + (rs->max_len + 1) + (sl + 1) + 1);
+    const uint32_t stride = hand_words(rs->max_len + 1, sl + 1, rs->idx->meta.ext != nullptr);
     size_t freeb = 0, totalb = 0;
     HIP_OK(hipMemGetInfo(&freeb, &totalb));
     const uint64_t limit = std::min<uint64_t>(HAND_BYTES, (uint64_t)(freeb + rs->hand_bytes) / 4);
@@ -3151,7 +3371,7 @@ int reserve_search(galn_hip_readset *rs, int n, int max_len, uint32_t flags)
         return r;
     };
     // hand-off slots (seed widths of seeds up to 32 bases included), within prepare_hand's limit
-    const uint64_t stride = (uint64_t)(1 + (max_len + 1) + 33 + 1);
+    const uint64_t stride = hand_words(max_len + 1, 33, rs->idx->meta.ext != nullptr);
     size_t freeb = 0, totalb = 0;
     HIP_OK(hipMemGetInfo(&freeb, &totalb));
     const uint64_t limit = std::min<uint64_t>(HAND_BYTES, (uint64_t)(freeb + rs->hand_bytes) / 4);
@@ -3302,7 +3522,7 @@ int launch_widths(galn_hip_readset *rs, const int32_t *list, int n, bool check)
     w.wlen = rs->max_len + 1;
     w.swlen = (rs->seed_len > 0 && rs->seed_len < rs->max_len) ? rs->seed_len + 1 : 1;
     w.check = check ? 1 : 0;
-    const int grid = n < 0 ? idx->n_cu * 8 : (int)std::max<int64_t>(1, std::min<int64_t>(idx->n_cu * 8, (2 * (int64_t)n + 255) / 256));
+    const int grid = n < 0 ? idx->n_cu * 8 : (int)std::max<int64_t>(1, std::min<int64_t>(idx->n_cu * 8, (3 * (int64_t)((n + HW - 1) / HW * HW) + 255) / 256));
     if (idx->meta.ext)
         hipLaunchKernelGGL(k_widths<true>, dim3(grid), dim3(256), 0, rs->ctx->stream, w);
     else
@@ -3543,7 +3763,6 @@ int readset_search(galn_hip_readset *rs, int form, uint32_t flags, const galn_hi
         slots = resident_slots(rs, block, trace, tune ? tune->waves_per_cu : 0);
         const bool sorted = !tune || tune->sort_by_cost != 0;
         const int hp = tune ? tune->heavy_pops : 0;
-        rs->heavy_wpe = tune && tune->heavy_waves_per_simd == 5 ? 5 : 4;
         budget = (hp < 0 || !heavy_ok(rs)) ? 0 : (uint64_t)(hp > 0 ? hp : DEFAULT_HEAVY_POPS);
         hwaves = heavy_grid(rs, flags, false);
         if (budget && (r = prepare_hand(rs))) return r;
@@ -3571,7 +3790,6 @@ int readset_search(galn_hip_readset *rs, int form, uint32_t flags, const galn_hi
             key.budget = budget, key.rec_cap = (uint32_t)t0.rec_cap, key.keep = (uint32_t)t0.keep, key.list = list;
             key.push_cap = heavy_push_cap();
             key.park_pops = heavy_park_pops();
-            key.heavy_wpe = rs->heavy_wpe;
             if ((!direct && (r = prepare_tier(rs, t0, slots, std::min(slots, rs->n)))) ||
                 (budget && (r = prepare_heavy(rs, hwaves, 256, flags))))
                 return r;
@@ -4041,9 +4259,8 @@ int galn_hip_readset_autotune(galn_hip_index *idx, galn_hip_readset *rs, uint32_
             const double ms = std::chrono::duration<double, std::milli>(std::chrono::steady_clock::now() - t0).count();
             if (verbose)
                 fprintf(stderr, "[galn_hip] autotune: cutoff %d, %d-thread groups, %d waves/CU, %d record slots, "
-                                "%d chunks kept, wave engine at %d waves/SIMD: %.1f ms\n",
-                        t.heavy_pops, t.block_threads, t.waves_per_cu, t.rec_per_lane, t.chunks_per_lane,
-                        t.heavy_waves_per_simd == 5 ? 5 : 4, ms);
+                                "%d chunks kept: %.1f ms\n",
+                        t.heavy_pops, t.block_threads, t.waves_per_cu, t.rec_per_lane, t.chunks_per_lane, ms);
             if (best_ms == 0 || ms < best_ms) {
                 best_ms = ms;
                 best = t;
@@ -4086,21 +4303,6 @@ int galn_hip_readset_autotune(galn_hip_index *idx, galn_hip_readset *rs, uint32_
             t = best;
             t.chunks_per_lane = v;
             if ((r = trial(t))) return r;
-        }
-        if (heavy_ok(rs) && best.heavy_pops >= 0) {
-            t = best;
-            t.heavy_waves_per_simd = 5;
-            if ((r = trial(t))) return r;
-            // with more waves in flight the best cutoff can move: the small ones again
-            if (best.heavy_waves_per_simd == 5) {
-                const galn_hip_tune_t at5 = best;
-                for (int c : {1, 16, 64, 128}) {
-                    if (c == at5.heavy_pops) continue;
-                    t = at5;
-                    t.heavy_pops = c;
-                    if ((r = trial(t))) return r;
-                }
-            }
         }
     }
     rs->tuned = best;

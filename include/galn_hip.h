@@ -124,9 +124,8 @@ typedef struct {
     int32_t sort_by_cost;      /* 1: claim reads longest-first */
     int32_t heavy_pops;        /* pops after which a read moves to the wave-per-read engine
                                   (0: the default, every read from its first pop; -1: never) */
-    int32_t heavy_waves_per_simd; /* wave-per-read engine occupancy: 4 (0: default) or 5 (fewer
-                                  registers, more of them spilled; more loads in flight, which pays
-                                  for indexes in HBM) */
+    int32_t heavy_waves_per_simd; /* any value: the wave-per-read engine runs four waves per SIMD (a variant
+                                  of five was no faster) */
 } galn_hip_tune_t;
 
 /* Serving loop configuration (0 = default). */
