@@ -3725,6 +3725,10 @@ int readset_search(galn_hip_readset *rs, int form, uint32_t flags, const galn_hi
     if (!tune && rs->has_tuned) tune = &rs->tuned;
     galn_hip_index *idx = rs->idx;
     HIP_OK(hipSetDevice(idx->device));
+// The plain form's: its lanes wait for the slowest of 64 at 6 us a pop. 100k reads of 100 bp 31 ms without a
+// limit, 8.8 after 512 pops, 7.2 after 128, 5.7 after 32, 5.5 after 16; 262,144 ancient DNA reads 67, 56, 51, 53.
+constexpr int PLAIN_POPS = 32;
+
     hipStream_t fst = rs->ctx->stream;
     rs->last_flags = flags;
     rs->launches.clear();
@@ -3748,13 +3752,19 @@ int readset_search(galn_hip_readset *rs, int form, uint32_t flags, const galn_hi
     int r = 0, slots = 0, hwaves = 0;
     uint64_t budget = 0;
     if (form == 0) {
-        // plain: one launch per 0x40000 reads, one lane per read, input order
+        // plain: one launch per 0x40000 reads, one lane per read, input order; the reads past PLAIN_POPS pops then
+        // get a wave each
         slots = 0x40000;
         for (int s = 0; s < rs->n && !r; s += 0x40000)
-            r = run_tier(rs, flags, t0, nullptr, s, std::min(0x40000, rs->n - s), false, 0, 0, block, 0);
+            r = run_tier(rs, flags, t0, nullptr, s, std::min(0x40000, rs->n - s), false, 0, 0, block, 0, budget);
+        int32_t nh = 0;
+        if (!r && budget && !(r = read_ctr(rs, 3, &nh)) && nh > 0) r = run_heavy(rs, flags, rs->d_heavy, nh, 256, 0, 10, hwaves);
     } else {
         // batched: one persistent launch over the reads, longest first; reads that spend their
         // pop budget go to the wave-per-read engine
+        budget = heavy_ok(rs) ? PLAIN_POPS : 0;
+        hwaves = heavy_grid(rs, flags, false);
+        if (budget && (r = prepare_hand(rs))) return r;
         // 64-thread workgroups unless tuned otherwise (the autotuner's choice on every workload
         // measured so far)
         block = 64;

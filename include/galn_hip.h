@@ -171,8 +171,9 @@ int galn_hip_index_open(const uint32_t *bwt, const galn_bwt_meta_t *meta, int de
 int galn_hip_index_close(galn_hip_index *idx);
 int galn_hip_index_device(const galn_hip_index *idx);
 
-/* Plain form: reads uploaded, one launch per 0x40000 reads (thread per read), re-runs of
- * reads that outgrow the first tier in larger tiers, results copied to `out`. */
+/* Plain form: reads uploaded, one launch per 0x40000 reads (thread per read), then a wave for each
+ * read past 32 pops, re-runs of reads that outgrow the first tier in larger tiers, results copied to
+ * `out`. */
 int galn_hip_search_plain(galn_hip_index *idx, const galn_hip_reads *reads, galn_hip_out *out,
                           uint32_t flags);
 
