@@ -3215,9 +3215,8 @@ size_t heavy_lds_of(const galn_hip_readset *rs, int nw, int cpl)
 
 typedef void (*HeavyKernel)(HArgs);
 
-HeavyKernel heavy_kernel(const galn_hip_readset *rs, bool trace, bool deep)
+HeavyKernel heavy_kernel(bool wide, bool trace, bool deep)
 {
-    const bool wide = rs->idx->meta.ext != nullptr;
     if (deep)
         return trace ? (wide ? k_heavy<true, true, DEEP_NW, DEEP_CPL> : k_heavy<true, false, DEEP_NW, DEEP_CPL>)
                      : (wide ? k_heavy<false, true, DEEP_NW, DEEP_CPL> : k_heavy<false, false, DEEP_NW, DEEP_CPL>);
@@ -3231,7 +3230,7 @@ int heavy_grid(galn_hip_readset *rs, uint32_t flags, bool deep)
     const int nw = deep ? DEEP_NW : 1, cpl = deep ? DEEP_CPL : HEAVY_CPL;
     int nb = 0;
     const hipError_t e = hipOccupancyMaxActiveBlocksPerMultiprocessor(
-        &nb, reinterpret_cast<const void *>(heavy_kernel(rs, (flags & GALN_HIP_TRACE) != 0, deep)), nw * HW, heavy_lds_of(rs, nw, cpl));
+        &nb, reinterpret_cast<const void *>(heavy_kernel(rs->idx->meta.ext != nullptr, (flags & GALN_HIP_TRACE) != 0, deep)), nw * HW, heavy_lds_of(rs, nw, cpl));
     if (e != hipSuccess || nb < 1) nb = 1;
     return nb * rs->idx->n_cu;
 }
@@ -3500,6 +3499,18 @@ uint32_t heavy_park_pops()
     return v && *v ? (uint32_t)strtoul(v, nullptr, 10) : PARK_POPS;
 }
 
+int launch_widths(galn_hip_index *idx, hipStream_t st, const WArgs &w)
+{
+    const int64_t threads = 3 * ((int64_t)w.n_list + HW - 1) / HW * HW;
+    const int grid = w.n_list_dev ? idx->n_cu * 8 : (int)std::max<int64_t>(1, std::min<int64_t>(idx->n_cu * 8, (threads + 255) / 256));
+    if (idx->meta.ext)
+        hipLaunchKernelGGL(k_widths<true>, dim3(grid), dim3(256), 0, st, w);
+    else
+        hipLaunchKernelGGL(k_widths<false>, dim3(grid), dim3(256), 0, st, w);
+    HIP_OK(hipGetLastError());
+    return 0;
+}
+
 // The widths of list[0..n) (n < 0: as many as k_search handed over) into the hand-off slots; `check`:
 // those that k_search filled stay.
 int launch_widths(galn_hip_readset *rs, const int32_t *list, int n, bool check)
@@ -3522,13 +3533,7 @@ int launch_widths(galn_hip_readset *rs, const int32_t *list, int n, bool check)
     w.wlen = rs->max_len + 1;
     w.swlen = (rs->seed_len > 0 && rs->seed_len < rs->max_len) ? rs->seed_len + 1 : 1;
     w.check = check ? 1 : 0;
-    const int grid = n < 0 ? idx->n_cu * 8 : (int)std::max<int64_t>(1, std::min<int64_t>(idx->n_cu * 8, (3 * (int64_t)((n + HW - 1) / HW * HW) + 255) / 256));
-    if (idx->meta.ext)
-        hipLaunchKernelGGL(k_widths<true>, dim3(grid), dim3(256), 0, rs->ctx->stream, w);
-    else
-        hipLaunchKernelGGL(k_widths<false>, dim3(grid), dim3(256), 0, rs->ctx->stream, w);
-    HIP_OK(hipGetLastError());
-    return 0;
+    return launch_widths(idx, rs->ctx->stream, w);
 }
 
 // The wave-per-read engine over list[0..n): one wave per read, `waves` resident waves
@@ -3616,7 +3621,7 @@ int run_heavy(galn_hip_readset *rs, uint32_t flags, const int32_t *list, int n, 
     a.algo_bytes = rs->d_algo + li;
     if (!rs->capturing) HIP_OK(hipEventRecord(rs->lev[2 * li], fst));
     if (a.hand && a.hand_cap > 0 && !widths_done && (r = launch_widths(rs, list, n, true))) return r;
-    hipLaunchKernelGGL(heavy_kernel(rs, tr, false), dim3(waves), dim3(HW), lds, fst, a);
+    hipLaunchKernelGGL(heavy_kernel(wide, tr, false), dim3(waves), dim3(HW), lds, fst, a);
     if (park_pops) {
         // the reads still running when the last one was taken, with more waves each (their count is read on
         // the device; the workgroups end at once when there are none)
@@ -3638,7 +3643,7 @@ int run_heavy(galn_hip_readset *rs, uint32_t flags, const int32_t *list, int n, 
         d.park_own_off = L.own_off;
         d.park_spill_off = L.spill_off;
         d.park_state_off = L.state_off;
-        hipLaunchKernelGGL(heavy_kernel(rs, tr, true), dim3(groups), dim3(DEEP_NW * HW), lds_deep, fst, d);
+        hipLaunchKernelGGL(heavy_kernel(wide, tr, true), dim3(groups), dim3(DEEP_NW * HW), lds_deep, fst, d);
     }
     HIP_OK(hipGetLastError());
     if (!rs->capturing) HIP_OK(hipEventRecord(rs->lev[2 * li + 1], fst));
@@ -3720,15 +3725,15 @@ int run_retries(galn_hip_readset *rs, uint32_t flags, int fi, int32_t n, Tier t,
 // pops, 7.2 ms in the wave engine; 262,144 ancient DNA reads: 20 ms + 39 against 39).
 constexpr int DEFAULT_HEAVY_POPS = 1;
 
+// The plain form's: its lanes wait for the slowest of 64 at 6 us a pop. 100k reads of 100 bp 31 ms without a
+// limit, 8.8 after 512 pops, 7.2 after 128, 5.7 after 32, 5.5 after 16; 262,144 ancient DNA reads 67, 56, 51, 53.
+constexpr int PLAIN_POPS = 32;
+
 int readset_search(galn_hip_readset *rs, int form, uint32_t flags, const galn_hip_tune_t *tune)
 {
     if (!tune && rs->has_tuned) tune = &rs->tuned;
     galn_hip_index *idx = rs->idx;
     HIP_OK(hipSetDevice(idx->device));
-// The plain form's: its lanes wait for the slowest of 64 at 6 us a pop. 100k reads of 100 bp 31 ms without a
-// limit, 8.8 after 512 pops, 7.2 after 128, 5.7 after 32, 5.5 after 16; 262,144 ancient DNA reads 67, 56, 51, 53.
-constexpr int PLAIN_POPS = 32;
-
     hipStream_t fst = rs->ctx->stream;
     rs->last_flags = flags;
     rs->launches.clear();
@@ -3755,6 +3760,9 @@ constexpr int PLAIN_POPS = 32;
         // plain: one launch per 0x40000 reads, one lane per read, input order; the reads past PLAIN_POPS pops then
         // get a wave each
         slots = 0x40000;
+        budget = heavy_ok(rs) ? PLAIN_POPS : 0;
+        hwaves = heavy_grid(rs, flags, false);
+        if (budget && (r = prepare_hand(rs))) return r;
         for (int s = 0; s < rs->n && !r; s += 0x40000)
             r = run_tier(rs, flags, t0, nullptr, s, std::min(0x40000, rs->n - s), false, 0, 0, block, 0, budget);
         int32_t nh = 0;
@@ -3762,9 +3770,6 @@ constexpr int PLAIN_POPS = 32;
     } else {
         // batched: one persistent launch over the reads, longest first; reads that spend their
         // pop budget go to the wave-per-read engine
-        budget = heavy_ok(rs) ? PLAIN_POPS : 0;
-        hwaves = heavy_grid(rs, flags, false);
-        if (budget && (r = prepare_hand(rs))) return r;
         // 64-thread workgroups unless tuned otherwise (the autotuner's choice on every workload
         // measured so far)
         block = 64;
@@ -4496,6 +4501,7 @@ constexpr size_t NA_SCRATCH_BYTES = 256ull << 20;  // the array's size
 constexpr int NA_MAX_READS = 1 << 20;              // reads per call
 constexpr int NA_MAX_BATCHES = 4096;               // per-batch option sets per call
 constexpr int NA_MAX_DEVICES = 64;
+constexpr int NA_PARK = 24;  // counters of parked reads, in the i32 at the array's start
 }  // namespace
 
 static __device__ __align__(256) uint8_t scratch[NA_SCRATCH_BYTES];
@@ -4546,7 +4552,7 @@ NaLayout na_layout()
     L.ctr = 0;      // 8 x i32: [0],[1] failure counts, [2] claim counter, [3] unused, [4..6] failure kinds
     L.top = 64;     // u64 records reserved in the caller's array
     L.algo = 72;    // u64 algorithmic index bytes
-    L.scan = 80;    // 2 x i32 (k_na_scan)
+    L.scan = 80;    // 2 x i32 (k_na_scan); from 96 (NA_PARK) 2 x i32, the parked reads and their claim counter
     L.ghead = 256;  // NSHARD x u64 free-granule stack heads
     L.gbump = L.ghead + NSHARD * 8;
     size_t off = align_up(L.gbump + 4, 256);
@@ -4562,6 +4568,55 @@ NaLayout na_layout()
     off += (size_t)NA_MAX_READS * 8;
     L.lanes = align_up(off, 256);
     return L;
+}
+
+// k_fill's counterpart for the first list of reads: 0, 1, 2, ...
+__global__ void k_iota(int32_t *p, int n)
+{
+    for (int i = blockIdx.x * blockDim.x + threadIdx.x; i < n; i += gridDim.x * blockDim.x) p[i] = i;
+}
+
+// The array's split for the wave engine. A lane of k_search needs two granules of pool, so 4096 lanes -- 64
+// waves on 256 CUs -- filled it, each lane on its read until the last pop; the wave engine's 512 waves each have
+// their log (128 KB) and some ten granules, reads take hand-off slots for their widths in turns of what
+// NA_HAND_BYTES hold, and NA_DEEP workgroups go on with parked reads: 30k reads of 100 bp 57 -> 7.0 ms.
+constexpr int NA_WAVES = 512;
+constexpr int NA_DEEP = 32;
+constexpr size_t NA_HAND_BYTES = 32ull << 20;
+
+struct NaWaves {
+    int waves = 0, groups = 0, turn = 0, own_cap = 0;  // turn: reads per launch
+    uint64_t n_gran = 0;
+    HLayout L, D;
+    size_t park, hand, slots, deep, pool, gnext;  // offsets
+};
+
+// At most `want` waves, halved until each has 12 granules (the last one: whatever is left, at least 32).
+// waves = 0: not even one fits.
+NaWaves na_waves(int want, int n, uint32_t hand_stride, int rec_cap, bool trace, bool wide, size_t state_bytes)
+{
+    NaWaves N;
+    for (int w = std::max(1, want);; w = w > 1 ? w / 2 : 0) {
+        if (w == 0) return N;
+        N.own_cap = w > 16 ? 1024 : 16384;
+        N.L = make_hlayout(rec_cap, N.own_cap, 1, trace, wide, state_bytes);
+        N.D = make_hlayout(0, 0, DEEP_NW, trace, wide, 0);
+        N.groups = std::min(w, NA_DEEP);
+        N.turn = (int)std::min<uint64_t>((uint64_t)n, std::max<uint64_t>(1, NA_HAND_BYTES / (hand_stride * 8ull)));
+        const int turns = (n + N.turn - 1) / N.turn;
+        N.turn = (n + turns - 1) / turns;
+        N.park = na_layout().lanes;
+        N.hand = align_up(N.park + (size_t)w * 4, 256);
+        N.slots = align_up(N.hand + (size_t)N.turn * hand_stride * 8, 256);
+        N.deep = N.slots + (size_t)w * N.L.slot_bytes;
+        N.pool = N.deep + (size_t)N.groups * N.D.slot_bytes;
+        if (N.pool + 256 >= NA_SCRATCH_BYTES) continue;
+        N.n_gran = (NA_SCRATCH_BYTES - N.pool - 256) / (GENT * sizeof(Ent) + 4);
+        if (N.n_gran < (w > 1 ? 12ull * (uint64_t)w : 32ull)) continue;
+        N.gnext = N.pool + N.n_gran * GENT * sizeof(Ent);
+        N.waves = w;
+        return N;
+    }
 }
 
 // Bytes of one pool granule with its chunk links and free-stack link.
@@ -4638,15 +4693,20 @@ int noalloc_search(galn_hip_index *idx, const galn_hip_reads *reads, galn_hip_ou
     // what readset_fill derives from the reads
     const int max_len = std::max(1, std::min(hs[0], MAXLEN));
     int seed_len = 0, max_stacks = 1, max_entries = 0;
-    bool nonneg = true;
+    bool nonneg = true, positive = true;
     for (int b = 0; b < nb; ++b) {
         const galn_search_opt_t &o = reads->bopts[b];
         if (o.seed_len < max_len) seed_len = std::max(seed_len, o.seed_len);
         max_stacks = std::max(max_stacks, reads->n_stacks[b]);
         max_entries = std::max(max_entries, std::max(o.max_entries, 0));
         nonneg = nonneg && o.s_mm >= 0 && o.s_gapo >= 0 && o.s_gape >= 0;
+        positive = positive && o.s_mm > 0 && o.s_gapo > 0 && o.s_gape > 0;
     }
     const int buckets = std::max(1, std::min(max_stacks, MAXB));
+    const bool wide = idx->meta.ext != nullptr;
+    const int wlen = max_len + 1, swlen = seed_len > 0 && seed_len < max_len ? seed_len + 1 : 1;
+    const size_t lds = heavy_lds_bytes(buckets, wlen, swlen, 1, HEAVY_CPL), lds_deep = heavy_lds_bytes(buckets, wlen, swlen, DEEP_NW, DEEP_CPL);
+    const bool engine = positive && std::max(lds, lds_deep) <= 65536;
     const int block = buckets * 128 * 4 <= 65536 ? 128 : 64;
     const int own_full = (int)(((int64_t)(max_entries + 16) / CH + MAXB + 2) / GRAN + 2);
 
@@ -4676,11 +4736,134 @@ int noalloc_search(galn_hip_index *idx, const galn_hip_reads *reads, galn_hip_ou
     a.fuse = ((flags & GALN_HIP_NOFUSE) || !nonneg) ? 0 : 1;
     a.heavy_n = ctr + 3;  // no pop budget: nothing is handed on
 
-    int rec_cap = 64, want = std::min(n, 4096), fi = 0;
+    int rec_cap = engine ? 256 : 64, want = std::min(n, engine ? NA_WAVES : 4096), fi = 0;
     int32_t n_todo = n;
     bool out_full = false;
+    if (engine) {
+        fi = 1;
+        hipLaunchKernelGGL(k_iota, dim3(std::min(1024, (n + 255) / 256)), dim3(256), 0, st, d_fail[1], n);
+        HIP_OK(hipGetLastError());
+    }
     for (int round = 0; n_todo > 0; ++round) {
         if (round >= 24) return fail(GALN_HIP_E_NOMEM, "search_device_noalloc: reads still failing after %d re-runs", round);
+        if (engine) {
+            // the wave engine over d_fail[fi][0..n_todo), a turn of reads after the other
+            const uint32_t stride = hand_words(wlen, swlen, wide);
+            const NaWaves N = na_waves(std::min(want, (int)n_todo), n_todo, stride, rec_cap, trace, wide, heavy_state_bytes(buckets, wlen, swlen));
+            if (N.waves == 0)
+                return fail(GALN_HIP_E_UNSUPPORTED, "search_device_noalloc: a wave's regions and its pool do not fit in %zu bytes", NA_SCRATCH_BYTES);
+            const int fo = fi ^ 1;
+            FILL(ctr + fo, 0, sizeof(int32_t));
+            FILL(ctr + 4, 0, 3 * sizeof(int32_t));
+            for (int at = 0; at < n_todo; at += N.turn) {
+                const int m = std::min(N.turn, (int)n_todo - at);
+                WArgs w{};
+                w.bwt = idx->d_bwt;
+                w.meta = idx->meta;
+                w.query = reads->query;
+                w.qoff = reads->qoff;
+                w.qlen = reads->qlen;
+                w.batch = reads->batch;
+                w.bopts = d_bopts;
+                w.list = d_fail[fi] + at;
+                w.n_list = m;
+                w.hand = reinterpret_cast<uint64_t *>(S + N.hand);
+                w.hand_stride = stride;
+                w.hand_cap = m;
+                w.wlen = wlen;
+                w.swlen = swlen;
+                if ((r = launch_widths(idx, st, w))) return r;
+                HArgs h{};
+                h.bwt = w.bwt;
+                h.meta = w.meta;
+                h.query = w.query;
+                h.qoff = w.qoff;
+                h.qlen = w.qlen;
+                h.maxdiff = reads->max_diff;
+                h.batch = w.batch;
+                h.bopts = d_bopts;
+                h.nstacks = d_nstacks;
+                h.list = w.list;
+                h.n_list = m;
+                h.hand = w.hand;
+                h.hand_stride = stride;
+                h.hand_cap = m;
+                h.qnext = ctr + 2;
+                h.n_slots = std::min(N.waves, m);
+                h.scratch = S + N.slots;
+                h.slot_bytes = N.L.slot_bytes;
+                h.rec_off = N.L.rec_off;
+                h.own_off = N.L.own_off;
+                h.spill_off = N.L.spill_off;
+                h.plog_off = N.L.plog_off;
+                h.slog_off = N.L.slog_off;
+                h.own_cap = N.own_cap;
+                h.rec_cap = rec_cap;
+                h.pool = reinterpret_cast<Ent *>(S + N.pool);
+                h.gnext = reinterpret_cast<uint32_t *>(S + N.gnext);
+                h.ghead = ghead;
+                h.gbump = gbump;
+                h.n_gran = (uint32_t)N.n_gran;
+                h.first_gran = (int)std::min<uint64_t>(FIRST_GRAN, N.n_gran / 2 / (uint64_t)N.waves);
+                h.out_n = out->n_aln;
+                h.out_off = out->rec_off;
+                h.out_pops = d_pops;
+                h.out_trace = out->trace;
+                h.out_bytes = out->occ_bytes;
+                h.out_rec = out->rec;
+                h.out_cap = out->rec_cap;
+                h.out_top = top;
+                h.fail_list = d_fail[fo];
+                h.fail_n = ctr + fo;
+                h.fail_kind = ctr + 4;
+                h.algo_bytes = algo;
+                h.buckets = buckets;
+                h.wlen = wlen;
+                h.swlen = swlen;
+                h.push_cap = heavy_push_cap();
+                h.park_pops = heavy_park_pops();
+                h.park_list = reinterpret_cast<int32_t *>(S + N.park);
+                h.park_n = ctr + NA_PARK;
+                h.state_off = N.L.state_off;
+                FILL(ctr + 2, 0, sizeof(int32_t));
+                FILL(ctr + NA_PARK, 0, 2 * sizeof(int32_t));
+                FILL(ghead, 0xffffffffu, NSHARD * 8);
+                FILL(gbump, (uint32_t)(h.first_gran * h.n_slots), 4);
+                hipLaunchKernelGGL(heavy_kernel(wide, trace, false), dim3(h.n_slots), dim3(HW), lds, st, h);
+                HIP_OK(hipGetLastError());
+                if (h.park_pops) {
+                    HArgs d = h;
+                    d.n_list_dev = ctr + NA_PARK;
+                    d.qnext = ctr + NA_PARK + 1;
+                    d.n_slots = std::min(N.groups, h.n_slots);
+                    d.scratch = S + N.deep;
+                    d.slot_bytes = N.D.slot_bytes;
+                    d.plog_off = N.D.plog_off;
+                    d.slog_off = N.D.slog_off;
+                    d.park_pops = 0;
+                    d.park_scratch = h.scratch;
+                    d.park_slot_bytes = N.L.slot_bytes;
+                    d.park_rec_off = N.L.rec_off;
+                    d.park_own_off = N.L.own_off;
+                    d.park_spill_off = N.L.spill_off;
+                    d.park_state_off = N.L.state_off;
+                    hipLaunchKernelGGL(heavy_kernel(wide, trace, true), dim3(d.n_slots), dim3(DEEP_NW * HW), lds_deep, st, d);
+                    HIP_OK(hipGetLastError());
+                }
+            }
+            int32_t c[8];
+            HIP_OK(hipMemcpyAsync(c, ctr, sizeof c, hipMemcpyDeviceToHost, st));
+            HIP_OK(hipStreamSynchronize(st));
+            if (c[4]) {  // the caller's record array is full: stop, and report what was reserved
+                out_full = true;
+                break;
+            }
+            if (c[5]) rec_cap *= 16;
+            if (c[6]) want = std::max(1, N.waves / 4);
+            fi = fo;
+            n_todo = c[fo];
+            continue;
+        }
         const Layout L0 = make_layout(max_len, seed_len, rec_cap, own_full);
         uint64_t n_gran = 0;
         const int lanes = na_lanes(L0.slot_bytes, std::min(want, (int)n_todo), &n_gran);

@@ -16,6 +16,7 @@ import fixtures as fx
 from conftest import golden_inputs, load_reads, run_opts
 from galn_amd import index as ix
 from galn_amd import native as nv
+from galn_amd import synth
 
 pytestmark = pytest.mark.gpu
 
@@ -158,3 +159,36 @@ def test_noalloc_record_array_too_small_and_size_limits(golden_dir):
         O = nv.Out()
         assert nv.hip_lib().galn_hip_search_device_noalloc(index.h, C.byref(R), C.byref(O), 0) == E_ARG
         assert "at most 1048576" in nv.last_error()
+
+
+# reads in several turns of hand-off slots (300 bp: some 9000 a turn), one wave less than a turn's, a single
+# read, records beyond the first slots' 256 (a re-run with larger ones), and penalties of zero, which the wave
+# engine does not take
+@pytest.mark.parametrize("n,length,opts", [(20_011, 300, ["-n", "0", "-o", "0"]), (511, 60, []), (1, 37, []),
+                                           (200, 9, ["-n", "3", "-o", "0", "-N", "-l", "1024"]), (300, 40, ["-M", "0"])])
+def test_noalloc_equals_batched_across_turns(n, length, opts):
+    print(f"case noalloc turns {n} x {length} {opts}", flush=True)
+    rng = np.random.default_rng(n)
+    ref = np.frombuffer(b"ACGT", np.uint8)[rng.integers(0, 4, 30_000)]
+    at = rng.integers(0, ref.size - length, n)
+    reads = ref[at[:, None] + np.arange(length)]
+    at = rng.integers(0, length, n)
+    reads[np.arange(n), at] = np.frombuffer(b"ACGT", np.uint8)[rng.integers(0, 4, n)]
+    lens = np.full(n, length, np.int32)
+    q, qoff = synth.encode_queries(reads, lens)
+    batch = np.zeros(n, np.int32)
+    bopts, nst, md = nv.prepare_batches(nv.gap_opt_from_args(opts), lens, batch)
+    prim, last = ix.bwt_from_forward(ix.encode_forward(ref))
+    L2, words = ix.pack_bwt(last)
+    meta = {"primary": prim, "L2": list(L2), "seq_len": int(last.size), "bwt_size": int(words.size)}
+    with nv.Index(words, meta, 0) as index:
+        rs = nv.ReadSet(index, q, qoff, lens, md, batch, bopts, nst)
+        rs.search(nv.FORM_BATCHED)
+        want = rs.results(want_pops=True)
+        rs.close()
+        rc, n_rec, got = _noalloc(index, (q, qoff, lens, md, batch, bopts, nst), 0, rec_cap=max(4 * n, want.rec.shape[0]) + 4096)
+    assert rc == 0, nv.last_error()
+    np.testing.assert_array_equal(got.n_aln, want.n_aln)
+    np.testing.assert_array_equal(got.pops, want.pops)
+    for i in range(n):
+        np.testing.assert_array_equal(got.records(i), want.records(i))
