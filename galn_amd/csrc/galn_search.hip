@@ -2801,6 +2801,25 @@ __global__ void k_fill_u32(uint32_t *p, uint32_t v, uint32_t n)
     for (uint32_t i = blockIdx.x * blockDim.x + threadIdx.x; i < n; i += gridDim.x * blockDim.x) p[i] = v;
 }
 
+// The resets before a search, and before a launch of the wave engine, in one kernel each.
+__global__ void k_reset_search(unsigned long long *algo, int n_algo, unsigned long long *stats, unsigned long long *top, int32_t *ctr)
+{
+    for (int i = threadIdx.x; i < n_algo; i += blockDim.x) algo[i] = 0;
+    if (threadIdx.x < 16) stats[threadIdx.x] = 0;
+    if (threadIdx.x < 8) ctr[threadIdx.x] = 0;
+    if (threadIdx.x == 0) *top = 0;
+}
+
+__global__ void k_reset_heavy(int32_t *qnext, int32_t *park_n, unsigned long long *ghead, uint32_t *gbump, uint32_t first)
+{
+    for (int i = threadIdx.x; i < NSHARD; i += blockDim.x) ghead[i] = ~0ull;  // an empty free stack
+    if (threadIdx.x == 0) {
+        *qnext = 0;
+        park_n[0] = park_n[1] = 0;
+        *gbump = first;  // granules handed out: those the workgroups start with
+    }
+}
+
 // ---------------------------------------------------------------------------
 // host side
 
@@ -2963,6 +2982,16 @@ struct galn_hip_readset {
     std::vector<hipEvent_t> lev;           // 2 per launch, reused across searches
     unsigned long long *d_algo = nullptr;  // per-launch algorithmic byte counters
     static constexpr int MAX_LAUNCH = 256;
+    struct Back {                          // pinned: what a search reads back at its end
+        unsigned long long algo[MAX_LAUNCH];
+        int32_t failed;
+        uint32_t used;
+    } *back = nullptr;
+    struct {
+        const void *kernel;
+        size_t lds;
+        int groups;
+    } occ[4] = {};                         // workgroups of the wave engine a CU holds, as asked of the runtime
 };
 
 namespace {
@@ -3047,9 +3076,10 @@ int ensure_pool(SearchCtx *idx, uint64_t want)
     static std::mutex mu;
     std::lock_guard<std::mutex> lk(mu);
     const uint64_t gbytes = (uint64_t)GRAN * CH * sizeof(Ent);
+    const uint64_t have = idx->n_gran;
+    if (!idx->grow && have >= std::max<uint64_t>(want, 1024)) return 0;
     size_t freeb = 0, totalb = 0;
     HIP_OK(hipMemGetInfo(&freeb, &totalb));
-    const uint64_t have = idx->n_gran;
     uint64_t cap = (uint64_t)((freeb + have * (gbytes + GRAN * 4 + 4)) / 2) / (gbytes + GRAN * 4 + 4);
     cap = std::min<uint64_t>(cap, MAX_POOL_CHUNKS / GRAN);
     cap = std::min<uint64_t>(cap, pool_test_cap());
@@ -3231,11 +3261,16 @@ HeavyKernel heavy_kernel(bool wide, bool trace, bool deep)
 int heavy_grid(galn_hip_readset *rs, uint32_t flags, bool deep)
 {
     const int nw = deep ? DEEP_NW : 1, cpl = deep ? DEEP_CPL : HEAVY_CPL;
-    int nb = 0;
-    const hipError_t e = hipOccupancyMaxActiveBlocksPerMultiprocessor(
-        &nb, reinterpret_cast<const void *>(heavy_kernel(rs->idx->meta.ext != nullptr, (flags & GALN_HIP_TRACE) != 0, deep)), nw * HW, heavy_lds_of(rs, nw, cpl));
-    if (e != hipSuccess || nb < 1) nb = 1;
-    return nb * rs->idx->n_cu;
+    const bool trace = (flags & GALN_HIP_TRACE) != 0;
+    const void *const kernel = reinterpret_cast<const void *>(heavy_kernel(rs->idx->meta.ext != nullptr, trace, deep));
+    const size_t lds = heavy_lds_of(rs, nw, cpl);
+    auto &o = rs->occ[(trace ? 2 : 0) + (deep ? 1 : 0)];
+    if (o.kernel != kernel || o.lds != lds) {
+        int nb = 0;
+        const hipError_t e = hipOccupancyMaxActiveBlocksPerMultiprocessor(&nb, kernel, nw * HW, lds);
+        o = {kernel, lds, e != hipSuccess || nb < 1 ? 1 : nb};
+    }
+    return o.groups * rs->idx->n_cu;
 }
 
 // A workgroup's first granules: FIRST_GRAN of them, fewer in a small pool (half of it is left to share).
@@ -3335,6 +3370,11 @@ int prepare_hand(galn_hip_readset *rs)
 {
     const int sl = (rs->seed_len > 0 && rs->seed_len < rs->max_len) ? rs->seed_len : 0;
     const uint32_t stride = hand_words(rs->max_len + 1, sl + 1, rs->idx->meta.ext != nullptr);
+    if (rs->d_hand && rs->hand_bytes >= (uint64_t)std::max(rs->n, 1) * stride * 8) {
+        rs->hand_stride = stride;
+        rs->hand_cap = rs->n;
+        return 0;
+    }
     size_t freeb = 0, totalb = 0;
     HIP_OK(hipMemGetInfo(&freeb, &totalb));
     const uint64_t limit = std::min<uint64_t>(HAND_BYTES, (uint64_t)(freeb + rs->hand_bytes) / 4);
@@ -3615,10 +3655,9 @@ int run_heavy(galn_hip_readset *rs, uint32_t flags, const int32_t *list, int n, 
     a.park_n = rs->d_ctr + 8;
     a.state_off = L.state_off;
     a.first_gran = first_gran(cx, waves);
-    FILL(rs->d_ctr + 2, 0, sizeof(int32_t));
-    FILL(rs->d_ctr + 8, 0, 2 * sizeof(int32_t));
-    FILL(cx->d_ghead, 0xffffffffu, NSHARD * 8);
-    FILL(cx->d_gbump, (uint32_t)(a.first_gran * waves), 4);
+    hipLaunchKernelGGL(k_reset_heavy, dim3(1), dim3(256), 0, fst, rs->d_ctr + 2, rs->d_ctr + 8, cx->d_ghead, cx->d_gbump,
+                       (uint32_t)(a.first_gran * waves));
+    HIP_OK(hipGetLastError());
     int li = 0;
     if ((r = new_launch(rs, tier_id, &li))) return r;
     a.algo_bytes = rs->d_algo + li;
@@ -3743,10 +3782,9 @@ int readset_search(galn_hip_readset *rs, int form, uint32_t flags, const galn_hi
     const bool trace = (flags & GALN_HIP_TRACE) != 0;
     const bool graph = form != 0 && (flags & GALN_HIP_GRAPH) != 0;
     auto prologue = [&]() -> int {
-        FILL(rs->d_algo, 0, sizeof(unsigned long long) * galn_hip_readset::MAX_LAUNCH);
-        FILL(rs->d_stats, 0, 16 * 8);
-        FILL(rs->d_top, 0, sizeof(unsigned long long));
-        FILL(rs->d_ctr, 0, 8 * sizeof(int32_t));
+        hipLaunchKernelGGL(k_reset_search, dim3(1), dim3(256), 0, fst, rs->d_algo, (int)galn_hip_readset::MAX_LAUNCH, rs->d_stats,
+                           rs->d_top, rs->d_ctr);
+        HIP_OK(hipGetLastError());
         return 0;
     };
     if (!graph) {
@@ -3778,7 +3816,6 @@ int readset_search(galn_hip_readset *rs, int form, uint32_t flags, const galn_hi
         block = 64;
         if (tune && tune->block_threads > 0 && buckets_of(rs) * tune->block_threads * 4 <= 65536)
             block = tune->block_threads;
-        slots = resident_slots(rs, block, trace, tune ? tune->waves_per_cu : 0);
         const bool sorted = !tune || tune->sort_by_cost != 0;
         const int hp = tune ? tune->heavy_pops : 0;
         budget = (hp < 0 || !heavy_ok(rs)) ? 0 : (uint64_t)(hp > 0 ? hp : DEFAULT_HEAVY_POPS);
@@ -3787,6 +3824,7 @@ int readset_search(galn_hip_readset *rs, int form, uint32_t flags, const galn_hi
         const int32_t *list = sorted ? rs->d_sorted : nullptr;
         // every read to the wave engine: the widths launch stands in the place of k_search's
         const bool direct = budget == 1;
+        slots = direct ? 0 : resident_slots(rs, block, trace, tune ? tune->waves_per_cu : 0);
         auto first_tier = [&]() -> int {
             if (!direct) return run_tier(rs, flags, t0, list, 0, rs->n, true, slots, 0, block, 0, budget);
             int li = 0, rc = new_launch(rs, 0, &li);
@@ -3873,25 +3911,30 @@ int readset_search(galn_hip_readset *rs, int form, uint32_t flags, const galn_hi
         }
     }
     if (r) return r;
-    int32_t nf = 0;
-    if ((r = read_ctr(rs, 0, &nf))) return r;
-    if (nf > 0 && (r = run_retries(rs, flags, 0, nf, t0, slots, budget, std::max(1, hwaves)))) return r;
-    HIP_OK(hipStreamSynchronize(fst));
-    if (rs->ctx->d_gbump) {
-        uint32_t used = 0;
-        HIP_OK(hipMemcpyAsync(&used, rs->ctx->d_gbump, 4, hipMemcpyDeviceToHost, fst));
+    // what the host needs of the search in one wait: the failures, the granules used, the launches' index bytes
+    galn_hip_readset::Back *const back = rs->back;
+    auto read_back = [&]() -> int {
+        back->used = 0;
+        HIP_OK(hipMemcpyAsync(&back->failed, rs->d_ctr, 4, hipMemcpyDeviceToHost, fst));
+        if (rs->ctx->d_gbump) HIP_OK(hipMemcpyAsync(&back->used, rs->ctx->d_gbump, 4, hipMemcpyDeviceToHost, fst));
+        if (!rs->launches.empty())
+            HIP_OK(hipMemcpyAsync(back->algo, rs->d_algo, rs->launches.size() * 8, hipMemcpyDeviceToHost, fst));
         HIP_OK(hipStreamSynchronize(fst));
-        if (used >= rs->ctx->n_gran) rs->ctx->grow = true;
+        return 0;
+    };
+    if ((r = read_back())) return r;
+    if (back->failed > 0) {
+        if (!slots) slots = resident_slots(rs, block, trace, tune ? tune->waves_per_cu : 0);
+        if ((r = run_retries(rs, flags, 0, back->failed, t0, slots, budget, std::max(1, hwaves)))) return r;
+        if ((r = read_back())) return r;
     }
-    std::vector<unsigned long long> ab(rs->launches.size());
-    if (!ab.empty())
-        HIP_OK(hipMemcpy(ab.data(), rs->d_algo, ab.size() * sizeof(unsigned long long), hipMemcpyDeviceToHost));
+    if (rs->ctx->d_gbump && back->used >= rs->ctx->n_gran) rs->ctx->grow = true;
     rs->first_ms = rs->total_ms = 0;
     for (size_t i = 0; i < rs->launches.size(); ++i) {
         float ms = 0;
         HIP_OK(hipEventElapsedTime(&ms, rs->lev[2 * i], rs->lev[2 * i + 1]));
         rs->launches[i].ms = ms;
-        rs->launches[i].bytes = ab[i];
+        rs->launches[i].bytes = back->algo[i];
         if (rs->launches[i].tier == 0) rs->first_ms += ms;
         rs->total_ms += ms;
     }
@@ -4192,6 +4235,7 @@ int galn_hip_readset_free(galn_hip_readset *rs)
                     rs->d_stats, rs->d_incl, rs->d_roff, rs->d_stage, rs->d_scan_tmp, rs->d_hand};
     for (void *p : ptrs)
         if (p) (void)hipFree(p);
+    if (rs->back) (void)hipHostFree(rs->back);
     for (auto &e : rs->ev)
         if (e) (void)hipEventDestroy(e);
     for (auto &e : rs->lev) (void)hipEventDestroy(e);
@@ -4221,7 +4265,8 @@ int galn_hip_readset_upload(galn_hip_index *idx, const galn_hip_reads *reads, ga
     idx->n_readsets.fetch_add(1);
     auto M = [&](void **p, size_t b) __attribute__((always_inline)) -> bool { return hipMalloc(p, b) == hipSuccess; };
     bool ok = M((void **)&rs->d_top, 8) && M((void **)&rs->d_ctr, 16 * sizeof(int32_t)) && M((void **)&rs->d_stats, 16 * 8) &&
-              M((void **)&rs->d_algo, sizeof(unsigned long long) * galn_hip_readset::MAX_LAUNCH);
+              M((void **)&rs->d_algo, sizeof(unsigned long long) * galn_hip_readset::MAX_LAUNCH) &&
+              hipHostMalloc((void **)&rs->back, sizeof *rs->back) == hipSuccess;
     if (!ok) {
         galn_hip_readset_free(rs);
         return fail(GALN_HIP_E_NOMEM, "readset_upload: device allocation failed");
@@ -4828,10 +4873,9 @@ int noalloc_search(galn_hip_index *idx, const galn_hip_reads *reads, galn_hip_ou
                 h.park_list = reinterpret_cast<int32_t *>(S + N.park);
                 h.park_n = ctr + NA_PARK;
                 h.state_off = N.L.state_off;
-                FILL(ctr + 2, 0, sizeof(int32_t));
-                FILL(ctr + NA_PARK, 0, 2 * sizeof(int32_t));
-                FILL(ghead, 0xffffffffu, NSHARD * 8);
-                FILL(gbump, (uint32_t)(h.first_gran * h.n_slots), 4);
+                hipLaunchKernelGGL(k_reset_heavy, dim3(1), dim3(256), 0, st, ctr + 2, ctr + NA_PARK, ghead, gbump,
+                                   (uint32_t)(h.first_gran * h.n_slots));
+                HIP_OK(hipGetLastError());
                 hipLaunchKernelGGL(heavy_kernel(wide, trace, false), dim3(h.n_slots), dim3(HW), lds, st, h);
                 HIP_OK(hipGetLastError());
                 if (h.park_pops) {
