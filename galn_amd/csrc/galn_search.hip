@@ -1,7 +1,10 @@
 // galn_search.hip -- BWA-aln backtracking search on gfx950 (MI355X), and its C ABI.
 //
-// One lane searches one read (thread-per-read). The lane runs the read as a
-// state machine whose every iteration performs exactly one occurrence (LF)
+// Two engines. k_heavy searches a read with a wave, many entries of its stack at a
+// time (its comment is further down); every form's reads end there. k_search
+// searches a read with a lane (thread-per-read): the plain form's first pops, the
+// batched form where it is tuned to hand reads over later, penalties that are not
+// positive, re-runs. The lane runs the read as a state machine whose every iteration performs exactly one occurrence (LF)
 // lookup, whatever the read is doing -- widths (bwt_cal_width), the seed
 // widths, expanding a popped stack entry (bwt_2occ4), or an exact-match tail
 // (bwt_match_exact_alt) -- so all 64 lanes of a wave issue their random index
@@ -23,9 +26,11 @@
 // record order, pop counts and trace hashes are those of the CPU search.
 //
 // Forms:
-//   plain    one launch per 0x40000 reads (one lane per read, input order);
-//   batched  one persistent launch over the whole read list; lanes claim the
-//            next read from a device counter as soon as theirs is done.
+//   plain    one launch per 0x40000 reads (one lane per read, input order), then a
+//            wave for each read past 32 pops;
+//   batched  one persistent launch over the whole read list; waves claim the next
+//            read from a device counter as soon as theirs is done;
+//   without allocation  the same inside a static device array.
 // Reads that outgrow their record slots, or find the pool exhausted, are re-run
 // from scratch in a later launch with more room, so results never depend on
 // the capacities chosen (the reference's contract, src/bwtgap_hd.h:10-22).
@@ -1554,6 +1559,9 @@ struct WArgs {
     int32_t check;  // slots may hold widths already
 };
 constexpr int H_ROOT = 127;  // steps of the root chain kept at most (one round's chains with the root itself)
+// Only of reads of this length on: a shorter descent saves little, and its pushes come all at once (2M ancient
+// DNA reads, median 45, 240 ms with all of them, 228 with those from 90 on, 224 with none).
+constexpr int H_ROOT_MIN = 90;
 constexpr uint64_t HAND_OK = 1ull << 63, HAND_SEARCH = 1ull << 62;  // a slot's flags: filled; by k_search
 
 template <bool WIDE>
@@ -1584,7 +1592,7 @@ __global__ void __launch_bounds__(256) k_widths(WArgs a)
             dst[a.hand_stride - 1] = cal_width_one<K>(a.bwt, a.meta, sl, q + (len - sl), [w](int i, uint64_t v, int bid) { w[i] = wpack(v, bid); });
         } else if constexpr (!WIDE) {
             uint64_t *const at = dst + 1 + a.wlen + a.swlen;
-            const int most = none ? 0 : min(len, min(a.wlen - 1, H_ROOT));
+            const int most = none || len < H_ROOT_MIN ? 0 : min(len, min(a.wlen - 1, H_ROOT));
             uint32_t k = 0, l = (uint32_t)a.meta.seq_len;
             int s = 0;
             while (s < most) {
@@ -3809,8 +3817,8 @@ int readset_search(galn_hip_readset *rs, int form, uint32_t flags, const galn_hi
         int32_t nh = 0;
         if (!r && budget && !(r = read_ctr(rs, 3, &nh)) && nh > 0) r = run_heavy(rs, flags, rs->d_heavy, nh, 256, 0, 10, hwaves);
     } else {
-        // batched: one persistent launch over the reads, longest first; reads that spend their
-        // pop budget go to the wave-per-read engine
+        // batched: one persistent launch over the reads, longest first; with a cutoff above 1 reads that
+        // spend their pop budget go from k_search to the wave-per-read engine
         // 64-thread workgroups unless tuned otherwise (the autotuner's choice on every workload
         // measured so far)
         block = 64;
@@ -4336,7 +4344,7 @@ int galn_hip_readset_autotune(galn_hip_index *idx, galn_hip_readset *rs, uint32_
         galn_hip_tune_t t{};
         t.sort_by_cost = 1;
         t.block_threads = 128;
-        // (1: every read that pops goes to the wave engine, k_search computing only its widths)
+        // (1: every read goes to the wave engine, k_search is not launched)
         const int cut[] = {1, 16, 64, 128, 256, 512, 1024, 4096};
         int r;
         if (heavy_ok(rs)) {
