@@ -3278,7 +3278,12 @@ int heavy_grid(galn_hip_readset *rs, uint32_t flags, bool deep)
         const hipError_t e = hipOccupancyMaxActiveBlocksPerMultiprocessor(&nb, kernel, nw * HW, lds);
         o = {kernel, lds, e != hipSuccess || nb < 1 ? 1 : nb};
     }
-    return o.groups * rs->idx->n_cu;
+    // Without seeds a read's stack, log and granules are several times larger, and those of 16 waves a CU go past L2:
+    // 12 take 2M ancient DNA reads from 230 to 221 ms, 262,144 from 39.4 to 38.6, 100,003 repeat-rich ones from 105
+    // to 101; 100k seeded reads of 100 bp take 4.1 ms with 16, 4.6 with 12. (From 2^32 symbols on the waves wait on
+    // the index in HBM: 16; and few reads get a wave each: 4001 take 13.1 ms either way.)
+    const bool fewer = !deep && rs->seed_len == 0 && rs->idx->meta.ext == nullptr && rs->n >= 16 * o.groups * rs->idx->n_cu;
+    return (fewer ? std::min(o.groups, 12) : o.groups) * rs->idx->n_cu;
 }
 
 // A workgroup's first granules: FIRST_GRAN of them, fewer in a small pool (half of it is left to share).
