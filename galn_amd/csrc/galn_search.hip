@@ -3206,6 +3206,8 @@ constexpr uint32_t PARK_POPS = 2048;
 // only shortens the tail: 16 reads of 100 bp 0.54 ms after 512 pops, 0.64 after 2048, 0.59 after 256.
 constexpr uint32_t PARK_POPS_FEW = 512;
 constexpr int FIRST_GRAN = 8;  // granules a workgroup of it starts with
+constexpr int HEAVY_REC = 256;  // record slots of its waves in a search's first launch
+constexpr int HEAVY_REC_MAX = 1 << 26;  // and in any (1.6 GB a wave; a slot's offsets are 32-bit)
 
 struct HLayout {
     uint64_t slot_bytes;
@@ -3441,7 +3443,7 @@ int reserve_search(galn_hip_readset *rs, int n, int max_len, uint32_t flags)
     uint64_t p2 = 1024;
     while (p2 < (uint64_t)waves * 256) p2 <<= 1;
     if (!soft(ensure_pool(cx, p2))) {
-        soft(grow_dev((void **)&rs->d_hscratch, rs->hscratch_bytes, heavy_scratch(rs, waves, 256, flags), s));
+        soft(grow_dev((void **)&rs->d_hscratch, rs->hscratch_bytes, heavy_scratch(rs, waves, HEAVY_REC, flags), s));
     }
     // the results: the record counts' scan over n reads and the staged records
     size_t tmp = 0;
@@ -3735,18 +3737,26 @@ int grow_records(galn_hip_readset *rs)
 
 // Re-run failed reads (fail buffer `fi`, count n) until none is left: a full output arena
 // grows, full record slots get 16 times more, an exhausted pool gets fewer lanes sharing it.
+// A read past `budget` pops ends in the wave engine, whose record slots grow with each such re-run
+// from the 256 of the first launch; where that many for each wave would take more than half of
+// the free memory, fewer waves run.
 int run_retries(galn_hip_readset *rs, uint32_t flags, int fi, int32_t n, Tier t, int slots, uint64_t budget,
                 int hwaves)
 {
     hipStream_t fst = rs->ctx->stream;
     const int block = pick_block(rs);
+    int heavy_rec = HEAVY_REC;
     for (int round = 0; n > 0; ++round) {
         if (round >= 24) return fail(GALN_HIP_E_NOMEM, "reads still failing after %d re-runs", round);
         int32_t kind[3] = {0, 0, 0};
         HIP_OK(hipMemcpy(kind, rs->d_ctr + 4, sizeof(kind), hipMemcpyDeviceToHost));
         int r;
         if (kind[0] && (r = grow_records(rs))) return r;
-        if (kind[1]) t.rec_cap *= 16;
+        if (kind[1]) {
+            // (a lane hands a read on after `budget` pops, each of which gives one record at most)
+            if (!budget || (uint64_t)t.rec_cap < budget) t.rec_cap *= 16;
+            heavy_rec = std::min(heavy_rec * 16, HEAVY_REC_MAX);
+        }
         if (kind[2]) {
             // an exhausted pool: twice the granules when there is room, else fewer lanes sharing it
             const uint32_t before = rs->ctx->n_gran;
@@ -3764,7 +3774,13 @@ int run_retries(galn_hip_readset *rs, uint32_t flags, int fi, int32_t n, Tier t,
         if ((r = run_tier(rs, flags, t, rs->d_fail[fi], 0, n, true, slots, fo, block, 1 + round, budget))) return r;
         int32_t nh = 0;
         if ((r = read_ctr(rs, 3, &nh))) return r;
-        if (nh > 0 && (r = run_heavy(rs, flags, rs->d_heavy, nh, 256 * (1 + round), fo, 11 + round, hwaves))) return r;
+        if (nh > 0) {
+            int waves = std::min(hwaves, (int)nh);
+            size_t freeb = 0, totalb = 0;
+            HIP_OK(hipMemGetInfo(&freeb, &totalb));
+            while (waves > 1 && heavy_scratch(rs, waves, heavy_rec, flags) > (freeb + rs->hscratch_bytes) / 2) waves /= 2;
+            if ((r = run_heavy(rs, flags, rs->d_heavy, nh, heavy_rec, fo, 11 + round, waves))) return r;
+        }
         int32_t nf = 0;
         if ((r = read_ctr(rs, fo, &nf))) return r;
         fi = fo;
@@ -3820,7 +3836,7 @@ int readset_search(galn_hip_readset *rs, int form, uint32_t flags, const galn_hi
         for (int s = 0; s < rs->n && !r; s += 0x40000)
             r = run_tier(rs, flags, t0, nullptr, s, std::min(0x40000, rs->n - s), false, 0, 0, block, 0, budget);
         int32_t nh = 0;
-        if (!r && budget && !(r = read_ctr(rs, 3, &nh)) && nh > 0) r = run_heavy(rs, flags, rs->d_heavy, nh, 256, 0, 10, hwaves);
+        if (!r && budget && !(r = read_ctr(rs, 3, &nh)) && nh > 0) r = run_heavy(rs, flags, rs->d_heavy, nh, HEAVY_REC, 0, 10, hwaves);
     } else {
         // batched: one persistent launch over the reads, longest first; with a cutoff above 1 reads that
         // spend their pop budget go from k_search to the wave-per-read engine
@@ -3848,7 +3864,8 @@ int readset_search(galn_hip_readset *rs, int form, uint32_t flags, const galn_hi
             return 0;
         };
         auto wave_tier = [&](int n) -> int {
-            return direct ? run_heavy(rs, flags, list, rs->n, 256, 0, 10, hwaves, true) : run_heavy(rs, flags, rs->d_heavy, n, 256, 0, 10, hwaves);
+            return direct ? run_heavy(rs, flags, list, rs->n, HEAVY_REC, 0, 10, hwaves, true)
+                          : run_heavy(rs, flags, rs->d_heavy, n, HEAVY_REC, 0, 10, hwaves);
         };
         if (graph) {
             // the prologue, the persistent launch and the wave-engine launch (its read count read
@@ -3860,7 +3877,7 @@ int readset_search(galn_hip_readset *rs, int form, uint32_t flags, const galn_hi
             key.push_cap = heavy_push_cap();
             key.park_pops = heavy_park_pops(direct && rs->n <= hwaves);
             if ((!direct && (r = prepare_tier(rs, t0, slots, std::min(slots, rs->n)))) ||
-                (budget && (r = prepare_heavy(rs, hwaves, 256, flags))))
+                (budget && (r = prepare_heavy(rs, hwaves, HEAVY_REC, flags))))
                 return r;
             while (rs->lev.size() < 4) {
                 hipEvent_t e;
@@ -4797,7 +4814,7 @@ int noalloc_search(galn_hip_index *idx, const galn_hip_reads *reads, galn_hip_ou
     a.fuse = ((flags & GALN_HIP_NOFUSE) || !nonneg) ? 0 : 1;
     a.heavy_n = ctr + 3;  // no pop budget: nothing is handed on
 
-    int rec_cap = engine ? 256 : 64, want = std::min(n, engine ? NA_WAVES : 4096), fi = 0;
+    int rec_cap = engine ? HEAVY_REC : 64, want = std::min(n, engine ? NA_WAVES : 4096), fi = 0;
     int32_t n_todo = n;
     bool out_full = false;
     if (engine) {
