@@ -1760,7 +1760,7 @@ __global__ void __launch_bounds__(64 * NW) __attribute__((amdgpu_waves_per_eu(4,
             }
             __syncthreads();
             const bool unsup = len < 1 || len > MAXLEN || len + 1 > HA(wlen) || F.n_stacks > HA(buckets) || F.md_read > MAXDIFF ||
-                               F.max_gapo > MAXDIFF || F.max_gapo + F.max_gape > 255;
+                               F.max_gapo > MAXDIFF || F.max_gapo + F.max_gape > 255 || F.max_gape < 0;
             const uint64_t h0 = (!unsup && HA(hand) && pos < HA(hand_cap)) ? HA(hand)[(uint64_t)pos * HA(hand_stride)] : 0;
             if (!unsup) {
                 if (h0 >> 63) {
