@@ -1388,7 +1388,7 @@ struct HShared {
 static_assert(sizeof(HShared) % 8 == 0, "the widths follow it in a parked read's state");
 
 // what a read's state is besides HShared: the widths, the buckets
-__host__ __device__ inline size_t heavy_state_bytes(int buckets, int wlen, int swlen)
+__host__ __device__ constexpr size_t heavy_state_bytes(int buckets, int wlen, int swlen)
 {
     return sizeof(HShared) + (size_t)(wlen + swlen + 2) * 8 + (size_t)buckets * 12;
 }
@@ -3244,11 +3244,10 @@ size_t heavy_lds_bytes(int buckets, int wlen, int swlen, int nw, int cpl)
            H_STEPS * 2 + (size_t)wlen;
 }
 
-size_t heavy_state_of(const galn_hip_readset *rs)
-{
-    const int swlen = (rs->seed_len > 0 && rs->seed_len < rs->max_len) ? rs->seed_len + 1 : 1;
-    return heavy_state_bytes(buckets_of(rs), rs->max_len + 1, swlen);
-}
+// A wave's scratch has room for the state of any read (5% of a slot): launches of other reads and options
+// then fit what the first one allocated (a regrowth of this buffer frees some 2 GB, which waits for every
+// stream of the device).
+constexpr size_t HEAVY_STATE = heavy_state_bytes(MAXB, MAXLEN + 1, MAXLEN + 1);
 
 size_t heavy_lds_of(const galn_hip_readset *rs, int nw, int cpl)
 {
@@ -3267,6 +3266,21 @@ HeavyKernel heavy_kernel(bool wide, bool trace, bool deep)
                  : (wide ? k_heavy<false, true, 1, HEAVY_CPL> : k_heavy<false, false, 1, HEAVY_CPL>);
 }
 
+// Workgroups of the wave engine a CU holds.
+int heavy_per_cu(galn_hip_readset *rs, uint32_t flags, bool deep, size_t lds)
+{
+    const void *const kernel = reinterpret_cast<const void *>(heavy_kernel(rs->idx->meta.ext != nullptr, (flags & GALN_HIP_TRACE) != 0, deep));
+    int nb = 0;
+    const hipError_t e = hipOccupancyMaxActiveBlocksPerMultiprocessor(&nb, kernel, (deep ? DEEP_NW : 1) * HW, lds);
+    return e != hipSuccess || nb < 1 ? 1 : nb;
+}
+
+// The most workgroups that heavy_grid gives for any reads and options (that of the least LDS).
+int heavy_grid_most(galn_hip_readset *rs, uint32_t flags, bool deep)
+{
+    return heavy_per_cu(rs, flags, deep, heavy_lds_bytes(1, 2, 1, deep ? DEEP_NW : 1, deep ? DEEP_CPL : HEAVY_CPL)) * rs->idx->n_cu;
+}
+
 // Workgroups of the wave engine that are resident at once.
 int heavy_grid(galn_hip_readset *rs, uint32_t flags, bool deep)
 {
@@ -3275,11 +3289,7 @@ int heavy_grid(galn_hip_readset *rs, uint32_t flags, bool deep)
     const void *const kernel = reinterpret_cast<const void *>(heavy_kernel(rs->idx->meta.ext != nullptr, trace, deep));
     const size_t lds = heavy_lds_of(rs, nw, cpl);
     auto &o = rs->occ[(trace ? 2 : 0) + (deep ? 1 : 0)];
-    if (o.kernel != kernel || o.lds != lds) {
-        int nb = 0;
-        const hipError_t e = hipOccupancyMaxActiveBlocksPerMultiprocessor(&nb, kernel, nw * HW, lds);
-        o = {kernel, lds, e != hipSuccess || nb < 1 ? 1 : nb};
-    }
+    if (o.kernel != kernel || o.lds != lds) o = {kernel, lds, heavy_per_cu(rs, flags, deep, lds)};
     // Without seeds a read's stack, log and granules are several times larger, and those of 16 waves a CU go past L2:
     // 12 take 2M ancient DNA reads from 230 to 221 ms, 262,144 from 39.4 to 38.6, 100,003 repeat-rich ones from 105
     // to 101; 100k seeded reads of 100 bp take 4.1 ms with 16, 4.6 with 12. (From 2^32 symbols on the waves wait on
@@ -3353,13 +3363,13 @@ int prepare_tier(galn_hip_readset *rs, const Tier &t, int slots, int pool_lanes)
 }
 
 // Bytes of scratch for the wave engine: `waves` workgroups of one wave, then the workgroups that go on with
-// parked reads (which read the former's).
-size_t heavy_scratch(galn_hip_readset *rs, int waves, int rec_cap, uint32_t flags)
+// parked reads (which read the former's), `deep` of them at most.
+size_t heavy_scratch(galn_hip_readset *rs, int waves, int deep, int rec_cap, uint32_t flags)
 {
     const bool trace = (flags & GALN_HIP_TRACE) != 0, wide = rs->idx->meta.ext != nullptr;
     const int own_cap = (int)std::min<uint64_t>(rs->ctx->n_gran, 32768);
-    const size_t one = (size_t)waves * make_hlayout(rec_cap, own_cap, 1, trace, wide, heavy_state_of(rs)).slot_bytes;
-    return one + (size_t)std::min(waves, heavy_grid(rs, flags, true)) * make_hlayout(0, 0, DEEP_NW, trace, wide, 0).slot_bytes;
+    const size_t one = (size_t)waves * make_hlayout(rec_cap, own_cap, 1, trace, wide, HEAVY_STATE).slot_bytes;
+    return one + (size_t)std::min(waves, deep) * make_hlayout(0, 0, DEEP_NW, trace, wide, 0).slot_bytes;
 }
 
 // The allocations of a wave-engine launch of `waves` waves.
@@ -3372,7 +3382,7 @@ int prepare_heavy(galn_hip_readset *rs, int waves, int rec_cap, uint32_t flags)
     int r = ensure_pool(cx, p2);
     if (r) return r;
     if ((r = grow_dev((void **)&rs->d_park, rs->park_bytes, (size_t)waves * 4, cx->stream))) return r;
-    return grow_dev((void **)&rs->d_hscratch, rs->hscratch_bytes, heavy_scratch(rs, waves, rec_cap, flags), cx->stream);
+    return grow_dev((void **)&rs->d_hscratch, rs->hscratch_bytes, heavy_scratch(rs, waves, heavy_grid(rs, flags, true), rec_cap, flags), cx->stream);
 }
 
 // Hand-off slots for the widths of reads moving to the wave engine: one per read, up to
@@ -3438,12 +3448,14 @@ int reserve_search(galn_hip_readset *rs, int n, int max_len, uint32_t flags)
         rs->hand_bytes = 0;
         rs->hand_cap = 0;
     }
-    // the stack pool and the wave engine's per-wave scratch, as prepare_heavy sizes them
-    const int waves = std::max(1, std::min(heavy_grid(rs, flags, false), n));
+    // the stack pool and the wave engine's per-wave scratch, as prepare_heavy sizes them for the reads and
+    // options that get the most waves (this launch's may be fewer)
+    const int waves = std::max(1, std::min(heavy_grid_most(rs, flags, false), n));
     uint64_t p2 = 1024;
     while (p2 < (uint64_t)waves * 256) p2 <<= 1;
     if (!soft(ensure_pool(cx, p2))) {
-        soft(grow_dev((void **)&rs->d_hscratch, rs->hscratch_bytes, heavy_scratch(rs, waves, HEAVY_REC, flags), s));
+        soft(grow_dev((void **)&rs->d_park, rs->park_bytes, (size_t)waves * 4, s));
+        soft(grow_dev((void **)&rs->d_hscratch, rs->hscratch_bytes, heavy_scratch(rs, waves, heavy_grid_most(rs, flags, true), HEAVY_REC, flags), s));
     }
     // the results: the record counts' scan over n reads and the staged records
     size_t tmp = 0;
@@ -3609,7 +3621,7 @@ int run_heavy(galn_hip_readset *rs, uint32_t flags, const int32_t *list, int n, 
     int r = prepare_heavy(rs, waves, rec_cap, flags);
     if (r) return r;
     const int own_cap = (int)std::min<uint64_t>(cx->n_gran, 32768);
-    const HLayout L = make_hlayout(rec_cap, own_cap, 1, tr, wide, heavy_state_of(rs));
+    const HLayout L = make_hlayout(rec_cap, own_cap, 1, tr, wide, HEAVY_STATE);
     const int wlen = rs->max_len + 1;
     const int swlen = (rs->seed_len > 0 && rs->seed_len < rs->max_len) ? rs->seed_len + 1 : 1;
     const size_t lds = heavy_lds_of(rs, 1, HEAVY_CPL);
@@ -3778,7 +3790,7 @@ int run_retries(galn_hip_readset *rs, uint32_t flags, int fi, int32_t n, Tier t,
             int waves = std::min(hwaves, (int)nh);
             size_t freeb = 0, totalb = 0;
             HIP_OK(hipMemGetInfo(&freeb, &totalb));
-            while (waves > 1 && heavy_scratch(rs, waves, heavy_rec, flags) > (freeb + rs->hscratch_bytes) / 2) waves /= 2;
+            while (waves > 1 && heavy_scratch(rs, waves, heavy_grid(rs, flags, true), heavy_rec, flags) > (freeb + rs->hscratch_bytes) / 2) waves /= 2;
             if ((r = run_heavy(rs, flags, rs->d_heavy, nh, heavy_rec, fo, 11 + round, waves))) return r;
         }
         int32_t nf = 0;
