@@ -1556,6 +1556,7 @@ struct WArgs {
     uint32_t hand_stride;
     int32_t hand_cap;
     int32_t wlen, swlen;
+    int32_t root;   // steps of a root chain that a slot has room for (0: none)
     int32_t check;  // slots may hold widths already
 };
 constexpr int H_ROOT = 127;  // steps of the root chain kept at most (one round's chains with the root itself)
@@ -1592,7 +1593,7 @@ __global__ void __launch_bounds__(256) k_widths(WArgs a)
             dst[a.hand_stride - 1] = cal_width_one<K>(a.bwt, a.meta, sl, q + (len - sl), [w](int i, uint64_t v, int bid) { w[i] = wpack(v, bid); });
         } else if constexpr (!WIDE) {
             uint64_t *const at = dst + 1 + a.wlen + a.swlen;
-            const int most = none || len < H_ROOT_MIN ? 0 : min(len, min(a.wlen - 1, H_ROOT));
+            const int most = none || len < H_ROOT_MIN ? 0 : min(len, a.root);
             uint32_t k = 0, l = (uint32_t)a.meta.seq_len;
             int s = 0;
             while (s < most) {
@@ -1616,11 +1617,11 @@ __global__ void __launch_bounds__(256) k_widths(WArgs a)
     }
 }
 
+// steps of the root chain that a hand-off slot of reads of up to max_len bases has room for
+inline int hand_root(int max_len, bool wide) { return wide || max_len < H_ROOT_MIN ? 0 : std::min(max_len, H_ROOT); }
+
 // words of a hand-off slot
-inline uint32_t hand_words(int wlen, int swlen, bool wide)
-{
-    return (uint32_t)(1 + wlen + swlen + (wide ? 0 : std::min(wlen - 1, H_ROOT)) + 2);
-}
+inline uint32_t hand_words(int wlen, int swlen, int root) { return (uint32_t)(1 + wlen + swlen + root + 2); }
 
 // A wave logs a round's pushes in the order it makes them, 16 bytes after 16 bytes. A logged push holds, beside
 // the entry, its chain, its rank among the chain's pushes to its bucket and the bucket's code, so that it can
@@ -2958,6 +2959,7 @@ struct galn_hip_readset {
     uint64_t *d_hand = nullptr;
     size_t hand_bytes = 0;
     uint32_t hand_stride = 0;
+    int32_t hand_root = 0;  // steps of a root chain in each
     int32_t hand_cap = 0;
     // results in read order: inclusive prefix sums of record counts, output offsets, staging
     uint64_t *d_incl = nullptr, *d_roff = nullptr;
@@ -3387,22 +3389,38 @@ int prepare_heavy(galn_hip_readset *rs, int waves, int rec_cap, uint32_t flags)
 
 // Hand-off slots for the widths of reads moving to the wave engine: one per read, up to
 // HAND_BYTES or a quarter of the free device memory (reads beyond recompute their widths there,
-// one lane walking the read while the wave waits: with every read sent to the wave engine, 10M
-// reads of up to 150 bp need 12 GB).
+// one lane walking the read while the wave waits). 10M unseeded reads of up to 150 bp, every read sent
+// to the wave engine, need 22.6 GB with their root chains (127 words of a slot's 282) and 12.4 without,
+// and where all reads fit only without, the chains are left out: a read then starts with one lane at
+// work, but every read has its widths.
 constexpr uint64_t HAND_BYTES = 32ull << 30;
+
+// HAND_BYTES, or the value of GALN_HIP_TEST_HAND_BYTES, with which the tests leave slots out.
+uint64_t hand_limit(const galn_hip_readset *rs, size_t freeb)
+{
+    const char *v = getenv("GALN_HIP_TEST_HAND_BYTES");
+    const uint64_t most = v && *v ? strtoull(v, nullptr, 10) : HAND_BYTES;
+    return std::min<uint64_t>(most, (uint64_t)(freeb + rs->hand_bytes) / 4);
+}
 
 int prepare_hand(galn_hip_readset *rs)
 {
     const int sl = (rs->seed_len > 0 && rs->seed_len < rs->max_len) ? rs->seed_len : 0;
-    const uint32_t stride = hand_words(rs->max_len + 1, sl + 1, rs->idx->meta.ext != nullptr);
-    if (rs->d_hand && rs->hand_bytes >= (uint64_t)std::max(rs->n, 1) * stride * 8) {
+    int root = hand_root(rs->max_len, rs->idx->meta.ext != nullptr);
+    uint32_t stride = hand_words(rs->max_len + 1, sl + 1, root);
+    if (!getenv("GALN_HIP_TEST_HAND_BYTES") && rs->d_hand && rs->hand_bytes >= (uint64_t)std::max(rs->n, 1) * stride * 8) {
         rs->hand_stride = stride;
+        rs->hand_root = root;
         rs->hand_cap = rs->n;
         return 0;
     }
     size_t freeb = 0, totalb = 0;
     HIP_OK(hipMemGetInfo(&freeb, &totalb));
-    const uint64_t limit = std::min<uint64_t>(HAND_BYTES, (uint64_t)(freeb + rs->hand_bytes) / 4);
+    const uint64_t limit = hand_limit(rs, freeb);
+    if ((uint64_t)rs->n * stride * 8 > limit) {
+        root = 0;
+        stride = hand_words(rs->max_len + 1, sl + 1, root);
+    }
     const int cap = (int)std::min<uint64_t>((uint64_t)rs->n, limit / (stride * 8ull));
     // slots of this stride in the bytes already held (another launch's stride may differ)
     const size_t need = (size_t)std::max(cap, 1) * stride * 8;
@@ -3417,6 +3435,7 @@ int prepare_hand(galn_hip_readset *rs)
         }
     }
     rs->hand_stride = stride;
+    rs->hand_root = root;
     rs->hand_cap = (int)std::min<uint64_t>((uint64_t)cap, rs->hand_bytes / (stride * 8ull));
     return 0;
 }
@@ -3438,10 +3457,10 @@ int reserve_search(galn_hip_readset *rs, int n, int max_len, uint32_t flags)
         return r;
     };
     // hand-off slots (seed widths of seeds up to 32 bases included), within prepare_hand's limit
-    const uint64_t stride = hand_words(max_len + 1, 33, rs->idx->meta.ext != nullptr);
+    const uint64_t stride = hand_words(max_len + 1, 33, hand_root(max_len, rs->idx->meta.ext != nullptr));
     size_t freeb = 0, totalb = 0;
     HIP_OK(hipMemGetInfo(&freeb, &totalb));
-    const uint64_t limit = std::min<uint64_t>(HAND_BYTES, (uint64_t)(freeb + rs->hand_bytes) / 4);
+    const uint64_t limit = hand_limit(rs, freeb);
     const uint64_t hand = std::min<uint64_t>((uint64_t)n, limit / (stride * 8)) * stride * 8;
     if (hand > rs->hand_bytes && soft(grow_dev((void **)&rs->d_hand, rs->hand_bytes, hand, s))) {
         rs->d_hand = nullptr;
@@ -3600,6 +3619,7 @@ int launch_widths(galn_hip_readset *rs, const int32_t *list, int n, bool check)
     w.hand = rs->d_hand;
     w.hand_stride = rs->hand_stride;
     w.hand_cap = rs->hand_cap;
+    w.root = rs->hand_root;
     w.wlen = rs->max_len + 1;
     w.swlen = (rs->seed_len > 0 && rs->seed_len < rs->max_len) ? rs->seed_len + 1 : 1;
     w.check = check ? 1 : 0;
@@ -4838,7 +4858,8 @@ int noalloc_search(galn_hip_index *idx, const galn_hip_reads *reads, galn_hip_ou
         if (round >= 24) return fail(GALN_HIP_E_NOMEM, "search_device_noalloc: reads still failing after %d re-runs", round);
         if (engine) {
             // the wave engine over d_fail[fi][0..n_todo), a turn of reads after the other
-            const uint32_t stride = hand_words(wlen, swlen, wide);
+            const int root = hand_root(max_len, wide);
+            const uint32_t stride = hand_words(wlen, swlen, root);
             const NaWaves N = na_waves(std::min(want, (int)n_todo), n_todo, stride, rec_cap, trace, wide, heavy_state_bytes(buckets, wlen, swlen));
             if (N.waves == 0)
                 return fail(GALN_HIP_E_UNSUPPORTED, "search_device_noalloc: a wave's regions and its pool do not fit in %zu bytes", NA_SCRATCH_BYTES);
@@ -4860,6 +4881,7 @@ int noalloc_search(galn_hip_index *idx, const galn_hip_reads *reads, galn_hip_ou
                 w.hand = reinterpret_cast<uint64_t *>(S + N.hand);
                 w.hand_stride = stride;
                 w.hand_cap = m;
+                w.root = root;
                 w.wlen = wlen;
                 w.swlen = swlen;
                 if ((r = launch_widths(idx, st, w))) return r;
