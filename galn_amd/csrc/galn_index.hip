@@ -44,6 +44,7 @@
 #include "galn_hip.h"
 
 __attribute__((visibility("hidden"))) void galn_hip_set_error(const char *msg);
+__attribute__((visibility("hidden"))) hipError_t galn_hip_dev_malloc(void **p, size_t bytes);
 
 namespace {
 
@@ -344,7 +345,7 @@ int dalloc(DevBuf &b, size_t bytes)
 {
     if (b.p) IHIP(hipFree(b.p));
     b.p = nullptr;
-    IHIP(hipMalloc(&b.p, std::max<size_t>(bytes, 16)));
+    IHIP(galn_hip_dev_malloc(&b.p, std::max<size_t>(bytes, 16)));
     return 0;
 }
 
@@ -363,11 +364,13 @@ struct Work {
 };
 
 // A chunk's arrays, all in one allocation: positions and keys twice (the sort goes from one to the other
-// and back), head and tie flags. Freeing is what it costs: once the card's memory has been handed out, a
-// free of 0.9 GB takes 26 ms, ten times a 5 Mbp build's kernels (64 MB and less: 0.02 ms). So the arrays of
-// the tied suffixes lie in the keys' place, or in an allocation of their own where many are tied, which
-// takes 34 bytes a suffix where 90 were taken before, and a freed arena of up to ARENA_KEPT bytes (builds
-// of up to 15 Mbp) waits for the next build, until an index is opened: 5 Mbp take 3.0 ms (30.4 before).
+// and back), head and tie flags; the arrays of the tied suffixes lie in the keys' place, or in an allocation
+// of their own where many are tied. That takes 34 bytes a suffix where 90 were taken before. A freed arena of
+// up to ARENA_KEPT bytes (builds of up to 15 Mbp) waits for the next build: freeing 0.3 GB or more takes
+// 0.3 ms, and 26 ms in a process that has been handed some 200 to 320 GB of memory in all, ten times a
+// 5 Mbp build's kernels. It is given back when an allocation of this library finds no room, and by
+// galn_hip_build_trim. A build owns the arena that it has taken from here: two at a time never count or use
+// the same one.
 struct Arena {
     void *p = nullptr;
     size_t bytes = 0;
@@ -391,7 +394,9 @@ struct ChunkBufs {
     uint8_t *H, *flag;
     uint64_t *cnt;
     explicit ChunkBufs(hipStream_t s) : st(s) {}
-    ~ChunkBufs()
+    ~ChunkBufs() { give(); }
+    // The chunks are done: the arena waits for the next build, or goes.
+    void give()
     {
         if (!a.p) return;
         const bool idle = hipStreamSynchronize(st) == hipSuccess;
@@ -399,17 +404,20 @@ struct ChunkBufs {
         if (idle && a.bytes <= ARENA_KEPT && a.bytes > g_arena.bytes) std::swap(a, g_arena);
         arena_drop(a);
     }
+    // The kept arena, when it lies on this device, is this build's from here on; its bytes.
+    size_t take(int device)
+    {
+        std::lock_guard<std::mutex> g(g_arena_mu);
+        if (g_arena.device == device) std::swap(a, g_arena);
+        return a.bytes;
+    }
     int alloc(int device, uint64_t m_)
     {
         m = m_;
         const size_t col = (m * 8 + 255) / 256 * 256, need = 256 + 4 * col + 2 * ((m + 255) / 256 * 256);
-        {
-            std::lock_guard<std::mutex> g(g_arena_mu);
-            std::swap(a, g_arena);
-        }
-        if (a.device != device || a.bytes < need) {
+        if (a.bytes < need) {
             arena_drop(a);
-            IHIP(hipMalloc(&a.p, need));
+            IHIP(galn_hip_dev_malloc(&a.p, need));
             a.bytes = need;
             a.device = device;
         }
@@ -544,11 +552,10 @@ int build(const uint8_t *fwd, uint64_t len, int device, galn_bwt_meta_t *meta, u
     const uint64_t *Pc = P.as<const uint64_t>();
     // chunk capacity from the free memory (the packed body, n/2 bytes, comes after the chunks)
     size_t freeb = 0, totalb = 0;
+    ChunkBufs cb(st);
+    const size_t kept = cb.take(device);  // (used, or freed before the chunks' arrays are allocated)
     IHIP(hipMemGetInfo(&freeb, &totalb));
-    {
-        std::lock_guard<std::mutex> g(g_arena_mu);  // this build's to use, or freed before it allocates
-        if (g_arena.device == device) freeb += g_arena.bytes;
-    }
+    freeb += kept;
     const uint64_t reserve = (uint64_t)1 << 30;
     uint64_t cap = freeb > reserve ? (freeb - reserve) / (CHUNK_BYTES_PER_SUFFIX + 8) : 0;
     cap = std::min(cap, CHUNK_MAX);
@@ -597,7 +604,6 @@ int build(const uint8_t *fwd, uint64_t len, int device, galn_bwt_meta_t *meta, u
     const char *vb = getenv("GALN_HIP_VERBOSE");
     const bool verbose = vb && *vb && strcmp(vb, "0") != 0;
     {
-        ChunkBufs cb(st);
         if ((r = cb.alloc(device, maxm))) return r;
         int max_rounds = 0;
         for (const Chunk &c : chunks) {
@@ -629,6 +635,7 @@ int build(const uint8_t *fwd, uint64_t len, int device, galn_bwt_meta_t *meta, u
             stats[1] = (double)max_rounds;
             stats[2] = (double)maxm;
         }
+        cb.give();
     }
     P.release();
     uint64_t prim = 0;
@@ -682,14 +689,24 @@ int build(const uint8_t *fwd, uint64_t len, int device, galn_bwt_meta_t *meta, u
 
 }  // namespace
 
-// Frees the chunk arena kept by earlier builds: an index is opened, the building is over (galn_search.hip).
-__attribute__((visibility("hidden"))) void galn_hip_build_trim()
+// hipMalloc for the whole library: where there is no room, the chunk arena kept by earlier builds goes first.
+__attribute__((visibility("hidden"))) hipError_t galn_hip_dev_malloc(void **p, size_t bytes)
 {
-    std::lock_guard<std::mutex> g(g_arena_mu);
-    arena_drop(g_arena);
+    const hipError_t e = hipMalloc(p, bytes);
+    if (e != hipErrorOutOfMemory || galn_hip_build_trim() == 0) return e;
+    (void)hipGetLastError();
+    return hipMalloc(p, bytes);
 }
 
 extern "C" {
+
+uint64_t galn_hip_build_trim(void)
+{
+    std::lock_guard<std::mutex> g(g_arena_mu);
+    const size_t bytes = g_arena.bytes;
+    arena_drop(g_arena);
+    return bytes;
+}
 
 uint64_t galn_hip_bwt_words(uint64_t n)
 {

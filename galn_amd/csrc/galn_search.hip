@@ -55,7 +55,7 @@
 
 #include "galn_hip.h"
 
-__attribute__((visibility("hidden"))) void galn_hip_build_trim();  // galn_index.hip
+__attribute__((visibility("hidden"))) hipError_t galn_hip_dev_malloc(void **p, size_t bytes);  // galn_index.hip
 
 namespace {
 
@@ -3008,6 +3008,13 @@ namespace {
 
 size_t align_up(size_t x, size_t a) { return (x + a - 1) / a * a; }
 
+// every device allocation of this file (one that finds no room takes back what earlier builds left)
+template <class T>
+hipError_t dev_malloc(T **p, size_t bytes)
+{
+    return galn_hip_dev_malloc(reinterpret_cast<void **>(p), bytes);
+}
+
 struct Layout {
     uint64_t slot_bytes;
     uint32_t sw_off, rec_off, own_off;
@@ -3042,11 +3049,11 @@ int grow_dev(void **p, size_t &cap, size_t need, hipStream_t s)
     if (*p) HIP_OK(hipFree(*p));
     *p = nullptr;
     const size_t c = std::max(need, cap * 2);
-    if (hipMalloc(p, c) != hipSuccess) {
+    if (dev_malloc(p, c) != hipSuccess) {
         (void)hipGetLastError();
         *p = nullptr;
         cap = 0;
-        if (hipMalloc(p, need) != hipSuccess) return fail(GALN_HIP_E_NOMEM, "device allocation of %zu bytes failed", need);
+        if (dev_malloc(p, need) != hipSuccess) return fail(GALN_HIP_E_NOMEM, "device allocation of %zu bytes failed", need);
         cap = need;
         return 0;
     }
@@ -3104,8 +3111,8 @@ int ensure_pool(SearchCtx *idx, uint64_t want)
     if (!idx->d_ghead) {
         unsigned long long *head = nullptr;
         uint32_t *bump = nullptr;
-        HIP_OK(hipMalloc(&head, NSHARD * 8));
-        if (hipMalloc(&bump, 4) != hipSuccess) {
+        HIP_OK(dev_malloc(&head, NSHARD * 8));
+        if (dev_malloc(&bump, 4) != hipSuccess) {
             (void)hipFree(head);
             return fail(GALN_HIP_E_NOMEM, "stack pool: allocation of its heads failed");
         }
@@ -3127,8 +3134,8 @@ int ensure_pool(SearchCtx *idx, uint64_t want)
     // half as many granules while the allocation fails (other allocations of the process, or of
     // other processes, since the free memory was read): a smaller pool only costs re-runs
     for (;;) {
-        if (hipMalloc(&chk, want * gbytes) == hipSuccess && hipMalloc(&link, want * GRAN * 4) == hipSuccess &&
-            hipMalloc(&gnext, want * 4) == hipSuccess)
+        if (dev_malloc(&chk, want * gbytes) == hipSuccess && dev_malloc(&link, want * GRAN * 4) == hipSuccess &&
+            dev_malloc(&gnext, want * 4) == hipSuccess)
             break;
         (void)hipGetLastError();
         for (void *p : {(void *)chk, (void *)link, (void *)gnext})
@@ -3755,7 +3762,7 @@ int grow_records(galn_hip_readset *rs)
     const uint64_t used = std::min<uint64_t>(top, rs->rec_cap);
     const uint64_t ncap = std::max<uint64_t>(rs->rec_cap * 2, top + 4096);
     galn_aln_rec_t *nrec = nullptr;
-    HIP_OK(hipMalloc(&nrec, ncap * sizeof(galn_aln_rec_t)));
+    HIP_OK(dev_malloc(&nrec, ncap * sizeof(galn_aln_rec_t)));
     if (used) HIP_OK(hipMemcpyAsync(nrec, rs->d_rec, used * sizeof(galn_aln_rec_t), hipMemcpyDeviceToDevice, st));
     HIP_OK(hipStreamSynchronize(st));
     HIP_OK(hipFree(rs->d_rec));
@@ -4026,7 +4033,7 @@ int readset_reserve(galn_hip_readset *rs, int n, uint64_t qbytes, int nb)
     auto regrow = [](void **p, size_t bytes) __attribute__((always_inline)) -> bool {
         if (*p) (void)hipFree(*p);
         *p = nullptr;
-        return hipMalloc(p, std::max<size_t>(bytes, 16)) == hipSuccess;
+        return dev_malloc(p, std::max<size_t>(bytes, 16)) == hipSuccess;
     };
     bool ok = true;
     if (grow_q) {
@@ -4204,7 +4211,6 @@ int galn_hip_index_open(const uint32_t *bwt, const galn_bwt_meta_t *meta, int de
     if (hipGetDeviceCount(&ndev) != hipSuccess || ndev == 0) return fail(GALN_HIP_E_DEVICE, "no HIP device");
     if (device < 0 || device >= ndev) return fail(GALN_HIP_E_DEVICE, "no HIP device %d (%d visible)", device, ndev);
     HIP_OK(hipSetDevice(device));
-    galn_hip_build_trim();
     galn_hip_index *idx = new galn_hip_index;
     idx->device = device;
     idx->hmeta = *meta;
@@ -4219,7 +4225,7 @@ int galn_hip_index_open(const uint32_t *bwt, const galn_bwt_meta_t *meta, int de
     const size_t bytes = (size_t)meta->bwt_size * 4;
     // whole 64-byte blocks are loaded: pad so the last block's load stays in bounds
     const size_t alloc = align_up(bytes + 256, 256);
-    if (hipMalloc(&idx->d_bwt, alloc) != hipSuccess) {
+    if (dev_malloc(&idx->d_bwt, alloc) != hipSuccess) {
         delete idx;
         return fail(GALN_HIP_E_NOMEM, "index of %zu bytes does not fit in device memory", bytes);
     }
@@ -4241,7 +4247,7 @@ int galn_hip_index_open(const uint32_t *bwt, const galn_bwt_meta_t *meta, int de
         wide = true;
     }
     const uint32_t n_ep = wide ? (uint32_t)((n_blocks >> eshift) + 1) : 1u;
-    bool up = hipMalloc(&idx->d_ext, (size_t)n_ep * 32) == hipSuccess;
+    bool up = dev_malloc(&idx->d_ext, (size_t)n_ep * 32) == hipSuccess;
     if (up && n_blocks > 0) {
         const uint64_t *const L2 = meta->L2;
         hipLaunchKernelGGL(k_epochs, dim3((4 * n_ep + 255) / 256), dim3(256), 0, idx->ctx0.stream, (const uint32_t *)idx->d_bwt, n_blocks,
@@ -4325,7 +4331,7 @@ int galn_hip_readset_upload(galn_hip_index *idx, const galn_hip_reads *reads, ga
     rs->idx = idx;
     rs->ctx = &idx->ctx0;
     idx->n_readsets.fetch_add(1);
-    auto M = [&](void **p, size_t b) __attribute__((always_inline)) -> bool { return hipMalloc(p, b) == hipSuccess; };
+    auto M = [&](void **p, size_t b) __attribute__((always_inline)) -> bool { return dev_malloc(p, b) == hipSuccess; };
     bool ok = M((void **)&rs->d_top, 8) && M((void **)&rs->d_ctr, 16 * sizeof(int32_t)) && M((void **)&rs->d_stats, 16 * 8) &&
               M((void **)&rs->d_algo, sizeof(unsigned long long) * galn_hip_readset::MAX_LAUNCH) &&
               hipHostMalloc((void **)&rs->back, sizeof *rs->back) == hipSuccess;
@@ -4547,7 +4553,7 @@ int galn_hip_index_set_sa(galn_hip_index *idx, const uint64_t *samples, uint64_t
     if (idx->d_sa) HIP_OK(hipFree(idx->d_sa));
     idx->d_sa = nullptr;
     idx->n_sa = 0;
-    HIP_OK(hipMalloc(&idx->d_sa, std::max<uint64_t>(n_samples, 1) * 8));
+    HIP_OK(dev_malloc(&idx->d_sa, std::max<uint64_t>(n_samples, 1) * 8));
     if (n_samples) HIP_OK(hipMemcpy(idx->d_sa, samples, n_samples * 8, hipMemcpyHostToDevice));
     idx->n_sa = n_samples;
     idx->sa_intv = intv;
@@ -4570,7 +4576,7 @@ int galn_hip_sa_positions(galn_hip_index *idx, const uint64_t *rows, uint64_t n,
     HIP_OK(hipSetDevice(idx->device));
     const uint64_t chunk = std::min<uint64_t>(n, 1ull << 24);
     uint64_t *d = nullptr;
-    HIP_OK(hipMalloc(&d, chunk * (ref_len ? 24 : 16)));
+    HIP_OK(dev_malloc(&d, chunk * (ref_len ? 24 : 16)));
     int32_t *const d_rl = ref_len ? reinterpret_cast<int32_t *>(d + 2 * chunk) : nullptr;
     int32_t *const d_st = ref_len ? d_rl + chunk : nullptr;
     hipStream_t s = idx->ctx0.stream;

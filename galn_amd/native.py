@@ -32,7 +32,7 @@ HIP_SYMBOLS = (
     "galn_hip_readset_engine_stats", "galn_hip_server_open", "galn_hip_server_submit", "galn_hip_server_wait",
     "galn_hip_server_result", "galn_hip_server_stats", "galn_hip_server_close", "galn_hip_gather_ceiling",
     "galn_hip_search_device_noalloc", "galn_hip_bwt_words", "galn_hip_build_bwt", "galn_hip_index_set_sa",
-    "galn_hip_sa_positions",
+    "galn_hip_sa_positions", "galn_hip_build_trim",
 )
 HOST_SYMBOLS = (
     "galn_gap_opt_default", "galn_parse_aln_args", "galn_cal_maxdiff", "galn_batch_opt", "galn_read_maxdiff",
@@ -137,6 +137,7 @@ def hip_lib():
         L.galn_hip_bwt_words.restype = C.c_uint64
         L.galn_hip_bwt_words.argtypes = [C.c_uint64]
         L.galn_hip_build_bwt.argtypes = [P, C.c_uint64, C.c_int, C.POINTER(BwtMeta), P, P, P]
+        L.galn_hip_build_trim.restype = C.c_uint64
         L.galn_hip_index_set_sa.argtypes = [P, P, C.c_uint64, C.c_uint32]
         L.galn_hip_sa_positions.argtypes = [P, P, C.c_uint64, P, P, P]
         L.galn_hip_get_limits.argtypes = [C.POINTER(Limits)]
@@ -222,6 +223,11 @@ def build_bwt(fwd2: np.ndarray, device: int = 0, want_sa: bool = False) -> tuple
         raise GalnError(f"build_bwt failed ({rc}): {last_error()}")
     info = {"chunks": int(st[0]), "rounds": int(st[1]), "largest_chunk": int(st[2])}
     return m, words, (sa[: (n + 32) // 32 - 1] if sa is not None else None), info
+
+
+def build_trim() -> int:
+    """galn_hip_build_trim: frees the device memory that finished builds keep for the next one; its bytes."""
+    return int(hip_lib().galn_hip_build_trim())
 
 
 # --------------------------------------------------------------------------

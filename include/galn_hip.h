@@ -287,9 +287,15 @@ uint64_t galn_hip_bwt_words(uint64_t n);
  *   sa_samples: optional, (n + 32) / 32 - 1 words: the suffix at rows 32, 64, ... (the .sa samples
  *         of bwt_cal_sa(bwt, 32)).
  *   stats: optional [4]: chunks, most refinement rounds of a chunk, largest chunk, 0.
- * Byte-identical to the reference builder's .bwt. */
+ * Byte-identical to the reference builder's .bwt.
+ * A build's working memory of up to 1 GiB (genomes of up to 15 Mbp; one build's per process) stays allocated for
+ * the next build. It is given back when an allocation of this library finds no room, or by: */
 int galn_hip_build_bwt(const uint8_t *fwd, uint64_t len, int device, galn_bwt_meta_t *meta, uint32_t *bwt,
                        uint64_t *sa_samples, double *stats);
+
+/* Frees the working memory that finished builds have left; returns its bytes (0: there was none). Any thread,
+ * also while a build runs (whose memory is its own). */
+uint64_t galn_hip_build_trim(void);
 
 /* Random-access ceiling of `device`: pointer chase over a `ws_bytes` buffer of
  * `line_bytes` (64 or 128) lines in one pseudo-random cycle, waves_per_cu * CUs
