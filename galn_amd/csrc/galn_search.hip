@@ -4398,9 +4398,9 @@ int galn_hip_readset_autotune(galn_hip_index *idx, galn_hip_readset *rs, uint32_
             }
             return 0;
         };
-        // the thread-vs-wave cutoff first (when the wave engine may run), then the workgroup size,
-        // then one change at a time from the best so far: the persistent grid's waves per CU, the
-        // record slots per lane, and the stack chunks a lane keeps between reads
+        // the thread-vs-wave cutoff first (when the wave engine may run), then, where k_search runs, the
+        // workgroup size, then one change at a time from the best so far: the persistent grid's waves
+        // per CU, the record slots per lane, and the stack chunks a lane keeps between reads
         galn_hip_tune_t t{};
         t.sort_by_cost = 1;
         t.block_threads = 128;
@@ -4416,24 +4416,28 @@ int galn_hip_readset_autotune(galn_hip_index *idx, galn_hip_readset *rs, uint32_
             t.heavy_pops = -1;
             if ((r = trial(t))) return r;
         }
-        t = best;
-        t.block_threads = 64;
-        if ((r = trial(t))) return r;
-        const int waves[] = {4, 6}, recs[] = {16, 256}, keeps[] = {GRAN, 16 * GRAN};
-        for (int v : waves) {
+        if (best.heavy_pops == 1) {
+            best.block_threads = 64;  // (the library's own; this and the remaining settings are k_search's)
+        } else {
             t = best;
-            t.waves_per_cu = v;
+            t.block_threads = 64;
             if ((r = trial(t))) return r;
-        }
-        for (int v : recs) {
-            t = best;
-            t.rec_per_lane = v;
-            if ((r = trial(t))) return r;
-        }
-        for (int v : keeps) {
-            t = best;
-            t.chunks_per_lane = v;
-            if ((r = trial(t))) return r;
+            const int waves[] = {4, 6}, recs[] = {16, 256}, keeps[] = {GRAN, 16 * GRAN};
+            for (int v : waves) {
+                t = best;
+                t.waves_per_cu = v;
+                if ((r = trial(t))) return r;
+            }
+            for (int v : recs) {
+                t = best;
+                t.rec_per_lane = v;
+                if ((r = trial(t))) return r;
+            }
+            for (int v : keeps) {
+                t = best;
+                t.chunks_per_lane = v;
+                if ((r = trial(t))) return r;
+            }
         }
     }
     rs->tuned = best;
