@@ -1638,7 +1638,9 @@ typedef const __attribute__((address_space(4))) HArgs HArgsC;
 #define HA(f) cold_ld(&((HArgsC *)__builtin_amdgcn_kernarg_segment_ptr())->f)
 
 // NW waves per read, at four waves per SIMD (128 VGPRs): a variant of five (96) was 4% faster on light reads, 2%
-// slower on heavy ones, before the light reads' descents were taken out of the loop.
+// slower on heavy ones, before the light reads' descents were taken out of the loop. (The upper bound changes the
+// schedule only, not the registers or scratch bytes of any variant; the traced ones and those above 2^32 symbols
+// keep the compiler's own, 8, with which their code does not change as the others' bound does.)
 template <bool TRACE, bool WIDE, int NW, int CPL>
 __global__ void __launch_bounds__(64 * NW) __attribute__((amdgpu_waves_per_eu(4, (TRACE || WIDE) ? 8 : 4))) k_heavy(HArgs a)
 {
@@ -1649,11 +1651,17 @@ __global__ void __launch_bounds__(64 * NW) __attribute__((amdgpu_waves_per_eu(4,
     extern __shared__ __align__(16) uint8_t hlds[];
     // the launch of NW > 1 waves goes on with reads that the launch of one wave parked
     constexpr bool RESUME = NW > 1;
-    // Steps of exact descents side by side (the root's round, a lone lane's descent), not in the trace build and
-    // not above 2^32 symbols: those variants spill most, and the code compiled for one of them with this in it
-    // read out of range, as a variant for five waves per SIMD (96 registers) gave wrong records, while the same
-    // source is right in the others and on the CPU.
+    // Steps of exact descents side by side (the root's round, a lone lane's descent): not in the trace build, whose
+    // step log has no place for steps that are walked ahead, and not above 2^32 symbols, where hand-off slots have
+    // no room for a root chain. Two other builds with this in it were wrong, for a reason that is not known: the
+    // traced one above 2^32 symbols read out of range, and one for five waves per SIMD (96 registers) gave records
+    // that changed from run to run. What is known: the same source gives the right results lane by lane on the CPU
+    // with unwritten memory and registers poisoned and the lanes and waves in any order between two wave operations;
+    // and both of those builds keep state of the round in scratch memory, stored from several branches of its loops,
+    // while the two kernels that have this code now store to scratch memory in their prologue only, with every
+    // lane on (tests/test_device_code.py holds them to that).
     constexpr bool AHEAD = !TRACE && !WIDE;
+    static_assert(!AHEAD || (!TRACE && !WIDE), "no step log, no root chain");
     constexpr int STEPS = AHEAD ? H_STEPS : H_STEPS_PLAIN;
     uint4 *const pieces = reinterpret_cast<uint4 *>(hlds);         // {bucket code, rank0, len, base}
     Ent *const hent = reinterpret_cast<Ent *>(pieces + H_PIECES);  // live chains' heads, in order
