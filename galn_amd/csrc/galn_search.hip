@@ -278,23 +278,31 @@ __device__ __forceinline__ uint32_t lf_pair(const uint32_t *__restrict__ bwt, co
     return occ_units<uint64_t>(Pk, Pl) << 6;
 }
 
+// What the .bwt header says of a body: the bases' first rows (L2[4] = the symbols), and the block that the
+// end of the text is counted in where the text fills the block before it (~0 otherwise). A position at the end
+// reads that block's counts, which are the totals of the header: of the body's own words only those of
+// blocks with symbols are taken, as the .bwt readers of the reference do.
+struct Totals {
+    uint64_t L2[5], end;
+};
+
 // `ext` of an uploaded .bwt body (before k_planes rewrites it): per epoch and base, the base's first row
 // plus its count before the epoch's first block
-__global__ void k_epochs(const uint32_t *bwt, uint64_t n_blocks, uint32_t eshift, uint4 l2lo, uint4 l2hi, uint64_t *ext, uint32_t n)
+__global__ void k_epochs(const uint32_t *bwt, uint64_t n_blocks, uint32_t eshift, Totals T, uint64_t *ext, uint32_t n)
 {
     const uint32_t t = blockIdx.x * blockDim.x + threadIdx.x;
     if (t >= 4 * n) return;
     const uint64_t blk = (uint64_t)(t >> 2) << eshift;
     const int c = (int)(t & 3);
-    const uint32_t lo[4] = {l2lo.x, l2lo.y, l2lo.z, l2lo.w}, hi[4] = {l2hi.x, l2hi.y, l2hi.z, l2hi.w};
     const uint64_t before = blk < n_blocks ? reinterpret_cast<const uint64_t *>(bwt + (blk << 4))[c] : 0;
-    ext[t] = ((uint64_t)hi[c] << 32 | lo[c]) + before;
+    ext[t] = blk == T.end ? T.L2[c + 1] : T.L2[c] + before;
 }
 
 // In-place conversion of the uploaded .bwt body (BWA's blocks: 4 x u64 exclusive counts, 8 words of 16
 // two-bit symbols, first symbol in bits 31-30) to the device layout, one block per thread (a last, shorter
 // block included: what lies past its symbols is never counted).
-__global__ void __launch_bounds__(256) k_planes(uint32_t *bwt, uint64_t n_blocks, const uint64_t *ext, uint32_t eshift, int wide)
+__global__ void __launch_bounds__(256)
+    k_planes(uint32_t *bwt, uint64_t n_blocks, Totals T, const uint64_t *ext, uint32_t eshift, int wide)
 {
     const uint64_t i = (uint64_t)blockIdx.x * blockDim.x + threadIdx.x;
     if (i >= n_blocks) return;
@@ -324,7 +332,10 @@ __global__ void __launch_bounds__(256) k_planes(uint32_t *bwt, uint64_t n_blocks
     const uint64_t *const e = ext + (wide ? 4 * (i >> eshift) : 0);
     uint64_t C[4] = {(uint64_t)c0.y << 32 | c0.x, (uint64_t)c0.w << 32 | c0.z, (uint64_t)c1.y << 32 | c1.x, (uint64_t)c1.w << 32 | c1.z};
 #pragma unroll
-    for (int c = 0; c < 4; ++c) C[c] = wide ? C[c] + ext[c] - e[c] : C[c] + ext[c];
+    for (int c = 0; c < 4; ++c) {
+        const uint64_t row = i == T.end ? T.L2[c + 1] : C[c] + ext[c];
+        C[c] = wide ? row - e[c] : row;
+    }
     p[0] = make_uint4((uint32_t)C[0], (uint32_t)C[1], (uint32_t)C[2], (uint32_t)C[3]);
     p[1] = make_uint4(hp[0], lp[0], pre[0], hp[1]);
     p[2] = make_uint4(lp[1], pre[1], hp[2], lp[2]);
@@ -4247,7 +4258,12 @@ int galn_hip_index_open(const uint32_t *bwt, const galn_bwt_meta_t *meta, int de
     }
     // 32-bit counts reach 2^32 - 1 (row seq_len + 1 included); a larger index counts per epoch of 2^24
     // blocks. GALN_HIP_TEST_EPOCH=n makes the epochs 2^n blocks on an index of any size (tests).
-    const uint64_t n_blocks = ((uint64_t)meta->bwt_size + 15) / 16;
+    Totals T;
+    for (int c = 0; c < 5; ++c) T.L2[c] = meta->L2[c];
+    T.end = meta->seq_len % 128 == 0 ? meta->seq_len / 128 : ~0ull;
+    // (the end's block may lie past the body, within the allocation's padding)
+    uint64_t n_blocks = ((uint64_t)meta->bwt_size + 15) / 16;
+    if (T.end == n_blocks) n_blocks += 1;
     uint32_t eshift = 24;
     bool wide = meta->seq_len >= 0xfffffffeull;
     if (const char *v = getenv("GALN_HIP_TEST_EPOCH"); v && *v) {
@@ -4257,13 +4273,10 @@ int galn_hip_index_open(const uint32_t *bwt, const galn_bwt_meta_t *meta, int de
     const uint32_t n_ep = wide ? (uint32_t)((n_blocks >> eshift) + 1) : 1u;
     bool up = dev_malloc(&idx->d_ext, (size_t)n_ep * 32) == hipSuccess;
     if (up && n_blocks > 0) {
-        const uint64_t *const L2 = meta->L2;
         hipLaunchKernelGGL(k_epochs, dim3((4 * n_ep + 255) / 256), dim3(256), 0, idx->ctx0.stream, (const uint32_t *)idx->d_bwt, n_blocks,
-                           eshift, make_uint4((uint32_t)L2[0], (uint32_t)L2[1], (uint32_t)L2[2], (uint32_t)L2[3]),
-                           make_uint4((uint32_t)(L2[0] >> 32), (uint32_t)(L2[1] >> 32), (uint32_t)(L2[2] >> 32), (uint32_t)(L2[3] >> 32)),
-                           idx->d_ext, n_ep);
+                           eshift, T, idx->d_ext, n_ep);
         hipLaunchKernelGGL(k_planes, dim3((unsigned)((n_blocks + 255) / 256)), dim3(256), 0, idx->ctx0.stream, idx->d_bwt,
-                           n_blocks, (const uint64_t *)idx->d_ext, eshift, wide ? 1 : 0);
+                           n_blocks, T, (const uint64_t *)idx->d_ext, eshift, wide ? 1 : 0);
     }
     if (!up || hipGetLastError() != hipSuccess || hipStreamSynchronize(idx->ctx0.stream) != hipSuccess) {
         (void)hipStreamDestroy(idx->ctx0.stream);
