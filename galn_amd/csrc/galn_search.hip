@@ -4725,6 +4725,16 @@ constexpr int NA_WAVES = 512;
 constexpr int NA_DEEP = 32;
 constexpr size_t NA_HAND_BYTES = 32ull << 20;
 
+// The array's bytes, or fewer: GALN_HIP_TEST_NA_BYTES, with which the tests reach its limits.
+size_t na_bytes()
+{
+    const char *v = getenv("GALN_HIP_TEST_NA_BYTES");
+    return v && *v ? std::min<size_t>(NA_SCRATCH_BYTES, strtoull(v, nullptr, 10)) : NA_SCRATCH_BYTES;
+}
+
+// Record slots of a wave at most: three eighths of the array (4,194,304 records), beside which one wave's pool fits.
+int na_rec_max() { return (int)(na_bytes() * 3 / 8 / sizeof(galn_aln_rec_t)); }
+
 struct NaWaves {
     int waves = 0, groups = 0, turn = 0, own_cap = 0;  // turn: reads per launch
     uint64_t n_gran = 0;
@@ -4751,8 +4761,8 @@ NaWaves na_waves(int want, int n, uint32_t hand_stride, int rec_cap, bool trace,
         N.slots = align_up(N.hand + (size_t)N.turn * hand_stride * 8, 256);
         N.deep = N.slots + (size_t)w * N.L.slot_bytes;
         N.pool = N.deep + (size_t)N.groups * N.D.slot_bytes;
-        if (N.pool + 256 >= NA_SCRATCH_BYTES) continue;
-        N.n_gran = (NA_SCRATCH_BYTES - N.pool - 256) / (GENT * sizeof(Ent) + 4);
+        if (N.pool + 256 >= na_bytes()) continue;
+        N.n_gran = (na_bytes() - N.pool - 256) / (GENT * sizeof(Ent) + 4);
         if (N.n_gran < (w > 1 ? 12ull * (uint64_t)w : 32ull)) continue;
         N.gnext = N.pool + N.n_gran * GENT * sizeof(Ent);
         N.waves = w;
@@ -4893,7 +4903,7 @@ int noalloc_search(galn_hip_index *idx, const galn_hip_reads *reads, galn_hip_ou
             const uint32_t stride = hand_words(wlen, swlen, root);
             const NaWaves N = na_waves(std::min(want, (int)n_todo), n_todo, stride, rec_cap, trace, wide, heavy_state_bytes(buckets, wlen, swlen));
             if (N.waves == 0)
-                return fail(GALN_HIP_E_UNSUPPORTED, "search_device_noalloc: a wave's regions and its pool do not fit in %zu bytes", NA_SCRATCH_BYTES);
+                return fail(GALN_HIP_E_UNSUPPORTED, "search_device_noalloc: a wave's regions and its pool do not fit in %zu bytes", na_bytes());
             const int fo = fi ^ 1;
             FILL(ctr + fo, 0, sizeof(int32_t));
             FILL(ctr + 4, 0, 3 * sizeof(int32_t));
@@ -5000,7 +5010,9 @@ int noalloc_search(galn_hip_index *idx, const galn_hip_reads *reads, galn_hip_ou
                 out_full = true;
                 break;
             }
-            if (c[5]) rec_cap *= 16;
+            if (c[5] && rec_cap >= na_rec_max())
+                return fail(GALN_HIP_E_UNSUPPORTED, "search_device_noalloc: a read has more than %d records", na_rec_max());
+            if (c[5]) rec_cap = std::min(rec_cap * 16, na_rec_max());
             if (c[6]) want = std::max(1, N.waves / 4);
             fi = fo;
             n_todo = c[fo];
