@@ -3234,6 +3234,10 @@ constexpr uint32_t PARK_POPS = 2048;
 // only shortens the tail: 16 reads of 100 bp 0.54 ms after 512 pops, 0.64 after 2048, 0.59 after 256.
 constexpr uint32_t PARK_POPS_FEW = 512;
 constexpr int FIRST_GRAN = 8;  // granules a workgroup of it starts with
+// Granules of the stack pool for each wave: 34 GB for a full grid. Unseeded reads on a repeat-rich genome take them:
+// 2M reads on 3.1 Gbp use 1.84M granules, and with 256 a wave the first search of an index ran dry and took 14.4 s,
+// each granule sought in 64 shards, where the second one took 3.5 (1M reads on 700 Mbp: 1.82 s and 1.45).
+constexpr int POOL_PER_WAVE = 512;
 constexpr int HEAVY_REC = 256;  // record slots of its waves in a search's first launch
 constexpr int HEAVY_REC_MAX = 1 << 26;  // and in any (1.6 GB a wave; a slot's offsets are 32-bit)
 
@@ -3405,7 +3409,7 @@ int prepare_heavy(galn_hip_readset *rs, int waves, int rec_cap, uint32_t flags)
 {
     SearchCtx *cx = rs->ctx;
     // granules for the waves that can get reads, rounded up to a power of two
-    uint64_t want = (uint64_t)std::max(1, std::min(waves, rs->n)) * 256, p2 = 1024;
+    uint64_t want = (uint64_t)std::max(1, std::min(waves, rs->n)) * POOL_PER_WAVE, p2 = 1024;
     while (p2 < want) p2 <<= 1;
     int r = ensure_pool(cx, p2);
     if (r) return r;
@@ -3497,7 +3501,7 @@ int reserve_search(galn_hip_readset *rs, int n, int max_len, uint32_t flags)
     // options that get the most waves (this launch's may be fewer)
     const int waves = std::max(1, std::min(heavy_grid_most(rs, flags, false), n));
     uint64_t p2 = 1024;
-    while (p2 < (uint64_t)waves * 256) p2 <<= 1;
+    while (p2 < (uint64_t)waves * POOL_PER_WAVE) p2 <<= 1;
     if (!soft(ensure_pool(cx, p2))) {
         soft(grow_dev((void **)&rs->d_park, rs->park_bytes, (size_t)waves * 4, s));
         soft(grow_dev((void **)&rs->d_hscratch, rs->hscratch_bytes, heavy_scratch(rs, waves, heavy_grid_most(rs, flags, true), HEAVY_REC, flags), s));
