@@ -3324,10 +3324,14 @@ int heavy_grid(galn_hip_readset *rs, uint32_t flags, bool deep)
     if (o.kernel != kernel || o.lds != lds) o = {kernel, lds, heavy_per_cu(rs, flags, deep, lds)};
     // Without seeds a read's stack, log and granules are several times larger, and those of 16 waves a CU go past L2:
     // 12 take 2M ancient DNA reads from 230 to 221 ms, 262,144 from 39.4 to 38.6, 100,003 repeat-rich ones from 105
-    // to 101; 100k seeded reads of 100 bp take 4.1 ms with 16, 4.6 with 12. (From 2^32 symbols on the waves wait on
-    // the index in HBM: 16; and few reads get a wave each: 4001 take 13.1 ms either way.)
-    const bool fewer = !deep && rs->seed_len == 0 && rs->idx->meta.ext == nullptr && rs->n >= 16 * o.groups * rs->idx->n_cu;
-    return (fewer ? std::min(o.groups, 12) : o.groups) * rs->idx->n_cu;
+    // to 101; 100k seeded reads of 100 bp take 4.1 ms with 16, 4.6 with 12, and few reads get a wave each (4001 take
+    // 13.1 ms either way). From 2^32 symbols on, where every lookup leaves L2 as well, it depends on the reads: of
+    // 30 to 150 bp, 2M on a 3.1 Gbp human-like genome take 3330 to 3480 ms with 16, 2860 to 3000 with 12, 2670 with 8,
+    // 2580 with 6, 2690 with 4 (200,000 of them 309 to 330, 290, 283, 278, 295), while 1M of median 45, whose stacks
+    // stay small, take 423 with 16, 444 with 12, 524 with 8. The line lies between their means, 90 and 48 bp.
+    const bool many = !deep && rs->seed_len == 0 && rs->n >= 16 * o.groups * rs->idx->n_cu;
+    const int most = !many ? o.groups : rs->idx->meta.ext == nullptr ? 12 : rs->qbytes >= (uint64_t)rs->n * 64 ? 8 : o.groups;
+    return std::min(o.groups, most) * rs->idx->n_cu;
 }
 
 // A workgroup's first granules: FIRST_GRAN of them, fewer in a small pool (half of it is left to share).

@@ -124,8 +124,8 @@ typedef struct {
     int32_t sort_by_cost;      /* 1: claim reads longest-first */
     int32_t heavy_pops;        /* pops after which a read moves to the wave-per-read engine
                                   (0: the default, every read from its first pop; -1: never) */
-    int32_t heavy_waves_per_simd; /* any value: the wave-per-read engine runs four waves per SIMD (a variant
-                                  of five was no faster) */
+    int32_t heavy_waves_per_simd; /* any value: the wave-per-read engine runs at most four waves per SIMD, fewer
+                                  where its reads' stacks are large */
 } galn_hip_tune_t;
 
 /* Serving loop configuration (0 = default). */

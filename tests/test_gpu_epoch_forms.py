@@ -10,6 +10,7 @@ import fixtures as fx
 from conftest import golden_inputs, load_reads, run_opts
 from galn_amd import index as ix
 from galn_amd import native as nv
+from galn_amd import synth
 from test_zz_no_alloc import _in_order, _noalloc
 
 pytestmark = pytest.mark.gpu
@@ -57,3 +58,31 @@ def test_untraced_search_on_an_index_of_many_epochs(name, key, epoch, golden_dir
         off, rec = _in_order(got, r["qlen"].size)
         np.testing.assert_array_equal(got.pops, exp[key + "_pops"])
         assert fx.md5_bytes(nv.sai_bytes(o, got.n_aln, off, rec)) == w["meta"]["runs"][key]["sai_md5"]
+
+
+@pytest.mark.parametrize("length", [40, 64, 100])
+def test_many_unseeded_reads_with_and_without_epochs(length, monkeypatch):
+    """65,536 unseeded reads and more get fewer waves, above 2^32 symbols by their mean length: the same results."""
+    print(f"case many unseeded reads of {length}", flush=True)
+    rng = np.random.default_rng(length)
+    ref = np.frombuffer(b"ACGT", np.uint8)[rng.integers(0, 4, 400_000)]
+    m, words, _, _ = nv.build_bwt(ix.encode_forward(ref), 0)
+    n = 70_000
+    lens = np.full(n, length, np.int32)
+    lens[::7] -= 1
+    reads = ref[rng.integers(0, ref.size - length, n)[:, None] + np.arange(length)].copy()
+    reads[np.arange(n), rng.integers(0, length - 1, n)] = ord("C")
+    q, qoff = synth.encode_queries(reads, lens)
+    batch = np.zeros(n, np.int32)
+    bopts, nst, md = nv.prepare_batches(nv.gap_opt_from_args(["-l", "1024", "-n", "2", "-o", "1"]), lens, batch)
+    got = []
+    for epoch in ("", "5"):
+        monkeypatch.setenv("GALN_HIP_TEST_EPOCH", epoch)
+        with nv.Index(words, m, 0) as idx:
+            rs = nv.ReadSet(idx, q, qoff, lens, md, batch, bopts, nst)
+            rs.search(nv.FORM_BATCHED)
+            got.append(rs.results(want_bytes=True))
+            rs.close()
+    a, b = got
+    for x, y in ((a.n_aln, b.n_aln), (a.pops, b.pops), (a.occ_bytes, b.occ_bytes), (a.rec, b.rec)):
+        np.testing.assert_array_equal(x, y)
