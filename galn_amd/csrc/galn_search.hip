@@ -2884,6 +2884,43 @@ struct Tier {
 
 }  // namespace
 
+// What a search reads back at its end, in pinned memory.
+constexpr int galn_max_launch = 256;
+struct SearchBack {
+    unsigned long long algo[galn_max_launch];
+    int32_t failed;
+    uint32_t used;
+};
+
+// A read set has one of its own; up to eight (2 KB each) wait here for the next read sets of the process, on any
+// device, since pinning and unpinning one takes most of what an upload of few reads costs.
+struct BackPool {
+    std::mutex mu;
+    SearchBack *kept[8] = {};
+    int n = 0;
+    SearchBack *take()
+    {
+        {
+            std::lock_guard<std::mutex> g(mu);
+            if (n > 0) return kept[--n];
+        }
+        SearchBack *b = nullptr;
+        return hipHostMalloc((void **)&b, sizeof *b, hipHostMallocPortable) == hipSuccess ? b : nullptr;
+    }
+    void give(SearchBack *b)
+    {
+        {
+            std::lock_guard<std::mutex> g(mu);
+            if (n < 8) {
+                kept[n++] = b;
+                return;
+            }
+        }
+        (void)hipHostFree(b);
+    }
+};
+static BackPool g_backs;
+
 // Where a search runs: a stream and a stack pool (grown on demand). The read sets of an index
 // share its context; a read set of a server slot has one of its own, so that slots' launches run
 // at the same time.
@@ -3009,13 +3046,9 @@ struct galn_hip_readset {
     GraphKey gkey{};
     std::vector<Launch> glaunches;
     std::vector<hipEvent_t> lev;           // 2 per launch, reused across searches
+    SearchBack *back = nullptr;
     unsigned long long *d_algo = nullptr;  // per-launch algorithmic byte counters
-    static constexpr int MAX_LAUNCH = 256;
-    struct Back {                          // pinned: what a search reads back at its end
-        unsigned long long algo[MAX_LAUNCH];
-        int32_t failed;
-        uint32_t used;
-    } *back = nullptr;
+    static constexpr int MAX_LAUNCH = galn_max_launch;
     struct {
         const void *kernel;
         size_t lds;
@@ -4008,7 +4041,7 @@ int readset_search(galn_hip_readset *rs, int form, uint32_t flags, const galn_hi
     }
     if (r) return r;
     // what the host needs of the search in one wait: the failures, the granules used, the launches' index bytes
-    galn_hip_readset::Back *const back = rs->back;
+    SearchBack *const back = rs->back;
     auto read_back = [&]() -> int {
         back->used = 0;
         HIP_OK(hipMemcpyAsync(&back->failed, rs->d_ctr, 4, hipMemcpyDeviceToHost, fst));
@@ -4332,7 +4365,7 @@ int galn_hip_readset_free(galn_hip_readset *rs)
                     rs->d_stats, rs->d_incl, rs->d_roff, rs->d_stage, rs->d_scan_tmp, rs->d_hand};
     for (void *p : ptrs)
         if (p) (void)hipFree(p);
-    if (rs->back) (void)hipHostFree(rs->back);
+    if (rs->back) g_backs.give(rs->back);
     for (auto &e : rs->ev)
         if (e) (void)hipEventDestroy(e);
     for (auto &e : rs->lev) (void)hipEventDestroy(e);
@@ -4362,8 +4395,7 @@ int galn_hip_readset_upload(galn_hip_index *idx, const galn_hip_reads *reads, ga
     idx->n_readsets.fetch_add(1);
     auto M = [&](void **p, size_t b) __attribute__((always_inline)) -> bool { return dev_malloc(p, b) == hipSuccess; };
     bool ok = M((void **)&rs->d_top, 8) && M((void **)&rs->d_ctr, 16 * sizeof(int32_t)) && M((void **)&rs->d_stats, 16 * 8) &&
-              M((void **)&rs->d_algo, sizeof(unsigned long long) * galn_hip_readset::MAX_LAUNCH) &&
-              hipHostMalloc((void **)&rs->back, sizeof *rs->back) == hipSuccess;
+              M((void **)&rs->d_algo, sizeof(unsigned long long) * galn_hip_readset::MAX_LAUNCH) && (rs->back = g_backs.take());
     if (!ok) {
         galn_hip_readset_free(rs);
         return fail(GALN_HIP_E_NOMEM, "readset_upload: device allocation failed");
