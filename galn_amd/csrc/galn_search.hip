@@ -1283,8 +1283,10 @@ __global__ void __launch_bounds__(256) k_sa_walk(const uint32_t *__restrict__ bw
 // granule each round gave a round only the last piece, 91 heads of up to 256 on average, and a read's
 // memory grew with its pushes, not with its stack.)
 //
-// What bounds it: vector issue, then the lookups' latency on a round's longest chain. A wave pays a full
-// iteration while one lane has a lookup left, and the chains of a heavy read are 2.3 steps long on average,
+// What bounds it: with few reads, the rounds of the longest ones, one after the other; with the chip full, memory
+// past L2, 3.2 TB/s of the 4.9 that a copy reaches (10M ancient DNA reads, 1.22 s: 3.9 TB for 1.66 TB of index
+// blocks, the vector units 28% busy; the one before, a chain a lane and round, was 70% busy and took 1.26 s). What
+// took it from vector issue to there: a wave pays a full iteration while one lane has a lookup left, and the chains of a heavy read are 2.3 steps long on average,
 // 5.5 the longest of 64: with one chain per lane and round 37% of the lane slots did work. Taking the next
 // chain when one ends, pruning dead heads before the loop, tails as iterations of the same loop (a nested
 // one held the wave for the longest tail of every step), 32-bit intervals and packed fields kept in
