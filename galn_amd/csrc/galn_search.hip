@@ -3269,10 +3269,15 @@ constexpr uint32_t PARK_POPS = 2048;
 // only shortens the tail: 16 reads of 100 bp 0.54 ms after 512 pops, 0.64 after 2048, 0.59 after 256.
 constexpr uint32_t PARK_POPS_FEW = 512;
 constexpr int FIRST_GRAN = 8;  // granules a workgroup of it starts with
-// Granules of the stack pool for each wave: 34 GB for a full grid. Unseeded reads on a repeat-rich genome take them:
-// 2M reads on 3.1 Gbp use 1.84M granules, and with 256 a wave the first search of an index ran dry and took 14.4 s,
-// each granule sought in 64 shards, where the second one took 3.5 (1M reads on 700 Mbp: 1.82 s and 1.45).
-constexpr int POOL_PER_WAVE = 512;
+// Granules of the stack pool: POOL_FIRST for each wave's first read and POOL_READ for each read more, up to POOL_MOST
+// (34 GB), or POOL_SEEDED where seeds keep the stacks small. It is the longest searches that take them, and more
+// reads hold more of those: unseeded ones on a 3.1 Gbp human-like genome use 48k granules (4000 reads), 123k (20,000),
+// 340k (60,000), 620k (200,000), 1.15M (2M; 1.84M with 16 waves a CU, where a first search with 1.05M ran dry, each
+// granule sought in 64 shards, and took 14.4 s against 3.5); seeded ones 16k (2000) to 247k (1M repeat-rich ones of
+// 250 bp). Not POOL_MOST for all: handing out and taking back 17 to 34 GB costs up to 2 s in some phases of the
+// driver. 24 times an index opened, one search, closed, 100 bp, default options: of 2000 reads 13.0 s with 512 granules
+// a wave and 0.06 so, of 6000 23.1 and 0.16, of 100,000 25.1 and 9.3.
+constexpr uint64_t POOL_FIRST = 32, POOL_READ = 4, POOL_SEEDED = 1 << 19, POOL_MOST = 1 << 21;
 constexpr int HEAVY_REC = 256;  // record slots of its waves in a search's first launch
 constexpr int HEAVY_REC_MAX = 1 << 26;  // and in any (1.6 GB a wave; a slot's offsets are 32-bit)
 
@@ -3443,14 +3448,28 @@ size_t heavy_scratch(galn_hip_readset *rs, int waves, int deep, int rec_cap, uin
     return one + (size_t)std::min(waves, deep) * make_hlayout(0, 0, DEEP_NW, trace, wide, 0).slot_bytes;
 }
 
+// Granules of the pool for n reads on `waves` waves, rounded up to a power of two; `most` (one itself) at most.
+uint64_t pool_granules(int waves, int n, uint64_t most)
+{
+    const uint64_t used = std::max(1, std::min(waves, n)), want = used * (POOL_FIRST - POOL_READ) + (uint64_t)std::max(n, 1) * POOL_READ;
+    uint64_t p2 = 1024;
+    while (p2 < std::min(want, most)) p2 <<= 1;
+    return p2;
+}
+
+// Seeds that keep every read's stack small: no longer than 32 bases and with 3 differences at most (those measured).
+bool pool_seeded(const galn_hip_readset *rs)
+{
+    for (const auto &o : rs->h_bopts)
+        if (o.seed_len > 32 || o.max_seed_diff > 3) return false;
+    return true;
+}
+
 // The allocations of a wave-engine launch of `waves` waves.
 int prepare_heavy(galn_hip_readset *rs, int waves, int rec_cap, uint32_t flags)
 {
     SearchCtx *cx = rs->ctx;
-    // granules for the waves that can get reads, rounded up to a power of two
-    uint64_t want = (uint64_t)std::max(1, std::min(waves, rs->n)) * POOL_PER_WAVE, p2 = 1024;
-    while (p2 < want) p2 <<= 1;
-    int r = ensure_pool(cx, p2);
+    int r = ensure_pool(cx, pool_granules(waves, rs->n, pool_seeded(rs) ? POOL_SEEDED : POOL_MOST));
     if (r) return r;
     if ((r = grow_dev((void **)&rs->d_park, rs->park_bytes, (size_t)waves * 4, cx->stream))) return r;
     return grow_dev((void **)&rs->d_hscratch, rs->hscratch_bytes, heavy_scratch(rs, waves, heavy_grid(rs, flags, true), rec_cap, flags), cx->stream);
@@ -3539,9 +3558,7 @@ int reserve_search(galn_hip_readset *rs, int n, int max_len, uint32_t flags)
     // the stack pool and the wave engine's per-wave scratch, as prepare_heavy sizes them for the reads and
     // options that get the most waves (this launch's may be fewer)
     const int waves = std::max(1, std::min(heavy_grid_most(rs, flags, false), n));
-    uint64_t p2 = 1024;
-    while (p2 < (uint64_t)waves * POOL_PER_WAVE) p2 <<= 1;
-    if (!soft(ensure_pool(cx, p2))) {
+    if (!soft(ensure_pool(cx, pool_granules(waves, n, POOL_MOST)))) {
         soft(grow_dev((void **)&rs->d_park, rs->park_bytes, (size_t)waves * 4, s));
         soft(grow_dev((void **)&rs->d_hscratch, rs->hscratch_bytes, heavy_scratch(rs, waves, heavy_grid_most(rs, flags, true), HEAVY_REC, flags), s));
     }
